@@ -62,6 +62,7 @@ extern "C" {
 #define SSSP_MODE_CHECK 3  /* trace only: the final fixpoint check (run dense) */
 #define SSSP_MODE_DENSE 4  /* trace only: an all-edge round run dense (see dense_all_frac) */
 #define SSSP_MODE_TAIL  5  /* trace only: a push round run as a tail round (see tail_edges) */
+#define SSSP_MODE_LIGHT 6  /* trace only: a dense round over the graph's light edges alone */
 
 /* ---- graph creation flags ------------------------------------------------ */
 #define SSSP_INPUT_DEVICE 1u   /* src/dst/w are device pointers on `device` */

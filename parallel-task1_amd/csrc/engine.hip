@@ -870,6 +870,7 @@ __global__ void k_init_solve(Ctrl *c, uint32_t *dist, int32_t *stamp, int32_t *q
     zero_slot(&c->slot[0], 0u);
     zero_slot(&c->slot[1], 0xFFFFFFFFu);
     for (int i = 0; i < 64; i++) c->changed[i] = 0;
+    c->ph_low[0] = 0;
     for (int i = 0; i < 8; i++) c->cert[i] = 0;
     c->n_reached = 0;
     c->err = 0;
@@ -928,6 +929,7 @@ __device__ __forceinline__ void round_sample(Ctrl *c, int32_t r, int pile,
     RoundSlot *nxt = &c->slot[(r + 1) & 1];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         zero_slot(nxt, 0xFFFFFFFFu);
+        c->ph_low[0] = 0;  // of a run of light passes this round may begin with
         cur->sample_n = n_sample;
     }
     const uint32_t minF = pile >= 0 ? min(cur->minw, c->pile_min[pile]) : cur->minw;
@@ -1410,19 +1412,21 @@ constexpr int kBlkPer = (1 << kBlkBits) / kBlkThreads;  // block vertices per th
 static_assert(kBlkPer <= 16, "a thread's appends of one tile fit a 16-bit mask");
 
 // One tile of the destination-blocked edge list, shared by the dense round
-// and the plain blocked pass: loads the tile's block of 2^kBlkBits distances
-// into LDS, then relaxes the tile's edges into it -- d[src] gathered from
-// global memory, the minimum taken with LDS atomics. The callers compare the
-// LDS minima with the block read again from global memory (64 KB per tile,
-// 2 % of a round's bytes at R-MAT scale 25): keeping the loaded values in
-// registers instead took 16 VGPRs per lane, which left room for one
-// 1024-thread workgroup per CU; with two per CU (8 waves per SIMD, 64 VGPRs
-// at most) a dense round at R-MAT scale 25 takes 1.04-1.24 ms instead of
-// 1.29-1.35 and a plain blocked pass 0.98-1.09 instead of 1.10-1.19. A wave takes one chunk of 256
+// and the plain blocked pass: relaxes the tile's edges into a block of
+// 2^kBlkBits minima in LDS that starts at INF -- d[src] gathered from global
+// memory, the minimum taken with LDS atomics. The callers compare the
+// minima with the distances in global memory, read for the touched vertices
+// alone (nothing needs the block's distances earlier: loading them first cost
+// a light pass, whose tiles hold few edges, 0.171 against 0.163 ms at R-MAT
+// scale 25, and 16 VGPRs at its start). Two 1024-thread workgroups per CU (8
+// waves per SIMD, 64 VGPRs at most): a dense round at R-MAT scale 25 took
+// 1.04-1.24 ms instead of 1.29-1.35 with one. A wave takes one chunk of 256
 // edge slots per step, 4 per lane: the sources are the chunk's first source
 // plus a wave prefix sum of the packed deltas (or, for a chunk with a large
-// gap, read whole). Returns the number of relaxed edges with a reached source
-// (counted only when COUNT).
+// gap, read whole). Bound by the HBM stream and the d[src] lines: 1.05 ms for
+// 537 M edges (6.7 GB, 6.4 TB/s); on graphs without hubs by the gathers.
+// Returns the number of relaxed edges with a reached source (counted only when
+// COUNT).
 struct BlkList {
     const uint32_t *pk;     // packed edges: source delta << kBlkBits | destination offset
     const int32_t *cbase;   // per chunk: first source, or -(1 + index) of whole sources
@@ -1434,28 +1438,15 @@ BlkList blk_list(const sssp_graph *g) { return BlkList{g->b_pk, g->b_cbase, g->b
 
 template <class WT, bool COUNT>
 __device__ __forceinline__ int64_t blk_relax_tile(const BlkTile &t, const BlkList L,
-                                                  const uint32_t *dist, int64_t base, int nb,
-                                                  uint32_t *s_d)
+                                                  const uint32_t *dist, uint32_t *s_d)
 {
     typedef int32_t v4i __attribute__((ext_vector_type(4)));
     typedef uint32_t v4u __attribute__((ext_vector_type(4)));
     constexpr uint32_t INF = WT::INF;
     constexpr uint32_t kOffMask = (1u << kBlkBits) - 1;
     static_assert(kBlkChunk == 4 * 64, "a chunk is 4 slots per lane of one wave");
-    // the block's distances: all rows' loads in flight before the first LDS
-    // store (a load per row under its bounds test made the compiler wait for
-    // each row in turn: 16 memory round trips per tile)
-    uint32_t row[kBlkPer];
 #pragma unroll
-    for (int k = 0; k < kBlkPer; k++) {
-        const int i = k * kBlkThreads + threadIdx.x;
-        row[k] = dist[base + min(i, nb - 1)];  // nb >= 1: an in-bounds read
-    }
-#pragma unroll
-    for (int k = 0; k < kBlkPer; k++) {
-        const int i = k * kBlkThreads + threadIdx.x;
-        s_d[i] = i < nb ? row[k] : INF;
-    }
+    for (int k = 0; k < kBlkPer; k++) s_d[k * kBlkThreads + threadIdx.x] = INF;
     __syncthreads();
     const v4u *p4 = reinterpret_cast<const v4u *>(L.pk);
     const v4u *w4 = reinterpret_cast<const v4u *>(L.w);
@@ -1470,18 +1461,23 @@ __device__ __forceinline__ int64_t blk_relax_tile(const BlkTile &t, const BlkLis
         atomicMin(&s_d[loc], fin ? WT::add(du, ww) : INF);
     };
     // tiles hold whole chunks and the wave's 64 lanes cover one chunk per
-    // step, so the loop bound and the chunk index are wave-uniform. The next
-    // step's stream loads are issued before this step's gathers.
-    const int64_t gend = t.e1 >> 2;
-    int64_t g = (t.e0 >> 2) + threadIdx.x;
+    // step, so the loop bound and the chunk index are wave-uniform (kept in
+    // scalar registers); chunks nc0 and up are those of the tile's second
+    // run. The next step's stream loads are issued before this step's gathers.
+    const int nc0 = (int)((t.e1 - t.e0) / kBlkChunk);
+    const int nc = nc0 + (int)((t.f1 - t.f0) / kBlkChunk);
+    const int64_t ce = t.e0 / kBlkChunk, cf = t.f0 / kBlkChunk - nc0;
+    int c = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int32_t cb = 0;
     v4u pv = {0u, 0u, 0u, 0u}, wv = {0u, 0u, 0u, 0u};
-    if (g < gend) {
-        cb = L.cbase[g >> 6];
-        pv = __builtin_nontemporal_load(&p4[g]);
-        wv = __builtin_nontemporal_load(&w4[g]);
-    }
-    for (; g < gend; g += kBlkThreads) {
+    auto load = [&](int i, int32_t &b, v4u &p, v4u &ww) {
+        const int64_t k = (i < nc0 ? ce : cf) + i;  // chunk of the list
+        b = L.cbase[k];
+        p = __builtin_nontemporal_load(&p4[k * (kBlkChunk / 4) + lane]);
+        ww = __builtin_nontemporal_load(&w4[k * (kBlkChunk / 4) + lane]);
+    };
+    if (c < nc) load(c, cb, pv, wv);
+    for (; c < nc; c += kBlkThreads / 64) {
         int32_t s0, s1, s2, s3;
         if (cb >= 0) {
             const int32_t a0 = (int32_t)(pv.x >> kBlkBits);
@@ -1510,14 +1506,9 @@ __device__ __forceinline__ int64_t blk_relax_tile(const BlkTile &t, const BlkLis
         // the src-sorted runs, hit the same line); a reuse test between them
         // would serialise them behind one another's latency
         const uint32_t u0 = dist[s0], u1 = dist[s1], u2 = dist[s2], u3 = dist[s3];
-        const int64_t gn = g + kBlkThreads;
         int32_t cbn = 0;
         v4u pvn = {0u, 0u, 0u, 0u}, wvn = {0u, 0u, 0u, 0u};
-        if (gn < gend) {
-            cbn = L.cbase[gn >> 6];
-            pvn = __builtin_nontemporal_load(&p4[gn]);
-            wvn = __builtin_nontemporal_load(&w4[gn]);
-        }
+        if (c + kBlkThreads / 64 < nc) load(c + kBlkThreads / 64, cbn, pvn, wvn);
         relax(u0, pv.x & kOffMask, wv.x);
         relax(u1, pv.y & kOffMask, wv.y);
         relax(u2, pv.z & kOffMask, wv.z);
@@ -1595,26 +1586,31 @@ __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))
     RoundAcc acc;
     const BlkTile t = tiles[blockIdx.x];
     const int64_t base = (int64_t)t.blk << kBlkBits;
-    const int nb = (int)min((int64_t)(1 << kBlkBits), V - base);
-    acc.relaxed = blk_relax_tile<WT, true>(t, L, dist, base, nb, s_d);
-    // write-back: the distance loads of the thread's 16 rows in flight together
+    acc.relaxed = blk_relax_tile<WT, true>(t, L, dist, s_d);
+    // write-back of the vertices whose LDS minimum is below their distance,
+    // eight rows' distance loads in flight together (vertices past the end,
+    // and those no reached source led to, are INF)
     uint32_t lowm = 0;  // bit k: this lane lowered its vertex of row k
 #pragma unroll
-    for (int k = 0; k < kBlkPer; k++) {
-        const int i = k * kBlkThreads + threadIdx.x;
-        if (i < nb) {
-            // below the value in global memory: this tile lowers v (for a
-            // block of one tile that value is the one loaded; for a split
-            // block another tile may lower it further before the returning
-            // atomicMin, which then reports no change)
-            const int32_t v = (int32_t)(base + i);
+    for (int k0 = 0; k0 < kBlkPer; k0 += 8) {
+        uint32_t cur[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (k0 + j) * kBlkThreads + threadIdx.x;
+            cur[j] = s_d[i] != WT::INF ? dist[base + i] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (k0 + j) * kBlkThreads + threadIdx.x;
             const uint32_t nv = s_d[i];
-            if (nv < dist[v]) {
+            if (nv < cur[j]) {
+                // in a split block another tile may lower the vertex further
+                // before the returning atomicMin, which then reports no change
                 bool low = true;
-                if (t.split) low = atomicMin(&dist[v], nv) > nv;
-                else dist[v] = nv;  // only this workgroup writes the block
+                if (t.split) low = atomicMin(&dist[base + i], nv) > nv;
+                else dist[base + i] = nv;  // only this workgroup writes the block
                 if (low) {
-                    lowm |= 1u << k;
+                    lowm |= 1u << (k0 + j);
                     acc.lowered++;
                     acc.minw = min(acc.minw, nv);
                 }
@@ -1727,38 +1723,118 @@ __global__ __launch_bounds__(kBlock) void k_frontier_from_bits(const BlkTile *__
     }
 }
 
-// Plain Bellman-Ford pass (bellman_ford.cu:62-99) over the destination-blocked
-// edge list: the tile relaxation of the dense round without its frontier
-// (no stamps, no appends, no counters), and the change flag protocol of
-// k_el_pass -- pass p zeroes the flag of pass p+1, returns at once when pass
-// p-1 changed nothing, and sets its own flag when it lowers a distance -- so
-// passes are queued without a host round trip. A tile sets the flag only
-// when its minimum for a vertex is below that vertex's distance in global
-// memory, which its write then lowers: the flag never reports a change that
-// did not happen, and a pass that leaves it clear relaxed every edge against
-// the final distances: the fixpoint.
+// Passes over the destination-blocked edge list without a frontier (no
+// stamps, no appends): the tile relaxation of the dense round, over every edge
+// (full) or over the light edges alone. Passes are queued ahead of the host;
+// each finds out on the device what it runs, from what the pass before it
+// ran and how many vertices that pass lowered, and one that has nothing to
+// do returns at once:
+//   kRunFull   full passes until one lowers nothing: the plain Bellman-Ford
+//              (bellman_ford.cu:62-99);
+//   kRunLight  light passes until they lower few vertices: the prelude of a
+//              dense round, which then relaxes every edge;
+//   kRunMixed  light passes until they lower few vertices, a full pass, light
+//              passes again if that lowered anything, and so on until a full
+//              pass lowers nothing -- the same fixpoint test as kRunFull.
+// Why light passes: a shortest path takes mostly light edges, so relaxing the
+// lightest sixteenth of the edges to near convergence costs a fraction of the
+// full passes it replaces, and the full passes after it find the distances
+// nearly final. R-MAT 25 x 16: 13 light passes of 0.15 ms and one dense round
+// instead of 9 dense rounds of 1.1 ms (a learned solve 13.4 -> 5.6 ms); R-MAT
+// 22 x 32 4.75 -> 2.1; uniform 6 M x 16, u32 6.85 -> 4.8; power-law 1.2 M x 9 in the
+// pass loop 2.33 -> 1.2.
+// A tile counts a vertex as lowered only when its minimum is below the
+// vertex's distance in global memory, which its write then lowers: the count
+// never reports a change that did not happen, and a full pass that leaves
+// it zero relaxed every edge against the final distances: the fixpoint.
+enum { kRunFull = 0, kRunLight = 1, kRunMixed = 2 };
+enum { kPassLight = 1, kPassFull = 2, kPassIdle = 3 };
+
+struct PassArgs {
+    const BlkTile *full, *light;
+    int32_t n_full, n_light;
+    int32_t run;          // kRunFull / kRunLight / kRunMixed
+    int32_t pass;         // index in the run
+    int32_t light_stop;   // light passes go on while they lower this many vertices, or
+                          // more than the light pass before
+    int32_t tag;          // of the run, in the progress word
+    Ctrl *ctrl;
+    unsigned long long *pos;  // device address of the host mirror's progress word
+};
+
+// Progress word: tag (6 bits), passes begun (28), full passes among them
+// (28), kind of the last one (2). An idle pass reports the count of the first
+// idle one.
+__host__ __device__ inline unsigned long long pass_word(int32_t tag, int32_t begun, int32_t full,
+                                                        int32_t kind)
+{
+    return ((unsigned long long)(tag & 63) << 58) | ((unsigned long long)begun << 30) |
+           ((unsigned long long)full << 2) | (unsigned)kind;
+}
+
+// What pass a.pass runs; every workgroup reads the same values (written by
+// the passes before).
+__device__ __forceinline__ int pass_kind(const PassArgs &a)
+{
+    const Ctrl *c = a.ctrl;
+    if (a.pass == 0) return a.run == kRunFull ? kPassFull : kPassLight;
+    const int i1 = (a.pass - 1) & 63, i2 = (a.pass - 2) & 63;
+    const int prev = c->ph_kind[i1];
+    const int32_t low = c->ph_low[i1];
+    if (prev == kPassIdle) return kPassIdle;
+    if (prev == kPassFull) {
+        if (low == 0) return kPassIdle;
+        return a.run == kRunMixed && a.pass < kLightMaxPasses ? kPassLight : kPassFull;
+    }
+    const int32_t before = a.pass > 1 && c->ph_kind[i2] == kPassLight ? c->ph_low[i2] : 0;
+    if ((low >= a.light_stop || low > before) && low > 0 && a.pass < kLightMaxPasses)
+        return kPassLight;
+    return a.run == kRunLight ? kPassIdle : kPassFull;
+}
+
 template <class WT>
 __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blk_plain(
-    const BlkTile *__restrict__ tiles, const BlkList L, uint32_t *dist, int64_t V,
-    int32_t *changed, int32_t pass)
+    const PassArgs a, const BlkList L, uint32_t *dist)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) changed[(pass + 1) & 63] = 0;
-    if (pass > 0 && __hip_atomic_load(&changed[(pass - 1) & 63], __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT) == 0)
-        return;
     __shared__ uint32_t s_d[1 << kBlkBits];
-    const BlkTile t = tiles[blockIdx.x];
+    __shared__ int s_low;
+    const int kind = pass_kind(a);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        Ctrl *c = a.ctrl;
+        const int32_t full = (a.pass == 0 ? 0 : c->ph_full) + (kind == kPassFull ? 1 : 0);
+        int32_t begun = a.pass + 1;
+        if (kind == kPassIdle) {
+            if (c->ph_kind[(a.pass - 1) & 63] != kPassIdle) c->ph_done = begun;
+            else begun = c->ph_done;
+        }
+        c->ph_kind[a.pass & 63] = kind;
+        c->ph_low[(a.pass + 1) & 63] = 0;
+        c->ph_full = full;
+        __hip_atomic_store(a.pos, pass_word(a.tag, begun, full, kind), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (kind == kPassIdle) return;
+    const bool light = kind == kPassLight;
+    if ((int)blockIdx.x >= (light ? a.n_light : a.n_full)) return;
+    const BlkTile t = (light ? a.light : a.full)[blockIdx.x];
+    if (threadIdx.x == 0) s_low = 0;  // before the relaxation's barriers
     const int64_t base = (int64_t)t.blk << kBlkBits;
-    const int nb = (int)min((int64_t)(1 << kBlkBits), V - base);
-    blk_relax_tile<WT, false>(t, L, dist, base, nb, s_d);
-    bool low = false;
+    blk_relax_tile<WT, false>(t, L, dist, s_d);
+    int low = 0;
 #pragma unroll
-    for (int k = 0; k < kBlkPer; k++) {
-        const int i = k * kBlkThreads + threadIdx.x;
-        if (i < nb) {
+    for (int k0 = 0; k0 < kBlkPer; k0 += 8) {
+        uint32_t cur[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (k0 + j) * kBlkThreads + threadIdx.x;
+            cur[j] = s_d[i] != WT::INF ? dist[base + i] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (k0 + j) * kBlkThreads + threadIdx.x;
             const uint32_t nv = s_d[i];
-            if (nv < dist[base + i]) {
-                low = true;
+            if (nv < cur[j]) {
+                low++;
                 if (t.split)  // the result of the min is not needed
                     __hip_atomic_fetch_min(&dist[base + i], nv, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
@@ -1767,7 +1843,12 @@ __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))
             }
         }
     }
-    if (__ballot(low) != 0 && __lane_id() == 0) changed[pass & 63] = 1;
+    if (__ballot(low != 0) != 0) {
+        low = wave_sum32(low);
+        if (__lane_id() == 0) atomicAdd(&s_low, low);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && s_low != 0) atomicAdd(&a.ctrl->ph_low[a.pass & 63], s_low);
 }
 
 // ---------------------------------------------------------------------------
@@ -1985,8 +2066,11 @@ void frontier_to_queue(sssp_graph *g, int32_t r)
 // round reads; the host mirror of the control block holds its counters.
 // Returns true when a push round wrote the next pile (the caller swaps).
 template <class WT>
+void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st);
+
+template <class WT>
 bool run_round(sssp_graph *g, int mode, int kidx, int32_t r, int32_t tick0, const RoundSlot &cur,
-               bool verify)
+               bool verify, bool light, sssp_stats *st)
 {
     AdvArgs a = base_args<WT>(g, r, tick0);
     hipStream_t s = g->stream;
@@ -2019,6 +2103,13 @@ bool run_round(sssp_graph *g, int mode, int kidx, int32_t r, int32_t tick0, cons
             // against a snapshot
             g->last_round_dense = true;
             if (g->dense_kernel == 0 && g->n_btile > 0) {
+                // the light edges first, to near convergence: a round that
+                // relaxes every edge then finds the distances nearly final
+                // (the vertices light passes lower need no frontier: this
+                // round relaxes every reached source)
+                if (light && !verify && WT::kWeighted && g->n_ltile > 0)
+                    run_passes<WT>(g, kRunLight, INT64_MAX, st);
+                if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
                 k_blk_pass<WT><<<(unsigned)g->n_btile, kBlkThreads, 0, s>>>(
                     g->b_tile, blk_list(g), g->dist, g->V, g->stamp, a.tick_cur,
                     g->row_ptr, g->b_app, a.slot);
@@ -2131,16 +2222,132 @@ void read_slot(sssp_graph *g, int32_t r)
     SSSP_HIP(hipStreamSynchronize(s));
 }
 
+// Waits until the decision kernel has written round `seq` into the host
+// mirror: a spin on the mirror's sequence number (coherent host memory),
+// which sees the write about a microsecond after it lands -- a stream
+// synchronize wakes the host up later, and the GPU idles until the round's
+// kernels are launched. After kSpinPolls polls it falls back to the stream
+// synchronize, which also reports a failed kernel.
+constexpr int64_t kSpinPolls = (int64_t)1 << 22;
+
+void wait_decision(sssp_graph *g, int32_t seq)
+{
+    volatile int32_t *p = &g->ctrl_host->dec_seq;
+    for (int64_t i = 0; g->decide_spin && i < kSpinPolls; i++) {
+        if (*p == seq) {
+            std::atomic_thread_fence(std::memory_order_acquire);
+            return;
+        }
+        if ((i & 1023) == 1023 && hipStreamQuery(g->stream) != hipErrorNotReady) break;
+    }
+    SSSP_HIP(hipStreamSynchronize(g->stream));
+}
+
+// Passes queued ahead of the one the host has seen begin: enough to cover the
+// host's poll and launch, few enough that the idle ones left in the queue
+// when a run ends (3-6 us each) cost little.
+constexpr int kPassAhead = 3;
+
+// Runs a run of blocked passes (k_blk_plain) to its end on the device, the
+// host queueing passes as it sees them begin in the mirror's progress word.
+// With trace_events every pass is launched alone between events. Adds the
+// passes to the stats and the trace; full_limit: full passes at most (then
+// SSSP_ERR_NOT_CONVERGED).
 template <class WT>
-void solve_plain(sssp_graph *g, sssp_stats *st)
+void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
+{
+    hipStream_t s = g->stream;
+    PassArgs a{};
+    a.full = g->b_tile;
+    a.light = g->b_ltile;
+    a.n_full = g->n_btile;
+    a.n_light = g->n_ltile;
+    a.run = run;
+    a.light_stop = (int32_t)(kLightStopFrac * g->n_nzo);
+    a.tag = ++g->ph_tag;
+    a.ctrl = g->ctrl;
+    a.pos = &g->ctrl_host_dev->ph_pos;
+    const unsigned grid = (unsigned)(run == kRunFull    ? g->n_btile
+                                     : run == kRunLight ? g->n_ltile
+                                                        : std::max(g->n_btile, g->n_ltile));
+    // the mirror still holds the last run's word (another tag) or none
+    volatile unsigned long long *pos = &g->ctrl_host->ph_pos;
+    const unsigned long long mine = pass_word(a.tag, 0, 0, 0) >> 58;
+    const int ahead = g->trace_events ? 1 : kPassAhead;
+    int32_t queued = 0, begun = 0, full = 0;
+    int kind = 0;
+    while (kind != kPassIdle) {
+        while (queued < begun + ahead) {
+            a.pass = queued++;
+            if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
+            k_blk_plain<WT><<<grid, kBlkThreads, 0, s>>>(a, blk_list(g), g->dist);
+            SSSP_LAUNCH_CHECK("k_blk_plain");
+            if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r1, s));
+        }
+        unsigned long long w = 0;
+        bool drained = false;
+        for (int64_t i = 0;; i++) {
+            w = *pos;
+            if (w >> 58 == mine && ((int32_t)(w >> 30 & 0xFFFFFFF) > begun ||
+                                    (int)(w & 3) == kPassIdle))
+                break;
+            if (drained) throw Error{SSSP_ERR_INTERNAL, "blocked passes made no progress"};
+            if ((i & 1023) == 1023 && hipStreamQuery(s) != hipErrorNotReady) {
+                SSSP_HIP(hipStreamSynchronize(s));  // reports a failed kernel
+                drained = true;                      // the word is final: read it once more
+            }
+        }
+        const int32_t was = begun;
+        begun = (int32_t)(w >> 30 & 0xFFFFFFF);
+        full = (int32_t)(w >> 2 & 0xFFFFFFF);
+        kind = (int)(w & 3);
+        if (g->trace_events && kind != kPassIdle && begun > was) {
+            TraceRow tr{};
+            tr.mode = kind == kPassLight ? SSSP_MODE_LIGHT : SSSP_MODE_ALL;
+            tr.frontier = g->V;
+            tr.frontier_edges = kind == kPassLight ? g->light_edges : g->E;
+            SSSP_HIP(hipEventSynchronize(g->ev_r1));
+            SSSP_HIP(hipEventElapsedTime(&tr.ms, g->ev_r0, g->ev_r1));
+            g->trace.push_back(tr);
+        }
+        if (kind != kPassIdle && full > full_limit) {
+            SSSP_HIP(hipStreamSynchronize(s));
+            throw Error{SSSP_ERR_NOT_CONVERGED,
+                        "plain Bellman-Ford did not converge within max_rounds or V passes"};
+        }
+    }
+    const int32_t passes = begun - 1, light = passes - full;
+    if (!g->trace_events && run == kRunLight) {
+        TraceRow tr{};
+        tr.mode = SSSP_MODE_LIGHT;
+        tr.frontier = tr.frontier_edges = -1;
+        for (int32_t i = 0; i < light; i++) g->trace.push_back(tr);
+    }
+    st->iterations += passes;
+    st->n_all += passes;
+    st->edges_relaxed += (int64_t)full * g->E + (int64_t)light * g->light_edges;
+}
+
+// The plain pass loop: full passes until one changes nothing (mixed: with
+// light passes between them, see k_blk_plain).
+template <class WT>
+void solve_plain(sssp_graph *g, bool mixed, sssp_stats *st)
 {
     hipStream_t s = g->stream;
     const int64_t E = g->E;
+    // passes at most: max_rounds and V + 1, in whole groups of four
+    const int64_t limit = std::min<int64_t>(4 * ((int64_t)g->max_rounds / 4 + 1),
+                                            std::max<int64_t>(8, ((int64_t)g->V + 4) / 4 * 4));
+    st->verify_passes = 1;  // the last pass changed nothing: the fixpoint check
+    if (plain_uses_blocked(g)) {
+        run_passes<WT>(g, mixed && WT::kWeighted && g->n_ltile > 0 ? kRunMixed : kRunFull, limit,
+                       st);
+        return;
+    }
     const int64_t ng = E >> 2;
     int64_t nblocks = (int64_t)g->cu_count * 8;
     if (nblocks < 8) nblocks = 8;
     const int64_t per_block = (ng + nblocks - 1) / nblocks;
-    const bool blocked = plain_uses_blocked(g);
     int32_t pass = 0;
     // with trace_events every pass is bracketed by events (one pass per batch)
     const int batch = g->trace_events ? 1 : 4;
@@ -2148,17 +2355,10 @@ void solve_plain(sssp_graph *g, sssp_stats *st)
     while (done_at < 0) {
         for (int i = 0; i < batch; i++) {
             if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
-            if (blocked) {
-                k_blk_plain<WT><<<(unsigned)g->n_btile, kBlkThreads, 0, s>>>(
-                    g->b_tile, blk_list(g), g->dist, g->V, g->ctrl->changed,
-                    pass + i);
-                SSSP_LAUNCH_CHECK("k_blk_plain");
-            } else {
-                k_el_pass<WT, uint32_t, 4, true><<<(unsigned)nblocks, kBlock, 0, s>>>(
-                    g->x_src, g->x_dst, g->x_w, E, g->dist, g->ctrl->changed, pass + i,
-                    per_block, g->xgoff);
-                SSSP_LAUNCH_CHECK("k_el_pass");
-            }
+            k_el_pass<WT, uint32_t, 4, true><<<(unsigned)nblocks, kBlock, 0, s>>>(
+                g->x_src, g->x_dst, g->x_w, E, g->dist, g->ctrl->changed, pass + i, per_block,
+                g->xgoff);
+            SSSP_LAUNCH_CHECK("k_el_pass");
             if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r1, s));
         }
         SSSP_HIP(hipMemcpyAsync(g->ctrl_host->changed, g->ctrl->changed, sizeof(int32_t) * 64,
@@ -2186,29 +2386,7 @@ void solve_plain(sssp_graph *g, sssp_stats *st)
     }
     st->iterations = done_at + 1;
     st->n_all = done_at + 1;
-    st->verify_passes = 1;  // the last pass changed nothing: the fixpoint check
     st->edges_relaxed = (int64_t)(done_at + 1) * E;
-}
-
-// Waits until the decision kernel has written round `seq` into the host
-// mirror: a spin on the mirror's sequence number (coherent host memory),
-// which sees the write about a microsecond after it lands -- a stream
-// synchronize wakes the host up later, and the GPU idles until the round's
-// kernels are launched. After kSpinPolls polls it falls back to the stream
-// synchronize, which also reports a failed kernel.
-constexpr int64_t kSpinPolls = (int64_t)1 << 22;
-
-void wait_decision(sssp_graph *g, int32_t seq)
-{
-    volatile int32_t *p = &g->ctrl_host->dec_seq;
-    for (int64_t i = 0; g->decide_spin && i < kSpinPolls; i++) {
-        if (*p == seq) {
-            std::atomic_thread_fence(std::memory_order_acquire);
-            return;
-        }
-        if ((i & 1023) == 1023 && hipStreamQuery(g->stream) != hipErrorNotReady) break;
-    }
-    SSSP_HIP(hipStreamSynchronize(g->stream));
 }
 
 // Tail rounds from round r on, tail_group queued per host check, until one
@@ -2401,7 +2579,9 @@ int32_t step_round(sssp_graph *g, int32_t r, int sched, int32_t tick0, sssp_stat
         // (the first tail round always runs: its frontier was checked here)
     }
     if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
-    if (run_round<WT>(g, mode, kidx, r, tick0, cur, verify)) g->pile_cur ^= 1;
+    const bool light =
+        (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) && force_mode < 0;
+    if (run_round<WT>(g, mode, kidx, r, tick0, cur, verify, light, st)) g->pile_cur ^= 1;
     float ms = 0.f;
     if (g->trace_events) {
         SSSP_HIP(hipEventRecord(g->ev_r1, s));
@@ -2442,7 +2622,7 @@ int32_t solve_rounds(sssp_graph *g, int sched, int32_t tick0, sssp_stats *st)
         if (used == 0) break;
         r += used;
     }
-    st->edges_relaxed = relaxed;
+    st->edges_relaxed += relaxed;
     return r;
 }
 
@@ -2491,7 +2671,7 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
     const bool small = (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) &&
                        n_src == 1 && g->E < g->plain_below_edges;
     if (sched == SSSP_SCHED_PLAIN || small) {
-        solve_plain<WT>(g, st);
+        solve_plain<WT>(g, small, st);
         g->tick = tick0 + 1;
     } else {
         if (g->pile_dirty) {

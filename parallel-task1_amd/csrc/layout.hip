@@ -332,14 +332,35 @@ __global__ __launch_bounds__(kBlock) void k_group_gather(const uint32_t *perm, c
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_blk_keys(const int32_t *dst, int64_t E, uint32_t *keys)
+// Run of an edge: its destination block, light before heavy.
+__global__ __launch_bounds__(kBlock) void k_blk_keys(const int32_t *dst, const uint32_t *w,
+                                                     int64_t E, uint32_t thr, uint32_t *keys)
 {
     for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < E;
          e += (int64_t)gridDim.x * kBlock)
-        keys[e] = (uint32_t)dst[e] >> kBlkBits;
+        keys[e] = (((uint32_t)dst[e] >> kBlkBits) << 1) | (w[e] > thr ? 1u : 0u);
 }
 
-// Sorted position j of block b = skeys[j] goes to boff[b] + (j - bptr[b]);
+// out[i] = w[i * E / n]: a fixed-stride sample of the weights
+__global__ __launch_bounds__(kBlock) void k_weight_sample(const uint32_t *w, int64_t E, int32_t n,
+                                                          uint32_t *out)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) out[i] = w[i * E / n];
+}
+
+// largest out-degree
+__global__ __launch_bounds__(kBlock) void k_max_degree(const int64_t *ptr, int64_t V, uint32_t *mx)
+{
+    uint32_t m = 0;
+    for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < V;
+         v += (int64_t)gridDim.x * kBlock)
+        m = max(m, (uint32_t)(ptr[v + 1] - ptr[v]));
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor(m, o));
+    if (__lane_id() == 0 && m) atomicMax(mx, m);
+}
+
+// Sorted position j of run b = skeys[j] goes to boff[b] + (j - bptr[b]);
 // perm[j] is its position in the src-sorted list, whose order is kept.
 __global__ __launch_bounds__(kBlock) void k_blk_gather(const uint32_t *skeys, const uint32_t *perm,
                                                        int64_t E, const int64_t *bptr,
@@ -353,12 +374,12 @@ __global__ __launch_bounds__(kBlock) void k_blk_gather(const uint32_t *skeys, co
         const int64_t o = boff[b] + (j - bptr[b]);
         const uint32_t p = perm[j];
         bs[o] = src[p];
-        bd[o] = (uint16_t)(dst[p] - (int32_t)(b << kBlkBits));
+        bd[o] = (uint16_t)(dst[p] - (int32_t)((b >> 1) << kBlkBits));
         bw[o] = w[p];
     }
 }
 
-// The padding slots of each block (up to kBlkChunk - 1) copy the block's last
+// The padding slots of each run (up to kBlkChunk - 1) copy the run's last
 // edge: relaxing it again changes nothing, and its source delta is 0.
 __global__ __launch_bounds__(kBlock) void k_blk_pad(const int64_t *bptr, const int64_t *boff,
                                                     int32_t nblk, int32_t *bs, uint16_t *bd,
@@ -369,7 +390,7 @@ __global__ __launch_bounds__(kBlock) void k_blk_pad(const int64_t *bptr, const i
         const int32_t b = (int32_t)(i / kBlkChunk);
         const int64_t last = boff[b] + (bptr[b + 1] - bptr[b]) - 1;
         const int64_t o = last + 1 + i % kBlkChunk;
-        if (o < boff[b + 1]) {  // only blocks with edges have slots
+        if (o < boff[b + 1]) {  // only runs with edges have slots
             bs[o] = bs[last];
             bd[o] = bd[last];
             bw[o] = bw[last];
@@ -727,7 +748,7 @@ void build_multi_layout(sssp_graph *g)
         const int64_t nt = (c + kMTileEdges - 1) / kMTileEdges;
         for (int64_t k = 0; k < nt; k++) {
             const int64_t e0 = bp[(size_t)b] + k * kMTileEdges;
-            tiles.push_back(BlkTile{b, nt > 1 ? 1 : 0, e0, std::min(e0 + kMTileEdges, bp[(size_t)b + 1])});
+            tiles.push_back(BlkTile{b, nt > 1 ? 1 : 0, e0, std::min(e0 + kMTileEdges, bp[(size_t)b + 1]), 0, 0});
         }
     }
     BlkTile *td = dmalloc<BlkTile>(std::max<size_t>(tiles.size(), 1));
@@ -775,38 +796,63 @@ void validate_edges(const int32_t *src, const int32_t *dst, const void *w, int w
     if (hb[1]) throw Error{SSSP_ERR_ARG, std::to_string(hb[1]) + " edges have a negative or NaN weight"};
 }
 
-// The tiles of the destination-blocked list: runs of at most `cap` edge slots
-// (a multiple of kBlkChunk) of one block, `split` when a block has several.
-// Without source ranges (R.stride == 0) a tile is a run of its block's slots;
+// The tiles of the destination-blocked list: at most `cap` edge slots (a
+// multiple of kBlkChunk) of one block, `split` when a block has several.
+// Without source ranges (R.stride == 0) a tile is one run of its block's slots;
 // order 0 = smallest tiles first (stable by block), 1 = by block, 2 = largest
-// first, 3 = by descending block. With source ranges each block's run is cut
+// first, 3 = by descending block. With source ranges each run is cut
 // at the (chunk-aligned) slots where its sources reach multiples of the range
 // size, and the tiles are dispatched range by range (by block within one):
 // the workgroups running at one time then gather d[src] from one range of
-// the distance array, which an XCD's L2 holds. bo: padded block offsets,
-// nblk + 1 values.
+// the distance array, which an XCD's L2 holds; a tile then holds its range's
+// light and heavy slots as two runs. bo: padded run offsets (light and heavy
+// run of each block), 2 nblk + 1 values; light: the light runs alone.
 std::vector<BlkTile> make_blk_tiles(const std::vector<int64_t> &bo, int64_t cap, int order,
-                                    const BlkRanges &R)
+                                    const BlkRanges &R, bool light)
 {
     struct T {
         BlkTile t;
         int32_t range;
     };
     std::vector<T> tiles;
-    const int32_t nblk = (int32_t)bo.size() - 1;
+    const int32_t nblk = (int32_t)((bo.size() - 1) / 2);
     const bool ranged = R.stride > 0 && !R.off.empty();
     const int32_t nr = ranged ? (R.n_fine + R.stride - 1) / R.stride : 1;
     for (int32_t b = 0; b < nblk; b++) {
         const size_t first = tiles.size();
         for (int32_t r = 0; r < nr; r++) {
-            int64_t lo = bo[(size_t)b], hi = bo[(size_t)b + 1];
-            if (ranged) {
-                const size_t row = (size_t)b * (size_t)(R.n_fine + 1);
-                lo = R.off[row + (size_t)std::min(r * R.stride, R.n_fine)];
-                hi = R.off[row + (size_t)std::min((r + 1) * R.stride, R.n_fine)];
+            int64_t lo[2], hi[2];  // the slots of the block's two runs
+            for (int h = 0; h < 2; h++) {
+                const size_t run = 2 * (size_t)b + (size_t)h;
+                lo[h] = bo[run];
+                hi[h] = bo[run + 1];
+                if (ranged) {
+                    const size_t row = run * (size_t)(R.n_fine + 1);
+                    lo[h] = R.off[row + (size_t)std::min(r * R.stride, R.n_fine)];
+                    hi[h] = R.off[row + (size_t)std::min((r + 1) * R.stride, R.n_fine)];
+                }
             }
-            for (int64_t e0 = lo; e0 < hi; e0 += cap)
-                tiles.push_back(T{BlkTile{b, 0, e0, std::min(e0 + cap, hi)}, r});
+            if (light) {
+                lo[1] = hi[1] = 0;
+            } else if (hi[0] == lo[1]) {  // one run
+                hi[0] = hi[1];
+                lo[1] = hi[1] = 0;
+            }
+            while (lo[0] < hi[0] || lo[1] < hi[1]) {
+                const int64_t n0 = std::min(cap, hi[0] - lo[0]);
+                const int64_t n1 = std::min(cap - n0, hi[1] - lo[1]);
+                BlkTile t{b, 0, lo[0], lo[0] + n0, 0, 0};
+                if (n0 == 0) {
+                    t.e0 = lo[1];
+                    t.e1 = lo[1] + n1;
+                } else if (n1 > 0) {
+                    t.f0 = lo[1];
+                    t.f1 = lo[1] + n1;
+                }
+                lo[0] += n0;
+                lo[1] += n1;
+                tiles.push_back(T{t, r});
+            }
         }
         if (tiles.size() - first > 1)
             for (size_t i = first; i < tiles.size(); i++) tiles[i].t.split = 1;
@@ -828,6 +874,15 @@ std::vector<BlkTile> make_blk_tiles(const std::vector<int64_t> &bo, int64_t cap,
     return out;
 }
 
+// Slots of a light tile at most: about kLightTiles tiles over the light
+// edges, a power of two (whole chunks), never above the full tiles' cap.
+static int64_t light_cap(const sssp_graph *g, int64_t cap)
+{
+    int64_t c = kLightTileMin;
+    while (c < cap && c * kLightTiles < g->light_edges) c <<= 1;
+    return std::min(c, cap);
+}
+
 void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits)
 {
     if (g->b_off_host.empty()) return;
@@ -838,21 +893,89 @@ void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits)
             throw Error{SSSP_ERR_ARG, "blk_range_bits: source ranges unavailable for this size"};
         R.stride = 1 << (range_bits - R.fine_bits);
     }
-    std::vector<BlkTile> tiles = make_blk_tiles(g->b_off_host, cap, order, R);
-    BlkTile *td = dmalloc<BlkTile>(std::max<size_t>(tiles.size(), 1));
-    SSSP_HIP(hipMemcpyAsync(td, tiles.data(), sizeof(BlkTile) * tiles.size(), hipMemcpyHostToDevice,
-                            g->stream));
+    const std::vector<BlkTile> tiles = make_blk_tiles(g->b_off_host, cap, order, R, false);
+    std::vector<BlkTile> ltiles;
+    if (g->light_edges > 0)
+        ltiles = make_blk_tiles(g->b_off_host, light_cap(g, cap), order, R, true);
+    auto upload = [&](const std::vector<BlkTile> &t) {
+        BlkTile *d = dmalloc<BlkTile>(std::max<size_t>(t.size(), 1));
+        SSSP_HIP(hipMemcpyAsync(d, t.data(), sizeof(BlkTile) * t.size(), hipMemcpyHostToDevice,
+                                g->stream));
+        return d;
+    };
+    struct Own {
+        void *p[3] = {};
+        ~Own()
+        {
+            for (void *x : p) dfree(x);
+        }
+    } own;
+    BlkTile *td = upload(tiles);
+    own.p[0] = td;
+    BlkTile *ltd = upload(ltiles);
+    own.p[1] = ltd;
+    const size_t n_mask = std::max<size_t>(std::max(tiles.size(), ltiles.size()), 1);
+    uint16_t *ad = dmalloc<uint16_t>(n_mask * kBlkThreads);
+    own.p[2] = ad;
     SSSP_HIP(hipStreamSynchronize(g->stream));
-    uint16_t *ad = dmalloc<uint16_t>(std::max<size_t>(tiles.size(), 1) * kBlkThreads);
-    dfree(g->b_tile);
-    dfree(g->b_app);
+    own.p[0] = g->b_tile;
+    own.p[1] = g->b_ltile;
+    own.p[2] = g->b_app;
     g->b_tile = td;
+    g->b_ltile = ltd;
     g->b_app = ad;
     g->frontier_bits = false;
     g->n_btile = (int32_t)tiles.size();
+    g->n_ltile = (int32_t)ltiles.size();
     g->blk_tile_cap = cap;
     g->blk_tile_order = order;
     g->blk_range_bits = range_bits;
+}
+
+// The weight threshold of the light class: the quantile `frac` of a sample
+// of the weights (patterns order like the weights). frac leaves every vertex
+// with out-edges about one light edge on a graph with hubs, six on one without
+// (the light edges alone have to reach most vertices; hubs shorten the paths),
+// between 1/16 and 1/2 of the edges. Measured (ms of a solve, frac 1/16 / 1/8 /
+// 1/4 / 3/8 / 1/2; mean degrees are over vertices with out-edges): R-MAT 25 x 16
+// 5.6 / 6.7 / 8.2 / 9.2 / - (mean 60), 22 x 32 2.1 / 2.05 / 2.9 / 2.9 / -,
+// power-law 4 M x 8 3.2 / 2.5 / 3.0 / 2.9 / 2.8 (mean 8), uniform 6 M x 16
+// 9.1 / 9.5 / 5.1 / 4.8 / 5.1, 16 M x 8 - / - / 14.5 / 12.5 / 11.6. The line
+// between hubs and none is a largest out-degree of 16 times the mean.
+// With many equal weights the class can come out far from that share; below
+// half or above three times the target there are no classes (0xFFFFFFFF: every
+// edge is light and light passes do not run).
+static uint32_t light_threshold(const sssp_graph *g)
+{
+    const int64_t n = std::min<int64_t>(g->E, kLightSample);
+    uint32_t *d = dmalloc<uint32_t>((size_t)n + 1);
+    struct F {
+        void *p;
+        ~F() { dfree(p); }
+    } f{d};
+    k_weight_sample<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, g->stream>>>(
+        g->el_w, g->E, (int32_t)n, d);
+    SSSP_LAUNCH_CHECK("k_weight_sample");
+    SSSP_HIP(hipMemsetAsync(d + n, 0, 4, g->stream));
+    k_max_degree<<<grid_for(g->V), kBlock, 0, g->stream>>>(g->row_ptr, g->V, d + n);
+    SSSP_LAUNCH_CHECK("k_max_degree");
+    std::vector<uint32_t> s((size_t)n + 1);
+    SSSP_HIP(hipMemcpyAsync(s.data(), d, 4 * s.size(), hipMemcpyDeviceToHost, g->stream));
+    SSSP_HIP(hipStreamSynchronize(g->stream));
+    const double mean = (double)g->E / std::max(g->n_nzo, 1);
+    const double per_vertex = (double)s.back() >= 16.0 * mean ? 1.0 : 6.0;
+    const double frac = std::min(0.5, std::max(1.0 / 16, per_vertex / mean));
+    s.pop_back();
+    std::sort(s.begin(), s.end());
+    const double target = frac * (double)n;
+    const uint32_t at = s[(size_t)std::min<int64_t>(n - 1, (int64_t)target)];
+    // the class is w <= thr: `at` itself, or the value before it
+    const int64_t up = std::upper_bound(s.begin(), s.end(), at) - s.begin();
+    const int64_t lo = std::lower_bound(s.begin(), s.end(), at) - s.begin();
+    const bool use_lo = at > 0 && std::abs((double)lo - target) < std::abs((double)up - target);
+    const double got = use_lo ? (double)lo : (double)up;
+    if (got < 0.5 * target || got > 3.0 * target || got > 0.75 * (double)n) return 0xFFFFFFFFu;
+    return use_lo ? at - 1 : at;
 }
 
 void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, const uint32_t *d_w,
@@ -1045,9 +1168,11 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
     // ---- destination-blocked edge list ----
     if (E > 0) {
         const int32_t nblk = (int32_t)(((int64_t)V + (1 << kBlkBits) - 1) >> kBlkBits);
+        const int32_t nrun = 2 * nblk;  // light and heavy run of each block
+        g->light_thr = light_threshold(g);
         uint32_t *keys = dmalloc<uint32_t>((size_t)E);
-        int64_t *bptr = dmalloc<int64_t>((size_t)nblk + 1);
-        int64_t *boff = dmalloc<int64_t>((size_t)nblk + 1);
+        int64_t *bptr = dmalloc<int64_t>((size_t)nrun + 1);
+        int64_t *boff = dmalloc<int64_t>((size_t)nrun + 1);
         struct F3 {
             void *p[3];
             ~F3()
@@ -1055,13 +1180,13 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
                 for (void *x : p) dfree(x);
             }
         } f3{{keys, bptr, boff}};
-        k_blk_keys<<<grid_for(E), kBlock, 0, s>>>(g->el_dst, E, keys);
+        k_blk_keys<<<grid_for(E), kBlock, 0, s>>>(g->el_dst, g->el_w, E, g->light_thr, keys);
         SSSP_LAUNCH_CHECK("k_blk_keys");
         uint32_t *bkeys = nullptr, *bperm = nullptr;
-        radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), E, nblk - 1, kA, kB, vA, vB,
+        radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), E, nrun - 1, kA, kB, vA, vB,
                          counts, g->blk_a, g->blk_b, g->n_blk, s, &bkeys, &bperm);
-        rowptr_from_sorted(bkeys, E, nblk, bptr, s);
-        std::vector<int64_t> bp((size_t)nblk + 1), bo((size_t)nblk + 1);
+        rowptr_from_sorted(bkeys, E, nrun, bptr, s);
+        std::vector<int64_t> bp((size_t)nrun + 1), bo((size_t)nrun + 1);
         SSSP_HIP(hipMemcpyAsync(bp.data(), bptr, 8 * bp.size(), hipMemcpyDeviceToHost, s));
         SSSP_HIP(hipStreamSynchronize(s));
         bo[0] = 0;
@@ -1072,12 +1197,15 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         // 37.5 at 0.15, R-MAT 22 x 32 6.1 ms at 0.15 against 6.5 at 0.4.
         int64_t max_blk = 0;
         for (int32_t b = 0; b < nblk; b++)
-            max_blk = std::max(max_blk, bp[(size_t)b + 1] - bp[(size_t)b]);
+            max_blk = std::max(max_blk, bp[2 * (size_t)b + 2] - bp[2 * (size_t)b]);
         const bool no_hubs = (double)max_blk * nblk < 2.0 * (double)E;
         if (no_hubs) g->dense_all_frac = 0.4;
-        for (int32_t b = 0; b < nblk; b++)
+        for (int32_t b = 0; b < nrun; b++)
             bo[(size_t)b + 1] = bo[(size_t)b] +
                                 (bp[(size_t)b + 1] - bp[(size_t)b] + kBlkChunk - 1) / kBlkChunk * kBlkChunk;
+        if (g->light_thr != 0xFFFFFFFFu)
+            for (int32_t b = 0; b < nrun; b += 2)
+                g->light_edges += bp[(size_t)b + 1] - bp[(size_t)b];
         // Tile cap: 2^17 edges up to 2^29 edges, doubled while more than
         // kBlkTileCount tiles of the cap fit in the graph -- the 2.08 G-edge
         // R-MAT graph ran 50.9 GTEPS with 2^19-edge tiles, 46.7 with 2^17;
@@ -1089,10 +1217,7 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         int64_t tcap = kBlkTileEdges;
         while (tcap * kBlkTileCount < E) tcap <<= 1;
         g->b_off_host = bo;
-        std::vector<BlkTile> tiles = make_blk_tiles(bo, tcap, 0, BlkRanges{});
-        g->blk_tile_cap = tcap;
-        g->blk_tile_order = 0;
-        const int64_t Ep = bo[(size_t)nblk];
+        const int64_t Ep = bo[(size_t)nrun];
         const int64_t nch = Ep / kBlkChunk;
         SSSP_HIP(hipMemcpyAsync(boff, bo.data(), 8 * bo.size(), hipMemcpyHostToDevice, s));
         // whole sources and destination offsets first, packed below
@@ -1108,16 +1233,11 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
             }
         } f4{{bs, bd, wflag, widx}};
         g->b_w = dmalloc<uint32_t>((size_t)Ep);
-        g->n_btile = (int32_t)tiles.size();
         g->b_edges = Ep;
-        g->b_tile = dmalloc<BlkTile>(tiles.size());
-        g->b_app = dmalloc<uint16_t>(tiles.size() * kBlkThreads);
-        SSSP_HIP(hipMemcpyAsync(g->b_tile, tiles.data(), sizeof(BlkTile) * tiles.size(),
-                                hipMemcpyHostToDevice, s));
         k_blk_gather<<<grid_for(E), kBlock, 0, s>>>(bkeys, bperm, E, bptr, boff, g->el_src,
                                                     g->el_dst, g->el_w, bs, bd, g->b_w);
         SSSP_LAUNCH_CHECK("k_blk_gather");
-        k_blk_pad<<<grid_for((int64_t)nblk * kBlkChunk), kBlock, 0, s>>>(bptr, boff, nblk, bs, bd,
+        k_blk_pad<<<grid_for((int64_t)nrun * kBlkChunk), kBlock, 0, s>>>(bptr, boff, nrun, bs, bd,
                                                                          g->b_w);
         SSSP_LAUNCH_CHECK("k_blk_pad");
         const unsigned chunk_grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
@@ -1140,13 +1260,13 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         // (for tiles dispatched range by range), when the table is small
         const int64_t nfine = ((int64_t)V + (1 << kBlkRangeFineBits) - 1) >> kBlkRangeFineBits;
         if ((int64_t)nblk * (nfine + 1) <= kBlkRangeMaxEntries) {
-            const int64_t n_off = (int64_t)nblk * (nfine + 1);
+            const int64_t n_off = (int64_t)nrun * (nfine + 1);
             int64_t *roff = dmalloc<int64_t>((size_t)n_off);
             struct F1 {
                 void *p;
                 ~F1() { dfree(p); }
             } f1{roff};
-            k_blk_range_offsets<<<grid_for(n_off), kBlock, 0, s>>>(bs, boff, nblk, kBlkRangeFineBits,
+            k_blk_range_offsets<<<grid_for(n_off), kBlock, 0, s>>>(bs, boff, nrun, kBlkRangeFineBits,
                                                                   (int32_t)nfine, roff);
             SSSP_LAUNCH_CHECK("k_blk_range_offsets");
             g->b_ranges.off.resize((size_t)n_off);
@@ -1165,11 +1285,13 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         // 7.75 / 11.1 / 0.38 by block, 7.09 / 7.93 / 0.38 in 8 ranges). Graphs
         // with hubs lose by it (R-MAT 25 x 16: 17.2 / 24.7 ms by block, 18.5 /
         // 26.4 in 8 ranges).
+        int range_bits = 0;
         if (no_hubs && V >= (1 << kBlkRangeMinVertexBits) && !g->b_ranges.off.empty()) {
             int lg = 0;
             while (((int64_t)1 << lg) < (int64_t)V) lg++;
-            retile_blocked(g, tcap, 0, std::max(kBlkRangeFineBits, lg - 3));
+            range_bits = std::max(kBlkRangeFineBits, lg - 3);
         }
+        retile_blocked(g, tcap, 0, range_bits);
     }
 
     // ---- CSC ----

@@ -37,6 +37,13 @@ struct alignas(64) RoundSlot {
 struct Ctrl {
     RoundSlot slot[2];
     int32_t changed[64];   // plain passes: changed[p & 63] = 1 when pass p lowered a distance
+    // passes over the blocked list (k_blk_plain), rings of 64: what pass p ran
+    // and how many vertices it lowered; full passes so far; first idle pass
+    int32_t ph_kind[64];
+    int32_t ph_low[64];
+    int32_t ph_full;
+    int32_t ph_done;
+    unsigned long long ph_pos;  // host mirror: progress word of the passes
     int64_t n_compact;     // lb scan: entries
     int64_t lb_total;      // lb scan: total edges
     int64_t cert[8];       // certificate counters
@@ -86,9 +93,20 @@ struct BlkTile {
     int32_t blk;
     int32_t split;
     int64_t e0, e1;
+    int64_t f0, f1;  // second run of slots (f0 == f1: none)
 };
-// Source-range cuts of the blocked list's block runs (host copy): off[b *
-// (n_fine + 1) + k] = first slot of block b whose source is at least
+// Weight classes of the blocked list. A block's run is its light edges
+// (weight at most the threshold, ascending sources, padded to whole chunks)
+// followed by its heavy ones; a light round relaxes the light edges alone.
+constexpr int kLightSample = 1 << 16;        // weights sampled for the threshold
+constexpr int64_t kLightTileMin = 1 << 12;   // edge slots of a light tile at least
+constexpr int64_t kLightTiles = 1024;        // ... and the tile count its cap aims at
+constexpr int kLightMaxPasses = 64;          // light passes stop after this many passes of a run
+constexpr double kLightStopFrac = 0.05;      // light passes stop once a pass lowers fewer than
+                                             // this share of the vertices with out-edges
+// Source-range cuts of the blocked list's runs (host copy; run 2 b = block
+// b's light edges, 2 b + 1 its heavy ones): off[run *
+// (n_fine + 1) + k] = first slot of the run whose source is at least
 // k << fine_bits, aligned down to its chunk (k = n_fine: the run's end).
 // Tiles cut at every stride-th cut (stride 0: no cuts).
 constexpr int kBlkRangeFineBits = 18;
@@ -166,7 +184,12 @@ struct sssp_graph {
     int32_t n_btile = 0;
     uint16_t *b_app = nullptr;  // dense rounds' append masks: kBlkThreads per tile
     bool frontier_bits = false;  // the coming round's frontier is in b_app, not yet queued
-    std::vector<int64_t> b_off_host;  // padded block offsets (tiles are rebuilt from them)
+    sssp::BlkTile *b_ltile = nullptr;  // tiles of the light edges (n_ltile 0: no weight classes)
+    int32_t n_ltile = 0;
+    int64_t light_edges = 0;      // edges in the light class
+    uint32_t light_thr = 0xFFFFFFFFu;  // largest weight pattern of the light class
+    std::vector<int64_t> b_off_host;  // padded run offsets, two runs per block (tiles are rebuilt
+                                      // from them)
     int64_t blk_tile_cap = 0;         // edges per tile at most
     int blk_tile_order = 0;           // dispatch order of the tiles (make_blk_tiles)
     sssp::BlkRanges b_ranges;         // source-range cuts of the block runs (may be empty)
@@ -247,6 +270,7 @@ struct sssp_graph {
     sssp::Ctrl *ctrl_host_dev = nullptr;  // the mirror's device address
     int32_t tick = 1;
     int32_t dec_seq = 0;  // sequence number of the last decision enqueued
+    int32_t ph_tag = 0;   // tag of the last run of blocked passes
     int decide_spin = 1;  // 1: poll the mirror for the decision; 0: stream synchronize
     hipEvent_t ev_a = nullptr, ev_b = nullptr, ev_r0 = nullptr, ev_r1 = nullptr;
 

@@ -99,6 +99,7 @@ inline void dfree(void *p)
 // serves both types.
 // ---------------------------------------------------------------------------
 struct WF32 {
+    static constexpr bool kWeighted = true;
     static constexpr uint32_t INF = 0x7F7FFFFFu;  // FLT_MAX
     __device__ __forceinline__ static uint32_t add(uint32_t d, uint32_t w)
     {
@@ -109,6 +110,7 @@ struct WF32 {
 };
 
 struct WU32 {
+    static constexpr bool kWeighted = true;
     static constexpr uint32_t INF = 0xFFFFFFFFu;
     __device__ __forceinline__ static uint32_t add(uint32_t d, uint32_t w)
     {
@@ -121,6 +123,7 @@ struct WU32 {
 // of d[v] <= d[u] + 1 is the hop distance, and d != INF is the reference's
 // visited flag (bfs.cu:25-39). Callers never add to INF; levels stay < V.
 struct WUnit {
+    static constexpr bool kWeighted = false;
     static constexpr uint32_t INF = 0xFFFFFFFFu;
     __device__ __forceinline__ static uint32_t add(uint32_t d, uint32_t) { return d + 1u; }
 };

@@ -902,3 +902,62 @@ def test_python_mirror_cache_follows_in_place_edits(gpu, oracle):
     op.gpu_bellman_ford(g, d, 0)
     assert np.array_equal(bits(d), bits(oracle.dijkstra(g.src_ids, g.dst_ids, g.weights,
                                                           g.vertices_count, 0)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["one_block", "block_edge", "split", "ties", "equal", "u32",
+                                  "ranges", "path"])
+def test_light_passes_bit_exact(gpu, oracle, case):
+    """Light passes (the lightest edges alone, before a dense round and between
+    the full passes of small graphs) end on the oracle's fixpoint: a graph
+    of one destination block, one vertex past a block, tiles down to 256 slots
+    (split blocks), a few distinct weights, equal weights (no light class), u32,
+    tiles by source range, and a long path whose passes outlast the light
+    ones. Bit equality: no tolerance."""
+    rng = np.random.default_rng(17)
+    V = {"one_block": 1 << 14, "block_edge": (1 << 14) + 1, "path": 40000}.get(case, 50021)
+    n = 8 * V
+    src = (rng.random(n) ** 3 * V).astype(np.int32)
+    dst = (rng.random(n) ** 2 * V).astype(np.int32)
+    if case in ("u32", "ranges"):
+        src, dst = (rng.integers(0, V, n).astype(np.int32) for _ in range(2))
+    w = rng.random(n, dtype=np.float32)
+    if case == "ties":
+        w = (rng.integers(0, 8, n) / 8).astype(np.float32)
+    elif case == "equal":
+        w = np.full(n, 0.25, np.float32)
+    elif case == "u32":
+        w = rng.integers(1, 256, n).astype(np.uint32)
+    elif case == "path":
+        hop = np.arange(V, dtype=np.int32)[::-1].copy()  # against the ids: one hop a pass
+        src, dst = np.concatenate([hop[:400], src[:200]]), np.concatenate([hop[1:401], dst[:200]])
+        w = np.concatenate([rng.random(400, dtype=np.float32), np.full(200, 9, np.float32)])
+    source = int(src[0])
+    ref = oracle.dijkstra(src, dst, w, V, source)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        g.set_param("dense_unreached", 0.0)  # every all-edge round dense
+        if case == "split":
+            g.set_param("blk_tile_cap", 256)
+        if case == "ranges":
+            g.set_param("blk_range_bits", 18)
+        g.set_param("trace_events", 1)
+        light = 0
+        for below, kernel in ((2 ** 26, 2), (0, 2)):  # pass loop, round engine
+            g.set_param("plain_below_edges", below)
+            g.set_param("plain_kernel", kernel)
+            for frac in (0.05, 0.0):  # push rounds first, or none
+                g.set_param("push_edge_frac", frac)
+                for traced in (1, 0):
+                    g.set_param("trace_events", traced)
+                    print(f"light passes: {case} below {below} push {frac} traced {traced}",
+                          flush=True)
+                    d, st = g.solve(source, "heuristic")
+                    assert np.array_equal(bits(d), bits(ref)), (below, frac, traced)
+                    if traced:
+                        tr = g.trace()
+                        assert len(tr["mode"]) == st["iterations"]
+                        light += int((tr["mode"] == S.MODE_LIGHT).sum())
+        assert (light == 0) == (case == "equal"), light
+        d, st = g.solve(source, "plain")  # the plain schedule stays all-edge passes
+        assert np.array_equal(bits(d), bits(ref))
+        assert st["edges_relaxed"] == st["iterations"] * len(src)
