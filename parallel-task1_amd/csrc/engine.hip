@@ -1462,22 +1462,20 @@ __device__ __forceinline__ int64_t blk_relax_tile(const BlkTile &t, const BlkLis
     };
     // tiles hold whole chunks and the wave's 64 lanes cover one chunk per
     // step, so the loop bound and the chunk index are wave-uniform (kept in
-    // scalar registers); chunks nc0 and up are those of the tile's second
-    // run. The next step's stream loads are issued before this step's gathers.
-    const int nc0 = (int)((t.e1 - t.e0) / kBlkChunk);
-    const int nc = nc0 + (int)((t.f1 - t.f0) / kBlkChunk);
-    const int64_t ce = t.e0 / kBlkChunk, cf = t.f0 / kBlkChunk - nc0;
-    int c = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // scalar registers). The next step's stream loads are issued before this
+    // step's gathers.
+    constexpr int kStep = kBlkThreads / 64;
+    const int c1 = (int)(t.e1 / kBlkChunk);
+    int c = (int)(t.e0 / kBlkChunk) + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int32_t cb = 0;
     v4u pv = {0u, 0u, 0u, 0u}, wv = {0u, 0u, 0u, 0u};
-    auto load = [&](int i, int32_t &b, v4u &p, v4u &ww) {
-        const int64_t k = (i < nc0 ? ce : cf) + i;  // chunk of the list
+    auto load = [&](int64_t k, int32_t &b, v4u &p, v4u &ww) {
         b = L.cbase[k];
         p = __builtin_nontemporal_load(&p4[k * (kBlkChunk / 4) + lane]);
         ww = __builtin_nontemporal_load(&w4[k * (kBlkChunk / 4) + lane]);
     };
-    if (c < nc) load(c, cb, pv, wv);
-    for (; c < nc; c += kBlkThreads / 64) {
+    if (c < c1) load(c, cb, pv, wv);
+    for (; c < c1; c += kStep) {
         int32_t s0, s1, s2, s3;
         if (cb >= 0) {
             const int32_t a0 = (int32_t)(pv.x >> kBlkBits);
@@ -1508,7 +1506,7 @@ __device__ __forceinline__ int64_t blk_relax_tile(const BlkTile &t, const BlkLis
         const uint32_t u0 = dist[s0], u1 = dist[s1], u2 = dist[s2], u3 = dist[s3];
         int32_t cbn = 0;
         v4u pvn = {0u, 0u, 0u, 0u}, wvn = {0u, 0u, 0u, 0u};
-        if (c + kBlkThreads / 64 < nc) load(c + kBlkThreads / 64, cbn, pvn, wvn);
+        if (c + kStep < c1) load(c + kStep, cbn, pvn, wvn);
         relax(u0, pv.x & kOffMask, wv.x);
         relax(u1, pv.y & kOffMask, wv.y);
         relax(u2, pv.z & kOffMask, wv.z);
@@ -1794,7 +1792,7 @@ __device__ __forceinline__ int pass_kind(const PassArgs &a)
 
 template <class WT>
 __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blk_plain(
-    const PassArgs a, const BlkList L, uint32_t *dist)
+    const PassArgs a, const BlkList L, const BlkList LL, uint32_t *dist)
 {
     __shared__ uint32_t s_d[1 << kBlkBits];
     __shared__ int s_low;
@@ -1819,7 +1817,7 @@ __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))
     const BlkTile t = (light ? a.light : a.full)[blockIdx.x];
     if (threadIdx.x == 0) s_low = 0;  // before the relaxation's barriers
     const int64_t base = (int64_t)t.blk << kBlkBits;
-    blk_relax_tile<WT, false>(t, L, dist, s_d);
+    blk_relax_tile<WT, false>(t, light ? LL : L, dist, s_d);
     int low = 0;
 #pragma unroll
     for (int k0 = 0; k0 < kBlkPer; k0 += 8) {
@@ -2270,6 +2268,7 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
     const unsigned grid = (unsigned)(run == kRunFull    ? g->n_btile
                                      : run == kRunLight ? g->n_ltile
                                                         : std::max(g->n_btile, g->n_ltile));
+    const BlkList light_list{g->l_pk, g->l_cbase, g->l_wide, g->l_w};
     // the mirror still holds the last run's word (another tag) or none
     volatile unsigned long long *pos = &g->ctrl_host->ph_pos;
     const unsigned long long mine = pass_word(a.tag, 0, 0, 0) >> 58;
@@ -2280,7 +2279,7 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
         while (queued < begun + ahead) {
             a.pass = queued++;
             if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
-            k_blk_plain<WT><<<grid, kBlkThreads, 0, s>>>(a, blk_list(g), g->dist);
+            k_blk_plain<WT><<<grid, kBlkThreads, 0, s>>>(a, blk_list(g), light_list, g->dist);
             SSSP_LAUNCH_CHECK("k_blk_plain");
             if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r1, s));
         }

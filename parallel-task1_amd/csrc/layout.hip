@@ -332,13 +332,49 @@ __global__ __launch_bounds__(kBlock) void k_group_gather(const uint32_t *perm, c
     }
 }
 
-// Run of an edge: its destination block, light before heavy.
-__global__ __launch_bounds__(kBlock) void k_blk_keys(const int32_t *dst, const uint32_t *w,
-                                                     int64_t E, uint32_t thr, uint32_t *keys)
+__global__ __launch_bounds__(kBlock) void k_blk_keys(const int32_t *dst, int64_t E, uint32_t *keys)
 {
     for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < E;
          e += (int64_t)gridDim.x * kBlock)
-        keys[e] = (((uint32_t)dst[e] >> kBlkBits) << 1) | (w[e] > thr ? 1u : 0u);
+        keys[e] = (uint32_t)dst[e] >> kBlkBits;
+}
+
+// Sorted position j of block b = skeys[j] goes to boff[b] + (j - bptr[b]);
+// perm[j] is its position in the src-sorted list, whose order is kept.
+__global__ __launch_bounds__(kBlock) void k_blk_gather(const uint32_t *skeys, const uint32_t *perm,
+                                                       int64_t E, const int64_t *bptr,
+                                                       const int64_t *boff, const int32_t *src,
+                                                       const int32_t *dst, const uint32_t *w,
+                                                       int32_t *bs, uint16_t *bd, uint32_t *bw)
+{
+    for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < E;
+         j += (int64_t)gridDim.x * kBlock) {
+        const uint32_t b = skeys[j];
+        const int64_t o = boff[b] + (j - bptr[b]);
+        const uint32_t p = perm[j];
+        bs[o] = src[p];
+        bd[o] = (uint16_t)(dst[p] - (int32_t)(b << kBlkBits));
+        bw[o] = w[p];
+    }
+}
+
+// The padding slots of each block (up to kBlkChunk - 1) copy the block's last
+// edge: relaxing it again changes nothing, and its source delta is 0.
+__global__ __launch_bounds__(kBlock) void k_blk_pad(const int64_t *bptr, const int64_t *boff,
+                                                    int32_t nblk, int32_t *bs, uint16_t *bd,
+                                                    uint32_t *bw)
+{
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < (int64_t)nblk * kBlkChunk;
+         i += (int64_t)gridDim.x * kBlock) {
+        const int32_t b = (int32_t)(i / kBlkChunk);
+        const int64_t last = boff[b] + (bptr[b + 1] - bptr[b]) - 1;
+        const int64_t o = last + 1 + i % kBlkChunk;
+        if (o < boff[b + 1]) {  // only blocks with edges have slots
+            bs[o] = bs[last];
+            bd[o] = bd[last];
+            bw[o] = bw[last];
+        }
+    }
 }
 
 // out[i] = w[i * E / n]: a fixed-stride sample of the weights
@@ -358,44 +394,6 @@ __global__ __launch_bounds__(kBlock) void k_max_degree(const int64_t *ptr, int64
         m = max(m, (uint32_t)(ptr[v + 1] - ptr[v]));
     for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor(m, o));
     if (__lane_id() == 0 && m) atomicMax(mx, m);
-}
-
-// Sorted position j of run b = skeys[j] goes to boff[b] + (j - bptr[b]);
-// perm[j] is its position in the src-sorted list, whose order is kept.
-__global__ __launch_bounds__(kBlock) void k_blk_gather(const uint32_t *skeys, const uint32_t *perm,
-                                                       int64_t E, const int64_t *bptr,
-                                                       const int64_t *boff, const int32_t *src,
-                                                       const int32_t *dst, const uint32_t *w,
-                                                       int32_t *bs, uint16_t *bd, uint32_t *bw)
-{
-    for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < E;
-         j += (int64_t)gridDim.x * kBlock) {
-        const uint32_t b = skeys[j];
-        const int64_t o = boff[b] + (j - bptr[b]);
-        const uint32_t p = perm[j];
-        bs[o] = src[p];
-        bd[o] = (uint16_t)(dst[p] - (int32_t)((b >> 1) << kBlkBits));
-        bw[o] = w[p];
-    }
-}
-
-// The padding slots of each run (up to kBlkChunk - 1) copy the run's last
-// edge: relaxing it again changes nothing, and its source delta is 0.
-__global__ __launch_bounds__(kBlock) void k_blk_pad(const int64_t *bptr, const int64_t *boff,
-                                                    int32_t nblk, int32_t *bs, uint16_t *bd,
-                                                    uint32_t *bw)
-{
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < (int64_t)nblk * kBlkChunk;
-         i += (int64_t)gridDim.x * kBlock) {
-        const int32_t b = (int32_t)(i / kBlkChunk);
-        const int64_t last = boff[b] + (bptr[b + 1] - bptr[b]) - 1;
-        const int64_t o = last + 1 + i % kBlkChunk;
-        if (o < boff[b + 1]) {  // only runs with edges have slots
-            bs[o] = bs[last];
-            bd[o] = bd[last];
-            bw[o] = bw[last];
-        }
-    }
 }
 
 // Source deltas of one chunk (one wave, 4 slots per lane, in slot order):
@@ -451,6 +449,70 @@ __global__ __launch_bounds__(kBlock) void k_blk_pack(const int32_t *bs, const ui
     if (wi >= 0)
         for (int k = 0; k < 4; k++) wide[(int64_t)wi * kBlkChunk + 4 * __lane_id() + k] = s[k];
     if (__lane_id() == 0) cbase[c] = wi < 0 ? s[0] : -(1 + wi);
+}
+
+// Light edges of one chunk of the blocked list (one wave, 4 slots per lane):
+// bit k of the result is set when the lane's slot k holds a light edge.
+__device__ __forceinline__ int chunk_light(const uint32_t *bw, int64_t c, uint32_t thr)
+{
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    const v4u v = reinterpret_cast<const v4u *>(bw)[c * (kBlkChunk / 4) + __lane_id()];
+    return (v.x <= thr ? 1 : 0) | (v.y <= thr ? 2 : 0) | (v.z <= thr ? 4 : 0) |
+           (v.w <= thr ? 8 : 0);
+}
+
+__global__ __launch_bounds__(kBlock) void k_light_count(const uint32_t *bw, int64_t nch,
+                                                        uint32_t thr, int64_t *cnt)
+{
+    const int64_t c = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+    if (c >= nch) return;  // wave-uniform
+    const int n = wave_sum32(__popc(chunk_light(bw, c, thr)));
+    if (__lane_id() == 0) cnt[c] = n;
+}
+
+// out[b] = pos[boff[b] / kBlkChunk]: light edges before block b (nblk + 1 values)
+__global__ __launch_bounds__(kBlock) void k_light_starts(const int64_t *pos, const int64_t *boff,
+                                                         int32_t nblk, int64_t *out)
+{
+    for (int64_t b = (int64_t)blockIdx.x * kBlock + threadIdx.x; b <= nblk;
+         b += (int64_t)gridDim.x * kBlock)
+        out[b] = pos[boff[b] / kBlkChunk];
+}
+
+// The light edges of chunk c, in order, to their block's run of the light list:
+// pos = light edges before each chunk, lptr / loff = light edges before and
+// first slot of each block.
+__global__ __launch_bounds__(kBlock) void k_light_gather(const int32_t *bs, const uint16_t *bd,
+                                                         const uint32_t *bw, int64_t nch,
+                                                         uint32_t thr, const int64_t *pos,
+                                                         const int64_t *boff, int32_t nblk,
+                                                         const int64_t *lptr, const int64_t *loff,
+                                                         int32_t *ls, uint16_t *ld, uint32_t *lw)
+{
+    const int64_t c = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+    if (c >= nch) return;  // wave-uniform
+    const int m = chunk_light(bw, c, thr);
+    int32_t lo = 0, hi = nblk - 1;  // the chunk's block: the last with boff <= its first slot
+    while (lo < hi) {
+        const int32_t mid = (lo + hi + 1) >> 1;
+        if (boff[mid] <= c * kBlkChunk) lo = mid;
+        else hi = mid - 1;
+    }
+    int inc = __popc(m);  // inclusive scan of the counts over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o);
+        if (__lane_id() >= o) inc += y;
+    }
+    int64_t o = loff[lo] + (pos[c] - lptr[lo]) + inc - __popc(m);
+    for (int k = 0; k < 4; k++) {
+        if (!((m >> k) & 1)) continue;
+        const int64_t e = c * kBlkChunk + 4 * __lane_id() + k;
+        ls[o] = bs[e];
+        ld[o] = bd[e];
+        lw[o] = bw[e];
+        o++;
+    }
 }
 
 // off[b * (nfine + 1) + k] = the first slot of block b whose source is at
@@ -748,7 +810,7 @@ void build_multi_layout(sssp_graph *g)
         const int64_t nt = (c + kMTileEdges - 1) / kMTileEdges;
         for (int64_t k = 0; k < nt; k++) {
             const int64_t e0 = bp[(size_t)b] + k * kMTileEdges;
-            tiles.push_back(BlkTile{b, nt > 1 ? 1 : 0, e0, std::min(e0 + kMTileEdges, bp[(size_t)b + 1]), 0, 0});
+            tiles.push_back(BlkTile{b, nt > 1 ? 1 : 0, e0, std::min(e0 + kMTileEdges, bp[(size_t)b + 1])});
         }
     }
     BlkTile *td = dmalloc<BlkTile>(std::max<size_t>(tiles.size(), 1));
@@ -796,63 +858,38 @@ void validate_edges(const int32_t *src, const int32_t *dst, const void *w, int w
     if (hb[1]) throw Error{SSSP_ERR_ARG, std::to_string(hb[1]) + " edges have a negative or NaN weight"};
 }
 
-// The tiles of the destination-blocked list: at most `cap` edge slots (a
-// multiple of kBlkChunk) of one block, `split` when a block has several.
-// Without source ranges (R.stride == 0) a tile is one run of its block's slots;
+// The tiles of the destination-blocked list: runs of at most `cap` edge slots
+// (a multiple of kBlkChunk) of one block, `split` when a block has several.
+// Without source ranges (R.stride == 0) a tile is a run of its block's slots;
 // order 0 = smallest tiles first (stable by block), 1 = by block, 2 = largest
-// first, 3 = by descending block. With source ranges each run is cut
+// first, 3 = by descending block. With source ranges each block's run is cut
 // at the (chunk-aligned) slots where its sources reach multiples of the range
 // size, and the tiles are dispatched range by range (by block within one):
 // the workgroups running at one time then gather d[src] from one range of
-// the distance array, which an XCD's L2 holds; a tile then holds its range's
-// light and heavy slots as two runs. bo: padded run offsets (light and heavy
-// run of each block), 2 nblk + 1 values; light: the light runs alone.
+// the distance array, which an XCD's L2 holds. bo: padded block offsets,
+// nblk + 1 values (of the blocked list or the light list); off: its cuts.
 std::vector<BlkTile> make_blk_tiles(const std::vector<int64_t> &bo, int64_t cap, int order,
-                                    const BlkRanges &R, bool light)
+                                    const BlkRanges &R, const std::vector<int64_t> &off)
 {
     struct T {
         BlkTile t;
         int32_t range;
     };
     std::vector<T> tiles;
-    const int32_t nblk = (int32_t)((bo.size() - 1) / 2);
-    const bool ranged = R.stride > 0 && !R.off.empty();
+    const int32_t nblk = (int32_t)bo.size() - 1;
+    const bool ranged = R.stride > 0 && !off.empty();
     const int32_t nr = ranged ? (R.n_fine + R.stride - 1) / R.stride : 1;
     for (int32_t b = 0; b < nblk; b++) {
         const size_t first = tiles.size();
         for (int32_t r = 0; r < nr; r++) {
-            int64_t lo[2], hi[2];  // the slots of the block's two runs
-            for (int h = 0; h < 2; h++) {
-                const size_t run = 2 * (size_t)b + (size_t)h;
-                lo[h] = bo[run];
-                hi[h] = bo[run + 1];
-                if (ranged) {
-                    const size_t row = run * (size_t)(R.n_fine + 1);
-                    lo[h] = R.off[row + (size_t)std::min(r * R.stride, R.n_fine)];
-                    hi[h] = R.off[row + (size_t)std::min((r + 1) * R.stride, R.n_fine)];
-                }
+            int64_t lo = bo[(size_t)b], hi = bo[(size_t)b + 1];
+            if (ranged) {
+                const size_t row = (size_t)b * (size_t)(R.n_fine + 1);
+                lo = off[row + (size_t)std::min(r * R.stride, R.n_fine)];
+                hi = off[row + (size_t)std::min((r + 1) * R.stride, R.n_fine)];
             }
-            if (light) {
-                lo[1] = hi[1] = 0;
-            } else if (hi[0] == lo[1]) {  // one run
-                hi[0] = hi[1];
-                lo[1] = hi[1] = 0;
-            }
-            while (lo[0] < hi[0] || lo[1] < hi[1]) {
-                const int64_t n0 = std::min(cap, hi[0] - lo[0]);
-                const int64_t n1 = std::min(cap - n0, hi[1] - lo[1]);
-                BlkTile t{b, 0, lo[0], lo[0] + n0, 0, 0};
-                if (n0 == 0) {
-                    t.e0 = lo[1];
-                    t.e1 = lo[1] + n1;
-                } else if (n1 > 0) {
-                    t.f0 = lo[1];
-                    t.f1 = lo[1] + n1;
-                }
-                lo[0] += n0;
-                lo[1] += n1;
-                tiles.push_back(T{t, r});
-            }
+            for (int64_t e0 = lo; e0 < hi; e0 += cap)
+                tiles.push_back(T{BlkTile{b, 0, e0, std::min(e0 + cap, hi)}, r});
         }
         if (tiles.size() - first > 1)
             for (size_t i = first; i < tiles.size(); i++) tiles[i].t.split = 1;
@@ -893,10 +930,10 @@ void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits)
             throw Error{SSSP_ERR_ARG, "blk_range_bits: source ranges unavailable for this size"};
         R.stride = 1 << (range_bits - R.fine_bits);
     }
-    const std::vector<BlkTile> tiles = make_blk_tiles(g->b_off_host, cap, order, R, false);
+    const std::vector<BlkTile> tiles = make_blk_tiles(g->b_off_host, cap, order, R, R.off);
     std::vector<BlkTile> ltiles;
     if (g->light_edges > 0)
-        ltiles = make_blk_tiles(g->b_off_host, light_cap(g, cap), order, R, true);
+        ltiles = make_blk_tiles(g->l_off_host, light_cap(g, cap), order, R, R.loff);
     auto upload = [&](const std::vector<BlkTile> &t) {
         BlkTile *d = dmalloc<BlkTile>(std::max<size_t>(t.size(), 1));
         SSSP_HIP(hipMemcpyAsync(d, t.data(), sizeof(BlkTile) * t.size(), hipMemcpyHostToDevice,
@@ -963,7 +1000,9 @@ static uint32_t light_threshold(const sssp_graph *g)
     SSSP_HIP(hipMemcpyAsync(s.data(), d, 4 * s.size(), hipMemcpyDeviceToHost, g->stream));
     SSSP_HIP(hipStreamSynchronize(g->stream));
     const double mean = (double)g->E / std::max(g->n_nzo, 1);
-    const double per_vertex = (double)s.back() >= 16.0 * mean ? 1.0 : 6.0;
+    const bool hubs = (double)s.back() >= 16.0 * mean;
+    if (!hubs && mean < kLightMinDegree) return 0xFFFFFFFFu;
+    const double per_vertex = hubs ? 1.0 : 6.0;
     const double frac = std::min(0.5, std::max(1.0 / 16, per_vertex / mean));
     s.pop_back();
     std::sort(s.begin(), s.end());
@@ -976,6 +1015,115 @@ static uint32_t light_threshold(const sssp_graph *g)
     const double got = use_lo ? (double)lo : (double)up;
     if (got < 0.5 * target || got > 3.0 * target || got > 0.75 * (double)n) return 0xFFFFFFFFu;
     return use_lo ? at - 1 : at;
+}
+
+// Packs nch chunks of whole sources and destination offsets (k_blk_pack).
+static void pack_chunks(const int32_t *bs, const uint16_t *bd, int64_t nch, hipStream_t s,
+                        uint32_t **pk, int32_t **cbase, int32_t **wide, int64_t *nwide)
+{
+    uint8_t *wflag = dmalloc<uint8_t>((size_t)nch);
+    struct F {
+        void *p[2] = {};
+        ~F()
+        {
+            for (void *x : p) dfree(x);
+        }
+    } f;
+    f.p[0] = wflag;
+    int32_t *widx = dmalloc<int32_t>((size_t)nch);
+    f.p[1] = widx;
+    const unsigned chunk_grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
+    k_blk_chunk_wide<<<chunk_grid, kBlock, 0, s>>>(bs, nch, wflag);
+    SSSP_LAUNCH_CHECK("k_blk_chunk_wide");
+    std::vector<uint8_t> wf((size_t)nch);
+    SSSP_HIP(hipMemcpyAsync(wf.data(), wflag, (size_t)nch, hipMemcpyDeviceToHost, s));
+    SSSP_HIP(hipStreamSynchronize(s));
+    std::vector<int32_t> wi((size_t)nch);
+    int64_t nw = 0;
+    for (int64_t c = 0; c < nch; c++) wi[(size_t)c] = wf[(size_t)c] ? (int32_t)nw++ : -1;
+    SSSP_HIP(hipMemcpyAsync(widx, wi.data(), 4 * (size_t)nch, hipMemcpyHostToDevice, s));
+    *pk = dmalloc<uint32_t>((size_t)(nch * kBlkChunk));
+    *cbase = dmalloc<int32_t>((size_t)nch);
+    *wide = nw ? dmalloc<int32_t>((size_t)(nw * kBlkChunk)) : nullptr;
+    *nwide = nw;
+    k_blk_pack<<<chunk_grid, kBlock, 0, s>>>(bs, bd, widx, nch, *pk, *cbase, *wide);
+    SSSP_LAUNCH_CHECK("k_blk_pack");
+    SSSP_HIP(hipStreamSynchronize(s));
+}
+
+// Source-range cuts of every block's run (k_blk_range_offsets), to the host.
+static void range_cuts(const int32_t *bs, const int64_t *boff, int32_t nblk, int32_t nfine,
+                       hipStream_t s, std::vector<int64_t> *out)
+{
+    const int64_t n_off = (int64_t)nblk * (nfine + 1);
+    int64_t *roff = dmalloc<int64_t>((size_t)n_off);
+    struct F {
+        void *p;
+        ~F() { dfree(p); }
+    } f{roff};
+    k_blk_range_offsets<<<grid_for(n_off), kBlock, 0, s>>>(bs, boff, nblk, kBlkRangeFineBits, nfine,
+                                                          roff);
+    SSSP_LAUNCH_CHECK("k_blk_range_offsets");
+    out->resize((size_t)n_off);
+    SSSP_HIP(hipMemcpyAsync(out->data(), roff, 8 * (size_t)n_off, hipMemcpyDeviceToHost, s));
+    SSSP_HIP(hipStreamSynchronize(s));
+}
+
+// The light list, from the blocked list's edges (bs, bd and b_w, nch chunks,
+// boff: first slot of each block on the device): light edges counted per
+// chunk, scanned, and gathered in order, each block's run padded to whole
+// chunks as the blocked list's. (The padding of the blocked list may be light:
+// its copies of an edge are copied too.)
+static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *bd,
+                             const int64_t *boff, int32_t nblk, int64_t nch)
+{
+    hipStream_t s = g->stream;
+    const uint32_t thr = light_threshold(g);
+    if (thr == 0xFFFFFFFFu) return;
+    struct F {
+        void *p[5] = {};
+        ~F()
+        {
+            for (void *x : p) dfree(x);
+        }
+    } f;
+    int64_t *pos = dmalloc<int64_t>((size_t)nch + 1);
+    f.p[0] = pos;
+    int64_t *lptr = dmalloc<int64_t>(2 * ((size_t)nblk + 1));
+    f.p[1] = lptr;
+    int64_t *loff = lptr + nblk + 1;
+    const unsigned chunk_grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
+    k_light_count<<<chunk_grid, kBlock, 0, s>>>(g->b_w, nch, thr, pos);
+    SSSP_LAUNCH_CHECK("k_light_count");
+    k_fill_i64<<<1, 64, 0, s>>>(pos + nch, 1, 0);  // the last position: the total
+    device_exclusive_scan_i64(pos, pos, nch + 1, g->blk_a, g->blk_b, g->n_blk, s);
+    k_light_starts<<<grid_for((int64_t)nblk + 1), kBlock, 0, s>>>(pos, boff, nblk, lptr);
+    SSSP_LAUNCH_CHECK("k_light_starts");
+    std::vector<int64_t> lp((size_t)nblk + 1), lo((size_t)nblk + 1, 0);
+    SSSP_HIP(hipMemcpyAsync(lp.data(), lptr, 8 * lp.size(), hipMemcpyDeviceToHost, s));
+    SSSP_HIP(hipStreamSynchronize(s));
+    for (size_t b = 0; b < (size_t)nblk; b++)
+        lo[b + 1] = lo[b] + (lp[b + 1] - lp[b] + kBlkChunk - 1) / kBlkChunk * kBlkChunk;
+    const int64_t Lp = lo[(size_t)nblk];
+    if (Lp == 0) return;
+    SSSP_HIP(hipMemcpyAsync(loff, lo.data(), 8 * lo.size(), hipMemcpyHostToDevice, s));
+    int32_t *ls = dmalloc<int32_t>((size_t)Lp);
+    f.p[2] = ls;
+    uint16_t *ld = dmalloc<uint16_t>((size_t)Lp);
+    f.p[3] = ld;
+    g->l_w = dmalloc<uint32_t>((size_t)Lp);
+    k_light_gather<<<chunk_grid, kBlock, 0, s>>>(bs, bd, g->b_w, nch, thr, pos, boff, nblk, lptr,
+                                                 loff, ls, ld, g->l_w);
+    SSSP_LAUNCH_CHECK("k_light_gather");
+    k_blk_pad<<<grid_for((int64_t)nblk * kBlkChunk), kBlock, 0, s>>>(lptr, loff, nblk, ls, ld,
+                                                                     g->l_w);
+    SSSP_LAUNCH_CHECK("k_blk_pad light");
+    pack_chunks(ls, ld, Lp / kBlkChunk, s, &g->l_pk, &g->l_cbase, &g->l_wide, &g->l_nwide);
+    if (g->b_ranges.n_fine > 0)
+        range_cuts(ls, loff, nblk, g->b_ranges.n_fine, s, &g->b_ranges.loff);
+    g->l_off_host = lo;
+    g->l_edges = Lp;
+    g->light_edges = lp[(size_t)nblk];
 }
 
 void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, const uint32_t *d_w,
@@ -1168,11 +1316,9 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
     // ---- destination-blocked edge list ----
     if (E > 0) {
         const int32_t nblk = (int32_t)(((int64_t)V + (1 << kBlkBits) - 1) >> kBlkBits);
-        const int32_t nrun = 2 * nblk;  // light and heavy run of each block
-        g->light_thr = light_threshold(g);
         uint32_t *keys = dmalloc<uint32_t>((size_t)E);
-        int64_t *bptr = dmalloc<int64_t>((size_t)nrun + 1);
-        int64_t *boff = dmalloc<int64_t>((size_t)nrun + 1);
+        int64_t *bptr = dmalloc<int64_t>((size_t)nblk + 1);
+        int64_t *boff = dmalloc<int64_t>((size_t)nblk + 1);
         struct F3 {
             void *p[3];
             ~F3()
@@ -1180,13 +1326,13 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
                 for (void *x : p) dfree(x);
             }
         } f3{{keys, bptr, boff}};
-        k_blk_keys<<<grid_for(E), kBlock, 0, s>>>(g->el_dst, g->el_w, E, g->light_thr, keys);
+        k_blk_keys<<<grid_for(E), kBlock, 0, s>>>(g->el_dst, E, keys);
         SSSP_LAUNCH_CHECK("k_blk_keys");
         uint32_t *bkeys = nullptr, *bperm = nullptr;
-        radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), E, nrun - 1, kA, kB, vA, vB,
+        radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), E, nblk - 1, kA, kB, vA, vB,
                          counts, g->blk_a, g->blk_b, g->n_blk, s, &bkeys, &bperm);
-        rowptr_from_sorted(bkeys, E, nrun, bptr, s);
-        std::vector<int64_t> bp((size_t)nrun + 1), bo((size_t)nrun + 1);
+        rowptr_from_sorted(bkeys, E, nblk, bptr, s);
+        std::vector<int64_t> bp((size_t)nblk + 1), bo((size_t)nblk + 1);
         SSSP_HIP(hipMemcpyAsync(bp.data(), bptr, 8 * bp.size(), hipMemcpyDeviceToHost, s));
         SSSP_HIP(hipStreamSynchronize(s));
         bo[0] = 0;
@@ -1197,15 +1343,12 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         // 37.5 at 0.15, R-MAT 22 x 32 6.1 ms at 0.15 against 6.5 at 0.4.
         int64_t max_blk = 0;
         for (int32_t b = 0; b < nblk; b++)
-            max_blk = std::max(max_blk, bp[2 * (size_t)b + 2] - bp[2 * (size_t)b]);
+            max_blk = std::max(max_blk, bp[(size_t)b + 1] - bp[(size_t)b]);
         const bool no_hubs = (double)max_blk * nblk < 2.0 * (double)E;
         if (no_hubs) g->dense_all_frac = 0.4;
-        for (int32_t b = 0; b < nrun; b++)
+        for (int32_t b = 0; b < nblk; b++)
             bo[(size_t)b + 1] = bo[(size_t)b] +
                                 (bp[(size_t)b + 1] - bp[(size_t)b] + kBlkChunk - 1) / kBlkChunk * kBlkChunk;
-        if (g->light_thr != 0xFFFFFFFFu)
-            for (int32_t b = 0; b < nrun; b += 2)
-                g->light_edges += bp[(size_t)b + 1] - bp[(size_t)b];
         // Tile cap: 2^17 edges up to 2^29 edges, doubled while more than
         // kBlkTileCount tiles of the cap fit in the graph -- the 2.08 G-edge
         // R-MAT graph ran 50.9 GTEPS with 2^19-edge tiles, 46.7 with 2^17;
@@ -1217,64 +1360,37 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         int64_t tcap = kBlkTileEdges;
         while (tcap * kBlkTileCount < E) tcap <<= 1;
         g->b_off_host = bo;
-        const int64_t Ep = bo[(size_t)nrun];
+        const int64_t Ep = bo[(size_t)nblk];
         const int64_t nch = Ep / kBlkChunk;
         SSSP_HIP(hipMemcpyAsync(boff, bo.data(), 8 * bo.size(), hipMemcpyHostToDevice, s));
         // whole sources and destination offsets first, packed below
         int32_t *bs = dmalloc<int32_t>((size_t)Ep);
         uint16_t *bd = dmalloc<uint16_t>((size_t)Ep);
-        uint8_t *wflag = dmalloc<uint8_t>((size_t)nch);
-        int32_t *widx = dmalloc<int32_t>((size_t)nch);
         struct F4 {
-            void *p[4];
+            void *p[2];
             ~F4()
             {
                 for (void *x : p) dfree(x);
             }
-        } f4{{bs, bd, wflag, widx}};
+        } f4{{bs, bd}};
         g->b_w = dmalloc<uint32_t>((size_t)Ep);
         g->b_edges = Ep;
         k_blk_gather<<<grid_for(E), kBlock, 0, s>>>(bkeys, bperm, E, bptr, boff, g->el_src,
                                                     g->el_dst, g->el_w, bs, bd, g->b_w);
         SSSP_LAUNCH_CHECK("k_blk_gather");
-        k_blk_pad<<<grid_for((int64_t)nrun * kBlkChunk), kBlock, 0, s>>>(bptr, boff, nrun, bs, bd,
+        k_blk_pad<<<grid_for((int64_t)nblk * kBlkChunk), kBlock, 0, s>>>(bptr, boff, nblk, bs, bd,
                                                                          g->b_w);
         SSSP_LAUNCH_CHECK("k_blk_pad");
-        const unsigned chunk_grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
-        k_blk_chunk_wide<<<chunk_grid, kBlock, 0, s>>>(bs, nch, wflag);
-        SSSP_LAUNCH_CHECK("k_blk_chunk_wide");
-        std::vector<uint8_t> wf((size_t)nch);
-        SSSP_HIP(hipMemcpyAsync(wf.data(), wflag, (size_t)nch, hipMemcpyDeviceToHost, s));
-        SSSP_HIP(hipStreamSynchronize(s));
-        std::vector<int32_t> wi((size_t)nch);
-        int64_t nw = 0;
-        for (int64_t c = 0; c < nch; c++) wi[(size_t)c] = wf[(size_t)c] ? (int32_t)nw++ : -1;
-        SSSP_HIP(hipMemcpyAsync(widx, wi.data(), 4 * (size_t)nch, hipMemcpyHostToDevice, s));
-        g->b_pk = dmalloc<uint32_t>((size_t)Ep);
-        g->b_cbase = dmalloc<int32_t>((size_t)nch);
-        g->b_wide = nw ? dmalloc<int32_t>((size_t)(nw * kBlkChunk)) : nullptr;
-        g->b_nwide = nw;
-        k_blk_pack<<<chunk_grid, kBlock, 0, s>>>(bs, bd, widx, nch, g->b_pk, g->b_cbase, g->b_wide);
-        SSSP_LAUNCH_CHECK("k_blk_pack");
+        pack_chunks(bs, bd, nch, s, &g->b_pk, &g->b_cbase, &g->b_wide, &g->b_nwide);
         // source-range cuts of every block at 2^kBlkRangeFineBits granularity
         // (for tiles dispatched range by range), when the table is small
         const int64_t nfine = ((int64_t)V + (1 << kBlkRangeFineBits) - 1) >> kBlkRangeFineBits;
         if ((int64_t)nblk * (nfine + 1) <= kBlkRangeMaxEntries) {
-            const int64_t n_off = (int64_t)nrun * (nfine + 1);
-            int64_t *roff = dmalloc<int64_t>((size_t)n_off);
-            struct F1 {
-                void *p;
-                ~F1() { dfree(p); }
-            } f1{roff};
-            k_blk_range_offsets<<<grid_for(n_off), kBlock, 0, s>>>(bs, boff, nrun, kBlkRangeFineBits,
-                                                                  (int32_t)nfine, roff);
-            SSSP_LAUNCH_CHECK("k_blk_range_offsets");
-            g->b_ranges.off.resize((size_t)n_off);
-            SSSP_HIP(hipMemcpyAsync(g->b_ranges.off.data(), roff, 8 * (size_t)n_off,
-                                    hipMemcpyDeviceToHost, s));
+            range_cuts(bs, boff, nblk, (int32_t)nfine, s, &g->b_ranges.off);
             g->b_ranges.fine_bits = kBlkRangeFineBits;
             g->b_ranges.n_fine = (int32_t)nfine;
         }
+        build_light_list(g, bs, bd, boff, nblk, nch);
         SSSP_HIP(hipStreamSynchronize(s));
         // Without hubs the d[src] gathers of a tile spread over the whole
         // distance array (degree order cannot gather them), so a graph whose

@@ -93,27 +93,29 @@ struct BlkTile {
     int32_t blk;
     int32_t split;
     int64_t e0, e1;
-    int64_t f0, f1;  // second run of slots (f0 == f1: none)
 };
-// Weight classes of the blocked list. A block's run is its light edges
-// (weight at most the threshold, ascending sources, padded to whole chunks)
-// followed by its heavy ones; a light round relaxes the light edges alone.
-constexpr int kLightSample = 1 << 16;        // weights sampled for the threshold
+// Light list: the blocked list's light edges (weight at most a threshold)
+// once more, as a blocked list of their own with its own tiles, for the light
+// passes. (Keeping the classes apart in one list instead of copying the light
+// edges cost the passes over all edges 5-18 %, their gathers no longer sharing
+// lines: uniform 1 M x 16 2.26 -> 2.77 ms of plain passes.)
+constexpr int kLightSample = 1 << 12;        // weights sampled for the threshold
+constexpr double kLightMinDegree = 8;        // no light class on sparser graphs without hubs
 constexpr int64_t kLightTileMin = 1 << 12;   // edge slots of a light tile at least
 constexpr int64_t kLightTiles = 1024;        // ... and the tile count its cap aims at
 constexpr int kLightMaxPasses = 64;          // light passes stop after this many passes of a run
 constexpr double kLightStopFrac = 0.05;      // light passes stop once a pass lowers fewer than
                                              // this share of the vertices with out-edges
-// Source-range cuts of the blocked list's runs (host copy; run 2 b = block
-// b's light edges, 2 b + 1 its heavy ones): off[run *
-// (n_fine + 1) + k] = first slot of the run whose source is at least
+// Source-range cuts of the blocked list's block runs (host copy): off[b *
+// (n_fine + 1) + k] = first slot of block b whose source is at least
 // k << fine_bits, aligned down to its chunk (k = n_fine: the run's end).
-// Tiles cut at every stride-th cut (stride 0: no cuts).
+// Tiles cut at every stride-th cut (stride 0: no cuts). loff: the same for the
+// light list.
 constexpr int kBlkRangeFineBits = 18;
 constexpr int64_t kBlkRangeMaxEntries = (int64_t)1 << 22;
 constexpr int kBlkRangeMinVertexBits = 22;  // source ranges by default from 2^22 vertices
 struct BlkRanges {
-    std::vector<int64_t> off;
+    std::vector<int64_t> off, loff;
     int32_t fine_bits = 0;
     int32_t n_fine = 0;
     int32_t stride = 0;
@@ -184,12 +186,17 @@ struct sssp_graph {
     int32_t n_btile = 0;
     uint16_t *b_app = nullptr;  // dense rounds' append masks: kBlkThreads per tile
     bool frontier_bits = false;  // the coming round's frontier is in b_app, not yet queued
-    sssp::BlkTile *b_ltile = nullptr;  // tiles of the light edges (n_ltile 0: no weight classes)
+    // the light list (n_ltile 0: none), laid out as the blocked list
+    uint32_t *l_pk = nullptr;
+    int32_t *l_cbase = nullptr;
+    int32_t *l_wide = nullptr;
+    uint32_t *l_w = nullptr;
+    int64_t l_edges = 0, l_nwide = 0;
+    sssp::BlkTile *b_ltile = nullptr;
     int32_t n_ltile = 0;
-    int64_t light_edges = 0;      // edges in the light class
-    uint32_t light_thr = 0xFFFFFFFFu;  // largest weight pattern of the light class
-    std::vector<int64_t> b_off_host;  // padded run offsets, two runs per block (tiles are rebuilt
-                                      // from them)
+    int64_t light_edges = 0;      // edges in the light list
+    std::vector<int64_t> b_off_host;  // padded block offsets (tiles are rebuilt from them)
+    std::vector<int64_t> l_off_host;  // ... of the light list
     int64_t blk_tile_cap = 0;         // edges per tile at most
     int blk_tile_order = 0;           // dispatch order of the tiles (make_blk_tiles)
     sssp::BlkRanges b_ranges;         // source-range cuts of the block runs (may be empty)

@@ -930,8 +930,10 @@ def test_light_passes_bit_exact(gpu, oracle, case):
         w = rng.integers(1, 256, n).astype(np.uint32)
     elif case == "path":
         hop = np.arange(V, dtype=np.int32)[::-1].copy()  # against the ids: one hop a pass
-        src, dst = np.concatenate([hop[:400], src[:200]]), np.concatenate([hop[1:401], dst[:200]])
-        w = np.concatenate([rng.random(400, dtype=np.float32), np.full(200, 9, np.float32)])
+        hub = np.full(64, hop[0])  # sparse graphs have a light class only with hubs
+        src = np.concatenate([hop[:400], hub, src[:200]])
+        dst = np.concatenate([hop[1:401], hop[1000:1064], dst[:200]])
+        w = np.concatenate([rng.random(400, dtype=np.float32), np.full(264, 9, np.float32)])
     source = int(src[0])
     ref = oracle.dijkstra(src, dst, w, V, source)
     with S.DeviceGraph(src, dst, w, V) as g:
