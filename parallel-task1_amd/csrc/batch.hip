@@ -830,9 +830,13 @@ int sssp_solve_batch(sssp_graph *g, const int32_t *sources, int32_t n, int32_t p
                 : (policy == 3) ? Config{3, kMThreads, 1, 0.0, 0}
                                 : Config{2, 256, 2, g->push_edge_frac, g->push_chunk};
         const std::vector<int32_t> slots = source_slots(g, sources, n);
+        const size_t bytes = 4 * (size_t)n * (size_t)g->V;
+        Prefault pages(dist_out, bytes);
         const double ms = batch_sources(g, slots.data(), n, c);
-        if (dist_out)
-            SSSP_HIP(hipMemcpy(dist_out, g->bdist, 4 * (size_t)n * (size_t)g->V, hipMemcpyDeviceToHost));
+        if (dist_out) {
+            pages.join();
+            download(g, dist_out, g->bdist, bytes);
+        }
         fill_stats(stats, ms, (double)g->E * n);
         if (stats) stats->iterations = c.policy;
     });
@@ -927,9 +931,12 @@ int sssp_pack_solve(sssp_pack *p, const int32_t *sources, int32_t policy, float 
         Config c{p->policy ? p->policy : 1, p->bs, p->wgpcu, p->frac, p->push_chunk};
         if (policy == 1) c = Config{1, p->policy == 1 ? p->bs : 1024, p->policy == 1 ? p->wgpcu : 1, 0.05, 1};
         if (policy == 2) c = Config{2, 256, 2, p->policy == 2 ? p->frac : 0.05, p->policy == 2 ? p->push_chunk : 1};
+        Prefault pages(dist_out, 4 * (size_t)p->g->V);
         const double ms = pack_run(p, sources, c);
-        if (dist_out)
-            SSSP_HIP(hipMemcpy(dist_out, p->g->bdist, 4 * (size_t)p->g->V, hipMemcpyDeviceToHost));
+        if (dist_out) {
+            pages.join();
+            download(p->g, dist_out, p->g->bdist, 4 * (size_t)p->g->V);
+        }
         fill_stats(stats, ms, (double)p->g->E);
         if (stats) stats->iterations = c.policy;
     });

@@ -2,6 +2,9 @@
 // launch helpers. Internal to the library.
 #pragma once
 
+#include <atomic>
+#include <thread>
+
 #include "sssp_internal.hpp"
 
 namespace sssp {
@@ -135,6 +138,9 @@ struct MRec {
     int32_t loc;  // dst - block base
     int32_t pad;
 };
+
+constexpr int kStageBufs = 4;
+constexpr size_t kStageBytes = (size_t)4 << 20;
 
 struct TraceRow {
     int32_t mode;
@@ -330,6 +336,10 @@ struct sssp_graph {
     int64_t bscratch_elems = 0;
     int64_t bscratch_stride = 0;
 
+    // one per staging buffer of large results (the buffers are shared, see download)
+    hipEvent_t stage_ev[sssp::kStageBufs] = {};
+    uint8_t *dvis = nullptr;  // visited flags of a BFS (on demand)
+
     int64_t device_bytes = 0;
 
     // multi-source solves: device copy of the source list
@@ -395,6 +405,25 @@ __device__ inline int64_t block_excl_scan_i64(int64_t x, int64_t *total, int64_t
     *total = tot;
     return wpre + inc - x;
 }
+
+// capi.cpp
+// Device memory -> the caller's host buffer (the graph's stream is idle).
+void download(sssp_graph *g, void *dst, const void *src, size_t bytes);
+// Faults in a large host buffer's pages on helper threads while the GPU
+// solves (the first touch of fresh memory costs more than the copy into it);
+// its contents stay as they are. Joined by the destructor.
+class Prefault {
+  public:
+    Prefault(void *dst, size_t bytes);
+    ~Prefault();
+    Prefault(const Prefault &) = delete;
+    Prefault &operator=(const Prefault &) = delete;
+    void join();
+
+  private:
+    std::atomic<bool> go_{false};
+    std::vector<std::thread> threads_;
+};
 
 // gen.hip
 void rmat_device(int scale, int ef, int a, int b, int c, int d, uint32_t base_seed, int T,

@@ -963,3 +963,45 @@ def test_light_passes_bit_exact(gpu, oracle, case):
         d, st = g.solve(source, "plain")  # the plain schedule stays all-edge passes
         assert np.array_equal(bits(d), bits(ref))
         assert st["edges_relaxed"] == st["iterations"] * len(src)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [1 << 20, (1 << 20) + 1, 4 * (1 << 20) + 3, 5000011])
+def test_large_results_reach_the_host_whole(gpu, V):
+    """Results above 4 MB are staged through pinned buffers, 4 MB at a time,
+    into pages faulted in ahead: at the threshold, one word past it, and sizes
+    that end inside a buffer, into memory that starts off a page, every word
+    arrives and none beyond it is written. The same copies from two threads
+    at once (one of them finds the buffers taken) agree too."""
+    import threading
+
+    rng = np.random.default_rng(3)
+    src = rng.integers(0, V, 4 * V).astype(np.int32)
+    dst = rng.integers(0, V, 4 * V).astype(np.int32)
+    w = rng.random(4 * V, dtype=np.float32)
+    with S.DeviceGraph(src, dst, w, V, csc=False) as g, \
+            S.DeviceGraph(src[:V], dst[:V], w[:V], V, csc=False) as h:
+        ref, _ = g.solve(int(src[0]), "plain")
+        href, _ = h.solve(int(src[0]), "plain")
+        # the fixpoint itself, in numpy: no edge can lower a distance
+        ok = ref[src] < S.F32_INF
+        assert ref[src[0]] == 0 and not np.any(ref[src[ok]] + w[ok] < ref[dst[ok]])
+        room = np.full(V + 64, 7, np.float32)
+        out = room[1:1 + V]
+        S._check(S.lib().sssp_get_distances(g.handle, S._ptr(out)))
+        assert np.array_equal(bits(out), bits(ref))
+        assert (room[0] == 7) and (room[1 + V:] == 7).all()
+        got = {}
+
+        def fetch(graph, key):
+            for k in range(4):
+                got[key, k] = graph.distances()
+
+        ts = [threading.Thread(target=fetch, args=a) for a in ((g, "g"), (h, "h"))]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        for k in range(4):
+            assert np.array_equal(bits(got["g", k]), bits(ref))
+            assert np.array_equal(bits(got["h", k]), bits(href))
