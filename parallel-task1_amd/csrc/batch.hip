@@ -16,13 +16,15 @@
 //   256 sources are one array D[v * n + s], so a vertex's distances are one
 //   contiguous row. All-edge passes over the edges sorted by 16-vertex
 //   destination block: a 256-thread workgroup (thread s = source s) holds its
-//   block's 16 x 256 distances in LDS, reads each edge record once for all its
+//   block's 16 x 256 minima in LDS, reads each edge record once for all its
 //   sources (a wave-uniform load), gathers the source vertex's row (coalesced,
-//   eight rows in flight)
+//   eight rows in flight) unless no source lowered it since the record was
+//   last relaxed,
 //   and lowers its own LDS column -- no atomics inside a block; the block is
 //   written back at the end (atomicMin for blocks split over several tiles).
-//   Passes run until one changes nothing, the plain Bellman-Ford fixpoint of
-//   every source; the rows are then transposed into the per-source output.
+//   Passes over the light edges alone alternate with full ones until a full
+//   pass changes nothing, the Bellman-Ford fixpoint of every source; the rows
+//   are then transposed into the per-source output.
 // The autotuner times block size x workgroups per CU for policy 1, frontier
 // threshold x push chunk width for policy 2, and policy 3, and keeps the
 // fastest.
@@ -353,101 +355,210 @@ double batch_sources(sssp_graph *g, const int32_t *sources, int32_t n, const Con
 constexpr int kMThreads = 256;  // sources per chunk: one thread per source
 constexpr int kMBlock = 1 << kMBits;
 
-// One tile of a vertex-major pass: thread s holds source s's distances of
-// the tile's 16-vertex destination block in its LDS column, lowers them with
-// the tile's records (a record's source row gathered for all sources at
-// once), and writes back what it lowered. Returns whether this lane lowered a
-// distance.
+// Pass state on the device: what each pass ran, whether it lowered anything,
+// an estimate of how many rows it lowered (one wave in MultiArgs::every counts:
+// one addition per wave to one counter, from 200 thousand waves, took 1.8 ms of
+// every light pass at R-MAT scale 20), the last full pass before each, and
+// the number of the first pass of the captured run.
+struct MultiCtl {
+    int32_t kind[64];
+    int32_t changed[64];
+    int32_t low[64];
+    int32_t full[64];
+    int32_t base;
+};
+enum { kMultiLight = 1, kMultiFull = 2, kMultiIdle = 3 };
+
+// One tile of a vertex-major pass: thread s holds source s's minima for the
+// tile's 16-vertex destination block in its LDS column, lowers them with the
+// tile's records (a record's source row gathered for all sources at once), and
+// writes back what is below the distances in global memory. A record is
+// relaxed only when its source's row was lowered in pass `since` or later
+// (stamp): before that, its list was last relaxed against the row as it still
+// is. Rows the tile lowers are stamped with this pass. Returns the rows this
+// wave lowered.
+// A wave takes 64 records at a time, one per lane: their stamps are one gather,
+// the live ones a ballot, and each live record is broadcast from its lane. The
+// next 64 records' stamps and the records after those load under this group's
+// row gathers. (With a record per step in scalar registers each step waited
+// for its records and then for their stamps: a pass took as long as relaxing
+// every record.)
 template <class WT>
-__device__ __forceinline__ bool multi_tile(const BlkTile &t, const MRec *__restrict__ rec,
-                                           uint32_t *D, int32_t n, int64_t V,
-                                           uint32_t (&ld)[kMBlock][kMThreads])
+__device__ __forceinline__ int multi_tile(const BlkTile &t, const MRec *__restrict__ rec,
+                                          uint32_t *D, int32_t n, int32_t *stamp, int32_t since,
+                                          int32_t pass, uint32_t (&ld)[kMBlock][kMThreads])
 {
     constexpr uint32_t INF = WT::INF;
-    const int s = threadIdx.x;
+    const int s = threadIdx.x, lane = __lane_id();
     const bool act = s < n;
     const int64_t base = (int64_t)t.blk << kMBits;
-    const int nb = (int)min((int64_t)kMBlock, V - base);
     // each thread touches only its own column: no barrier is needed
-    for (int v = 0; v < nb; v++) ld[v][s] = act ? D[(base + v) * n + s] : INF;
-    auto relax = [&](const MRec &r, uint32_t du) {
-        if (du == INF) return;
-        const uint32_t cand = WT::add(du, r.w);
-        if (cand < ld[r.loc][s]) ld[r.loc][s] = cand;
+#pragma unroll
+    for (int v = 0; v < kMBlock; v++) ld[v][s] = INF;
+    struct Rec {
+        int32_t src, loc;
+        uint32_t w;
     };
-    int64_t e = t.e0;
-    // eight records at a time: their row gathers are in flight together.
-    // Measured at R-MAT scale 20 x 256 sources (GTEPS): 64-vertex blocks (64
-    // KB of LDS, 2 waves per SIMD) 23.0 with 8 in flight, 25.8-27.4 with 16;
-    // 32-vertex blocks 44.0 (16); 16-vertex blocks (16 KB, 8 workgroups per
-    // CU) 51.4 (16), 54.7 (8); 8-vertex blocks 51.1 (16)
-    constexpr int R = 8;
-    MRec r[R];
-    if (e + R <= t.e1) {
-#pragma unroll
-        for (int k = 0; k < R; k++) r[k] = rec[e + k];
-    }
-    for (; e + R <= t.e1; e += R) {
-        uint32_t du[R];
-#pragma unroll
-        for (int k = 0; k < R; k++) du[k] = act ? D[(int64_t)r[k].src * n + s] : INF;
-        // the next step's records load under this step's gathers
-        MRec rn[R];
-        if (e + 2 * R <= t.e1) {
-#pragma unroll
-            for (int k = 0; k < R; k++) rn[k] = rec[e + R + k];
+    auto fetch = [&](int64_t e) {
+        Rec r{0, 0, 0u};
+        if (e < t.e1) {
+            const MRec m = rec[e];
+            r = Rec{m.src, m.loc, m.w};
         }
+        return r;
+    };
+    auto mark = [&](int64_t e, const Rec &r) { return e < t.e1 ? stamp[r.src] : since - 1; };
+    const uint32_t *const Ds = D + s;
+    auto row = [&](const Rec &r, int i) {  // of lane i's record, this thread's source
+        const int32_t u = __builtin_amdgcn_readlane(r.src, i);
+        return act ? Ds[(int64_t)u * n] : INF;
+    };
+    auto relax = [&](const Rec &r, int i, uint32_t du) {
+        const uint32_t w = __builtin_amdgcn_readlane(r.w, i);
+        const int32_t loc = __builtin_amdgcn_readlane(r.loc, i);
+        if (du == INF) return;
+        const uint32_t cand = WT::add(du, w);
+        if (cand < ld[loc][s]) ld[loc][s] = cand;
+    };
+    bool any = false;
+    Rec r0 = fetch(t.e0 + lane), r1 = fetch(t.e0 + 64 + lane);
+    int32_t st = mark(t.e0 + lane, r0);
+    for (int64_t e = t.e0; e < t.e1; e += 64) {
+        uint64_t m = __ballot(st >= since);
+        const Rec r2 = fetch(e + 128 + lane);
+        const int32_t st1 = mark(e + 64 + lane, r1);
+        any |= m != 0;
+        // eight row gathers in flight. Measured at R-MAT scale 20 x 256
+        // sources (GTEPS, all records live): 64-vertex blocks (64
+        // KB of LDS, 2 waves per SIMD) 23.0 with 8 in flight, 25.8-27.4 with 16;
+        // 32-vertex blocks 44.0 (16); 16-vertex blocks (16 KB, 8 workgroups per
+        // CU) 51.4 (16), 54.7 (8); 8-vertex blocks 51.1 (16)
+        constexpr int R = 8;
+        while (m != 0) {
+            int at[R];
+            uint32_t du[R];
+            int k = 0;
 #pragma unroll
-        for (int k = 0; k < R; k++) relax(r[k], du[k]);
-#pragma unroll
-        for (int k = 0; k < R; k++) r[k] = rn[k];
-    }
-    for (; e < t.e1; e++) {
-        const MRec r = rec[e];
-        relax(r, act ? D[(int64_t)r.src * n + s] : INF);
-    }
-    bool low = false;
-    if (act) {
-        for (int v = 0; v < nb; v++) {
-            const uint32_t nv = ld[v][s];
-            const int64_t idx = (base + v) * n + s;
-            if (nv < D[idx]) {
-                if (t.split)
-                    __hip_atomic_fetch_min(&D[idx], nv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                else
-                    D[idx] = nv;  // only this workgroup writes the block
-                low = true;
+            for (int q = 0; q < R; q++) {
+                at[q] = m != 0 ? __builtin_ctzll(m) : at[q > 0 ? q - 1 : 0];
+                if (m != 0) k = q + 1;
+                m &= m - 1;
             }
+#pragma unroll
+            for (int q = 0; q < R; q++)
+                if (q < k) du[q] = row(r0, at[q]);
+#pragma unroll
+            for (int q = 0; q < R; q++)
+                if (q < k) relax(r0, at[q], du[q]);
+        }
+        r0 = r1;
+        r1 = r2;
+        st = st1;
+    }
+    if (!any) return 0;  // wave-uniform
+    // the touched rows' distances, all in flight together (a minimum is INF past
+    // the end, and where nothing was relaxed into it)
+    int rows = 0;
+    uint32_t cur[kMBlock];
+#pragma unroll
+    for (int v = 0; v < kMBlock; v++) {
+        cur[v] = 0u;
+        if (ld[v][s] != INF) cur[v] = D[(base + v) * n + s];
+    }
+#pragma unroll
+    for (int v = 0; v < kMBlock; v++) {
+        const uint32_t nv = ld[v][s];
+        const bool low = nv < cur[v];
+        if (low) {
+            uint32_t *const p = &D[(base + v) * n + s];
+            if (t.split)
+                __hip_atomic_fetch_min(p, nv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else
+                *p = nv;  // only this workgroup writes the block
+        }
+        if (__ballot(low) != 0) {
+            rows++;
+            if (lane == 0) stamp[base + v] = pass;
         }
     }
-    return low;
+    return rows;
 }
 
-// One pass per launch, one workgroup per tile. The pass number is base[0] +
-// k (base in device memory, so a captured run of passes is replayed as the
-// next run); pass p zeroes the flag pass p+1 sets and returns at once when
-// pass p-1 changed nothing.
-template <class WT>
-__global__ __launch_bounds__(kMThreads) void k_multi_pass(const BlkTile *__restrict__ tiles,
-                                                          const MRec *__restrict__ rec,
-                                                          uint32_t *D, int32_t n, int64_t V,
-                                                          int32_t *changed, const int32_t *base,
-                                                          int32_t k)
+struct MultiArgs {
+    const BlkTile *tile, *ltile;  // of all records, of the light ones
+    const MRec *rec, *lrec;
+    int32_t n_tile, n_ltile;  // n_ltile 0: full passes only
+    uint32_t *D;
+    int32_t n;
+    int64_t V;
+    int32_t *stamp;
+    MultiCtl *ctl;
+    int32_t every;       // a power of two: blocks whose hash is 0 modulo it count their rows
+    int32_t light_stop;  // light passes go on while their count is this much, or more than
+                         // the light pass before
+};
+
+// What pass p (from 1) runs; every workgroup reads the same values.
+__device__ __forceinline__ int multi_kind(const MultiArgs &a, int32_t p)
 {
-    const int32_t pass = *base + k;
-    if (blockIdx.x == 0 && threadIdx.x == 0) changed[(pass + 1) & 63] = 0;
-    if (pass > 0 && __hip_atomic_load(&changed[(pass - 1) & 63], __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT) == 0)
-        return;
-    __shared__ uint32_t ld[kMBlock][kMThreads];
-    const bool low = multi_tile<WT>(tiles[blockIdx.x], rec, D, n, V, ld);
-    if (__ballot(low) != 0 && __lane_id() == 0) changed[pass & 63] = 1;
+    if (p == 1) return a.n_ltile > 0 ? kMultiLight : kMultiFull;
+    const MultiCtl *c = a.ctl;
+    const int i1 = (p - 1) & 63, i2 = (p - 2) & 63;
+    const int prev = c->kind[i1];
+    const int32_t low = c->low[i1];
+    if (prev == kMultiIdle) return kMultiIdle;
+    if (prev == kMultiFull) {
+        if (c->changed[i1] == 0) return kMultiIdle;
+        // few rows lowered: the stamps make another full pass cheap
+        return a.n_ltile > 0 && low >= a.light_stop && p < kLightMaxPasses ? kMultiLight
+                                                                           : kMultiFull;
+    }
+    const int32_t before = p > 2 && c->kind[i2] == kMultiLight ? c->low[i2] : 0;
+    return (low >= a.light_stop || low > before) && low > 0 && p < kLightMaxPasses ? kMultiLight
+                                                                                   : kMultiFull;
 }
 
-// D[v * n + s] = INF, D[sources[s] * n + s] = 0
+// One pass per launch, one workgroup per tile. The pass number is the run's
+// base + k (base in device memory, so a captured run of passes is replayed as
+// the next run). As the blocked passes of a single solve, a pass finds out
+// what it runs from the pass before it: light passes (the light records alone)
+// until they lower few rows, a full pass, light passes again, until a full pass
+// lowers nothing; passes after that return at once. R-MAT 20 x 16, 256 sources:
+// 21 passes over every record took 72.6 ms; now two full passes of 2.9 ms (17 GB
+// of row gathers at 6 TB/s), 24 light ones of 0.3 ms and a few full ones over the
+// few rows still changing, 15.4 ms in all.
+template <class WT>
+__global__ __launch_bounds__(kMThreads) void k_multi_pass(const MultiArgs a, int32_t k)
+{
+    MultiCtl *c = a.ctl;
+    const int32_t pass = c->base + k;
+    const int kind = multi_kind(a, pass);
+    const int32_t last_full = pass == 1 ? 0 : c->full[(pass - 1) & 63];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c->kind[pass & 63] = kind;
+        c->full[pass & 63] = kind == kMultiFull ? pass : last_full;
+        c->low[(pass + 1) & 63] = 0;
+        c->changed[(pass + 1) & 63] = 0;
+    }
+    if (kind == kMultiIdle) return;
+    const bool light = kind == kMultiLight;
+    if ((int)blockIdx.x >= (light ? a.n_ltile : a.n_tile)) return;
+    __shared__ uint32_t ld[kMBlock][kMThreads];
+    const BlkTile t = (light ? a.ltile : a.tile)[blockIdx.x];
+    const int rows = multi_tile<WT>(t, light ? a.lrec : a.rec, a.D, a.n, a.stamp,
+                                    light ? pass - 1 : last_full, pass, ld);
+    if (rows != 0 && __lane_id() == 0) {
+        c->changed[pass & 63] = 1;
+        if ((((uint32_t)t.blk * 0x9E3779B1u) >> 16 & (uint32_t)(a.every - 1)) == 0)
+            atomicAdd(&c->low[pass & 63], rows);
+    }
+}
+
+// D[v * n + s] = INF, D[sources[s] * n + s] = 0; stamps: -1 (never lowered),
+// k_multi_sources sets the sources'
 template <class WT>
 __global__ __launch_bounds__(kBlock) void k_multi_init(uint32_t *D, int32_t n, int64_t V,
-                                                       const int32_t *sources)
+                                                       const int32_t *sources, int32_t *stamp)
 {
     const int64_t total = V * n;
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < total;
@@ -455,6 +566,18 @@ __global__ __launch_bounds__(kBlock) void k_multi_init(uint32_t *D, int32_t n, i
         const int64_t v = i / n;
         const int32_t s = (int32_t)(i - v * n);
         D[i] = sources[s] == v ? 0u : WT::INF;
+        if (s == 0) stamp[v] = -1;
+    }
+}
+
+// the sources' rows count as lowered before the first pass; first pass: 1
+__global__ void k_multi_sources(const int32_t *sources, int32_t n, int32_t *stamp, MultiCtl *c)
+{
+    for (int i = threadIdx.x; i < n; i += blockDim.x) stamp[sources[i]] = 0;
+    if (threadIdx.x == 0) {
+        c->base = 1;
+        c->low[1] = 0;
+        c->changed[1] = 0;
     }
 }
 
@@ -480,31 +603,60 @@ __global__ __launch_bounds__(kBlock) void k_multi_out(const uint32_t *D, int32_t
     }
 }
 
-__global__ void k_zero_words(int32_t *p, int32_t n)
-{
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
-}
-
 // base[0] += k (the next run of captured passes)
 __global__ void k_advance_base(int32_t *base, int32_t k)
 {
     if (threadIdx.x == 0) base[0] += k;
 }
 
+// Light passes stop once they lower fewer rows than this share of the vertices
+// with out-edges: 0.02 / 0.05 / 0.1 / 0.2 took 17.2 / 17.1 / 15.4 / 17.1 ms at
+// R-MAT 20 x 16 with 256 sources (the stamps keep the next full pass cheap).
+constexpr double kMultiStopFrac = 0.1;
 constexpr int32_t kMultiRun = 32;  // passes per captured run (the flag ring has 64)
 
-template <class WT>
-void launch_multi_passes(sssp_graph *g, int32_t m, hipStream_t s)
+MultiArgs multi_args(sssp_graph *g, int32_t m)
 {
-    for (int32_t k = 0; k < kMultiRun; k++)
-        k_multi_pass<WT><<<(unsigned)g->n_mtile, kMThreads, 0, s>>>(
-            g->m_tile, g->m_rec, g->mdist, m, g->V, g->mflags, g->mflags + 64, k);
+    MultiArgs a{};
+    a.tile = g->m_tile;
+    a.ltile = g->m_ltile;
+    a.rec = g->m_rec;
+    a.lrec = g->m_lrec;
+    a.n_tile = g->n_mtile;
+    a.n_ltile = g->n_mltile;
+    a.D = g->mdist;
+    a.n = m;
+    a.V = g->V;
+    a.stamp = g->mstamp;
+    a.ctl = static_cast<MultiCtl *>(g->mctl);
+    a.every = 1;
+    // about 2048 blocks count; rows once per wave that lowers them
+    while (a.every < 1 << 15 && (g->V >> kMBits) / (2 * a.every) >= 2048) a.every *= 2;
+    a.light_stop = (int32_t)std::min<double>(
+        kMultiStopFrac * g->n_nzo * ((m + 63) / 64) / a.every, 1 << 30);
+    return a;
+}
+
+void launch_multi_pass(sssp_graph *g, const MultiArgs &a, int32_t k, hipStream_t s)
+{
+    const unsigned grid = (unsigned)std::max(a.n_tile, a.n_ltile);
+    if (g->wtype == SSSP_W_U32) k_multi_pass<WU32><<<grid, kMThreads, 0, s>>>(a, k);
+    else k_multi_pass<WF32><<<grid, kMThreads, 0, s>>>(a, k);
+}
+
+void launch_multi_init(sssp_graph *g, const MultiArgs &a, const int32_t *sources, hipStream_t s)
+{
+    const int64_t V = g->V;
+    const unsigned gi = (unsigned)std::min<int64_t>((V * a.n + kBlock - 1) / kBlock, 65536);
+    if (g->wtype == SSSP_W_U32)
+        k_multi_init<WU32><<<gi, kBlock, 0, s>>>(a.D, a.n, V, sources, a.stamp);
+    else k_multi_init<WF32><<<gi, kBlock, 0, s>>>(a.D, a.n, V, sources, a.stamp);
+    k_multi_sources<<<1, kBlock, 0, s>>>(sources, a.n, a.stamp, a.ctl);
 }
 
 // The captured launches of one chunk of at most 256 sources, keyed on chunk
-// shape and buffers: `first` clears the change flags and the pass base with a
-// kernel, initialises the vertex-major distances, runs kMultiRun passes and
-// transposes the result into the per-source output; `more` advances the pass
+// shape and buffers: `first` initialises the vertex-major distances, the stamps
+// and the pass state, runs kMultiRun passes and transposes the result into the per-source output; `more` advances the pass
 // base by kMultiRun and runs the next kMultiRun passes and the transpose.
 // Passes after the fixpoint return at once.
 struct MultiGraphs {
@@ -518,7 +670,7 @@ MultiGraphs multi_graphs(sssp_graph *g, int32_t c0, int32_t m)
                                     c0,
                                     V,
                                     g->n_mtile,
-                                    (int64_t)(uintptr_t)g->mflags,
+                                    (int64_t)(uintptr_t)g->mctl,
                                     (int64_t)(uintptr_t)g->mdist,
                                     (int64_t)(uintptr_t)g->bdist,
                                     (int64_t)(uintptr_t)g->msrc,
@@ -536,22 +688,17 @@ MultiGraphs multi_graphs(sssp_graph *g, int32_t c0, int32_t m)
         }
     hipStream_t s = g->stream;
     SSSP_HIP(hipStreamSynchronize(s));
-    const bool u32 = g->wtype == SSSP_W_U32;
-    const unsigned gi = (unsigned)std::min<int64_t>((V * m + kBlock - 1) / kBlock, 65536);
+    const MultiArgs a = multi_args(g, m);
     for (int j = 0; j < 2; j++) {
         hipGraph_t graph;
         SSSP_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         if (j == 0) {
-            k_zero_words<<<1, 128, 0, s>>>(g->mflags, 65);
-            if (u32) k_multi_init<WU32><<<gi, kBlock, 0, s>>>(g->mdist, m, V, g->msrc + c0);
-            else k_multi_init<WF32><<<gi, kBlock, 0, s>>>(g->mdist, m, V, g->msrc + c0);
+            launch_multi_init(g, a, g->msrc + c0, s);
         } else {
-            k_advance_base<<<1, 64, 0, s>>>(g->mflags + 64, kMultiRun);
+            k_advance_base<<<1, 64, 0, s>>>(&a.ctl->base, kMultiRun);
         }
-        if (g->n_mtile > 0) {
-            if (u32) launch_multi_passes<WU32>(g, m, s);
-            else launch_multi_passes<WF32>(g, m, s);
-        }
+        if (g->n_mtile > 0)
+            for (int32_t k = 0; k < kMultiRun; k++) launch_multi_pass(g, a, k, s);
         k_multi_out<<<dim3((unsigned)((V + 63) / 64), (unsigned)((m + 63) / 64)), kBlock, 0, s>>>(
             g->mdist, m, V, g->vperm, g->bdist + (int64_t)c0 * V);
         const hipError_t le = hipGetLastError();
@@ -571,34 +718,38 @@ MultiGraphs multi_graphs(sssp_graph *g, int32_t c0, int32_t m)
     return MultiGraphs{(hipGraphExec_t)g->mexec[slot][0], (hipGraphExec_t)g->mexec[slot][1]};
 }
 
+// Passes among [first, first + count) that did work, from the host's copy of
+// what they ran; *done: one of them was idle (the fixpoint was reached).
+int32_t multi_ran(const int32_t *kind, int32_t first, int32_t count, bool *done)
+{
+    for (int32_t i = 0; i < count; i++)
+        if (kind[(first + i) & 63] == kMultiIdle) {
+            *done = true;
+            return i;
+        }
+    return count;
+}
+
 // Passes of one chunk as queued launches (batch_capture = 0): four at a time,
-// the host reading the change flags after each four.
-int32_t multi_passes_launched(sssp_graph *g, int32_t m)
+// the host reading what they ran after each four. Returns the passes run.
+int32_t multi_passes_launched(sssp_graph *g, const MultiArgs &a)
 {
     hipStream_t s = g->stream;
-    const int64_t V = g->V;
-    int32_t *changed = g->mflags;
-    k_zero_words<<<1, 128, 0, s>>>(changed, 65);
-    int32_t pass = 0, done_at = -1;
-    while (done_at < 0 && g->n_mtile > 0) {
+    int32_t ran = 0;
+    bool done = g->n_mtile == 0;
+    while (!done) {
         for (int i = 0; i < 4; i++) {
-            if (g->wtype == SSSP_W_U32)
-                k_multi_pass<WU32><<<(unsigned)g->n_mtile, kMThreads, 0, s>>>(
-                    g->m_tile, g->m_rec, g->mdist, m, V, changed, changed + 64, pass + i);
-            else
-                k_multi_pass<WF32><<<(unsigned)g->n_mtile, kMThreads, 0, s>>>(
-                    g->m_tile, g->m_rec, g->mdist, m, V, changed, changed + 64, pass + i);
+            launch_multi_pass(g, a, ran + i, s);
             SSSP_LAUNCH_CHECK("k_multi_pass");
         }
-        SSSP_HIP(hipMemcpyAsync(g->ctrl_host->changed, changed, 4 * 64, hipMemcpyDeviceToHost, s));
+        SSSP_HIP(hipMemcpyAsync(g->ctrl_host->changed, a.ctl->kind, 4 * 64, hipMemcpyDeviceToHost,
+                                s));
         SSSP_HIP(hipStreamSynchronize(s));
-        for (int i = 0; i < 4 && done_at < 0; i++)
-            if (g->ctrl_host->changed[(pass + i) & 63] == 0) done_at = pass + i;
-        pass += 4;
-        if (done_at < 0 && pass > g->V + 4)
+        ran += multi_ran(g->ctrl_host->changed, ran + 1, 4, &done);
+        if (!done && ran > (int64_t)g->V + 4 + kLightMaxPasses)
             throw Error{SSSP_ERR_NOT_CONVERGED, "multi-source passes exceeded V passes"};
     }
-    return done_at + 1;
+    return ran;
 }
 
 double run_multi(sssp_graph *g, const int32_t *sources, int32_t n)
@@ -619,7 +770,8 @@ double run_multi(sssp_graph *g, const int32_t *sources, int32_t n)
         g->msrc = dmalloc<int32_t>((size_t)n);
         g->msrc_cap = n;
     }
-    if (!g->mflags) g->mflags = dmalloc<int32_t>(65);  // 64 change flags, the pass base
+    if (!g->mctl) g->mctl = dmalloc<MultiCtl>(1);
+    if (!g->mstamp) g->mstamp = dmalloc<int32_t>((size_t)V);
     SSSP_HIP(hipMemcpyAsync(g->msrc, sources, 4 * (size_t)n, hipMemcpyHostToDevice, s));
     float total = 0.f;
     g->multi_passes = 0;
@@ -628,38 +780,29 @@ double run_multi(sssp_graph *g, const int32_t *sources, int32_t n)
         if (g->batch_capture) {
             const MultiGraphs mg = multi_graphs(g, c0, m);
             SSSP_HIP(hipEventRecord(g->ev_a, s));
-            int32_t done_at = -1;
-            // replay until a run holds a pass that changed nothing (at most
-            // V + 1 passes, as the pass loop)
-            for (int32_t run = 0; done_at < 0; run++) {
-                if (g->n_mtile == 0) {
-                    SSSP_HIP(hipGraphLaunch(mg.first, s));
-                    done_at = 0;
-                    break;
-                }
-                if ((int64_t)run * kMultiRun > V + 1)
+            bool done = g->n_mtile == 0;
+            if (done) SSSP_HIP(hipGraphLaunch(mg.first, s));
+            // replay until a run holds an idle pass (at most V + 1 passes and the
+            // light ones, as the pass loop)
+            for (int32_t run = 0; !done; run++) {
+                if ((int64_t)run * kMultiRun > V + 1 + kLightMaxPasses)
                     throw Error{SSSP_ERR_NOT_CONVERGED, "multi-source passes exceeded V passes"};
                 SSSP_HIP(hipGraphLaunch(run == 0 ? mg.first : mg.more, s));
-                SSSP_HIP(hipMemcpyAsync(g->ctrl_host->changed, g->mflags, 4 * 64,
+                SSSP_HIP(hipMemcpyAsync(g->ctrl_host->changed,
+                                        static_cast<MultiCtl *>(g->mctl)->kind, 4 * 64,
                                         hipMemcpyDeviceToHost, s));
                 SSSP_HIP(hipStreamSynchronize(s));
-                for (int32_t i = 0; i < kMultiRun && done_at < 0; i++) {
-                    const int32_t p = run * kMultiRun + i;
-                    if (g->ctrl_host->changed[p & 63] == 0) done_at = p;
-                }
+                g->multi_passes +=
+                    multi_ran(g->ctrl_host->changed, 1 + run * kMultiRun, kMultiRun, &done);
             }
             SSSP_HIP(hipEventRecord(g->ev_b, s));
             SSSP_HIP(hipEventSynchronize(g->ev_b));
-            g->multi_passes += done_at + 1;
         } else {
             SSSP_HIP(hipEventRecord(g->ev_a, s));
-            const unsigned gi = (unsigned)std::min<int64_t>((V * m + kBlock - 1) / kBlock, 65536);
-            if (g->wtype == SSSP_W_U32)
-                k_multi_init<WU32><<<gi, kBlock, 0, s>>>(g->mdist, m, V, g->msrc + c0);
-            else
-                k_multi_init<WF32><<<gi, kBlock, 0, s>>>(g->mdist, m, V, g->msrc + c0);
+            const MultiArgs a = multi_args(g, m);
+            launch_multi_init(g, a, g->msrc + c0, s);
             SSSP_LAUNCH_CHECK("k_multi_init");
-            g->multi_passes += multi_passes_launched(g, m);
+            g->multi_passes += multi_passes_launched(g, a);
             k_multi_out<<<dim3((unsigned)((V + 63) / 64), (unsigned)((m + 63) / 64)), kBlock, 0,
                           s>>>(g->mdist, m, V, g->vperm, g->bdist + (int64_t)c0 * V);
             SSSP_LAUNCH_CHECK("k_multi_out");

@@ -451,23 +451,63 @@ __global__ __launch_bounds__(kBlock) void k_blk_pack(const int32_t *bs, const ui
     if (__lane_id() == 0) cbase[c] = wi < 0 ? s[0] : -(1 + wi);
 }
 
-// Light edges of one chunk of the blocked list (one wave, 4 slots per lane):
+// Light edges of chunk c of a list of n weights (one wave, 4 slots per lane):
 // bit k of the result is set when the lane's slot k holds a light edge.
-__device__ __forceinline__ int chunk_light(const uint32_t *bw, int64_t c, uint32_t thr)
+__device__ __forceinline__ int chunk_light(const uint32_t *w, int64_t n, int64_t c, uint32_t thr)
 {
     typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-    const v4u v = reinterpret_cast<const v4u *>(bw)[c * (kBlkChunk / 4) + __lane_id()];
-    return (v.x <= thr ? 1 : 0) | (v.y <= thr ? 2 : 0) | (v.z <= thr ? 4 : 0) |
-           (v.w <= thr ? 8 : 0);
+    const int64_t e = c * kBlkChunk + 4 * __lane_id();
+    if (e + 4 <= n) {
+        const v4u v = *reinterpret_cast<const v4u *>(w + e);
+        return (v.x <= thr ? 1 : 0) | (v.y <= thr ? 2 : 0) | (v.z <= thr ? 4 : 0) |
+               (v.w <= thr ? 8 : 0);
+    }
+    int m = 0;
+    for (int k = 0; k < 4; k++)
+        if (e + k < n && w[e + k] <= thr) m |= 1 << k;
+    return m;
 }
 
-__global__ __launch_bounds__(kBlock) void k_light_count(const uint32_t *bw, int64_t nch,
+// light edges of each lane before this one, over the wave
+__device__ __forceinline__ int light_before(int m)
+{
+    int inc = __popc(m);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o);
+        if (__lane_id() >= o) inc += y;
+    }
+    return inc - __popc(m);
+}
+
+__global__ __launch_bounds__(kBlock) void k_light_count(const uint32_t *w, int64_t n, int64_t nch,
                                                         uint32_t thr, int64_t *cnt)
 {
     const int64_t c = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
     if (c >= nch) return;  // wave-uniform
-    const int n = wave_sum32(__popc(chunk_light(bw, c, thr)));
-    if (__lane_id() == 0) cnt[c] = n;
+    const int k = wave_sum32(__popc(chunk_light(w, n, c, thr)));
+    if (__lane_id() == 0) cnt[c] = k;
+}
+
+// The light edges of an edge list of n edges, in order (pos: light edges before
+// each chunk).
+__global__ __launch_bounds__(kBlock) void k_light_select(const int32_t *src, const int32_t *dst,
+                                                         const uint32_t *w, int64_t n, int64_t nch,
+                                                         uint32_t thr, const int64_t *pos,
+                                                         int32_t *ls, int32_t *ld, uint32_t *lw)
+{
+    const int64_t c = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+    if (c >= nch) return;  // wave-uniform
+    const int m = chunk_light(w, n, c, thr);
+    int64_t o = pos[c] + light_before(m);
+    for (int k = 0; k < 4; k++) {
+        if (!((m >> k) & 1)) continue;
+        const int64_t e = c * kBlkChunk + 4 * __lane_id() + k;
+        ls[o] = src[e];
+        ld[o] = dst[e];
+        lw[o] = w[e];
+        o++;
+    }
 }
 
 // out[b] = pos[boff[b] / kBlkChunk]: light edges before block b (nblk + 1 values)
@@ -491,20 +531,14 @@ __global__ __launch_bounds__(kBlock) void k_light_gather(const int32_t *bs, cons
 {
     const int64_t c = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
     if (c >= nch) return;  // wave-uniform
-    const int m = chunk_light(bw, c, thr);
+    const int m = chunk_light(bw, nch * kBlkChunk, c, thr);
     int32_t lo = 0, hi = nblk - 1;  // the chunk's block: the last with boff <= its first slot
     while (lo < hi) {
         const int32_t mid = (lo + hi + 1) >> 1;
         if (boff[mid] <= c * kBlkChunk) lo = mid;
         else hi = mid - 1;
     }
-    int inc = __popc(m);  // inclusive scan of the counts over the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(inc, o);
-        if (__lane_id() >= o) inc += y;
-    }
-    int64_t o = loff[lo] + (pos[c] - lptr[lo]) + inc - __popc(m);
+    int64_t o = loff[lo] + (pos[c] - lptr[lo]) + light_before(m);
     for (int k = 0; k < 4; k++) {
         if (!((m >> k) & 1)) continue;
         const int64_t e = c * kBlkChunk + 4 * __lane_id() + k;
@@ -773,16 +807,18 @@ void split_records(const uint32_t *rec, int64_t n, int32_t *src, int32_t *dst, u
     SSSP_LAUNCH_CHECK("k_split_records");
 }
 
-void build_multi_layout(sssp_graph *g)
+// Multi-source records of an edge list of n edges sorted by source (device
+// arrays): sorted by destination block, sources ascending within one, and the
+// tiles over them.
+static void build_records(sssp_graph *g, const int32_t *src, const int32_t *dst, const uint32_t *w,
+                          int64_t n, MRec **rec_out, BlkTile **tile_out, int32_t *n_tile)
 {
-    if (g->m_rec || g->E == 0) return;
     hipStream_t s = g->stream;
-    const int64_t E = g->E;
     const int32_t nblk = (int32_t)(((int64_t)g->V + (1 << kMBits) - 1) >> kMBits);
-    const int64_t rs_tiles = (E + kRsTile - 1) / kRsTile;
-    uint32_t *keys = dmalloc<uint32_t>((size_t)E);
-    uint32_t *kA = dmalloc<uint32_t>((size_t)E), *kB = dmalloc<uint32_t>((size_t)E);
-    uint32_t *vA = dmalloc<uint32_t>((size_t)E), *vB = dmalloc<uint32_t>((size_t)E);
+    const int64_t rs_tiles = (n + kRsTile - 1) / kRsTile;
+    uint32_t *keys = dmalloc<uint32_t>((size_t)n);
+    uint32_t *kA = dmalloc<uint32_t>((size_t)n), *kB = dmalloc<uint32_t>((size_t)n);
+    uint32_t *vA = dmalloc<uint32_t>((size_t)n), *vB = dmalloc<uint32_t>((size_t)n);
     int64_t *counts = dmalloc<int64_t>((size_t)std::max<int64_t>(256 * rs_tiles, (int64_t)nblk + 1));
     int64_t *bptr = dmalloc<int64_t>((size_t)nblk + 1);
     struct Scratch {
@@ -792,15 +828,16 @@ void build_multi_layout(sssp_graph *g)
             for (void *x : p) dfree(x);
         }
     } scratch{{keys, kA, kB, vA, vB, counts, bptr}};
-    k_m_keys<<<grid_for(E), kBlock, 0, s>>>(g->el_dst, E, keys);
+    k_m_keys<<<grid_for(n), kBlock, 0, s>>>(dst, n, keys);
     SSSP_LAUNCH_CHECK("k_m_keys");
     uint32_t *skeys = nullptr, *perm = nullptr;
-    radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), E, nblk - 1, kA, kB, vA, vB, counts,
+    radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), n, nblk - 1, kA, kB, vA, vB, counts,
                      g->blk_a, g->blk_b, g->n_blk, s, &skeys, &perm);
-    MRec *rec = dmalloc<MRec>((size_t)E);
-    k_m_gather<<<grid_for(E), kBlock, 0, s>>>(skeys, perm, E, g->el_src, g->el_dst, g->el_w, rec);
+    MRec *rec = dmalloc<MRec>((size_t)n);
+    *rec_out = rec;
+    k_m_gather<<<grid_for(n), kBlock, 0, s>>>(skeys, perm, n, src, dst, w, rec);
     SSSP_LAUNCH_CHECK("k_m_gather");
-    rowptr_from_sorted(skeys, E, nblk, bptr, s);
+    rowptr_from_sorted(skeys, n, nblk, bptr, s);
     std::vector<int64_t> bp((size_t)nblk + 1);
     SSSP_HIP(hipMemcpyAsync(bp.data(), bptr, 8 * bp.size(), hipMemcpyDeviceToHost, s));
     SSSP_HIP(hipStreamSynchronize(s));
@@ -814,11 +851,72 @@ void build_multi_layout(sssp_graph *g)
         }
     }
     BlkTile *td = dmalloc<BlkTile>(std::max<size_t>(tiles.size(), 1));
+    *tile_out = td;
     SSSP_HIP(hipMemcpyAsync(td, tiles.data(), sizeof(BlkTile) * tiles.size(), hipMemcpyHostToDevice, s));
     SSSP_HIP(hipStreamSynchronize(s));
+    *n_tile = (int32_t)tiles.size();
+}
+
+void build_multi_layout(sssp_graph *g)
+{
+    if (g->m_rec || g->E == 0) return;
+    hipStream_t s = g->stream;
+    struct Made {
+        void *p[4] = {};
+        ~Made()
+        {
+            for (void *x : p) dfree(x);
+        }
+    } made;
+    MRec *rec = nullptr, *lrec = nullptr;
+    BlkTile *tile = nullptr, *ltile = nullptr;
+    int32_t nt = 0, nlt = 0;
+    auto hold = [&] { made.p[0] = rec, made.p[1] = lrec, made.p[2] = tile, made.p[3] = ltile; };
+    try {
+        build_records(g, g->el_src, g->el_dst, g->el_w, g->E, &rec, &tile, &nt);
+        if (g->light_thr != 0xFFFFFFFFu) {
+            // the light edges of the src-sorted list, in order
+            const int64_t E = g->E, nch = (E + kBlkChunk - 1) / kBlkChunk;
+            int64_t *pos = dmalloc<int64_t>((size_t)nch + 1);
+            struct F {
+                void *p[4] = {};
+                ~F()
+                {
+                    for (void *x : p) dfree(x);
+                }
+            } f;
+            f.p[0] = pos;
+            const unsigned grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
+            k_light_count<<<grid, kBlock, 0, s>>>(g->el_w, E, nch, g->light_thr, pos);
+            SSSP_LAUNCH_CHECK("k_light_count");
+            k_fill_i64<<<1, 64, 0, s>>>(pos + nch, 1, 0);
+            device_exclusive_scan_i64(pos, pos, nch + 1, g->blk_a, g->blk_b, g->n_blk, s);
+            int64_t nl = 0;
+            SSSP_HIP(hipMemcpyAsync(&nl, pos + nch, 8, hipMemcpyDeviceToHost, s));
+            SSSP_HIP(hipStreamSynchronize(s));
+            if (nl > 0) {
+                int32_t *ls = dmalloc<int32_t>((size_t)nl);
+                f.p[1] = ls;
+                int32_t *ld = dmalloc<int32_t>((size_t)nl);
+                f.p[2] = ld;
+                uint32_t *lw = dmalloc<uint32_t>((size_t)nl);
+                f.p[3] = lw;
+                k_light_select<<<grid, kBlock, 0, s>>>(g->el_src, g->el_dst, g->el_w, E, nch,
+                                                       g->light_thr, pos, ls, ld, lw);
+                SSSP_LAUNCH_CHECK("k_light_select");
+                build_records(g, ls, ld, lw, nl, &lrec, &ltile, &nlt);
+            }
+        }
+    } catch (...) {
+        hold();
+        throw;
+    }
     g->m_rec = rec;
-    g->m_tile = td;
-    g->n_mtile = (int32_t)tiles.size();
+    g->m_tile = tile;
+    g->n_mtile = nt;
+    g->m_lrec = lrec;
+    g->m_ltile = ltile;
+    g->n_mltile = nlt;
 }
 
 // Edge-list check on the device: every id in [0, V) and (wtype >= 0) every
@@ -1093,7 +1191,7 @@ static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *b
     f.p[1] = lptr;
     int64_t *loff = lptr + nblk + 1;
     const unsigned chunk_grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
-    k_light_count<<<chunk_grid, kBlock, 0, s>>>(g->b_w, nch, thr, pos);
+    k_light_count<<<chunk_grid, kBlock, 0, s>>>(g->b_w, nch * kBlkChunk, nch, thr, pos);
     SSSP_LAUNCH_CHECK("k_light_count");
     k_fill_i64<<<1, 64, 0, s>>>(pos + nch, 1, 0);  // the last position: the total
     device_exclusive_scan_i64(pos, pos, nch + 1, g->blk_a, g->blk_b, g->n_blk, s);
@@ -1124,6 +1222,7 @@ static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *b
     g->l_off_host = lo;
     g->l_edges = Lp;
     g->light_edges = lp[(size_t)nblk];
+    g->light_thr = thr;
 }
 
 void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, const uint32_t *d_w,

@@ -127,11 +127,15 @@ struct BlkRanges {
 // Multi-source batches on one graph: edges as 16-byte records sorted by
 // (dst >> kMBits, src) -- 16-vertex destination blocks, so a 256-source block
 // of distances is 16 KB of LDS; tiles of at most kMTileEdges edges of one
-// block.
+// block, short enough that a hub block's tiles do not outlast the pass (a wave
+// relaxes a record in about 0.25 us; ms at 4096 / 1024 / 512 / 256 / 128 / 64 edges:
+// R-MAT 20 x 16 with 256 sources 59 / 54.9 / 17.9 / 16.7 / 17.3 / 20.7 -- the last four
+// without the pass counter's contention --, R-MAT 16 x 12 with 33 6.2 / 3.3 / 2.0 /
+// 1.4 / 1.2 / 0.94).
 constexpr int kMBits = 4;
 constexpr int kMultiSlots = 4;  // captured chunk launches kept per graph
 constexpr int kMultiKey = 10;
-constexpr int64_t kMTileEdges = 4096;
+constexpr int64_t kMTileEdges = 128;
 struct MRec {
     int32_t src;
     uint32_t w;
@@ -201,6 +205,7 @@ struct sssp_graph {
     sssp::BlkTile *b_ltile = nullptr;
     int32_t n_ltile = 0;
     int64_t light_edges = 0;      // edges in the light list
+    uint32_t light_thr = 0xFFFFFFFFu;  // its largest weight pattern (0xFFFFFFFF: no light list)
     std::vector<int64_t> b_off_host;  // padded block offsets (tiles are rebuilt from them)
     std::vector<int64_t> l_off_host;  // ... of the light list
     int64_t blk_tile_cap = 0;         // edges per tile at most
@@ -213,13 +218,17 @@ struct sssp_graph {
     sssp::MRec *m_rec = nullptr;
     sssp::BlkTile *m_tile = nullptr;
     int32_t n_mtile = 0;
+    sssp::MRec *m_lrec = nullptr;  // the light edges' records and tiles (n_mltile 0: none)
+    sssp::BlkTile *m_ltile = nullptr;
+    int32_t n_mltile = 0;
+    int32_t *mstamp = nullptr;     // per vertex: last pass that lowered its row
     uint32_t *mdist = nullptr;
     int64_t mdist_elems = 0;
     // the batch's sources on the device, and the captured launches of its
     // chunks (hipGraphExec_t), keyed on chunk shape and buffers
     int32_t *msrc = nullptr;
     int32_t msrc_cap = 0;
-    int32_t *mflags = nullptr;  // 64 change flags of the passes, then the pass base
+    void *mctl = nullptr;  // pass state (MultiCtl)
     void *mexec[sssp::kMultiSlots][2] = {};  // first run, next runs
     int64_t mkey[sssp::kMultiSlots][sssp::kMultiKey] = {};
     int mnext = 0;

@@ -1005,3 +1005,36 @@ def test_large_results_reach_the_host_whole(gpu, V):
         for k in range(4):
             assert np.array_equal(bits(got["g", k]), bits(ref))
             assert np.array_equal(bits(got["h", k]), bits(href))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,n,kind", [(1, 3, "f32"), (17, 1, "f32"), (4099, 65, "f32"),
+                                      (4099, 300, "u32"), (4099, 64, "equal"), (20011, 33, "hub")])
+def test_batch_light_and_live_records(gpu, oracle, V, n, kind):
+    """Policy 3 relaxes the records whose source row was lowered since, light
+    records first: one vertex, a part of one destination block, one source, a
+    chunk and a part, u32, equal weights (no light records), a hub block split
+    over many tiles, captured and queued. Bit equality: no tolerance."""
+    rng = np.random.default_rng(29)
+    m = 11 * V
+    src = (rng.random(m) ** 2 * V).astype(np.int32)
+    dst = rng.integers(0, V, m).astype(np.int32)
+    if kind == "hub":
+        dst[: m // 2] = 5
+    w = rng.random(m, dtype=np.float32)
+    if kind == "equal":
+        w[:] = 0.5
+    elif kind == "u32":
+        w = rng.integers(1, 256, m).astype(np.uint32)
+    sources = rng.integers(0, V, n).astype(np.int32)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        for capture in (1, 0):
+            g.set_param("batch_capture", capture)
+            for rep in range(2):
+                print(f"batch records: {kind} V {V} n {n} capture {capture} {rep}", flush=True)
+                D, _ = g.solve_batch(sources, policy=3)
+                for i in range(0, n, max(1, n // 7)):
+                    ref = oracle.dijkstra(src, dst, w, V, int(sources[i]))
+                    assert np.array_equal(bits(D[i]), bits(ref)), (capture, i)
+                D1, _ = g.solve_batch(sources, policy=1)
+                assert np.array_equal(bits(D), bits(D1))
