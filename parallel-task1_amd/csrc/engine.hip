@@ -2578,8 +2578,7 @@ int32_t step_round(sssp_graph *g, int32_t r, int sched, int32_t tick0, sssp_stat
         // (the first tail round always runs: its frontier was checked here)
     }
     if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
-    const bool light =
-        (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) && force_mode < 0;
+    const bool light = sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED;
     if (run_round<WT>(g, mode, kidx, r, tick0, cur, verify, light, st)) g->pile_cur ^= 1;
     float ms = 0.f;
     if (g->trace_events) {

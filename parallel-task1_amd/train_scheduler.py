@@ -19,13 +19,11 @@ JSON sidecar describing the run.
 
     python parallel-task1_amd/train_scheduler.py [--scales 19 20 21 22 23 24]
 
-The committed network (models/scheduler_mlp.f32) was trained on the rows of
-two collections over the default graphs -- one whose rollouts continued with
-the previous network (--rollout-weights), one whose rollouts followed the
-rule -- concatenated:
-    python parallel-task1_amd/train_scheduler.py --rollout-weights prev.f32 --out A.f32
-    python parallel-task1_amd/train_scheduler.py --out B.f32
-    python parallel-task1_amd/train_scheduler.py --data A_data.npz B_data.npz
+The committed network (models/scheduler_mlp.f32) was trained in two steps over
+the default graphs, the second one's rollouts continuing with the first one's
+network:
+    python parallel-task1_amd/train_scheduler.py --out rule.f32
+    python parallel-task1_amd/train_scheduler.py --rollout-weights rule.f32
 """
 import argparse
 import json
