@@ -82,7 +82,7 @@ void graph_free(sssp_graph *g)
                     g->src_list, g->btasks, g->bcounter, g->bround, g->x_src, g->x_dst,
                     g->x_w, g->xgoff, g->pile[0], g->pile[1], g->farst, g->snap,
                     g->b_pk, g->b_cbase, g->b_wide, g->b_w, g->b_tile, g->b_ltile, g->l_pk, g->l_cbase, g->l_wide, g->l_w, g->b_app, g->fbits, g->m_rec, g->m_tile, g->mdist,
-                    g->vperm, g->vinv, g->dout != g->dist ? g->dout : nullptr, g->msrc, g->mctl, g->mstamp, g->m_lrec, g->m_ltile, g->dvis};
+                    g->vperm, g->vinv, g->dout != g->dist ? g->dout : nullptr, g->msrc, g->mctl, g->mstamp, g->m_lrec, g->m_ltile, g->dvis, g->el_first};
     if (g->batch_exec) (void)hipGraphExecDestroy((hipGraphExec_t)g->batch_exec);
     for (auto &pair : g->mexec)
         for (void *e : pair)

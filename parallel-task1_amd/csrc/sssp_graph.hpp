@@ -357,7 +357,8 @@ struct sssp_graph {
     // batch policy chosen by the autotuner (0 = not tuned)
     int batch_policy = 0, batch_bs = 256, batch_wgpcu = 2;
     void *batch_exec = nullptr;  // hipGraphExec_t of the captured persistent launch
-    int64_t batch_key[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int64_t batch_key[10] = {};
+    int32_t *el_first = nullptr;  // source of every 256th edge, V at the end (on demand)
     void *btasks = nullptr;      // device BatchTask array
     int32_t btask_cap = 0;
     int32_t *bcounter = nullptr;  // task counter + error flag

@@ -1038,3 +1038,53 @@ def test_batch_light_and_live_records(gpu, oracle, V, n, kind):
                     assert np.array_equal(bits(D[i]), bits(ref)), (capture, i)
                 D1, _ = g.solve_batch(sources, policy=1)
                 assert np.array_equal(bits(D), bits(D1))
+
+
+@pytest.mark.gpu
+def test_pack_graphs_at_the_edges_of_the_lds_classes(gpu, oracle):
+    """Graphs of a pack are solved in LDS up to 2^15 vertices, in classes of
+    2^11, 2^14 and 2^15, larger ones together: sizes at and one past each edge,
+    a single vertex, a graph without edges, edge ranges that start and end
+    inside a 256-edge chunk and span one chunk or less. Bit equality: no
+    tolerance."""
+    rng = np.random.default_rng(41)
+    sizes = [(1, 0), (1, 3), (33, 5), (2047, 9001), (2048, 4096), (2049, 10007), (300, 256),
+             (16384, 70001), (16385, 50021), (32768, 100003), (32769, 90001), (40000, 80001),
+             (5, 0)]
+    for reorder in (False, True):
+        if reorder:
+            sizes = [sizes[i] for i in rng.permutation(len(sizes))]
+        src = [np.minimum((rng.random(m) ** 2 * v).astype(np.int32), v - 1) for v, m in sizes]
+        dst = [rng.integers(0, v, m).astype(np.int32) for v, m in sizes]
+        w = [rng.random(m, dtype=np.float32) for _, m in sizes]
+        offs = np.concatenate([[0], np.cumsum([m for _, m in sizes])]).astype(np.int64)
+        vc = np.array([v for v, _ in sizes], np.int32)
+        srcs = np.array([int(s[0]) if len(s) else v - 1 for s, (v, _) in zip(src, sizes)], np.int32)
+        voff = np.concatenate([[0], np.cumsum(vc)])
+        p = S.GraphPack(np.concatenate(src), np.concatenate(dst), np.concatenate(w), offs, vc)
+        try:
+            for rep in range(2):
+                print(f"pack at class edges: reorder {reorder} {rep}", flush=True)
+                D, _ = p.solve(srcs, policy=1)
+                for k, (v, m) in enumerate(sizes):
+                    ref = oracle.dijkstra(src[k], dst[k], w[k], v, int(srcs[k])) if m else \
+                        np.where(np.arange(v) == srcs[k], np.float32(0), S.F32_INF)
+                    assert np.array_equal(bits(D[voff[k]:voff[k + 1]]), bits(ref)), (rep, v, m)
+        finally:
+            p.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [700, 2048, 9001, 20000, 33000])
+def test_batch_policy_1_in_lds_u32(gpu, oracle, V):
+    """Policy 1 over the sources of one graph, in each LDS class and past the
+    largest, u32 weights with values that saturate."""
+    rng = np.random.default_rng(43)
+    src, dst = (rng.integers(0, V, 7 * V + 13).astype(np.int32) for _ in range(2))
+    w = rng.integers(1, 256, len(src)).astype(np.uint32)
+    w[::5] = 0xFFFFFF00
+    sources = rng.integers(0, V, 11).astype(np.int32)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        D, _ = g.solve_batch(sources, policy=1)
+        for i, s in enumerate(sources):
+            assert np.array_equal(D[i], oracle.dijkstra(src, dst, w, V, int(s))), i
