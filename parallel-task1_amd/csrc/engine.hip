@@ -1755,6 +1755,7 @@ struct PassArgs {
     int32_t pass;         // index in the run
     int32_t light_stop;   // light passes go on while they lower this many vertices, or
                           // more than the light pass before
+    int32_t full_stop;    // ... and follow a full pass that lowered at least this many
     int32_t tag;          // of the run, in the progress word
     Ctrl *ctrl;
     unsigned long long *pos;  // device address of the host mirror's progress word
@@ -1782,7 +1783,8 @@ __device__ __forceinline__ int pass_kind(const PassArgs &a)
     if (prev == kPassIdle) return kPassIdle;
     if (prev == kPassFull) {
         if (low == 0) return kPassIdle;
-        return a.run == kRunMixed && a.pass < kLightMaxPasses ? kPassLight : kPassFull;
+        return a.run == kRunMixed && a.pass < kLightMaxPasses && low >= a.full_stop ? kPassLight
+                                                                                    : kPassFull;
     }
     const int32_t before = a.pass > 1 && c->ph_kind[i2] == kPassLight ? c->ph_low[i2] : 0;
     if ((low >= a.light_stop || low > before) && low > 0 && a.pass < kLightMaxPasses)
@@ -2262,6 +2264,15 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
     a.n_light = g->n_ltile;
     a.run = run;
     a.light_stop = (int32_t)(kLightStopFrac * g->n_nzo);
+    // Light passes after every full pass that changed something, or only
+    // after one that changed as many vertices as keep light passes going: a
+    // full pass over few edges costs what a light pass costs, its launch and
+    // one tile's chain. Four plain solves, ms, always / from light_stop on:
+    // R-MAT 16 x 16 1.31 / 1.09, R-MAT 18 x 24 1.52 / 1.38, skewed 1 M x 4
+    // 2.73 / 2.34, uniform 400 K x 16 3.08 / 3.17, R-MAT 19 x 16 (2^23 edges)
+    // 1.94 / 1.78; above it skewed 1.2 M x 9 4.0 / 4.2, uniform 2 M x 14 10.5
+    // / 12.1, R-MAT 22 x 32 7.9 / 8.1.
+    a.full_stop = g->E <= kLightAlwaysEdges ? a.light_stop : 1;
     a.tag = ++g->ph_tag;
     a.ctrl = g->ctrl;
     a.pos = &g->ctrl_host_dev->ph_pos;

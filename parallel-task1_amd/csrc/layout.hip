@@ -1448,15 +1448,26 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         for (int32_t b = 0; b < nblk; b++)
             bo[(size_t)b + 1] = bo[(size_t)b] +
                                 (bp[(size_t)b + 1] - bp[(size_t)b] + kBlkChunk - 1) / kBlkChunk * kBlkChunk;
-        // Tile cap: 2^17 edges up to 2^29 edges, doubled while more than
-        // kBlkTileCount tiles of the cap fit in the graph -- the 2.08 G-edge
+        // Tile cap. A pass over a small list lasts as long as its longest
+        // tile, so the list is cut into about as many parts as run at once
+        // (kBlkTileWave); shorter tiles than that only add block write-backs
+        // and a second, part-filled wave. Plain solves, ms, at 2^17-edge tiles
+        // / at this cap: uniform 400 K x 16 2.2 / 0.74 (2^14), R-MAT 18 x 16
+        // 0.95 / 0.34 (2^13), R-MAT 20 x 16 1.32 / 1.25 (2^15), uniform 2 M x 6
+        // 3.16 / 2.3 (2^15), skewed 1.2 M x 9 2.33 / 1.45 (2^15); skewed 4 M x
+        // 14 2.70 at 2^17 (489 tiles), 3.14 at 2^16. Learned solves: skewed
+        // 1.2 M x 9 1.27 / 1.0, R-MAT 22 x 32 and larger graphs the same at
+        // 2^16 and 2^17. The cap stays 2^17 up to 2^29 edges and is doubled
+        // while more than kBlkTileCount tiles of it fit in the graph -- the
+        // 2.08 G-edge
         // R-MAT graph ran 50.9 GTEPS with 2^19-edge tiles, 46.7 with 2^17;
         // R-MAT 25 x 16 (2^29 edges), learned / plain ms, with the dense
         // round's stream loaded a step ahead: 14.9 / 22.3 at 2^17, 15.6 /
         // 23.3 at 2^18, 17.0 / 26.3 at 2^19 (before that change 2^18 was the
         // faster: 19.2 against 19.6 ms). A power of two, so every tile holds
         // whole chunks.
-        int64_t tcap = kBlkTileEdges;
+        int64_t tcap = kBlkTileFloor;
+        while (tcap * kBlkTileWave < E && tcap < kBlkTileEdges) tcap <<= 1;
         while (tcap * kBlkTileCount < E) tcap <<= 1;
         g->b_off_host = bo;
         const int64_t Ep = bo[(size_t)nblk];

@@ -82,14 +82,18 @@ struct Ctrl {
 // 32-bit word holding its destination's offset in the block (low kBlkBits
 // bits) and its source as the delta to the previous edge of the chunk, and
 // its weight; each chunk keeps its first source whole. A tile is a run of
-// at most kBlkTileEdges slots of one block, whole chunks (the cap doubles
-// while the graph holds more than kBlkTileCount tiles' worth of edges);
+// at most a cap of slots of one block, whole chunks: the smallest power of two
+// from kBlkTileFloor that cuts the edges into at most kBlkTileWave parts (two
+// 1024-thread workgroups on each of the 256 CUs), up to kBlkTileEdges, then
+// doubled while the graph holds more than kBlkTileCount tiles' worth of edges.
 // `split` = the block has more than one tile.
 constexpr int kBlkBits = 14;
 constexpr int kBlkThreads = 1024;  // threads of a blocked-pass workgroup
 static_assert(kBlkBits <= 16, "block offsets fit the low half of a packed edge");
 constexpr int kBlkDeltaBits = 32 - kBlkBits;  // source delta bits of a packed edge
 constexpr int64_t kBlkChunk = 256;  // edge slots per chunk: 4 per lane of one wave
+constexpr int64_t kBlkTileFloor = (int64_t)1 << 13;
+constexpr int64_t kBlkTileWave = 512;
 constexpr int64_t kBlkTileEdges = (int64_t)1 << 17;
 constexpr int64_t kBlkTileCount = 4096;
 struct BlkTile {
@@ -109,6 +113,8 @@ constexpr int64_t kLightTiles = 1024;        // ... and the tile count its cap a
 constexpr int kLightMaxPasses = 64;          // light passes stop after this many passes of a run
 constexpr double kLightStopFrac = 0.05;      // light passes stop once a pass lowers fewer than
                                              // this share of the vertices with out-edges
+constexpr int64_t kLightAlwaysEdges = (int64_t)1 << 23;  // light passes after every full pass
+                                                         // on graphs of more edges
 // Source-range cuts of the blocked list's block runs (host copy): off[b *
 // (n_fine + 1) + k] = first slot of block b whose source is at least
 // k << fine_bits, aligned down to its chunk (k = n_fine: the run's end).
@@ -371,9 +377,10 @@ namespace sssp {
 // blocked list has at least kPlainBlkMinTiles tiles (one 1024-thread
 // workgroup each), else the XCD-partitioned edge-list pass, whose grid fills
 // the chip whatever the graph's block structure. Measured crossover (plain
-// solve, R-MAT edge factor 16): 44 tiles (scale 18) 1.08 against 0.96 ms for
-// the edge-list pass, 83 tiles (scale 19) 1.27 against 1.57 ms; R-MAT
-// 22 x 32 (1196 tiles) 7.1 against 15.6 ms.
+// solve, R-MAT edge factor 16, tiles of 2^13 edges): scale 15 (65 tiles) 0.24
+// against 0.29 ms for the edge-list pass, scale 18 0.34 against 0.95 ms; R-MAT
+// 22 x 32 (1196 tiles) 5.3 against 15.6 ms. Below 64 tiles too few CUs hold
+// one.
 constexpr int64_t kPlainBlkMinTiles = 64;
 
 inline bool plain_uses_blocked(const sssp_graph *g)

@@ -556,6 +556,28 @@ def test_blocked_tiles_any_cap_and_order(gpu, oracle):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("E,cap", [(1, 1 << 13), (1 << 22, 1 << 13), ((1 << 22) + 1, 1 << 14),
+                                   (1 << 23, 1 << 14), ((1 << 23) + 1, 1 << 15)])
+def test_default_tile_cap(gpu, oracle, E, cap):
+    """The tile cap a graph gets by its edge count, on both sides of a step of
+    the rule and of the size up to which light passes wait for a full pass
+    that changed much: every schedule ends on the oracle's fixpoint (bits)."""
+    rng = np.random.default_rng(5)
+    V = 70001
+    src = (rng.random(E) ** 3 * V).astype(np.int32)
+    dst = (rng.random(E) ** 2 * V).astype(np.int32)
+    w = rng.random(E, dtype=np.float32)
+    source = int(src[0])
+    ref = oracle.dijkstra(src, dst, w, V, source)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        assert g.get_param("blk_tile_cap") == cap
+        for sched in ("heuristic", "learned", "plain"):
+            print(f"default tile cap: E {E}, {sched}", flush=True)
+            d, _ = g.solve(source, sched)
+            assert np.array_equal(bits(d), bits(ref)), sched
+
+
+@pytest.mark.gpu
 def test_batch_u32(gpu, oracle):
     src, dst, w = S.er(1 << 12, 8, seed=4, weight_mode=1)
     V = 1 << 12
