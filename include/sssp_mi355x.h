@@ -209,11 +209,15 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * collection ran.
  * plain_below_edges (default 2^26): a single-source heuristic or learned
  * solve (or BFS) of a graph with fewer edges runs the plain pass loop, whose
- * passes then cost less than the rounds with their fixed per-round cost.
+ * passes then cost less than the rounds with their fixed per-round cost: light
+ * passes (the lightest edges alone) before and between the passes over all
+ * edges, or, on sparse graphs without hubs whose edges mostly join near ids
+ * (grids, road networks), passes that relax each tile of edges several times
+ * and leave out the tiles no source of which changed.
  * plain_kernel picks the plain pass: 0 (default) the destination-blocked pass
  * (block minima in LDS, as the dense rounds) once the blocked list has 64
  * tiles or more, else the XCD-partitioned edge-list pass; 1 always the
- * edge-list pass, 2 always the blocked pass. "plain_blocked" (read-only) = 1
+ * edge-list pass (also for those graphs), 2 always the blocked pass. "plain_blocked" (read-only) = 1
  * when plain solves use the blocked pass.
  * tail_edges (default 2^23): once a heuristic or learned solve's frontier has
  * had more than tail_edges out-edges, a round decided as a push round over a

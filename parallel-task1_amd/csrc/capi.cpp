@@ -81,7 +81,7 @@ void graph_free(sssp_graph *g)
                     g->blk_a, g->blk_b, g->parent, g->ctrl, g->bdist, g->bscratch,
                     g->src_list, g->btasks, g->bcounter, g->bround, g->x_src, g->x_dst,
                     g->x_w, g->xgoff, g->pile[0], g->pile[1], g->farst, g->snap,
-                    g->b_pk, g->b_cbase, g->b_wide, g->b_w, g->b_tile, g->b_ltile, g->l_pk, g->l_cbase, g->l_wide, g->l_w, g->b_app, g->fbits, g->m_rec, g->m_tile, g->mdist,
+                    g->b_pk, g->b_cbase, g->b_wide, g->b_w, g->b_tile, g->b_ltile, g->l_pk, g->l_cbase, g->l_wide, g->l_w, g->b_app, g->t_tile, g->t_state, g->t_seg, g->fbits, g->m_rec, g->m_tile, g->mdist,
                     g->vperm, g->vinv, g->dout != g->dist ? g->dout : nullptr, g->msrc, g->mctl, g->mstamp, g->m_lrec, g->m_ltile, g->dvis, g->el_first};
     if (g->batch_exec) (void)hipGraphExecDestroy((hipGraphExec_t)g->batch_exec);
     for (auto &pair : g->mexec)
@@ -378,6 +378,8 @@ void graph_finish(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, con
                       (g->b_nwide + g->l_nwide) * kBlkChunk * 4 +
                       (int64_t)(g->n_btile + g->n_ltile) * (int64_t)sizeof(BlkTile) +
                       (int64_t)std::max(g->n_btile, g->n_ltile) * kBlkThreads * 2 +
+                      (int64_t)g->n_ttile * (int64_t)(sizeof(BlkTile) + sizeof(TileState)) +
+                      (int64_t)g->n_seg * 4 +
                       (Vi + 1) * 8 + (g->has_csc ? Ei * 8 + (Vi + 1) * 8 : 0) + Vi * 4 * 7 +
                       (Vi + 1) * 4 * 3 + (Vi + 1) * 8 * 2 + Vi * 24 + (g->relabel ? Vi * 12 : 0);
 }

@@ -1771,6 +1771,12 @@ __host__ __device__ inline unsigned long long pass_word(int32_t tag, int32_t beg
            ((unsigned long long)full << 2) | (unsigned)kind;
 }
 
+struct LocalArgs {
+    TileState *state;
+    int32_t *seg;      // per segment: the pass that last lowered a vertex of it
+    int64_t *work;     // device address of the host mirror's count of relaxed chunks
+};
+
 // What pass a.pass runs; every workgroup reads the same values (written by
 // the passes before).
 __device__ __forceinline__ int pass_kind(const PassArgs &a)
@@ -1792,6 +1798,23 @@ __device__ __forceinline__ int pass_kind(const PassArgs &a)
     return a.run == kRunLight ? kPassIdle : kPassFull;
 }
 
+// Records what the pass runs and tells the host; one thread of the pass.
+__device__ __forceinline__ void pass_publish(const PassArgs &a, int kind)
+{
+    Ctrl *c = a.ctrl;
+    const int32_t full = (a.pass == 0 ? 0 : c->ph_full) + (kind == kPassFull ? 1 : 0);
+    int32_t begun = a.pass + 1;
+    if (kind == kPassIdle) {
+        if (c->ph_kind[(a.pass - 1) & 63] != kPassIdle) c->ph_done = begun;
+        else begun = c->ph_done;
+    }
+    c->ph_kind[a.pass & 63] = kind;
+    c->ph_low[(a.pass + 1) & 63] = 0;
+    c->ph_full = full;
+    __hip_atomic_store(a.pos, pass_word(a.tag, begun, full, kind), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <class WT>
 __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blk_plain(
     const PassArgs a, const BlkList L, const BlkList LL, uint32_t *dist)
@@ -1799,20 +1822,7 @@ __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))
     __shared__ uint32_t s_d[1 << kBlkBits];
     __shared__ int s_low;
     const int kind = pass_kind(a);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        Ctrl *c = a.ctrl;
-        const int32_t full = (a.pass == 0 ? 0 : c->ph_full) + (kind == kPassFull ? 1 : 0);
-        int32_t begun = a.pass + 1;
-        if (kind == kPassIdle) {
-            if (c->ph_kind[(a.pass - 1) & 63] != kPassIdle) c->ph_done = begun;
-            else begun = c->ph_done;
-        }
-        c->ph_kind[a.pass & 63] = kind;
-        c->ph_low[(a.pass + 1) & 63] = 0;
-        c->ph_full = full;
-        __hip_atomic_store(a.pos, pass_word(a.tag, begun, full, kind), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) pass_publish(a, kind);
     if (kind == kPassIdle) return;
     const bool light = kind == kPassLight;
     if ((int)blockIdx.x >= (light ? a.n_light : a.n_full)) return;
@@ -1849,6 +1859,225 @@ __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))
     }
     __syncthreads();
     if (threadIdx.x == 0 && s_low != 0) atomicAdd(&a.ctrl->ph_low[a.pass & 63], s_low);
+}
+
+// State of a tile between the passes of k_blk_local: the segments its
+// sources lie in and the pass that last relaxed it.
+__global__ __launch_bounds__(64) void k_tile_spans(const BlkTile *__restrict__ tiles,
+                                                   const BlkList L, TileState *state)
+{
+    const BlkTile t = tiles[blockIdx.x];
+    const int lane = threadIdx.x;
+    const int64_t c0 = t.e0 / kBlkChunk, c1 = t.e1 / kBlkChunk - 1;
+    const int32_t b0 = L.cbase[c0], b1 = L.cbase[c1];
+    int32_t sum = 0;  // sources ascend: the last one is the first plus all deltas
+    for (int k = lane; k < (int)kBlkChunk; k += 64)
+        sum += (int32_t)(L.pk[c1 * kBlkChunk + k] >> kBlkBits);
+    sum = wave_sum32(sum);
+    if (lane != 0) return;
+    const int32_t first = b0 >= 0 ? b0 : L.wide[(int64_t)(-1 - b0) * kBlkChunk];
+    const int32_t last = b1 >= 0 ? b1 + sum : L.wide[(int64_t)(-b1) * kBlkChunk - 1];
+    state[blockIdx.x] = TileState{first >> kSegBits, last >> kSegBits, 1, 0};
+}
+
+// Before the first pass only the source's segment has changed.
+__global__ __launch_bounds__(kBlock) void k_local_reset(int32_t *seg, int32_t n_seg,
+                                                        TileState *state, int32_t n_tiles,
+                                                        int32_t source)
+{
+    const int32_t i = (int32_t)(blockIdx.x * kBlock + threadIdx.x);
+    if (i < n_seg) seg[i] = i == source >> kSegBits ? 1 : 0;
+    if (i < n_tiles) {
+        state[i].done = 1;
+        state[i].work = 0;
+    }
+}
+
+// A pass of graphs whose edges join near ids and whose paths are long (grids,
+// road networks numbered along the map; TileState, light_threshold). Their
+// plain passes cost a launch and one tile's chain of dependent loads, 9 us,
+// for one hop of every path. Here a tile keeps its edges in registers and
+// relaxes those whose source lies in its own block again, from the block's
+// minima in LDS, up to kLocalRounds * kLocalSweeps times, so a pass moves
+// paths on by several hops; and a tile none of whose source segments was
+// written since the pass that last relaxed it returns at once. A vertex
+// lowered by the pass a tile last ran in may have come too late for it, so
+// that counts as written since. A pass that lowers nothing relaxed every
+// tile with a source changed after the tile was relaxed: the fixpoint. Bound
+// by LDS latency (0.4 us a sweep) and the chain of a pass (12 us with its
+// launch). Four solves, ms, plain passes / 12 sweeps (8 / 16 / 24) a pass: grid
+// 517 x 389 27.5 / 7.6 (8.2 / 7.9 / 9.1), 700 x 700 47 / 17.4 (16.2 / 18.5 /
+// 21.6), 100 x 100 7.2 / 1.3 (1.5 / 1.1 / 1.0), 20000 x 5 1000 / 148 (185 /
+// 125 / 106); two solves of 3000 x 2000 478 / 127 (118 / 135 / 154). Tiles of
+// four chunks per wave, 12-16 sweeps: 517 x 389 8.3, 700 x 700 15.6, 20000 x 5
+// 197, 3000 x 2000 99, 300 x 12000 790 against 509. On R-MAT and random
+// graphs of 10^6 edges the passes took 1.3-1.5 times as long and were no
+// fewer.
+template <class WT>
+__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))) void
+k_blk_local(const PassArgs a, const LocalArgs la, const BlkList L, uint32_t *dist)
+{
+    __shared__ uint32_t s_d[1 << kBlkBits];
+    __shared__ unsigned long long s_work;
+    __shared__ int s_more[3];
+    typedef int32_t v4i __attribute__((ext_vector_type(4)));
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    constexpr uint32_t kOffMask = (1u << kBlkBits) - 1;
+    const int tid = threadIdx.x, lane = __lane_id();
+    const BlkTile t = a.full[blockIdx.x];
+    TileState ts = la.state[blockIdx.x];
+    const int kind = pass_kind(a);
+    if (blockIdx.x == 0) {
+        if (kind == kPassIdle && a.ctrl->ph_kind[(a.pass - 1) & 63] != kPassIdle) {
+            // the run is over: the chunks its tiles relaxed, for the host
+            if (tid == 0) s_work = 0;
+            __syncthreads();
+            int64_t n = 0;
+            for (int i = tid; i < a.n_full; i += kBlkThreads) n += la.state[i].work;
+            n = wave_sum64(n);
+            if (lane == 0) atomicAdd(&s_work, (unsigned long long)n);
+            __syncthreads();
+            if (tid == 0) {
+                *la.work = (int64_t)s_work;
+                __threadfence_system();
+            }
+        }
+        if (tid == 0) pass_publish(a, kind);
+    }
+    if (kind == kPassIdle) return;
+    int pend = 0;
+    for (int i = ts.lo + tid; i <= ts.hi; i += kBlkThreads) pend |= la.seg[i] >= ts.done;
+#pragma unroll
+    for (int k = 0; k < kBlkPer; k++) s_d[k * kBlkThreads + tid] = WT::INF;
+    if (tid < 3) s_more[tid] = 0;
+    if (!__syncthreads_or(pend)) return;
+    const int p = a.pass + 2;  // above the passes of k_local_reset
+    if (tid == 0) {
+        la.state[blockIdx.x].done = p;
+        la.state[blockIdx.x].work = ts.work + (int32_t)((t.e1 - t.e0) / kBlkChunk);
+    }
+    const v4u *p4 = reinterpret_cast<const v4u *>(L.pk);
+    const v4u *w4 = reinterpret_cast<const v4u *>(L.w);
+    const v4i *x4 = reinterpret_cast<const v4i *>(L.wide);
+    const int64_t base = (int64_t)t.blk << kBlkBits;
+    const int c1 = (int)(t.e1 / kBlkChunk);
+    const int c0 = (int)(t.e0 / kBlkChunk) + __builtin_amdgcn_readfirstlane(tid >> 6);
+    v4u pv[kLocalChunks], wv[kLocalChunks];
+    int32_t cb[kLocalChunks];
+#pragma unroll
+    for (int h = 0; h < kLocalChunks; h++) {
+        const int64_t c = c0 + h * (kBlkThreads / 64);
+        cb[h] = 0;
+        pv[h] = v4u{0u, 0u, 0u, 0u};
+        wv[h] = pv[h];
+        if (c < c1) {
+            cb[h] = L.cbase[c];
+            pv[h] = p4[c * (kBlkChunk / 4) + lane];
+            wv[h] = w4[c * (kBlkChunk / 4) + lane];
+        }
+    }
+    // per edge: LDS byte addresses of its source (high half; meaningful when
+    // the source is of this block) and its destination, and the source's
+    // distance as last relaxed
+    uint32_t ed[kLocalChunks * 4], eu[kLocalChunks * 4], inner = 0;
+    char *const lds = reinterpret_cast<char *>(s_d);
+    auto at = [&](uint32_t byte) { return reinterpret_cast<uint32_t *>(lds + byte); };
+#pragma unroll
+    for (int h = 0; h < kLocalChunks; h++) {
+        const bool has = c0 + h * (kBlkThreads / 64) < c1;
+        int32_t s[4];
+        if (cb[h] >= 0) {
+            int32_t a4[4];
+            a4[0] = (int32_t)(pv[h].x >> kBlkBits);
+            a4[1] = a4[0] + (int32_t)(pv[h].y >> kBlkBits);
+            a4[2] = a4[1] + (int32_t)(pv[h].z >> kBlkBits);
+            a4[3] = a4[2] + (int32_t)(pv[h].w >> kBlkBits);
+            int32_t incl = a4[3];
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int32_t y = __shfl_up(incl, o);
+                if (lane >= o) incl += y;
+            }
+            const int32_t b0 = cb[h] + (incl - a4[3]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) s[j] = b0 + a4[j];
+        } else {
+            const v4i sv = x4[(int64_t)(-1 - cb[h]) * (kBlkChunk / 4) + lane];
+            s[0] = sv.x;
+            s[1] = sv.y;
+            s[2] = sv.z;
+            s[3] = sv.w;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int e = h * 4 + j;
+            eu[e] = has ? dist[s[j]] : WT::INF;
+            ed[e] = (pv[h][j] & kOffMask) << 2 | ((uint32_t)s[j] & kOffMask) << 18;
+            if (has && s[j] >> kBlkBits == t.blk) inner |= 1u << e;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < kLocalChunks * 4; e++) {
+        atomicMin(at(ed[e] & 0xFFFFu),
+                  eu[e] != WT::INF ? WT::add(eu[e], wv[e >> 2][e & 3]) : WT::INF);
+        if (!(inner >> e & 1u)) eu[e] = 0u;  // never lowered
+    }
+    __syncthreads();
+    for (int it = 0; it < kLocalRounds; it++) {
+        bool ch = false;
+        for (int r = 0; r < kLocalSweeps; r++) {
+            uint32_t nu[kLocalChunks * 4];
+#pragma unroll
+            for (int e = 0; e < kLocalChunks * 4; e++)
+                nu[e] = *(volatile uint32_t *)at(ed[e] >> 16);
+            bool lower = false;
+#pragma unroll
+            for (int e = 0; e < kLocalChunks * 4; e++) lower |= nu[e] < eu[e];
+            if (__ballot(lower) == 0) continue;  // most waves, most sweeps
+            ch = true;
+#pragma unroll
+            for (int e = 0; e < kLocalChunks * 4; e++) {
+                if (nu[e] >= eu[e]) continue;
+                eu[e] = nu[e];
+                atomicMin(at(ed[e] & 0xFFFFu), WT::add(nu[e], wv[e >> 2][e & 3]));
+            }
+        }
+        // one barrier a round: the flag of the round after next is cleared
+        // while this round's is set, so no reader still waits for it
+        if (tid == 0) s_more[(it + 1) % 3] = 0;
+        if (ch && lane == 0) s_more[it % 3] = 1;
+        __syncthreads();
+        if (s_more[it % 3] == 0) break;
+    }
+    bool any = false;
+#pragma unroll
+    for (int k0 = 0; k0 < kBlkPer; k0 += 8) {
+        uint32_t cur[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (k0 + j) * kBlkThreads + tid;
+            cur[j] = s_d[i] != WT::INF ? dist[base + i] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (k0 + j) * kBlkThreads + tid;
+            const uint32_t nv = s_d[i];
+            const bool lower = nv < cur[j];
+            if (lower) {
+                if (t.split)  // the result of the min is not needed
+                    __hip_atomic_fetch_min(&dist[base + i], nv, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                else
+                    dist[base + i] = nv;  // only this workgroup writes the block
+            }
+            if (__ballot(lower) != 0) {
+                any = true;
+                if (lane == 0) la.seg[(t.blk << (kBlkBits - kSegBits)) + k0 + j] = p;
+            }
+        }
+    }
+    // the run only asks whether the pass lowered anything
+    if (any && lane == 0) a.ctrl->ph_low[a.pass & 63] = 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -2065,8 +2294,10 @@ void frontier_to_queue(sssp_graph *g, int32_t r)
 // Runs one relaxation round in the given mode. `pile` is the pile buffer the
 // round reads; the host mirror of the control block holds its counters.
 // Returns true when a push round wrote the next pile (the caller swaps).
+constexpr int32_t kNotLocal = -1;
 template <class WT>
-void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st);
+void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st,
+                int32_t local = kNotLocal);
 
 template <class WT>
 bool run_round(sssp_graph *g, int mode, int kidx, int32_t r, int32_t tick0, const RoundSlot &cur,
@@ -2222,6 +2453,15 @@ void read_slot(sssp_graph *g, int32_t r)
     SSSP_HIP(hipStreamSynchronize(s));
 }
 
+}  // namespace
+
+void tile_spans(const sssp_graph *g, const BlkTile *tiles, int32_t n, TileState *state)
+{
+    if (n > 0) k_tile_spans<<<(unsigned)n, 64, 0, g->stream>>>(tiles, blk_list(g), state);
+    SSSP_LAUNCH_CHECK("k_tile_spans");
+}
+
+namespace {
 // Waits until the decision kernel has written round `seq` into the host
 // mirror: a spin on the mirror's sequence number (coherent host memory),
 // which sees the write about a microsecond after it lands -- a stream
@@ -2252,9 +2492,10 @@ constexpr int kPassAhead = 3;
 // host queueing passes as it sees them begin in the mirror's progress word.
 // With trace_events every pass is launched alone between events. Adds the
 // passes to the stats and the trace; full_limit: full passes at most (then
-// SSSP_ERR_NOT_CONVERGED).
+// SSSP_ERR_NOT_CONVERGED). local: source of a run of local passes
+// (k_blk_local), or kNotLocal: k_blk_plain.
 template <class WT>
-void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
+void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int32_t local)
 {
     hipStream_t s = g->stream;
     PassArgs a{};
@@ -2280,6 +2521,18 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
                                      : run == kRunLight ? g->n_ltile
                                                         : std::max(g->n_btile, g->n_ltile));
     const BlkList light_list{g->l_pk, g->l_cbase, g->l_wide, g->l_w};
+    LocalArgs la{};
+    if (local != kNotLocal) {
+        const int32_t n = std::max(g->n_seg, g->n_ttile);
+        la.state = g->t_state;
+        la.seg = g->t_seg;
+        a.full = g->t_tile;
+        a.n_full = g->n_ttile;
+        la.work = &g->ctrl_host_dev->ph_work;
+        k_local_reset<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+            la.seg, g->n_seg, la.state, g->n_ttile, local);
+        SSSP_LAUNCH_CHECK("k_local_reset");
+    }
     // the mirror still holds the last run's word (another tag) or none
     volatile unsigned long long *pos = &g->ctrl_host->ph_pos;
     const unsigned long long mine = pass_word(a.tag, 0, 0, 0) >> 58;
@@ -2290,8 +2543,11 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
         while (queued < begun + ahead) {
             a.pass = queued++;
             if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
-            k_blk_plain<WT><<<grid, kBlkThreads, 0, s>>>(a, blk_list(g), light_list, g->dist);
-            SSSP_LAUNCH_CHECK("k_blk_plain");
+            if (local != kNotLocal)
+                k_blk_local<WT><<<(unsigned)a.n_full, kBlkThreads, 0, s>>>(a, la, blk_list(g), g->dist);
+            else
+                k_blk_plain<WT><<<grid, kBlkThreads, 0, s>>>(a, blk_list(g), light_list, g->dist);
+            SSSP_LAUNCH_CHECK("blocked pass");
             if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r1, s));
         }
         unsigned long long w = 0;
@@ -2335,13 +2591,16 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st)
     }
     st->iterations += passes;
     st->n_all += passes;
-    st->edges_relaxed += (int64_t)full * g->E + (int64_t)light * g->light_edges;
+    st->edges_relaxed += local != kNotLocal
+                             ? *(volatile int64_t *)&g->ctrl_host->ph_work * kBlkChunk
+                             : (int64_t)full * g->E + (int64_t)light * g->light_edges;
 }
 
 // The plain pass loop: full passes until one changes nothing (mixed: with
-// light passes between them, see k_blk_plain).
+// light passes between them, see k_blk_plain, or local passes where the graph
+// has their tiles: one source then).
 template <class WT>
-void solve_plain(sssp_graph *g, bool mixed, sssp_stats *st)
+void solve_plain(sssp_graph *g, bool mixed, int32_t source, sssp_stats *st)
 {
     hipStream_t s = g->stream;
     const int64_t E = g->E;
@@ -2349,6 +2608,10 @@ void solve_plain(sssp_graph *g, bool mixed, sssp_stats *st)
     const int64_t limit = std::min<int64_t>(4 * ((int64_t)g->max_rounds / 4 + 1),
                                             std::max<int64_t>(8, ((int64_t)g->V + 4) / 4 * 4));
     st->verify_passes = 1;  // the last pass changed nothing: the fixpoint check
+    if (mixed && g->n_ttile > 0 && g->plain_kernel != 1) {
+        run_passes<WT>(g, kRunFull, limit, st, source);
+        return;
+    }
     if (plain_uses_blocked(g)) {
         run_passes<WT>(g, mixed && WT::kWeighted && g->n_ltile > 0 ? kRunMixed : kRunFull, limit,
                        st);
@@ -2680,7 +2943,7 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
     const bool small = (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) &&
                        n_src == 1 && g->E < g->plain_below_edges;
     if (sched == SSSP_SCHED_PLAIN || small) {
-        solve_plain<WT>(g, small, st);
+        solve_plain<WT>(g, small, source, st);
         g->tick = tick0 + 1;
     } else {
         if (g->pile_dirty) {

@@ -378,11 +378,20 @@ __global__ __launch_bounds__(kBlock) void k_blk_pad(const int64_t *bptr, const i
 }
 
 // out[i] = w[i * E / n]: a fixed-stride sample of the weights
-__global__ __launch_bounds__(kBlock) void k_weight_sample(const uint32_t *w, int64_t E, int32_t n,
-                                                          uint32_t *out)
+// out[0 .. n) = sampled weights, out[n + 1] += sampled edges between near ids
+__global__ __launch_bounds__(kBlock) void k_edge_sample(const int32_t *src, const int32_t *dst,
+                                                        const uint32_t *w, int64_t E, int32_t n,
+                                                        int32_t near_ids, uint32_t *out)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) out[i] = w[i * E / n];
+    bool near = false;
+    if (i < n) {
+        const int64_t e = i * E / n;
+        out[i] = w[e];
+        near = abs(src[e] - dst[e]) < near_ids;
+    }
+    const unsigned long long m = __ballot(near);
+    if (m != 0 && __lane_id() == 0) atomicAdd(&out[n + 1], (uint32_t)__popcll(m));
 }
 
 // largest out-degree
@@ -1067,6 +1076,24 @@ void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits)
     g->blk_range_bits = range_bits;
 }
 
+// The tiles of the local passes (k_blk_local), on graphs they are for.
+static void build_local_tiles(sssp_graph *g)
+{
+    if (!g->local_graph) return;
+    const std::vector<BlkTile> tiles =
+        make_blk_tiles(g->b_off_host, kLocalTileMax, 0, BlkRanges{}, {});
+    const size_t n_seg = (g->b_off_host.size() - 1) << (kBlkBits - kSegBits);
+    g->t_tile = dmalloc<BlkTile>(tiles.size());
+    g->t_state = dmalloc<TileState>(tiles.size());
+    g->t_seg = dmalloc<int32_t>(n_seg);
+    SSSP_HIP(hipMemcpyAsync(g->t_tile, tiles.data(), sizeof(BlkTile) * tiles.size(),
+                            hipMemcpyHostToDevice, g->stream));
+    tile_spans(g, g->t_tile, (int32_t)tiles.size(), g->t_state);
+    SSSP_HIP(hipStreamSynchronize(g->stream));
+    g->n_ttile = (int32_t)tiles.size();
+    g->n_seg = (int32_t)n_seg;
+}
+
 // The weight threshold of the light class: the quantile `frac` of a sample
 // of the weights (patterns order like the weights). frac leaves every vertex
 // with out-edges about one light edge on a graph with hubs, six on one without
@@ -1080,29 +1107,36 @@ void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits)
 // With many equal weights the class can come out far from that share; below
 // half or above three times the target there are no classes (0xFFFFFFFF: every
 // edge is light and light passes do not run).
-static uint32_t light_threshold(const sssp_graph *g)
+static uint32_t light_threshold(sssp_graph *g)
 {
     const int64_t n = std::min<int64_t>(g->E, kLightSample);
-    uint32_t *d = dmalloc<uint32_t>((size_t)n + 1);
+    uint32_t *d = dmalloc<uint32_t>((size_t)n + 2);
     struct F {
         void *p;
         ~F() { dfree(p); }
     } f{d};
-    k_weight_sample<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, g->stream>>>(
-        g->el_w, g->E, (int32_t)n, d);
-    SSSP_LAUNCH_CHECK("k_weight_sample");
-    SSSP_HIP(hipMemsetAsync(d + n, 0, 4, g->stream));
+    SSSP_HIP(hipMemsetAsync(d + n, 0, 8, g->stream));
+    k_edge_sample<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, g->stream>>>(
+        g->el_src, g->el_dst, g->el_w, g->E, (int32_t)n,
+        std::min(kLocalNear, std::max(16, g->V / 32)), d);
+    SSSP_LAUNCH_CHECK("k_edge_sample");
     k_max_degree<<<grid_for(g->V), kBlock, 0, g->stream>>>(g->row_ptr, g->V, d + n);
     SSSP_LAUNCH_CHECK("k_max_degree");
-    std::vector<uint32_t> s((size_t)n + 1);
+    std::vector<uint32_t> s((size_t)n + 2);
     SSSP_HIP(hipMemcpyAsync(s.data(), d, 4 * s.size(), hipMemcpyDeviceToHost, g->stream));
     SSSP_HIP(hipStreamSynchronize(g->stream));
     const double mean = (double)g->E / std::max(g->n_nzo, 1);
-    const bool hubs = (double)s.back() >= 16.0 * mean;
-    if (!hubs && mean < kLightMinDegree) return 0xFFFFFFFFu;
+    const bool hubs = (double)s[(size_t)n] >= 16.0 * mean;
+    if (!hubs && mean < kLightMinDegree) {
+        // local passes: half the sampled edges join near ids (on random graphs
+        // of 2000-7000 vertices, whose edges all lie in one block, they took
+        // 1.4 times as long as the edge-list passes)
+        g->local_graph = (int64_t)s.back() * 2 >= n;
+        return 0xFFFFFFFFu;
+    }
     const double per_vertex = hubs ? 1.0 : 6.0;
     const double frac = std::min(0.5, std::max(1.0 / 16, per_vertex / mean));
-    s.pop_back();
+    s.resize((size_t)n);
     std::sort(s.begin(), s.end());
     const double target = frac * (double)n;
     const uint32_t at = s[(size_t)std::min<int64_t>(n - 1, (int64_t)target)];
@@ -1518,6 +1552,7 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
             range_bits = std::max(kBlkRangeFineBits, lg - 3);
         }
         retile_blocked(g, tcap, 0, range_bits);
+        build_local_tiles(g);
     }
 
     // ---- CSC ----

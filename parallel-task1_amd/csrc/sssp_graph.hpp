@@ -46,6 +46,7 @@ struct Ctrl {
     int32_t ph_low[64];
     int32_t ph_full;
     int32_t ph_done;
+    int64_t ph_work;            // host mirror: chunks relaxed by a run of local passes
     unsigned long long ph_pos;  // host mirror: progress word of the passes
     int64_t n_compact;     // lb scan: entries
     int64_t lb_total;      // lb scan: total edges
@@ -100,6 +101,22 @@ struct BlkTile {
     int32_t blk;
     int32_t split;
     int64_t e0, e1;
+};
+// Tiles of the local passes (k_blk_local): short enough to keep their edges in
+// registers, kLocalChunks chunks per wave; relaxed kLocalSweeps times between
+// barriers, kLocalRounds barriers at most, and only when a source may have
+// changed.
+constexpr int kLocalChunks = 2;
+constexpr int kLocalRounds = 3, kLocalSweeps = 4;
+constexpr int64_t kLocalTileMax = kLocalChunks * kBlkChunk * (kBlkThreads / 64);
+constexpr int kSegBits = 10;  // vertices of a segment whose changes are tracked together: a block's
+                              // row of one vertex per thread
+static_assert(1 << kSegBits == kBlkThreads, "a segment is a row of the write-back");
+constexpr int32_t kLocalNear = 1 << 12;  // edges between ids closer than this, and V / 32, are near
+struct TileState {
+    int32_t lo, hi;  // segments of its first and last source
+    int32_t done;    // pass that last relaxed it
+    int32_t work;    // chunks relaxed in the run
 };
 // Light list: the blocked list's light edges (weight at most a threshold)
 // once more, as a blocked list of their own with its own tiles, for the light
@@ -210,6 +227,12 @@ struct sssp_graph {
     int64_t l_edges = 0, l_nwide = 0;
     sssp::BlkTile *b_ltile = nullptr;
     int32_t n_ltile = 0;
+    // tiles of the local passes (n_ttile 0: the graph runs none)
+    sssp::BlkTile *t_tile = nullptr;
+    sssp::TileState *t_state = nullptr;
+    int32_t *t_seg = nullptr;  // pass of every segment's last change
+    int32_t n_ttile = 0, n_seg = 0;
+    bool local_graph = false;  // sparse, no hubs, most edges between near ids
     int64_t light_edges = 0;      // edges in the light list
     uint32_t light_thr = 0xFFFFFFFFu;  // its largest weight pattern (0xFFFFFFFF: no light list)
     std::vector<int64_t> b_off_host;  // padded block offsets (tiles are rebuilt from them)
@@ -465,6 +488,7 @@ void build_multi_layout(sssp_graph *g);
 // rebuilds the destination-blocked list's tile table (cap: edge slots per
 // tile, a multiple of kBlkChunk; order: 0 smallest first, 1 by block, 2 largest first, 3 by
 // descending block)
+void tile_spans(const sssp_graph *g, const BlkTile *tiles, int32_t n, TileState *state);
 void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits = 0);
 void device_exclusive_scan_i64(const int64_t *in, int64_t *out, int64_t n, int64_t *blk_a,
                                int64_t *blk_b, int64_t n_blk_cap, hipStream_t s);

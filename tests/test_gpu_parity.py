@@ -555,6 +555,63 @@ def test_blocked_tiles_any_cap_and_order(gpu, oracle):
                 g.set_param(name, bad)
 
 
+def _local_graph(case, rng):
+    """Edges between near ids, no hubs, fewer than 8 per vertex."""
+    if case in ("grid", "grid_u32", "grid_zero"):
+        r, c = 173, 97  # 16781 vertices: one past the first block's rows
+        v = np.arange(r * c, dtype=np.int32).reshape(r, c)
+        a = np.concatenate([v[:, :-1].ravel(), v[:-1].ravel()])
+        b = np.concatenate([v[:, 1:].ravel(), v[1:].ravel()])
+        return r * c, np.concatenate([a, b]), np.concatenate([b, a])
+    if case == "path":  # against the ids, then on with them: tiles wake each other
+        a = np.arange(30000, 0, -1, dtype=np.int32)
+        return 60002, np.concatenate([a, [0], np.arange(30001, 60001)]), np.concatenate(
+            [a - 1, [30001], np.arange(30002, 60002)])
+    if case == "one_edge":
+        return 7, np.array([3]), np.array([5])
+    if case == "tile_edges":  # one block: a tile of 8192 slots, and one of one chunk
+        V, E, span = 3000, 8193, 80
+    else:  # "band": near ids with far jumps, some of them over whole chunks of gaps
+        V, E, span = 600000, 1200000, 900
+    s = rng.integers(0, V, E)
+    d = np.clip(s + rng.integers(-span, span + 1, E), 0, V - 1)
+    if case == "band":
+        d[::50] = rng.integers(0, V, len(d[::50]))
+    return V, s, d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["grid", "grid_u32", "grid_zero", "path", "one_edge",
+                                  "tile_edges", "band"])
+def test_local_passes_bit_exact(gpu, oracle, case):
+    """Graphs of near ids (local passes: tiles relaxed several times a pass, and
+    only when a source changed) end on the oracle's fixpoint, for weights,
+    zero weights, u32 and hops, from sources in the first, a middle and the
+    last block, twice each (no state outlives a solve). Bit equality."""
+    rng = np.random.default_rng(23)
+    V, src, dst = _local_graph(case, rng)
+    src, dst = src.astype(np.int32), dst.astype(np.int32)
+    w = rng.random(len(src), dtype=np.float32)
+    if case == "grid_u32":
+        w = rng.integers(1, 256, len(src)).astype(np.uint32)
+    elif case == "grid_zero":
+        w[rng.random(len(src)) < 0.5] = 0
+    with S.DeviceGraph(src, dst, w, V) as g:
+        for source in (int(src[0]), V // 2, V - 1):
+            ref = oracle.dijkstra(src, dst, w, V, source)
+            for sched in ("heuristic", "learned", "heuristic"):
+                print(f"local passes: {case}, source {source}, {sched}", flush=True)
+                d, st = g.solve(source, sched)
+                assert np.array_equal(bits(d), bits(ref)), (case, source, sched)
+            hops = oracle.dijkstra(src, dst, np.ones(len(src), np.uint32), V, source)
+            lv = g.bfs(source, "heuristic")[1]
+            assert np.array_equal(lv, hops)
+        if case in ("grid", "path"):
+            d, plain = g.solve(int(src[0]), "plain")
+            st = g.solve(int(src[0]), "heuristic")[1]
+            assert st["iterations"] * 2 < plain["iterations"]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("E,cap", [(1, 1 << 13), (1 << 22, 1 << 13), ((1 << 22) + 1, 1 << 14),
                                    (1 << 23, 1 << 14), ((1 << 23) + 1, 1 << 15)])
