@@ -321,8 +321,10 @@ int sssp_init_distances_f64(double *d_dist, int32_t vertices, int32_t source);
 int sssp_init_distances_u32(uint32_t *d_dist, int32_t vertices, int32_t source);
 /* bellman_ford_wrapper<W> (bellman_ford.cu:103-144): all-edge passes over the
  * caller's edge list, in its order, until a pass changes nothing (at most
- * `vertices` passes). Convergence is tested on the device; *passes (may be
- * NULL) receives the pass count. The edge arrays are checked on the device
+ * `vertices` passes). A pass leaves out the edges whose source did not change
+ * since the pass before, told by a copy of the distances allocated for the call
+ * (without memory for it every pass relaxes every edge). Convergence is tested
+ * on the device; *passes (may be NULL) receives the pass count. The edge arrays are checked on the device
  * first: a vertex id outside [0, vertices) or a negative or NaN weight returns
  * SSSP_ERR_ARG before any pass (the distances are compared as unsigned bit
  * patterns, which order non-negative values only). */
@@ -338,7 +340,8 @@ int sssp_bellman_ford_u32(const int32_t *d_src, const int32_t *d_dst, const uint
 /* Allocation-free sssp_bellman_ford_f32: no counterpart in the reference. For
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc). Same arguments,
- * checks, passes and results as sssp_bellman_ford_f32, on the current device;
+ * checks and results as sssp_bellman_ford_f32, on the current device, every
+ * pass over every edge;
  * it calls no hipMalloc/hipFree. Its scratch (64 change flags and 2 validation
  * counters, 272 of 512 bytes) is a file-scope device array that each device
  * keeps until the process ends; the scratch does not grow with the graph, so

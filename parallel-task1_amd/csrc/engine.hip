@@ -3319,10 +3319,211 @@ void ref_init(DT *d, int32_t V, int32_t source)
     SSSP_HIP(hipDeviceSynchronize());
 }
 
+// The wrappers' passes over the caller's edges, in the caller's order: an edge
+// is relaxed only when its source changed since the pass before. Whether it
+// did is one bit in the workgroup's LDS, so an edge that is not relaxed costs
+// 4 bytes of stream and no gather, and its line of destinations and weights is
+// read only where another edge needs it. The pass over every edge (k_el_pass)
+// took 0.275 ms on a power-law graph of 2^20 vertices and 2^24 edges, bound
+// by the two random distance reads per edge (a distance array as large as an
+// XCD's L2); now 0.02-0.09 ms but for six passes of 0.14-0.41, at 22 passes
+// instead of 16 (a pass no longer sees the changes of its own): a call 4.8 ->
+// 2.7 ms. Uniform 500 K x 16, u32 2.9 -> 1.6 ms, power-law 300 K x 14 f64 1.15 ->
+// 0.86. kActBits bits fill most of a CU's LDS; half of them with two
+// workgroups per CU 3.0 ms, a quarter 3.2. kActUnroll 1 / 2 / 4 groups of four
+// edges in flight per lane: 2.79 / 2.69 / 2.62 ms, f64 0.88 / 0.85 / 0.92.
+constexpr int kActUnroll = 2;
+constexpr int32_t kActBits = 1 << 20;
+constexpr int kActThreads = 1024;
+constexpr size_t kActFlagBytes = 256;
+// Fewer edges run every edge in one launch a pass: R-MAT 14 x 16 0.287 ms against
+// 0.305, uniform 2000 x 4 0.26 against 0.30, power-law 100 K x 16 0.88 against 0.65.
+constexpr int64_t kActMinEdges = 1 << 19;
+constexpr int kActBatch = 6;  // passes queued per host check (an idle pass and mark: 4-8 us)
+
+// Vertices changed since the mark before, one bit each in bits[] (bit v & mask;
+// several vertices share one where V exceeds the mask). The first mark takes
+// every vertex with a distance. flags[p & 63] = 1 when mark p found any; a mark
+// after one that found none returns at once, and so does pass p.
+template <class DT>
+__global__ __launch_bounds__(kBlock) void k_mark_changed(const DT *__restrict__ dist, DT *snap,
+                                                         int32_t V, int32_t n_bits,
+                                                         unsigned long long *bits, int32_t *flags,
+                                                         int32_t p, DT inf)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) flags[(p + 1) & 63] = 0;
+    if (p > 0 && flags[(p - 1) & 63] == 0) return;
+    const int lane = __lane_id();
+    bool found = false;
+    const int words = (n_bits + 63) / 64;
+    const int wave = (int)(blockIdx.x * (kBlock / 64)) + ((int)threadIdx.x >> 6);
+    for (int i = wave; i < words; i += (int)gridDim.x * (kBlock / 64)) {
+        bool ch = false;
+        for (int64_t v = (int64_t)i * 64 + lane; v < V; v += n_bits) {
+            const DT d = dist[v];
+            if (d != (p > 0 ? snap[v] : inf)) {
+                ch = true;
+                snap[v] = d;
+            } else if (p == 0) {
+                snap[v] = d;
+            }
+        }
+        const unsigned long long m = __ballot(ch);
+        if (lane == 0) bits[i] = m;
+        found |= m != 0;
+    }
+    if (found && lane == 0) flags[p & 63] = 1;
+}
+
+template <class WT, class DT, int VEC>
+__global__ __launch_bounds__(kActThreads) void k_el_active(const int32_t *__restrict__ src,
+                                                    const int32_t *__restrict__ dst,
+                                                    const DT *__restrict__ w, int64_t E, DT *dist,
+                                                    const unsigned long long *__restrict__ bits,
+                                                    int32_t n_bits, int32_t mask,
+                                                    const int32_t *flags, int32_t p,
+                                                    int64_t per_block)
+{
+    extern __shared__ uint32_t s_bits[];
+    if (flags[p & 63] == 0) return;
+    const int tid = threadIdx.x;
+    {
+        const int words = (n_bits + 63) / 64;
+        uint64_t *s64 = reinterpret_cast<uint64_t *>(s_bits);
+        for (int i = tid; i < words; i += kActThreads) s64[i] = bits[i];
+    }
+    __syncthreads();
+    auto active = [&](int32_t v) {
+        const int32_t b = v & mask;
+        return (s_bits[b >> 5] >> (b & 31) & 1u) != 0;
+    };
+    auto relax = [&](DT du, DT dv, int32_t t, DT ww) {
+        if (du == WT::INF) return;
+        const DT cand = WT::add(du, ww);
+        if (cand < dv)
+            __hip_atomic_fetch_min(&dist[t], cand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    const int64_t b = xcd_tile(blockIdx.x, gridDim.x);
+    if constexpr (VEC == 4) {
+        typedef int32_t v4i __attribute__((ext_vector_type(4)));
+        typedef DT v4w __attribute__((ext_vector_type(4)));
+        const v4i *s4 = reinterpret_cast<const v4i *>(src);
+        const v4i *t4 = reinterpret_cast<const v4i *>(dst);
+        const v4w *w4 = reinterpret_cast<const v4w *>(w);
+        const int64_t g0 = b * per_block, g1 = min(g0 + per_block, E >> 2);
+        for (int64_t g = g0 + tid; g < g1; g += kActThreads * kActUnroll) {
+            v4i s[kActUnroll];
+#pragma unroll
+            for (int u = 0; u < kActUnroll; u++) {
+                s[u] = v4i{0, 0, 0, 0};
+                if (g + u * kActThreads < g1) s[u] = __builtin_nontemporal_load(&s4[g + u * kActThreads]);
+            }
+            uint32_t act = 0;
+#pragma unroll
+            for (int u = 0; u < kActUnroll; u++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (active(s[u][j])) act |= 1u << (u * 4 + j);
+#pragma unroll
+            for (int u = 0; u < kActUnroll; u++)
+                if (g + u * kActThreads >= g1) act &= ~(15u << (u * 4));
+            v4i t[kActUnroll];
+            v4w ww[kActUnroll];
+            DT du[kActUnroll * 4];
+#pragma unroll
+            for (int u = 0; u < kActUnroll; u++) {
+                if (!(act >> (u * 4) & 15u)) continue;
+                t[u] = __builtin_nontemporal_load(&t4[g + u * kActThreads]);
+                ww[u] = __builtin_nontemporal_load(&w4[g + u * kActThreads]);
+            }
+#pragma unroll
+            for (int e = 0; e < kActUnroll * 4; e++)
+                du[e] = act >> e & 1u ? dist[s[e >> 2][e & 3]] : (DT)WT::INF;
+            DT dv[kActUnroll * 4];
+#pragma unroll
+            for (int e = 0; e < kActUnroll * 4; e++)
+                if (act >> e & 1u) dv[e] = dist[t[e >> 2][e & 3]];
+#pragma unroll
+            for (int e = 0; e < kActUnroll * 4; e++)
+                if (act >> e & 1u) relax(du[e], dv[e], t[e >> 2][e & 3], ww[e >> 2][e & 3]);
+        }
+        if (b == 0 && tid < (E & 3)) {
+            const int64_t e = ((E >> 2) << 2) + tid;
+            if (active(src[e])) relax(dist[src[e]], dist[dst[e]], dst[e], w[e]);
+        }
+    } else {
+        const int64_t e0 = b * per_block, e1 = min(e0 + per_block, E);
+        for (int64_t e = e0 + tid; e < e1; e += kActThreads) {
+            const int32_t s = src[e];
+            if (active(s)) relax(dist[s], dist[dst[e]], dst[e], w[e]);
+        }
+    }
+}
+
+template <class WT, class DT>
+void ref_bf_active(const int32_t *src, const int32_t *dst, const DT *w, int32_t V, int64_t E, DT *d,
+                   int32_t *passes_out, unsigned char *mem)
+{
+    int dev = 0, cus = 0;
+    SSSP_HIP(hipGetDevice(&dev));
+    SSSP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int32_t n_bits = std::min(V, kActBits), mask = V <= kActBits ? INT32_MAX : kActBits - 1;
+    const size_t lds = ((size_t)n_bits + 63) / 64 * 8;
+    int32_t *flags = reinterpret_cast<int32_t *>(mem);
+    unsigned long long *bits = reinterpret_cast<unsigned long long *>(mem + kActFlagBytes);
+    DT *snap = reinterpret_cast<DT *>(mem + kActFlagBytes + kActBits / 8);
+    k_fill<int32_t><<<1, 64>>>(flags, 64, 0);
+    SSSP_LAUNCH_CHECK("clear change flags");
+    const bool vec = reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(dst) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(w) % 16 == 0;
+    const int64_t units = vec ? E >> 2 : E;
+    const int64_t full = (int64_t)cus * (lds <= 80 * 1024 ? 2 : 1);
+    const int64_t nblocks = std::max<int64_t>(1, std::min(full, (units + kActThreads - 1) / kActThreads));
+    const int64_t per_block = (units + nblocks - 1) / nblocks;
+    const unsigned mgrid = grid_for(n_bits, 1024);
+    int32_t hc[64], pass = 0, done = -1;
+    while (done < 0) {
+        for (int i = 0; i < kActBatch; i++) {
+            k_mark_changed<DT><<<mgrid, kBlock>>>(d, snap, V, n_bits, bits, flags, pass + i,
+                                                  (DT)WT::INF);
+            if (vec)
+                k_el_active<WT, DT, 4><<<(unsigned)nblocks, kActThreads, lds>>>(
+                    src, dst, w, E, d, bits, n_bits, mask, flags, pass + i, per_block);
+            else
+                k_el_active<WT, DT, 1><<<(unsigned)nblocks, kActThreads, lds>>>(
+                    src, dst, w, E, d, bits, n_bits, mask, flags, pass + i, per_block);
+            SSSP_LAUNCH_CHECK("bellman_ford pass");
+        }
+        SSSP_HIP(hipMemcpy(hc, flags, sizeof(hc), hipMemcpyDeviceToHost));
+        for (int i = 0; i < kActBatch && done < 0; i++)
+            if (hc[(pass + i) & 63] == 0) done = pass + i;
+        pass += kActBatch;
+        if (done < 0 && pass >= V + 4)
+            throw Error{SSSP_ERR_NOT_CONVERGED, "Bellman-Ford did not converge within V passes"};
+    }
+    if (passes_out) *passes_out = std::max(done, 1);
+}
+
 template <class WT, class DT>
 void ref_bf(const int32_t *src, const int32_t *dst, const DT *w, int32_t V, int64_t E, DT *d,
             int32_t *passes_out, int32_t *changed_buf)
 {
+    if (!changed_buf && E >= kActMinEdges) {
+        // the passes that keep the distances of the pass before; when there
+        // is no memory for those, the passes over every edge
+        void *mem = nullptr;
+        if (hipMalloc(&mem, kActFlagBytes + kActBits / 8 + sizeof(DT) * (size_t)V) == hipSuccess) {
+            struct Free {
+                void *p;
+                ~Free() { dfree(p); }
+            } fr{mem};
+            ref_bf_active<WT, DT>(src, dst, w, V, E, d, passes_out,
+                                  static_cast<unsigned char *>(mem));
+            return;
+        }
+        (void)hipGetLastError();
+    }
     int dev = 0;
     SSSP_HIP(hipGetDevice(&dev));
     hipDeviceProp_t prop;

@@ -96,3 +96,38 @@ def test_wrappers_reject_bad_arrays(gpu, lib):
             assert ("weight" in msg) if "weight" in name else ("outside" in msg), msg
     with HipBuffer(s) as a, HipBuffer(bad_id) as b, HipBuffer(np.zeros(V, np.uint8)) as vis:
         assert lib.sssp_bfs_edges(a.ptr, b.ptr, V, len(s), vis.ptr, 0, None) == S.ERR_ARG
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.uint32], ids=["f32", "f64", "u32"])
+@pytest.mark.parametrize("V,E,shift", [(1, 3, 0), (65, (1 << 19) - 1, 0),
+                                       (1, (1 << 19) + 3, 0), (65, 1 << 19, 1), (1 << 20, 3 << 20, 0), ((1 << 20) + 1, (3 << 20) + 2, 0),
+                                       (3000000, 4000003, 1)])
+def test_wrapper_change_bits(gpu, lib, oracle, dtype, V, E, shift):
+    """The change bits of the wrappers' passes, on both sides of the edge count they
+    start at: fewer vertices than a word,
+    exactly as many as bits, one and many more (vertices share bits), edge
+    counts off the vector width, arrays one element off their alignment; and
+    a second call that goes on from distances the caller lowered. Bit
+    equality with the oracle."""
+    rng = np.random.default_rng(V + E)
+    s = (rng.random(E) ** 2 * V).astype(np.int32)
+    d = rng.integers(0, V, E).astype(np.int32)
+    w = rng.integers(1, 256, E).astype(dtype) if dtype == np.uint32 else rng.random(E).astype(dtype)
+    a, b = int(s[0]), int(s[-1])
+    pad = [np.concatenate([x[:shift], x]) for x in (s, d, w)]
+    k, size = SUFFIX[dtype], np.dtype(dtype).itemsize
+    refs = [oracle.bf(s, d, w, V, x)[0] for x in (a, b)]
+    with HipBuffer(pad[0]) as ds, HipBuffer(pad[1]) as dd, HipBuffer(pad[2]) as dw, \
+            HipBuffer(np.zeros(V, dtype)) as dist:
+        at = [C.c_void_p(C.cast(x.ptr, C.c_void_p).value + shift * n)
+              for x, n in ((ds, 4), (dd, 4), (dw, size))]
+        assert getattr(lib, "sssp_init_distances_" + k)(dist.ptr, V, a) == S.OK
+        for source, ref in ((a, refs[0]), (b, np.minimum(*refs))):
+            print(f"wrapper bits: {k} V {V} E {E} shift {shift} source {source}", flush=True)
+            if source != a:
+                one = C.c_void_p(C.cast(dist.ptr, C.c_void_p).value + source * size)
+                assert getattr(lib, "sssp_init_distances_" + k)(one, 1, 0) == S.OK
+            assert getattr(lib, "sssp_bellman_ford_" + k)(*at, V, E, source, dist.ptr,
+                                                           None) == S.OK, S.last_error()
+            assert np.array_equal(_bits(dist.get()), _bits(ref))
