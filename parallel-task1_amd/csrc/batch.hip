@@ -209,11 +209,22 @@ __global__ __launch_bounds__(kBlock) void k_chunk_sources(const int32_t *src, in
 // a round lowers nothing. Bound by latency: LDS and the chunk loads.
 // 1024 R-MAT graphs of 2^8-2^14 vertices x 8: 0.39 ms, against 3.86 with
 // distances, queues and stamps in global memory (k_wg_solve); 1500 of 2^8-2^10 x 6
-// 0.068 against 0.31. The class sizes let two workgroups of 1024 threads (2^14
+// 0.068 against 0.31. One R-MAT graph of 2^11 vertices x 16: 56 us on the device,
+// 141 in the pass loop. The class sizes let two workgroups of 1024 threads (2^14
 // vertices) or eight of 256 (2^11) share a CU's 160 KB.
-template <class WT, int BS, int NV>
+// SOLO: one solve of a whole graph (launch_solo), its task in `solo`; the
+// workgroup also writes the caller-order copy and reports to the host mirror.
+struct SoloArgs {
+    BatchTask task;
+    const int32_t *vperm;  // slot of the caller's vertex, when relabelled
+    uint32_t *dout;        // distances by the caller's ids, when relabelled
+    Ctrl *mirror;
+    int32_t limit;         // rounds at most
+};
+
+template <class WT, int BS, int NV, bool SOLO = false>
 __global__ __launch_bounds__(BS) void k_lds_solve(const BatchTask *__restrict__ tasks,
-                                                  int32_t *counter,
+                                                  const SoloArgs solo, int32_t *counter,
                                                   const int64_t *__restrict__ row_ptr,
                                                   const int32_t *__restrict__ src,
                                                   const int32_t *__restrict__ dst,
@@ -230,8 +241,9 @@ __global__ __launch_bounds__(BS) void k_lds_solve(const BatchTask *__restrict__ 
     __shared__ uint32_t s_bits[2][NW];
     const int tid = threadIdx.x, lane = __lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const BatchTask T = tasks[blockIdx.x];
+    const BatchTask T = SOLO ? solo.task : tasks[blockIdx.x];
     const int nv = T.nv;
+    int32_t chunks = 0, rounds = 0;  // SOLO: chunks this wave relaxed
     for (int v = tid; v < nv; v += BS) s_d[v] = INF;
     for (int i = tid; i < 2 * NW; i += BS) s_bits[0][i] = 0u;
     __syncthreads();
@@ -266,7 +278,13 @@ __global__ __launch_bounds__(BS) void k_lds_solve(const BatchTask *__restrict__ 
     };
     int cur = 0;
     for (int32_t round = 0;; round++) {
-        if (round > nv + 2) {  // cannot happen for w >= 0; bounded anyway
+        if (SOLO) {
+            if (round >= solo.limit) {
+                rounds = -1;
+                break;
+            }
+            rounds = round + 1;
+        } else if (round > nv + 2) {  // cannot happen for w >= 0; bounded anyway
             if (tid == 0) counter[1] = 1;
             break;
         }
@@ -288,6 +306,7 @@ __global__ __launch_bounds__(BS) void k_lds_solve(const BatchTask *__restrict__ 
                 }
             }
             uint64_t todo = __ballot(live);
+            if (SOLO) chunks += __popcll(todo);
             auto next = [&](Edges &x, int64_t &c) {
                 const int i = __builtin_ctzll(todo);
                 todo &= todo - 1;
@@ -329,6 +348,31 @@ __global__ __launch_bounds__(BS) void k_lds_solve(const BatchTask *__restrict__ 
     }
     uint32_t *const out = bdist + T.doff;
     for (int v = tid; v < nv; v += BS) out[v] = s_d[v];
+    if constexpr (SOLO) {
+        if (solo.vperm)
+            for (int v = tid; v < nv; v += BS) solo.dout[v] = s_d[solo.vperm[v]];
+        int reached = 0;
+        for (int v = tid; v < nv; v += BS) reached += s_d[v] != INF ? 1 : 0;
+        reached = wave_sum32(reached);
+        // the bitmaps are no longer needed: a wave's counts in their place
+        __syncthreads();
+        if (lane == 0) {
+            s_bits[0][wave] = (uint32_t)reached;
+            s_bits[1][wave] = (uint32_t)chunks;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            int64_t r = 0, c = 0;
+            for (int i = 0; i < kWaves; i++) {
+                r += s_bits[0][i];
+                c += s_bits[1][i];
+            }
+            solo.mirror->n_reached = r;
+            solo.mirror->ph_work = c;
+            solo.mirror->ph_full = rounds;
+            __threadfence_system();
+        }
+    }
 }
 
 template <class WT>
@@ -337,21 +381,35 @@ void launch_lds_t(int c, unsigned n, hipStream_t s, const BatchTask *tasks, sssp
     switch (c) {
     case 1:
         k_lds_solve<WT, 1024, kLdsVerts[1]><<<n, 1024, 0, s>>>(
-            tasks, g->bcounter, g->row_ptr, g->el_src, g->el_dst, g->el_w, g->E, g->el_first,
+            tasks, SoloArgs{}, g->bcounter, g->row_ptr, g->el_src, g->el_dst, g->el_w, g->E, g->el_first,
             g->bdist);
         break;
     case 2:
         k_lds_solve<WT, 1024, kLdsVerts[2]><<<n, 1024, 0, s>>>(
-            tasks, g->bcounter, g->row_ptr, g->el_src, g->el_dst, g->el_w, g->E, g->el_first,
+            tasks, SoloArgs{}, g->bcounter, g->row_ptr, g->el_src, g->el_dst, g->el_w, g->E, g->el_first,
             g->bdist);
         break;
     default:
         k_lds_solve<WT, 256, kLdsVerts[3]><<<n, 256, 0, s>>>(
-            tasks, g->bcounter, g->row_ptr, g->el_src, g->el_dst, g->el_w, g->E, g->el_first,
+            tasks, SoloArgs{}, g->bcounter, g->row_ptr, g->el_src, g->el_dst, g->el_w, g->E, g->el_first,
             g->bdist);
         break;
     }
     SSSP_LAUNCH_CHECK("k_lds_solve");
+}
+
+template <class WT>
+void launch_solo_t(sssp_graph *g, int32_t source, int32_t limit)
+{
+    SoloArgs a{};
+    a.task = BatchTask{0, 0, g->V, source};
+    a.vperm = g->vperm;
+    a.dout = g->dout;
+    a.mirror = g->ctrl_host_dev;
+    a.limit = limit;
+    k_lds_solve<WT, 1024, kLdsVerts[1], true><<<1, 1024, 0, g->stream>>>(
+        nullptr, a, nullptr, g->row_ptr, g->el_src, g->el_dst, g->el_w, g->E, g->el_first, g->dist);
+    SSSP_LAUNCH_CHECK("k_lds_solve (one graph)");
 }
 
 template <int BS>
@@ -431,13 +489,7 @@ double run_wg(sssp_graph *g, const TaskCounts &tc, int64_t maxv, int bs, int wgp
     int32_t nwg = g->cu_count * wgpcu;
     if (nwg > ntasks) nwg = ntasks;
     if (nwg < 1) nwg = 1;
-    if (!g->el_first) {
-        const int64_t nch = (g->E + kBlkChunk - 1) / kBlkChunk;
-        g->el_first = dmalloc<int32_t>((size_t)nch + 1);
-        k_chunk_sources<<<(unsigned)std::min<int64_t>(nch / kBlock + 1, 4096), kBlock, 0, s>>>(
-            g->el_src, nch, g->V, g->el_first);
-        SSSP_LAUNCH_CHECK("k_chunk_sources");
-    }
+    ensure_chunk_sources(g);
     const int64_t key[10] = {ntasks, maxv, bs, nwg, (int64_t)(uintptr_t)g->bdist,
                              (int64_t)(uintptr_t)g->bscratch, (int64_t)(uintptr_t)g->btasks,
                              (int64_t)(uintptr_t)g->bround, tc.n[1] + ((int64_t)tc.n[2] << 32),
@@ -1180,6 +1232,28 @@ void check_pack_sources(const sssp_pack *p, const int32_t *sources)
 }
 
 }  // namespace
+
+bool solo_fits(const sssp_graph *g)
+{
+    return g->V <= kLdsVerts[1] && g->E <= (g->n_ttile > 0 ? kSoloLocalEdges : kSoloEdges);
+}
+
+void ensure_chunk_sources(sssp_graph *g)
+{
+    if (g->el_first) return;
+    const int64_t nch = (g->E + kBlkChunk - 1) / kBlkChunk;
+    g->el_first = dmalloc<int32_t>((size_t)nch + 1);
+    k_chunk_sources<<<(unsigned)std::min<int64_t>(nch / kBlock + 1, 4096), kBlock, 0, g->stream>>>(
+        g->el_src, nch, g->V, g->el_first);
+    SSSP_LAUNCH_CHECK("k_chunk_sources");
+}
+
+void launch_solo(sssp_graph *g, int32_t source, bool hops, int32_t limit)
+{
+    if (hops) launch_solo_t<WUnit>(g, source, limit);
+    else if (g->wtype == SSSP_W_F32) launch_solo_t<WF32>(g, source, limit);
+    else launch_solo_t<WU32>(g, source, limit);
+}
 }  // namespace sssp
 
 extern "C" {

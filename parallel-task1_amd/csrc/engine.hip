@@ -2596,6 +2596,14 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int3
                              : (int64_t)full * g->E + (int64_t)light * g->light_edges;
 }
 
+// Passes at most of a plain solve: max_rounds and V + 1, in whole groups of
+// four.
+int64_t plain_limit(const sssp_graph *g)
+{
+    return std::min<int64_t>(4 * ((int64_t)g->max_rounds / 4 + 1),
+                             std::max<int64_t>(8, ((int64_t)g->V + 4) / 4 * 4));
+}
+
 // The plain pass loop: full passes until one changes nothing (mixed: with
 // light passes between them, see k_blk_plain, or local passes where the graph
 // has their tiles: one source then).
@@ -2604,9 +2612,7 @@ void solve_plain(sssp_graph *g, bool mixed, int32_t source, sssp_stats *st)
 {
     hipStream_t s = g->stream;
     const int64_t E = g->E;
-    // passes at most: max_rounds and V + 1, in whole groups of four
-    const int64_t limit = std::min<int64_t>(4 * ((int64_t)g->max_rounds / 4 + 1),
-                                            std::max<int64_t>(8, ((int64_t)g->V + 4) / 4 * 4));
+    const int64_t limit = plain_limit(g);
     st->verify_passes = 1;  // the last pass changed nothing: the fixpoint check
     if (mixed && g->n_ttile > 0 && g->plain_kernel != 1) {
         run_passes<WT>(g, kRunFull, limit, st, source);
@@ -2909,6 +2915,29 @@ void upload_sources(sssp_graph *g, const int32_t *sources, int32_t n)
     SSSP_HIP(hipMemcpyAsync(g->src_list, sources, 4 * (size_t)n, hipMemcpyHostToDevice, g->stream));
 }
 
+// A small graph solved whole in one workgroup's LDS: one launch, one host wait.
+template <class WT>
+void solve_solo(sssp_graph *g, int32_t source, sssp_stats *st)
+{
+    hipStream_t s = g->stream;
+    SSSP_HIP(hipEventRecord(g->ev_a, s));
+    launch_solo(g, source, !WT::kWeighted, (int32_t)std::min<int64_t>(plain_limit(g), INT32_MAX));
+    SSSP_HIP(hipEventRecord(g->ev_b, s));
+    SSSP_HIP(hipEventSynchronize(g->ev_b));
+    const Ctrl &h = *g->ctrl_host;
+    if (h.ph_full < 0)
+        throw Error{SSSP_ERR_NOT_CONVERGED,
+                    "plain Bellman-Ford did not converge within max_rounds or V passes"};
+    float ms = 0.f;
+    SSSP_HIP(hipEventElapsedTime(&ms, g->ev_a, g->ev_b));
+    st->t_solve_ms = ms;
+    st->gteps = ms > 0 ? (double)g->E / (ms * 1e-3) / 1e9 : 0.0;
+    st->verify_passes = 1;  // the last round lowered nothing
+    st->iterations = st->n_all = h.ph_full;
+    st->edges_relaxed = h.ph_work * kBlkChunk;
+    st->reached = (int32_t)h.n_reached;
+}
+
 template <class WT>
 void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, sssp_stats *st)
 {
@@ -2919,9 +2948,22 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
     }
     const int32_t tick0 = g->tick;
     const int32_t source = sources[0];
+    // Below plain_below_edges the rule and the network hand the whole solve
+    // to the plain pass loop: its passes (the blocked pass from 64 tiles)
+    // then cost less than the rounds with their fixed per-round cost.
+    // Measured (learned, ms): R-MAT 21 x 16 (2^25 edges) 2.98 plain against
+    // 3.66 in rounds, BFS 0.79 against 0.95; at 2^26 edges about even (R-MAT
+    // 22 x 16 5.12 / 5.00, R-MAT 21 x 32 4.46 / 4.71); R-MAT 22 x 32 (2^27)
+    // 7.1 against 5.6 in rounds.
+    const bool small = (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) &&
+                       n_src == 1 && g->E < g->plain_below_edges;
     if (n_src > 1) upload_sources(g, sources, n_src);
     g->trace.clear();
     g->snap_round = -1;
+    if (small && solo_fits(g) && g->plain_kernel == 0 && !g->trace_events) {
+        solve_solo<WT>(g, source, st);
+        return;
+    }
     SSSP_HIP(hipEventRecord(g->ev_a, s));
     k_fill<uint32_t><<<grid_for(g->V), kBlock, 0, s>>>(g->dist, g->V, WT::INF);
     SSSP_LAUNCH_CHECK("k_fill dist");
@@ -2933,15 +2975,6 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
             g->ctrl, g->dist, g->stamp, g->queue[0], g->row_ptr, g->src_list, n_src, tick0);
         SSSP_LAUNCH_CHECK("k_init_sources");
     }
-    // Below plain_below_edges the rule and the network hand the whole solve
-    // to the plain pass loop: its passes (the blocked pass from 64 tiles)
-    // then cost less than the rounds with their fixed per-round cost.
-    // Measured (learned, ms): R-MAT 21 x 16 (2^25 edges) 2.98 plain against
-    // 3.66 in rounds, BFS 0.79 against 0.95; at 2^26 edges about even (R-MAT
-    // 22 x 16 5.12 / 5.00, R-MAT 21 x 32 4.46 / 4.71); R-MAT 22 x 32 (2^27)
-    // 7.1 against 5.6 in rounds.
-    const bool small = (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) &&
-                       n_src == 1 && g->E < g->plain_below_edges;
     if (sched == SSSP_SCHED_PLAIN || small) {
         solve_plain<WT>(g, small, source, st);
         g->tick = tick0 + 1;

@@ -1137,12 +1137,13 @@ static uint32_t light_threshold(sssp_graph *g)
     const double per_vertex = hubs ? 1.0 : 6.0;
     const double frac = std::min(0.5, std::max(1.0 / 16, per_vertex / mean));
     s.resize((size_t)n);
-    std::sort(s.begin(), s.end());
     const double target = frac * (double)n;
-    const uint32_t at = s[(size_t)std::min<int64_t>(n - 1, (int64_t)target)];
+    const auto nth = s.begin() + std::min<int64_t>(n - 1, (int64_t)target);
+    std::nth_element(s.begin(), nth, s.end());
+    const uint32_t at = *nth;
     // the class is w <= thr: `at` itself, or the value before it
-    const int64_t up = std::upper_bound(s.begin(), s.end(), at) - s.begin();
-    const int64_t lo = std::lower_bound(s.begin(), s.end(), at) - s.begin();
+    const int64_t up = std::count_if(s.begin(), s.end(), [at](uint32_t x) { return x <= at; });
+    const int64_t lo = std::count_if(s.begin(), s.end(), [at](uint32_t x) { return x < at; });
     const bool use_lo = at > 0 && std::abs((double)lo - target) < std::abs((double)up - target);
     const double got = use_lo ? (double)lo : (double)up;
     if (got < 0.5 * target || got > 3.0 * target || got > 0.75 * (double)n) return 0xFFFFFFFFu;
@@ -1554,6 +1555,7 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         retile_blocked(g, tcap, 0, range_bits);
         build_local_tiles(g);
     }
+    if (solo_fits(g)) ensure_chunk_sources(g);
 
     // ---- CSC ----
     if (build_csc) {

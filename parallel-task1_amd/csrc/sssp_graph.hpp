@@ -387,7 +387,8 @@ struct sssp_graph {
     int batch_policy = 0, batch_bs = 256, batch_wgpcu = 2;
     void *batch_exec = nullptr;  // hipGraphExec_t of the captured persistent launch
     int64_t batch_key[10] = {};
-    int32_t *el_first = nullptr;  // source of every 256th edge, V at the end (on demand)
+    int32_t *el_first = nullptr;  // source of every 256th edge, V at the end (built with a
+                                  // graph that solo_fits, on demand for the others)
     void *btasks = nullptr;      // device BatchTask array
     int32_t btask_cap = 0;
     int32_t *bcounter = nullptr;  // task counter + error flag
@@ -464,6 +465,21 @@ class Prefault {
     std::atomic<bool> go_{false};
     std::vector<std::thread> threads_;
 };
+
+// batch.hip
+// Graphs solved whole in one workgroup's LDS (launch_solo): one launch and one
+// wait, where the pass loop has a launch per pass and a wait per four. One
+// workgroup reads every live chunk of a round itself, so the line lies where
+// that costs what the launches do. A whole call, us, pass loop / in LDS: R-MAT
+// 8 x 8 137 / 42, 11 x 16 (2^15 edges) 199 / 81, 13 x 8 222 / 124, 13 x 16 (2^17)
+// 259 / 200, 14 x 16 (2^18) 267 / 301, 15 x 15 351 / 530; uniform 10 K x 10
+// 263 / 195, 30 K x 7 355 / 426. Local passes take fewer rounds on long paths:
+// grid 20 x 20 149 / 78, 40 x 50 (2^13 edges) 177 / 169, 100 x 100 331 / 527.
+constexpr int64_t kSoloEdges = (int64_t)1 << 17;
+constexpr int64_t kSoloLocalEdges = (int64_t)1 << 13;
+bool solo_fits(const sssp_graph *g);
+void ensure_chunk_sources(sssp_graph *g);
+void launch_solo(sssp_graph *g, int32_t source, bool hops, int32_t limit);
 
 // gen.hip
 void rmat_device(int scale, int ef, int a, int b, int c, int d, uint32_t base_seed, int T,

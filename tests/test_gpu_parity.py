@@ -613,6 +613,45 @@ def test_local_passes_bit_exact(gpu, oracle, case):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("V,E,kind", [(1, 1, "f32"), (64, 255, "f32"), (65, 256, "u32"),
+                                      (1 << 15, 1 << 17, "f32"), (1 << 15, (1 << 17) + 1, "f32"),
+                                      ((1 << 15) + 1, 1 << 17, "f32"), (1 << 15, 100003, "relabel"),
+                                      (300, 70001, "ties"), (2001, 0, "f32")])
+def test_graphs_solved_whole_in_lds(gpu, oracle, V, E, kind):
+    """Both sides of the sizes up to which a single solve runs in one
+    workgroup, chunk remainders, a relabelled graph, no edges, hops, and a
+    round limit below what the solve needs. Bit equality with the oracle."""
+    rng = np.random.default_rng(V + E)
+    src = (rng.random(E) ** 2 * V).astype(np.int32)
+    dst = rng.integers(0, V, E).astype(np.int32)
+    w = rng.integers(1, 256, E).astype(np.uint32) if kind == "u32" else rng.random(E, np.float32)
+    if kind == "ties":
+        w = np.full(E, 0.5, np.float32)
+    with S.DeviceGraph(src, dst, w, V, relabel=kind == "relabel") as g:
+        for source in sorted({int(src[0]) if E else 0, V - 1}):
+            ref = oracle.dijkstra(src, dst, w, V, source)
+            hops = oracle.dijkstra(src, dst, np.ones(E, np.uint32), V, source)
+            for sched in ("heuristic", "learned", "plain"):
+                print(f"in LDS: V {V} E {E} {kind}, source {source}, {sched}", flush=True)
+                d, st = g.solve(source, sched)
+                assert np.array_equal(bits(d), bits(ref)), sched
+                assert st["reached"] == (ref != S.U32_INF if kind == "u32"
+                                         else ref != S.F32_INF).sum()
+                assert st["iterations"] >= 1 and st["verify_passes"] == 1
+            assert np.array_equal(g.bfs(source, "heuristic")[1], hops)
+            assert np.array_equal(bits(g.solve(source)[0]), bits(g.distances()))
+        if V == 64:
+            path = S.DeviceGraph(np.arange(63, dtype=np.int32), np.arange(1, 64, dtype=np.int32),
+                                 np.ones(63, np.float32), 64)
+            with path:
+                path.set_param("max_rounds", 1)
+                with pytest.raises(S.SSSPError):
+                    path.solve(0, "heuristic")
+                path.set_param("max_rounds", 1000)
+                assert path.solve(0, "heuristic")[0][63] == 63
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,cap", [(1, 1 << 13), (1 << 22, 1 << 13), ((1 << 22) + 1, 1 << 14),
                                    (1 << 23, 1 << 14), ((1 << 23) + 1, 1 << 15)])
 def test_default_tile_cap(gpu, oracle, E, cap):
