@@ -5,10 +5,10 @@
 //     (graph.hpp:316-361: per-source order = edge-list order);
 //   * the CSC (in-edges grouped by dst, stable) for pull rounds;
 //   * static lists of vertices with out-/in-degree > 0 and their tile tables.
-// Sorting is a stable LSD radix sort on the vertex id with the original edge
-// index as payload: per 4096-key tile an LDS digit histogram, one device-wide
-// scan of the (digit, tile) counts, then a scatter that ranks keys inside the
-// tile with 8 ballots per wave (stable by construction).
+// Sorting is a stable LSD radix sort that moves the edges themselves: per tile
+// of 8192 an LDS digit histogram, one device-wide scan of the (digit, tile)
+// counts, then a pass that ranks the keys inside the tile with ballots (stable
+// by construction) and writes keys and payloads out from LDS in runs.
 #include "sssp_graph.hpp"
 
 #include <algorithm>
@@ -19,8 +19,10 @@ namespace {
 
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kBlock * kScanItems;  // 2048 elements per block
+constexpr int kRsThreads = 512;
 constexpr int kRsItems = 16;
-constexpr int kRsTile = kBlock * kRsItems;  // 4096 keys per tile
+constexpr int kRsTile = kRsThreads * kRsItems;  // 8192 keys per tile
+constexpr int kRsWaves = kRsThreads / 64;
 
 // --------------------------------------------------------------------------
 // Generic exclusive scan of int64, three phases.
@@ -179,105 +181,10 @@ __global__ __launch_bounds__(kBlock) void k_validate(const int32_t *src, const i
 }
 
 // --------------------------------------------------------------------------
-// Stable LSD radix sort of (key, value) by 8-bit digits.
+// Stable LSD radix sort by digits of at most 8 bits.
 // counts layout: counts[digit * ntiles + tile] (digit-major) so that one
 // exclusive scan yields every tile's output base per digit, in tile order.
 // --------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_rs_hist(const uint32_t *keys, int64_t n, int shift,
-                                                    int64_t *counts, int64_t ntiles)
-{
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * kRsTile;
-#pragma unroll 4
-    for (int i = 0; i < kRsItems; i++) {
-        int64_t idx = base + i * kBlock + threadIdx.x;
-        if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    counts[(int64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
-}
-
-__global__ __launch_bounds__(kBlock) void k_rs_scatter(const uint32_t *keys_in,
-                                                       const uint32_t *vals_in,
-                                                       uint32_t *keys_out, uint32_t *vals_out,
-                                                       int64_t n, int shift,
-                                                       const int64_t *offsets, int64_t ntiles)
-{
-    __shared__ int64_t s_off[256];
-    __shared__ uint32_t s_cnt[kBlock / 64][256];
-    const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6;
-    s_off[tid] = offsets[(int64_t)tid * ntiles + blockIdx.x];
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; w++) s_cnt[w][tid] = 0;
-    __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * kRsTile;
-    for (int r = 0; r < kRsItems; r++) {
-        const int64_t idx = base + (int64_t)r * kBlock + tid;
-        const bool valid = idx < n;
-        uint32_t key = valid ? keys_in[idx] : 0u;
-        uint32_t val = valid ? (vals_in ? vals_in[idx] : (uint32_t)idx) : 0u;
-        uint32_t dg = (key >> shift) & 255u;
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            bool bit = (dg >> b) & 1u;
-            uint64_t bm = __ballot(bit);
-            peers &= bit ? bm : ~bm;
-        }
-        const uint32_t rank = __popcll(peers & lanemask_lt());
-        if (valid && (peers >> lane) == 1ull) s_cnt[wv][dg] = __popcll(peers);
-        __syncthreads();
-        if (valid) {
-            uint32_t pre = 0;
-            for (int w = 0; w < wv; w++) pre += s_cnt[w][dg];
-            int64_t pos = s_off[dg] + pre + rank;
-            keys_out[pos] = key;
-            vals_out[pos] = val;
-        }
-        __syncthreads();
-        uint32_t add = 0;
-#pragma unroll
-        for (int w = 0; w < kBlock / 64; w++) {
-            add += s_cnt[w][tid];
-            s_cnt[w][tid] = 0;
-        }
-        s_off[tid] += add;
-        __syncthreads();
-    }
-}
-
-// --------------------------------------------------------------------------
-// Layout assembly kernels.
-// --------------------------------------------------------------------------
-template <class W>
-__global__ __launch_bounds__(kBlock) void k_gather_pair(const uint32_t *perm, int64_t E,
-                                                        const int32_t *ids, const W *w,
-                                                        int32_t *ids_out, uint32_t *w_out)
-{
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < E;
-         i += (int64_t)gridDim.x * kBlock) {
-        uint32_t p = perm[i];
-        ids_out[i] = ids[p];
-        W x = w[p];
-        uint32_t b;
-        if constexpr (sizeof(W) == 4) {
-            b = *reinterpret_cast<const uint32_t *>(&x);
-        } else {
-            b = 0;
-        }
-        w_out[i] = b;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_copy_i32(const uint32_t *in, int32_t *out, int64_t n)
-{
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * kBlock)
-        out[i] = (int32_t)in[i];
-}
-
 // XCD group of an edge: a multiplicative hash of its destination's 64-vertex
 // block, so each XCD's L2 serves a disjoint, work-balanced eighth of the
 // distance array (R-MAT's per-bit skew makes any bit-sliced split uneven).
@@ -286,75 +193,221 @@ __device__ __forceinline__ uint32_t xcd_group(int32_t dst)
     return (((uint32_t)dst >> 6) * 0x9E3779B1u) >> 29;
 }
 
-__global__ __launch_bounds__(kBlock) void k_group_keys(const int32_t *dst, int64_t E, uint32_t *keys,
-                                                       int64_t *gcount)
+// GROUP: the digit is the key's XCD group, else the bits at `shift`.
+template <bool GROUP>
+__device__ __forceinline__ uint32_t rs_digit(uint32_t key, int shift, uint32_t mask)
 {
-    __shared__ int64_t h[8];
-    if (threadIdx.x < 8) h[threadIdx.x] = 0;
-    __syncthreads();
-    for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * kBlock) {
-        const uint32_t k = xcd_group(dst[e]);
-        keys[e] = k;
-        atomicAdd((unsigned long long *)&h[k], 1ull);
-    }
-    __syncthreads();
-    if (threadIdx.x < 8 && h[threadIdx.x])
-        atomicAdd((unsigned long long *)&gcount[threadIdx.x], (unsigned long long)h[threadIdx.x]);
+    return GROUP ? xcd_group((int32_t)key) : (key >> shift) & mask;
 }
 
-// out[goff[x] + j] = in[perm[cbase[x] + j]] for j < count[x]; the rest of
-// each group's region (up to 3 slots, so every group is a whole number of
-// 16-byte vectors) is a weight-0 self loop on vertex 0, which never changes
-// a distance.
-__global__ __launch_bounds__(kBlock) void k_group_gather(const uint32_t *perm, const int64_t *goff,
-                                                         const int64_t *cbase, const int32_t *src,
-                                                         const int32_t *dst, const uint32_t *w,
-                                                         int32_t *xs, int32_t *xd, uint32_t *xw)
+template <bool GROUP>
+__global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint32_t *keys, int64_t n, int shift,
+                                                        int bins, int64_t *counts, int64_t ntiles)
 {
-    const int64_t Et = goff[8];
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < Et;
-         i += (int64_t)gridDim.x * kBlock) {
-        int x = 0;
-        while (x < 7 && i >= goff[x + 1]) x++;
-        const int64_t j = i - goff[x];
-        const int64_t cnt = cbase[x + 1] - cbase[x];
-        if (j < cnt) {
-            const uint32_t p = perm[cbase[x] + j];
-            xs[i] = src[p];
-            xd[i] = dst[p];
-            xw[i] = w[p];
-        } else {
-            xs[i] = 0;
-            xd[i] = 0;
-            xw[i] = 0u;
+    __shared__ uint32_t h[256];
+    const int tid = threadIdx.x;
+    if (tid < 256) h[tid] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * kRsTile;
+#pragma unroll 4
+    for (int i = 0; i < kRsItems; i++) {
+        const int64_t idx = base + i * kRsThreads + tid;
+        if (idx < n) {
+            const uint32_t d = rs_digit<GROUP>(keys[idx], shift, (uint32_t)bins - 1);
+            // 32 copies of the eight group counters: lanes rarely meet
+            atomicAdd(&h[GROUP ? d << 5 | (tid & 31) : d], 1u);
+        }
+    }
+    __syncthreads();
+    if (tid < bins) {
+        uint32_t c = 0;
+        if (GROUP)
+            for (int k = 0; k < 32; k++) c += h[tid << 5 | k];
+        else
+            c = h[tid];
+        counts[(int64_t)tid * ntiles + blockIdx.x] = c;
+    }
+}
+
+// One pass: NA arrays (the first holds the keys) from in to out, by digit.
+// A wave ranks a run of 1024 keys of the tile on its own (its counters in LDS,
+// no barrier between rounds); the counters of the waves before it and the
+// digits below complete the rank. Every array then goes through LDS in rank
+// order, so a digit's keys are written in one run (128 bytes on average at 64
+// of them). Bound by the bandwidth of reading and writing the arrays; moving
+// the payloads along (12 bytes an edge each way, 0.13 ms a pass at 2^24 edges)
+// replaced a pass over keys and positions (0.31 ms, three barriers per round of
+// keys and scattered writes) and a gather of the payloads by position after the
+// last one (0.62 ms). in.a[1] null: the positions 0, 1, ... pad: added to every
+// position of a digit (or null).
+template <int NA>
+struct RsArrays {
+    uint32_t *a[NA];
+};
+
+template <int NA, bool GROUP>
+__global__ __launch_bounds__(kRsThreads) void k_rs_split(const RsArrays<NA> in,
+                                                         const RsArrays<NA> out, int64_t n,
+                                                         int shift, int bins,
+                                                         const int64_t *offsets, int64_t ntiles,
+                                                         const int64_t *pad)
+{
+    __shared__ uint32_t s_stage[kRsTile];
+    __shared__ uint32_t s_cnt[kRsWaves][256];
+    __shared__ uint32_t s_start[256], s_goff[256];
+    __shared__ uint32_t s_wave[4];
+    const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6;
+    const uint32_t mask = (uint32_t)bins - 1;
+    const int64_t tile = blockIdx.x, base = tile * kRsTile;
+    const int cnt = (int)min(n - base, (int64_t)kRsTile);
+    for (int i = tid; i < kRsWaves * 256; i += kRsThreads) s_cnt[i >> 8][i & 255] = 0;
+    uint32_t key[kRsItems], lp[kRsItems];
+    const int first = wv * (kRsTile / kRsWaves) + lane;
+#pragma unroll
+    for (int r = 0; r < kRsItems; r++) {
+        const int i = first + r * 64;
+        key[r] = i < cnt ? in.a[0][base + i] : 0u;
+    }
+    __syncthreads();
+    volatile uint32_t *const mine = s_cnt[wv];
+#pragma unroll
+    for (int r = 0; r < kRsItems; r++) {
+        const bool valid = first + r * 64 < cnt;
+        const uint32_t dg = rs_digit<GROUP>(key[r], shift, mask);
+        uint64_t peers = __ballot(valid);
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const bool bit = (dg >> b) & 1u;
+            const uint64_t bm = __ballot(bit);
+            peers &= bit ? bm : ~bm;
+        }
+        // every lane reads its digit's counter before the last peer adds to it
+        const uint32_t before = mine[dg];
+        __builtin_amdgcn_wave_barrier();
+        if (valid && (peers >> lane) == 1ull) mine[dg] = before + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        lp[r] = before + (uint32_t)__popcll(peers & lanemask_lt());
+    }
+    __syncthreads();
+    // counters -> keys of the digit in the waves before; exclusive scan of the
+    // digits' totals over the tile
+    uint32_t total = 0, inc = 0;
+    if (tid < 256) {
+#pragma unroll
+        for (int w = 0; w < kRsWaves; w++) {
+            const uint32_t c = s_cnt[w][tid];
+            s_cnt[w][tid] = total;
+            total += c;
+        }
+        inc = total;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o);
+            if (lane >= o) inc += y;
+        }
+        if (lane == 63) s_wave[wv] = inc;
+    }
+    __syncthreads();
+    if (tid < 256) {
+        uint32_t start = inc - total;
+        for (int w = 0; w < wv; w++) start += s_wave[w];
+        s_start[tid] = start;
+        if (tid < bins)
+            s_goff[tid] = (uint32_t)(offsets[(int64_t)tid * ntiles + tile] + (pad ? pad[tid] : 0)) -
+                          start;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRsItems; r++) {
+        if (first + r * 64 >= cnt) continue;
+        const uint32_t dg = rs_digit<GROUP>(key[r], shift, mask);
+        lp[r] += s_start[dg] + s_cnt[wv][dg];
+        s_stage[lp[r]] = key[r];
+    }
+    __syncthreads();
+    uint32_t gp[kRsItems];  // where slot r * kRsThreads + tid of the tile goes (n < 2^32)
+#pragma unroll
+    for (int r = 0; r < kRsItems; r++) {
+        const int i = r * kRsThreads + tid;
+        if (i >= cnt) continue;
+        const uint32_t k = s_stage[i];
+        gp[r] = s_goff[rs_digit<GROUP>(k, shift, mask)] + (uint32_t)i;
+        out.a[0][gp[r]] = k;
+    }
+#pragma unroll
+    for (int x = 1; x < NA; x++) {
+        uint32_t v[kRsItems];
+#pragma unroll
+        for (int r = 0; r < kRsItems; r++) {
+            const int i = first + r * 64;
+            v[r] = 0;
+            if (i < cnt) v[r] = x > 1 || in.a[x] ? in.a[x][base + i] : (uint32_t)(base + i);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kRsItems; r++)
+            if (first + r * 64 < cnt) s_stage[lp[r]] = v[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kRsItems; r++) {
+            const int i = r * kRsThreads + tid;
+            if (i < cnt) out.a[x][gp[r]] = s_stage[i];
         }
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_blk_keys(const int32_t *dst, int64_t E, uint32_t *keys)
+// --------------------------------------------------------------------------
+// Layout assembly kernels.
+// --------------------------------------------------------------------------
+// Of the counts scanned for the split into XCD groups: goff[x] = where group
+// x begins in the padded list (every group a whole number of 16-byte vectors),
+// pad[x] = how far that is past its place in the unpadded one.
+__global__ void k_group_offsets(const int64_t *offsets, int64_t ntiles, int64_t E, int64_t *goff,
+                                int64_t *pad)
 {
-    for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * kBlock)
-        keys[e] = (uint32_t)dst[e] >> kBlkBits;
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    int64_t o = 0;
+    for (int x = 0; x < 8; x++) {
+        const int64_t b = ntiles > 0 ? offsets[x * ntiles] : 0;
+        const int64_t e = x < 7 && ntiles > 0 ? offsets[(x + 1) * ntiles] : E;
+        goff[x] = o;
+        pad[x] = o - b;
+        o += (e - b + 3) / 4 * 4;
+    }
+    goff[8] = o;
+    pad[8] = o - E;
 }
 
-// Sorted position j of block b = skeys[j] goes to boff[b] + (j - bptr[b]);
-// perm[j] is its position in the src-sorted list, whose order is kept.
-__global__ __launch_bounds__(kBlock) void k_blk_gather(const uint32_t *skeys, const uint32_t *perm,
-                                                       int64_t E, const int64_t *bptr,
-                                                       const int64_t *boff, const int32_t *src,
-                                                       const int32_t *dst, const uint32_t *w,
-                                                       int32_t *bs, uint16_t *bd, uint32_t *bw)
+// The padding of each group's region (up to 3 slots) is a weight-0 self loop
+// on vertex 0, which never changes a distance. 32 threads, four per group.
+__global__ void k_group_pad(const int64_t *goff, const int64_t *pad, int64_t E, int32_t *xs,
+                            int32_t *xd, uint32_t *xw)
+{
+    const int x = threadIdx.x >> 2;
+    // group x ends, unpadded, where group x + 1 begins without its padding
+    const int64_t end = (x < 7 ? goff[x + 1] - pad[x + 1] : E) + pad[x];
+    const int64_t i = end + (threadIdx.x & 3);
+    if (i < goff[x + 1]) {
+        xs[i] = 0;
+        xd[i] = 0;
+        xw[i] = 0u;
+    }
+}
+
+// Position j of the edges sorted by block, b = dst[j]'s block, goes to
+// boff[b] + (j - bptr[b]).
+__global__ __launch_bounds__(kBlock) void k_blk_place(const int32_t *src, const uint32_t *dst,
+                                                      const uint32_t *w, int64_t E,
+                                                      const int64_t *bptr, const int64_t *boff,
+                                                      int32_t *bs, uint16_t *bd, uint32_t *bw)
 {
     for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < E;
          j += (int64_t)gridDim.x * kBlock) {
-        const uint32_t b = skeys[j];
+        const uint32_t d = dst[j], b = d >> kBlkBits;
         const int64_t o = boff[b] + (j - bptr[b]);
-        const uint32_t p = perm[j];
-        bs[o] = src[p];
-        bd[o] = (uint16_t)(dst[p] - (int32_t)(b << kBlkBits));
-        bw[o] = w[p];
+        bs[o] = src[j];
+        bd[o] = (uint16_t)(d & ((1u << kBlkBits) - 1));
+        bw[o] = w[j];
     }
 }
 
@@ -377,7 +430,7 @@ __global__ __launch_bounds__(kBlock) void k_blk_pad(const int64_t *bptr, const i
     }
 }
 
-// out[i] = w[i * E / n]: a fixed-stride sample of the weights
+// A fixed-stride sample of the edges:
 // out[0 .. n) = sampled weights, out[n + 1] += sampled edges between near ids
 __global__ __launch_bounds__(kBlock) void k_edge_sample(const int32_t *src, const int32_t *dst,
                                                         const uint32_t *w, int64_t E, int32_t n,
@@ -402,7 +455,13 @@ __global__ __launch_bounds__(kBlock) void k_max_degree(const int64_t *ptr, int64
          v += (int64_t)gridDim.x * kBlock)
         m = max(m, (uint32_t)(ptr[v + 1] - ptr[v]));
     for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor(m, o));
-    if (__lane_id() == 0 && m) atomicMax(mx, m);
+    __shared__ uint32_t s_m[kBlock / 64];
+    if (__lane_id() == 0) s_m[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {  // one update per workgroup (see k_count_reached)
+        for (int w = 1; w < kBlock / 64; w++) m = max(m, s_m[w]);
+        if (m) atomicMax(mx, m);
+    }
 }
 
 // Source deltas of one chunk (one wave, 4 slots per lane, in slot order):
@@ -586,25 +645,14 @@ __global__ __launch_bounds__(kBlock) void k_blk_range_offsets(const int32_t *bs,
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_m_keys(const int32_t *dst, int64_t E, uint32_t *keys)
+// record j = edge j of the list sorted by block: destinations, sources,
+// weights, n of each
+__global__ __launch_bounds__(kBlock) void k_m_place(const uint32_t *sorted, int64_t n, MRec *out)
 {
-    for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * kBlock)
-        keys[e] = (uint32_t)dst[e] >> kMBits;
-}
-
-// record j = the edge at sorted position j (perm: its position in the
-// src-sorted list, whose order is kept within a block)
-__global__ __launch_bounds__(kBlock) void k_m_gather(const uint32_t *skeys, const uint32_t *perm,
-                                                     int64_t E, const int32_t *src,
-                                                     const int32_t *dst, const uint32_t *w,
-                                                     MRec *out)
-{
-    for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < E;
-         j += (int64_t)gridDim.x * kBlock) {
-        const uint32_t p = perm[j];
-        out[j] = MRec{src[p], w[p], dst[p] - (int32_t)(skeys[j] << kMBits), 0};
-    }
+    for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < n;
+         j += (int64_t)gridDim.x * kBlock)
+        out[j] = MRec{(int32_t)sorted[n + j], sorted[2 * n + j],
+                      (int32_t)(sorted[j] & ((1u << kMBits) - 1)), 0};
 }
 
 // row_ptr[v] = first position whose sorted key is >= v; row_ptr[V] = E.
@@ -614,12 +662,13 @@ __global__ __launch_bounds__(kBlock) void k_m_gather(const uint32_t *skeys, cons
 // k_rowptr_search, so no thread loops over millions of vertices.
 constexpr int64_t kRowptrRun = 64;
 __global__ __launch_bounds__(kBlock) void k_rowptr_from_sorted(const uint32_t *keys, int64_t E,
-                                                               int32_t V, int64_t *row_ptr)
+                                                               int32_t V, int shift,
+                                                               int64_t *row_ptr)
 {
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i <= E;
          i += (int64_t)gridDim.x * kBlock) {
-        int64_t lo = (i == 0) ? 0 : (int64_t)keys[i - 1] + 1;  // first vertex not yet placed
-        int64_t hi = (i == E) ? (int64_t)V : (int64_t)keys[i];  // last vertex starting at i
+        int64_t lo = (i == 0) ? 0 : (int64_t)(keys[i - 1] >> shift) + 1;  // first vertex not yet placed
+        int64_t hi = (i == E) ? (int64_t)V : (int64_t)(keys[i] >> shift);  // last vertex starting at i
         if (hi - lo < kRowptrRun)
             for (int64_t v = lo; v <= hi; v++) row_ptr[v] = i;
     }
@@ -627,7 +676,8 @@ __global__ __launch_bounds__(kBlock) void k_rowptr_from_sorted(const uint32_t *k
 
 // the entries k_rowptr_from_sorted left at -1: lower bound of v in the keys
 __global__ __launch_bounds__(kBlock) void k_rowptr_search(const uint32_t *keys, int64_t E,
-                                                          int32_t V, int64_t *row_ptr)
+                                                          int32_t V, int shift,
+                                                          int64_t *row_ptr)
 {
     for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v <= V;
          v += (int64_t)gridDim.x * kBlock) {
@@ -635,7 +685,7 @@ __global__ __launch_bounds__(kBlock) void k_rowptr_search(const uint32_t *keys, 
         int64_t lo = 0, hi = E;  // first position with key >= v
         while (lo < hi) {
             const int64_t mid = (lo + hi) >> 1;
-            if ((int64_t)keys[mid] < v) lo = mid + 1;
+            if ((int64_t)(keys[mid] >> shift) < v) lo = mid + 1;
             else hi = mid;
         }
         row_ptr[v] = lo;
@@ -691,48 +741,63 @@ inline int grid_for(int64_t n, int64_t cap = 8192)
     return (int)(b < cap ? b : cap);
 }
 
+// row_ptr over the keys' bits from `shift` on
 void rowptr_from_sorted(const uint32_t *keys, int64_t E, int32_t V, int64_t *row_ptr,
-                        hipStream_t s)
+                        hipStream_t s, int shift = 0)
 {
     k_fill_i64<<<grid_for((int64_t)V + 1), kBlock, 0, s>>>(row_ptr, (int64_t)V + 1, -1);
-    k_rowptr_from_sorted<<<grid_for(E + 1), kBlock, 0, s>>>(keys, E, V, row_ptr);
-    k_rowptr_search<<<grid_for((int64_t)V + 1), kBlock, 0, s>>>(keys, E, V, row_ptr);
+    k_rowptr_from_sorted<<<grid_for(E + 1), kBlock, 0, s>>>(keys, E, V, shift, row_ptr);
+    k_rowptr_search<<<grid_for((int64_t)V + 1), kBlock, 0, s>>>(keys, E, V, shift, row_ptr);
     SSSP_LAUNCH_CHECK("rowptr_from_sorted");
 }
 
-// Sorts by key; returns the permutation (original indices) in *perm_out
-// (one of the two value buffers) and sorted keys in *keys_out.
-void radix_sort_pairs(const int32_t *keys_in, int64_t n, int32_t max_key, uint32_t *kA,
-                      uint32_t *kB, uint32_t *vA, uint32_t *vB, int64_t *counts, int64_t *blk_a,
-                      int64_t *blk_b, int64_t n_blk, hipStream_t s, uint32_t **keys_out,
-                      uint32_t **perm_out)
+// Scratch of a sort: counts for 256 digits of every tile, the scan's blocks.
+struct RsScratch {
+    int64_t *counts, *blk_a, *blk_b, n_blk;
+};
+
+int key_bits(int64_t max_key)
 {
     int bits = 0;
-    while (bits < 31 && ((int64_t)1 << bits) <= (int64_t)max_key) bits++;
-    int passes = (bits + 7) / 8;
-    if (passes < 1) passes = 1;
-    const int64_t ntiles = (n + kRsTile - 1) / kRsTile;
-    const uint32_t *kin = reinterpret_cast<const uint32_t *>(keys_in);
-    const uint32_t *vin = nullptr;  // iota on the first pass
-    uint32_t *kout = kA, *vout = vA;
-    for (int p = 0; p < passes; p++) {
-        const int shift = 8 * p;
-        if (ntiles > 0) {
-            k_rs_hist<<<(unsigned)ntiles, kBlock, 0, s>>>(kin, n, shift, counts, ntiles);
-            SSSP_LAUNCH_CHECK("k_rs_hist");
-            device_exclusive_scan_i64(counts, counts, 256 * ntiles, blk_a, blk_b, n_blk, s);
-            k_rs_scatter<<<(unsigned)ntiles, kBlock, 0, s>>>(kin, vin, kout, vout, n, shift,
-                                                              counts, ntiles);
-            SSSP_LAUNCH_CHECK("k_rs_scatter");
-        }
-        kin = kout;
-        vin = vout;
-        kout = (kout == kA) ? kB : kA;
-        vout = (vout == vA) ? vB : vA;
-    }
-    *keys_out = const_cast<uint32_t *>(kin);
-    *perm_out = const_cast<uint32_t *>(vin);
+    while (bits < 31 && ((int64_t)1 << bits) <= max_key) bits++;
+    return bits;
 }
+
+// Counts of one digit, scanned.
+template <bool GROUP>
+void rs_count(const uint32_t *keys, int64_t n, int shift, int bins, const RsScratch &t,
+              hipStream_t s)
+{
+    const int64_t ntiles = (n + kRsTile - 1) / kRsTile;
+    k_rs_hist<GROUP><<<(unsigned)ntiles, kRsThreads, 0, s>>>(keys, n, shift, bins, t.counts, ntiles);
+    SSSP_LAUNCH_CHECK("k_rs_hist");
+    device_exclusive_scan_i64(t.counts, t.counts, bins * ntiles, t.blk_a, t.blk_b, t.n_blk, s);
+}
+
+// Sorts the arrays by bits [lo, lo + bits) of the first, from in to fin, by way
+// of tmp (at least one pass: a copy when bits is 0).
+template <int NA>
+void radix_sort(const RsArrays<NA> &in, const RsArrays<NA> &fin, const RsArrays<NA> &tmp, int64_t n,
+                int lo, int bits, const RsScratch &t, hipStream_t s)
+{
+    if (n <= 0) return;
+    const int64_t ntiles = (n + kRsTile - 1) / kRsTile;
+    const int passes = std::max(1, (bits + 7) / 8);
+    const int width = std::max(1, (bits + passes - 1) / passes);
+    RsArrays<NA> from = in;
+    for (int p = 0; p < passes; p++) {
+        const RsArrays<NA> to = (passes - 1 - p) % 2 == 0 ? fin : tmp;
+        const int shift = lo + width * p;
+        const int bins = 1 << std::min(width, std::max(1, bits - width * p));
+        rs_count<false>(from.a[0], n, shift, bins, t, s);
+        k_rs_split<NA, false><<<(unsigned)ntiles, kRsThreads, 0, s>>>(from, to, n, shift, bins,
+                                                                      t.counts, ntiles, nullptr);
+        SSSP_LAUNCH_CHECK("k_rs_split");
+        from = to;
+    }
+}
+
+inline uint32_t *u32p(const void *p) { return static_cast<uint32_t *>(const_cast<void *>(p)); }
 
 void build_static_list(const int64_t *ptr, int32_t V, int64_t E, int64_t *tmp_flags,
                        int64_t *tmp_pos, int64_t *blk_a, int64_t *blk_b, int64_t n_blk,
@@ -825,28 +890,26 @@ static void build_records(sssp_graph *g, const int32_t *src, const int32_t *dst,
     hipStream_t s = g->stream;
     const int32_t nblk = (int32_t)(((int64_t)g->V + (1 << kMBits) - 1) >> kMBits);
     const int64_t rs_tiles = (n + kRsTile - 1) / kRsTile;
-    uint32_t *keys = dmalloc<uint32_t>((size_t)n);
-    uint32_t *kA = dmalloc<uint32_t>((size_t)n), *kB = dmalloc<uint32_t>((size_t)n);
-    uint32_t *vA = dmalloc<uint32_t>((size_t)n), *vB = dmalloc<uint32_t>((size_t)n);
+    uint32_t *sorted = dmalloc<uint32_t>(3 * (size_t)n);
     int64_t *counts = dmalloc<int64_t>((size_t)std::max<int64_t>(256 * rs_tiles, (int64_t)nblk + 1));
     int64_t *bptr = dmalloc<int64_t>((size_t)nblk + 1);
     struct Scratch {
-        void *p[7];
+        void *p[3];
         ~Scratch()
         {
             for (void *x : p) dfree(x);
         }
-    } scratch{{keys, kA, kB, vA, vB, counts, bptr}};
-    k_m_keys<<<grid_for(n), kBlock, 0, s>>>(dst, n, keys);
-    SSSP_LAUNCH_CHECK("k_m_keys");
-    uint32_t *skeys = nullptr, *perm = nullptr;
-    radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), n, nblk - 1, kA, kB, vA, vB, counts,
-                     g->blk_a, g->blk_b, g->n_blk, s, &skeys, &perm);
+    } scratch{{sorted, counts, bptr}};
     MRec *rec = dmalloc<MRec>((size_t)n);
     *rec_out = rec;
-    k_m_gather<<<grid_for(n), kBlock, 0, s>>>(skeys, perm, n, src, dst, w, rec);
-    SSSP_LAUNCH_CHECK("k_m_gather");
-    rowptr_from_sorted(skeys, n, nblk, bptr, s);
+    // sorted by way of the records' own memory, which is written afterwards
+    uint32_t *via = reinterpret_cast<uint32_t *>(rec);
+    radix_sort<3>({{u32p(dst), u32p(src), u32p(w)}}, {{sorted, sorted + n, sorted + 2 * n}},
+                  {{via, via + n, via + 2 * n}}, n, kMBits, key_bits(nblk - 1),
+                  RsScratch{counts, g->blk_a, g->blk_b, g->n_blk}, s);
+    k_m_place<<<grid_for(n), kBlock, 0, s>>>(sorted, n, rec);
+    SSSP_LAUNCH_CHECK("k_m_place");
+    rowptr_from_sorted(sorted, n, nblk, bptr, s, kMBits);
     std::vector<int64_t> bp((size_t)nblk + 1);
     SSSP_HIP(hipMemcpyAsync(bp.data(), bptr, 8 * bp.size(), hipMemcpyDeviceToHost, s));
     SSSP_HIP(hipStreamSynchronize(s));
@@ -1120,7 +1183,7 @@ static uint32_t light_threshold(sssp_graph *g)
         g->el_src, g->el_dst, g->el_w, g->E, (int32_t)n,
         std::min(kLocalNear, std::max(16, g->V / 32)), d);
     SSSP_LAUNCH_CHECK("k_edge_sample");
-    k_max_degree<<<grid_for(g->V), kBlock, 0, g->stream>>>(g->row_ptr, g->V, d + n);
+    k_max_degree<<<grid_for(g->V, 512), kBlock, 0, g->stream>>>(g->row_ptr, g->V, d + n);
     SSSP_LAUNCH_CHECK("k_max_degree");
     std::vector<uint32_t> s((size_t)n + 2);
     SSSP_HIP(hipMemcpyAsync(s.data(), d, 4 * s.size(), hipMemcpyDeviceToHost, g->stream));
@@ -1276,8 +1339,8 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
     g->n_blk = scan_blocks_needed(scan_n);
     g->blk_a = dmalloc<int64_t>((size_t)g->n_blk);
     g->blk_b = dmalloc<int64_t>((size_t)g->n_blk);
-    uint32_t *kA = dmalloc<uint32_t>((size_t)n_sort), *kB = dmalloc<uint32_t>((size_t)n_sort);
-    uint32_t *vA = dmalloc<uint32_t>((size_t)n_sort), *vB = dmalloc<uint32_t>((size_t)n_sort);
+    uint32_t *kA = dmalloc<uint32_t>(4 * (size_t)n_sort);  // four arrays in one allocation
+    uint32_t *kB = kA + n_sort, *vA = kB + n_sort, *vB = vA + n_sort;
     int64_t *counts = dmalloc<int64_t>((size_t)std::max<int64_t>(256 * rs_tiles, (int64_t)V + 1));
     int64_t *tmp_pos = dmalloc<int64_t>((size_t)V + 1);
     struct Scratch {
@@ -1286,7 +1349,8 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         {
             for (void *x : p) dfree(x);
         }
-    } scratch{{kA, kB, vA, vB, counts, tmp_pos, nullptr, nullptr}};
+    } scratch{{kA, counts, tmp_pos, nullptr, nullptr, nullptr, nullptr, nullptr}};
+    const RsScratch rs{counts, g->blk_a, g->blk_b, g->n_blk};
 
     // ---- vertex order: slot = rank by descending in- plus out-degree, ties
     // by descending out-degree, then by vertex id (two stable sorts: by
@@ -1324,7 +1388,7 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
                 ~F1() { dfree(p); }
             } f1{mx};
             SSSP_HIP(hipMemsetAsync(mx, 0, 4, s));
-            k_max_u32<<<grid_for(V), kBlock, 0, s>>>(tot, V, mx);
+            k_max_u32<<<grid_for(V, 256), kBlock, 0, s>>>(tot, V, mx);
             SSSP_LAUNCH_CHECK("k_max_u32");
             uint32_t hmax = 0;
             SSSP_HIP(hipMemcpyAsync(&hmax, mx, 4, hipMemcpyDeviceToHost, s));
@@ -1343,16 +1407,15 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
                 for (void *x : p) dfree(x);
             }
         } f0{{okeys, by_out}};
-        uint32_t *sk = nullptr, *ord = nullptr;
+        // sorted keys with their positions: kB, and by_out, then vB
+        uint32_t *const ord = vB;
         k_order_keys<<<grid_for(V), kBlock, 0, s>>>(outd, nullptr, V, okeys);
         SSSP_LAUNCH_CHECK("k_order_keys out");
-        radix_sort_pairs(reinterpret_cast<const int32_t *>(okeys), V, (int32_t)kOrderCap, kA, kB,
-                         vA, vB, counts, g->blk_a, g->blk_b, g->n_blk, s, &sk, &ord);
-        SSSP_HIP(hipMemcpyAsync(by_out, ord, 4 * (size_t)V, hipMemcpyDeviceToDevice, s));
+        radix_sort<2>({{okeys, nullptr}}, {{kB, by_out}}, {{kA, vA}}, V, 0, key_bits(kOrderCap), rs,
+                      s);
         k_order_keys<<<grid_for(V), kBlock, 0, s>>>(tot, by_out, V, okeys);
         SSSP_LAUNCH_CHECK("k_order_keys total");
-        radix_sort_pairs(reinterpret_cast<const int32_t *>(okeys), V, (int32_t)kOrderCap, kA, kB,
-                         vA, vB, counts, g->blk_a, g->blk_b, g->n_blk, s, &sk, &ord);
+        radix_sort<2>({{okeys, nullptr}}, {{kB, ord}}, {{kA, vA}}, V, 0, key_bits(kOrderCap), rs, s);
         g->vperm = dmalloc<int32_t>((size_t)V);
         g->vinv = dmalloc<int32_t>((size_t)V);
         k_invert_order<<<grid_for(V), kBlock, 0, s>>>(by_out, ord, V, g->vperm, g->vinv);
@@ -1382,90 +1445,64 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
     }
 
     // ---- CSR / src-sorted edge list ----
-    uint32_t *skeys = nullptr, *perm = nullptr;
-    radix_sort_pairs(d_src, E, V > 0 ? V - 1 : 0, kA, kB, vA, vB, counts, g->blk_a, g->blk_b,
-                     g->n_blk, s, &skeys, &perm);
     g->el_src = dmalloc<int32_t>((size_t)E);
     g->el_dst = dmalloc<int32_t>((size_t)E);
     g->el_w = dmalloc<uint32_t>((size_t)E);
     g->row_ptr = dmalloc<int64_t>((size_t)V + 1);
-    if (E > 0) {
-        k_copy_i32<<<grid_for(E), kBlock, 0, s>>>(skeys, g->el_src, E);
-        k_gather_pair<uint32_t><<<grid_for(E), kBlock, 0, s>>>(perm, E, d_dst, d_w, g->el_dst, g->el_w);
-        SSSP_LAUNCH_CHECK("csr gather");
-    }
-    rowptr_from_sorted(skeys, E, V, g->row_ptr, s);
+    const int vbits = key_bits((int64_t)V - 1);
+    radix_sort<3>({{u32p(d_src), u32p(d_dst), u32p(d_w)}},
+                  {{u32p(g->el_src), u32p(g->el_dst), g->el_w}}, {{kA, kB, vA}}, E, 0, vbits, rs, s);
+    rowptr_from_sorted(u32p(g->el_src), E, V, g->row_ptr, s);
     build_static_list(g->row_ptr, V, E, counts, tmp_pos, g->blk_a, g->blk_b, g->n_blk, s,
                       &g->nzo_v, &g->nzo_scan, &g->n_nzo, g->nzo_tile);
 
     // ---- XCD-partitioned edge list: stable split of the src-sorted list into
     // 8 destination groups (src order kept inside each group) ----
     {
-        int64_t *gcnt = dmalloc<int64_t>(8);
-        struct F {
-            void *p;
-            ~F() { dfree(p); }
-        } fg{gcnt};
-        SSSP_HIP(hipMemsetAsync(gcnt, 0, 64, s));
+        const size_t Et = (size_t)E + 32;  // at most 3 slots of padding per group
+        g->x_src = dmalloc<int32_t>(Et);
+        g->x_dst = dmalloc<int32_t>(Et);
+        g->x_w = dmalloc<uint32_t>(Et);
+        g->xgoff = dmalloc<int64_t>(18);  // the groups' offsets, then the padding before them
+        int64_t *const pad = g->xgoff + 9;
+        const int64_t ntiles = (E + kRsTile - 1) / kRsTile;
+        if (E > 0) rs_count<true>(u32p(g->el_dst), E, 0, 8, rs, s);
+        k_group_offsets<<<1, 64, 0, s>>>(counts, ntiles, E, g->xgoff, pad);
+        SSSP_LAUNCH_CHECK("k_group_offsets");
         if (E > 0) {
-            k_group_keys<<<grid_for(E), kBlock, 0, s>>>(g->el_dst, E, kA, gcnt);
-            SSSP_LAUNCH_CHECK("k_group_keys");
+            k_rs_split<3, true><<<(unsigned)ntiles, kRsThreads, 0, s>>>(
+                {{u32p(g->el_dst), u32p(g->el_src), g->el_w}},
+                {{u32p(g->x_dst), u32p(g->x_src), g->x_w}}, E, 0, 8, counts, ntiles, pad);
+            SSSP_LAUNCH_CHECK("k_rs_split (XCD groups)");
+            k_group_pad<<<1, 32, 0, s>>>(g->xgoff, pad, E, g->x_src, g->x_dst, g->x_w);
+            SSSP_LAUNCH_CHECK("k_group_pad");
         }
-        int64_t hc[8];
-        SSSP_HIP(hipMemcpyAsync(hc, gcnt, 64, hipMemcpyDeviceToHost, s));
-        SSSP_HIP(hipStreamSynchronize(s));
-        int64_t hoff[9], hbase[9];
-        hoff[0] = hbase[0] = 0;
-        for (int x = 0; x < 8; x++) {
-            hbase[x + 1] = hbase[x] + hc[x];
-            hoff[x + 1] = hoff[x] + (hc[x] + 3) / 4 * 4;
-        }
-        g->xgoff_host.assign(hoff, hoff + 9);
-        uint32_t *gperm = nullptr, *gkeys = nullptr;
-        // one radix pass on the 3-bit group key; values = positions in the
-        // src-sorted list (stable)
-        radix_sort_pairs(reinterpret_cast<const int32_t *>(kA), E, 7, kB, kB, vA, vB, counts,
-                         g->blk_a, g->blk_b, g->n_blk, s, &gkeys, &gperm);
-        int64_t *dgo = dmalloc<int64_t>(18);
-        struct F2 {
-            void *p;
-            ~F2() { dfree(p); }
-        } fg2{dgo};
-        SSSP_HIP(hipMemcpyAsync(dgo, hoff, 72, hipMemcpyHostToDevice, s));
-        SSSP_HIP(hipMemcpyAsync(dgo + 9, hbase, 72, hipMemcpyHostToDevice, s));
-        g->x_src = dmalloc<int32_t>((size_t)hoff[8] + 4);
-        g->x_dst = dmalloc<int32_t>((size_t)hoff[8] + 4);
-        g->x_w = dmalloc<uint32_t>((size_t)hoff[8] + 4);
-        g->xgoff = dmalloc<int64_t>(9);
-        SSSP_HIP(hipMemcpyAsync(g->xgoff, hoff, 72, hipMemcpyHostToDevice, s));
-        if (hoff[8] > 0) {
-            k_group_gather<<<grid_for(hoff[8]), kBlock, 0, s>>>(gperm, dgo, dgo + 9, g->el_src,
-                                                                g->el_dst, g->el_w, g->x_src,
-                                                                g->x_dst, g->x_w);
-            SSSP_LAUNCH_CHECK("k_group_gather");
-        }
+        g->xgoff_host.resize(9);
+        SSSP_HIP(hipMemcpyAsync(g->xgoff_host.data(), g->xgoff, 72, hipMemcpyDeviceToHost, s));
         SSSP_HIP(hipStreamSynchronize(s));
     }
 
     // ---- destination-blocked edge list ----
     if (E > 0) {
         const int32_t nblk = (int32_t)(((int64_t)V + (1 << kBlkBits) - 1) >> kBlkBits);
-        uint32_t *keys = dmalloc<uint32_t>((size_t)E);
         int64_t *bptr = dmalloc<int64_t>((size_t)nblk + 1);
         int64_t *boff = dmalloc<int64_t>((size_t)nblk + 1);
+        // room for every block's padding to whole chunks
+        const size_t Em = (size_t)E + (size_t)nblk * (kBlkChunk - 1);
+        int32_t *bs = dmalloc<int32_t>(Em);
+        uint16_t *bd = dmalloc<uint16_t>(Em);
         struct F3 {
-            void *p[3];
+            void *p[4];
             ~F3()
             {
                 for (void *x : p) dfree(x);
             }
-        } f3{{keys, bptr, boff}};
-        k_blk_keys<<<grid_for(E), kBlock, 0, s>>>(g->el_dst, E, keys);
-        SSSP_LAUNCH_CHECK("k_blk_keys");
-        uint32_t *bkeys = nullptr, *bperm = nullptr;
-        radix_sort_pairs(reinterpret_cast<const int32_t *>(keys), E, nblk - 1, kA, kB, vA, vB,
-                         counts, g->blk_a, g->blk_b, g->n_blk, s, &bkeys, &bperm);
-        rowptr_from_sorted(bkeys, E, nblk, bptr, s);
+        } f3{{bptr, boff, bs, bd}};
+        g->b_w = dmalloc<uint32_t>(Em);
+        // into kA, kB, vA, by way of vB and the list's own arrays
+        radix_sort<3>({{u32p(g->el_dst), u32p(g->el_src), g->el_w}}, {{kA, kB, vA}},
+                      {{vB, u32p(bs), g->b_w}}, E, kBlkBits, key_bits(nblk - 1), rs, s);
+        rowptr_from_sorted(kA, E, nblk, bptr, s, kBlkBits);
         std::vector<int64_t> bp((size_t)nblk + 1), bo((size_t)nblk + 1);
         SSSP_HIP(hipMemcpyAsync(bp.data(), bptr, 8 * bp.size(), hipMemcpyDeviceToHost, s));
         SSSP_HIP(hipStreamSynchronize(s));
@@ -1509,20 +1546,9 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         const int64_t nch = Ep / kBlkChunk;
         SSSP_HIP(hipMemcpyAsync(boff, bo.data(), 8 * bo.size(), hipMemcpyHostToDevice, s));
         // whole sources and destination offsets first, packed below
-        int32_t *bs = dmalloc<int32_t>((size_t)Ep);
-        uint16_t *bd = dmalloc<uint16_t>((size_t)Ep);
-        struct F4 {
-            void *p[2];
-            ~F4()
-            {
-                for (void *x : p) dfree(x);
-            }
-        } f4{{bs, bd}};
-        g->b_w = dmalloc<uint32_t>((size_t)Ep);
         g->b_edges = Ep;
-        k_blk_gather<<<grid_for(E), kBlock, 0, s>>>(bkeys, bperm, E, bptr, boff, g->el_src,
-                                                    g->el_dst, g->el_w, bs, bd, g->b_w);
-        SSSP_LAUNCH_CHECK("k_blk_gather");
+        k_blk_place<<<grid_for(E), kBlock, 0, s>>>(reinterpret_cast<const int32_t *>(kB), kA, vA, E, bptr, boff, bs, bd, g->b_w);
+        SSSP_LAUNCH_CHECK("k_blk_place");
         k_blk_pad<<<grid_for((int64_t)nblk * kBlkChunk), kBlock, 0, s>>>(bptr, boff, nblk, bs, bd,
                                                                          g->b_w);
         SSSP_LAUNCH_CHECK("k_blk_pad");
@@ -1559,16 +1585,12 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
 
     // ---- CSC ----
     if (build_csc) {
-        radix_sort_pairs(d_dst, E, V > 0 ? V - 1 : 0, kA, kB, vA, vB, counts, g->blk_a, g->blk_b,
-                         g->n_blk, s, &skeys, &perm);
         g->csc_src = dmalloc<int32_t>((size_t)E);
         g->csc_w = dmalloc<uint32_t>((size_t)E);
         g->col_ptr = dmalloc<int64_t>((size_t)V + 1);
-        if (E > 0) {
-            k_gather_pair<uint32_t><<<grid_for(E), kBlock, 0, s>>>(perm, E, d_src, d_w, g->csc_src, g->csc_w);
-            SSSP_LAUNCH_CHECK("csc gather");
-        }
-        rowptr_from_sorted(skeys, E, V, g->col_ptr, s);
+        radix_sort<3>({{u32p(d_dst), u32p(d_src), u32p(d_w)}}, {{vB, u32p(g->csc_src), g->csc_w}},
+                      {{kA, kB, vA}}, E, 0, vbits, rs, s);
+        rowptr_from_sorted(vB, E, V, g->col_ptr, s);
         build_static_list(g->col_ptr, V, E, counts, tmp_pos, g->blk_a, g->blk_b, g->n_blk, s,
                           &g->nzi_v, &g->nzi_scan, &g->n_nzi, g->nzi_tile);
         g->has_csc = true;

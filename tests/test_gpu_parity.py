@@ -555,6 +555,34 @@ def test_blocked_tiles_any_cap_and_order(gpu, oracle):
                 g.set_param(name, bad)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,E,relabel", [(1, 8192, False), (256, 8191, False), (257, 8193, False),
+                                         (40000, 3, False), (65537, 16385, True),
+                                         (70001, 100003, False)])
+def test_layouts_at_the_edges_of_the_sort_tiles(gpu, oracle, V, E, relabel):
+    """Edge counts around the sort's tiles of 8192, one digit against two and
+    three, empty digits, and edges that pile up in one digit: solves over every
+    layout the sorts build (out-edges, in-edges, blocked list, XCD groups,
+    batch records) end on the oracle's fixpoint. Bit equality."""
+    rng = np.random.default_rng(V + E)
+    src = (rng.random(E) ** 4 * V).astype(np.int32)
+    dst = np.where(rng.random(E) < 0.5, V - 1, rng.integers(0, V, E)).astype(np.int32)
+    w = rng.random(E, dtype=np.float32)
+    sources = [int(x) for x in src[:3]]
+    refs = [oracle.dijkstra(src, dst, w, V, x) for x in sources]
+    with S.DeviceGraph(src, dst, w, V, relabel=relabel) as g:
+        g.set_param("plain_below_edges", 0)
+        g.set_param("dense_all_frac", 0.0)
+        for sched, kernel in (("push", 0), ("pull", 0), ("all", 0), ("plain", 1), ("plain", 2)):
+            print(f"layouts: V {V} E {E} relabel {relabel}, {sched} {kernel}", flush=True)
+            g.set_param("plain_kernel", kernel)
+            d, _ = g.solve(sources[0], sched)
+            assert np.array_equal(bits(d), bits(refs[0])), (sched, kernel)
+        got = g.solve_batch(np.array(sources, np.int32), policy=3)[0]
+        for x, ref in zip(got, refs):
+            assert np.array_equal(bits(x), bits(ref))
+
+
 def _local_graph(case, rng):
     """Edges between near ids, no hubs, fewer than 8 per vertex."""
     if case in ("grid", "grid_u32", "grid_zero"):
