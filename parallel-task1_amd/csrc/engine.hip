@@ -2942,7 +2942,7 @@ void solve_solo(sssp_graph *g, int32_t source, sssp_stats *st)
     st->gteps = ms > 0 ? (double)g->E / (ms * 1e-3) / 1e9 : 0.0;
     st->verify_passes = 1;  // the last round lowered nothing
     st->iterations = st->n_all = h.ph_full;
-    st->edges_relaxed = h.ph_work * kBlkChunk;
+    st->edges_relaxed = h.ph_work;
     st->reached = (int32_t)h.n_reached;
 }
 

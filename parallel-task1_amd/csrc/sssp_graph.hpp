@@ -470,13 +470,15 @@ class Prefault {
 // Graphs solved whole in one workgroup's LDS (launch_solo): one launch and one
 // wait, where the pass loop has a launch per pass and a wait per four. One
 // workgroup reads every live chunk of a round itself, so the line lies where
-// that costs what the launches do. A whole call, us, pass loop / in LDS: R-MAT
-// 8 x 8 137 / 42, 11 x 16 (2^15 edges) 199 / 81, 13 x 8 222 / 124, 13 x 16 (2^17)
-// 259 / 200, 14 x 16 (2^18) 267 / 301, 15 x 15 351 / 530; uniform 10 K x 10
-// 263 / 195, 30 K x 7 355 / 426. Local passes take fewer rounds on long paths:
-// grid 20 x 20 149 / 78, 40 x 50 (2^13 edges) 177 / 169, 100 x 100 331 / 527.
+// that costs what the launches do (up to 2^15 edges it keeps them in
+// registers). A whole call, us, pass loop / in LDS: R-MAT 8 x 8 137 / 37, 11 x
+// 16 (2^15 edges) 199 / 63, 13 x 8 222 / 124, 13 x 16 (2^17) 259 / 200, 14 x 16
+// (2^18) 267 / 301, 15 x 15 351 / 530; uniform 10 K x 10 263 / 195, 30 K x 7 355 /
+// 426. Local passes take fewer rounds on long paths, and are better than rounds
+// that read the edges: grid 20 x 20 149 / 55, 40 x 50 177 / 86, 100 x 100
+// (39600 edges) 331 / 527.
 constexpr int64_t kSoloEdges = (int64_t)1 << 17;
-constexpr int64_t kSoloLocalEdges = (int64_t)1 << 13;
+constexpr int64_t kSoloLocalEdges = (int64_t)1 << 15;
 bool solo_fits(const sssp_graph *g);
 void ensure_chunk_sources(sssp_graph *g);
 void launch_solo(sssp_graph *g, int32_t source, bool hops, int32_t limit);

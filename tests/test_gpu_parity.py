@@ -642,6 +642,9 @@ def test_local_passes_bit_exact(gpu, oracle, case):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("V,E,kind", [(1, 1, "f32"), (64, 255, "f32"), (65, 256, "u32"),
+                                      (2000, 8192, "f32"), (1 << 15, 8193, "u32"),
+                                      (2000, 16384, "relabel"), (2000, 16385, "f32"),
+                                      (1 << 15, 32768, "f32"), (2000, 32769, "f32"),
                                       (1 << 15, 1 << 17, "f32"), (1 << 15, (1 << 17) + 1, "f32"),
                                       ((1 << 15) + 1, 1 << 17, "f32"), (1 << 15, 100003, "relabel"),
                                       (300, 70001, "ties"), (2001, 0, "f32")])
