@@ -3361,59 +3361,175 @@ void ref_init(DT *d, int32_t V, int32_t source)
 }
 
 // The wrappers' passes over the caller's edges, in the caller's order: an edge
-// is relaxed only when its source changed since the pass before. Whether it
-// did is one bit in the workgroup's LDS, so an edge that is not relaxed costs
-// 4 bytes of stream and no gather, and its line of destinations and weights is
-// read only where another edge needs it. The pass over every edge (k_el_pass)
-// took 0.275 ms on a power-law graph of 2^20 vertices and 2^24 edges, bound
-// by the two random distance reads per edge (a distance array as large as an
-// XCD's L2); now 0.02-0.09 ms but for six passes of 0.14-0.41, at 22 passes
-// instead of 16 (a pass no longer sees the changes of its own): a call 4.8 ->
-// 2.7 ms. Uniform 500 K x 16, u32 2.9 -> 1.6 ms, power-law 300 K x 14 f64 1.15 ->
-// 0.86. kActBits bits fill most of a CU's LDS; half of them with two
-// workgroups per CU 3.0 ms, a quarter 3.2. kActUnroll 1 / 2 / 4 groups of four
-// edges in flight per lane: 2.79 / 2.69 / 2.62 ms, f64 0.88 / 0.85 / 0.92.
+// is relaxed only when its source changed since it was last relaxed, and in a
+// light pass only when its weight is light. Whether the source changed is one
+// bit in the workgroup's LDS, so an edge that is not relaxed costs 4 or 8 bytes
+// of stream and no gather, and a line of destinations or weights is read only
+// where some edge needs it. The pass over every edge (k_el_pass) took 0.275 ms
+// on a power-law graph of 2^20 vertices and 2^24 edges, bound by the two random
+// distance reads per edge (a distance array as large as an XCD's L2), 16 passes,
+// 4.8 ms a call. With the bits 22 passes, since a pass no longer sees the changes
+// of its own, six of them 0.14-0.41 ms and the others 0.02-0.09: 2.7 ms. With
+// light passes between them 1.9. Uniform 500 K x 16, u32 2.9 / 1.6 / 1.4 ms,
+// power-law 300 K x 14 f64 1.15 / 0.86 / 0.79. kActBits bits fill most of a CU's
+// LDS; half of them with two workgroups per CU 3.0 ms without light passes, a
+// quarter 3.2. kActUnroll 1 / 2 / 4 groups of four edges in flight per lane:
+// 2.79 / 2.69 / 2.62 ms, f64 0.88 / 0.85 / 0.92.
 constexpr int kActUnroll = 2;
 constexpr int32_t kActBits = 1 << 20;
 constexpr int kActThreads = 1024;
-constexpr size_t kActFlagBytes = 256;
 // Fewer edges run every edge in one launch a pass: R-MAT 14 x 16 0.287 ms against
 // 0.305, uniform 2000 x 4 0.26 against 0.30, power-law 100 K x 16 0.88 against 0.65.
 constexpr int64_t kActMinEdges = 1 << 19;
-constexpr int kActBatch = 6;  // passes queued per host check (an idle pass and mark: 4-8 us)
+// Passes queued per host check: a third of those that ran, between these (an
+// idle pass and mark take 4-8 us, a check 30).
+constexpr int kActBatch = 6, kActBatchMax = 32;
 
-// Vertices changed since the mark before, one bit each in bits[] (bit v & mask;
-// several vertices share one where V exceeds the mask). The first mark takes
-// every vertex with a distance. flags[p & 63] = 1 when mark p found any; a mark
-// after one that found none returns at once, and so does pass p.
+// State of a run of passes on the device, rings of 64 by pass. Light edges
+// (weight pattern at most thr) are relaxed to near convergence between full
+// passes, as in the pass loop of a graph (k_blk_plain).
 template <class DT>
-__global__ __launch_bounds__(kBlock) void k_mark_changed(const DT *__restrict__ dist, DT *snap,
-                                                         int32_t V, int32_t n_bits,
-                                                         unsigned long long *bits, int32_t *flags,
-                                                         int32_t p, DT inf)
+struct ActCtl {
+    int32_t low[64];   // vertices the pass before lowered (pass 0: vertices with a distance)
+    int32_t pend[64];  // some vertex changed since the last full pass
+    int32_t kind[64];
+    DT thr;
+    int32_t light;     // 1: there is a light class
+    int32_t stop;      // light passes go on while they lower this many vertices
+};
+
+template <class DT>
+__device__ __forceinline__ int act_kind(const ActCtl<DT> *c, int32_t p)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) flags[(p + 1) & 63] = 0;
-    if (p > 0 && flags[(p - 1) & 63] == 0) return;
+    // no branches: every load is in flight at once
+    const int32_t pend = c->pend[p & 63], low = c->low[p & 63], low1 = c->low[(p - 1) & 63];
+    const int32_t kind1 = c->kind[(p - 1) & 63], kind2 = c->kind[(p - 2) & 63];
+    const int32_t light = c->light, stop = c->stop;
+    // rings hold zeros, no kind, before the first pass
+    const int32_t before = kind2 == kPassLight ? low1 : 0;
+    const bool grows = (kind1 == kPassLight) & (low > before);
+    const bool again = (p == 0) | (low >= stop) | grows;
+    const int kind = (light != 0) & (p < kLightMaxPasses) & again ? kPassLight : kPassFull;
+    return pend == 0 ? kPassIdle : kind;
+}
+
+// Clears the state and picks the light class from a sample of the edges: the
+// sampled weight whose share of weights up to it is nearest to the one wanted,
+// none when that is off by more than half or three times (many equal weights).
+// Wanted: one edge per vertex on a graph with hubs (sampled endpoints meet far
+// more often than even ones would), six on one without (none when the mean
+// degree is below kLightMinDegree), between 1/16 and 1/2 of the edges; no class
+// when `weighted` is 0. One workgroup of kActSamples threads. Per vertex 0.5 /
+// 1 / 2 / 4 / 6 edges, ms a call: power-law 1 M x 16 1.89 / 1.89 / 1.97 / 2.17 /
+// 2.39, 2 M x 5 1.82 / 1.67 / 1.88 / 2.02 / 2.01, 300 K x 14 f64 0.77 / 0.77 / 0.77
+// / 0.79 / 0.83; uniform 500 K x 16 1.80 / 1.79 / 1.83 / 1.68 / 1.42, 2 M x 16 6.2 /
+// 6.2 / 5.9 / 6.7 / 5.4; without a class 2.7, 2.2, 0.88; 1.6, 6.2.
+constexpr int kActSamples = 512;
+template <class DT>
+__global__ __launch_bounds__(kActSamples) void k_act_begin(const int32_t *src, const int32_t *dst,
+                                                           const DT *w, int32_t V, int64_t E,
+                                                           int weighted, int32_t stop,
+                                                           ActCtl<DT> *c)
+{
+    __shared__ DT s_w[kActSamples];
+    __shared__ int32_t s_s[kActSamples], s_t[kActSamples];
+    __shared__ uint32_t s_best;
+    __shared__ int s_meet;
+    const int tid = threadIdx.x;
+    if (tid < 64) c->low[tid] = c->pend[tid] = c->kind[tid] = 0;
+    if (tid == 0) {
+        s_best = 0xFFFFFFFFu;
+        s_meet = 0;
+        c->light = 0;
+        c->stop = stop;
+    }
+    if (!weighted) return;
+    const DT mine = w[tid * E / kActSamples];
+    const int32_t from = src[tid * E / kActSamples], to = dst[tid * E / kActSamples];
+    s_w[tid] = mine;
+    s_s[tid] = from;
+    s_t[tid] = to;
+    __syncthreads();
+    int upto = 0, meet = -2;  // not with itself
+    for (int i = 0; i < kActSamples; i++) {
+        upto += s_w[i] <= mine ? 1 : 0;
+        meet += (s_s[i] == from ? 1 : 0) + (s_t[i] == to ? 1 : 0);
+    }
+    if (meet > 0) atomicAdd(&s_meet, meet);
+    __syncthreads();
+    const float mean = (float)E / (float)V;
+    const bool hubs = (float)s_meet > 8.f + 16.f * kActSamples * kActSamples / (float)V;
+    if (!hubs && mean < (float)kLightMinDegree) return;
+    const float target =
+        kActSamples * fminf(0.5f, fmaxf(1.f / 16.f, (hubs ? 1.f : 6.f) / mean));
+    if ((float)upto >= 0.5f * target && (float)upto <= 3.f * target && upto <= kActSamples * 3 / 4)
+        atomicMin(&s_best, (uint32_t)(fabsf((float)upto - target) * 16.f) << 10 | (uint32_t)tid);
+    __syncthreads();
+    if (s_best != 0xFFFFFFFFu && (s_best & 1023u) == (uint32_t)tid) {
+        c->thr = mine;
+        c->light = 1;
+    }
+}
+
+// Before pass p: the vertices changed by the pass before (bits[0]) and since
+// the last full pass began (bits[1]), one bit each (bit v & mask; several
+// vertices share one where V exceeds the mask), against the copies last[] and
+// full[]. The first mark takes every vertex with a distance. A mark after one
+// that left nothing pending returns at once, and so does pass p.
+template <class DT>
+__global__ __launch_bounds__(kActThreads) void k_mark_changed(const DT *__restrict__ dist, DT *last,
+                                                              DT *full, int32_t V, int32_t n_bits,
+                                                              unsigned long long *bits,
+                                                              ActCtl<DT> *c, int32_t p, DT inf)
+{
+    __shared__ int s_low, s_pend;
+    if (blockIdx.x == 0 && threadIdx.x == 0) c->low[(p + 1) & 63] = c->pend[(p + 1) & 63] = 0;
+    if (p > 0 && c->pend[(p - 1) & 63] == 0) return;
     const int lane = __lane_id();
-    bool found = false;
+    const bool light = c->light != 0;
+    const bool was_full = p > 0 && c->kind[(p - 1) & 63] == kPassFull;
+    if (light) {
+        if (threadIdx.x == 0) s_low = s_pend = 0;
+        __syncthreads();
+    }
     const int words = (n_bits + 63) / 64;
-    const int wave = (int)(blockIdx.x * (kBlock / 64)) + ((int)threadIdx.x >> 6);
-    for (int i = wave; i < words; i += (int)gridDim.x * (kBlock / 64)) {
-        bool ch = false;
+    const int wave = (int)(blockIdx.x * (kActThreads / 64)) + ((int)threadIdx.x >> 6);
+    int low = 0;
+    bool pend = false;
+    for (int i = wave; i < words; i += (int)gridDim.x * (kActThreads / 64)) {
+        bool ch = false, chf = false;
         for (int64_t v = (int64_t)i * 64 + lane; v < V; v += n_bits) {
-            const DT d = dist[v];
-            if (d != (p > 0 ? snap[v] : inf)) {
-                ch = true;
-                snap[v] = d;
-            } else if (p == 0) {
-                snap[v] = d;
+            const DT d = dist[v], l = p > 0 ? last[v] : inf;
+            ch |= d != l;
+            low += d != l ? 1 : 0;
+            if (p == 0 || d != l) last[v] = d;
+            if (light) {
+                const DT f = p == 0 || was_full ? l : full[v];
+                if (p == 0 || was_full) full[v] = f;
+                chf |= d != f;
             }
         }
-        const unsigned long long m = __ballot(ch);
-        if (lane == 0) bits[i] = m;
-        found |= m != 0;
+        const unsigned long long m = __ballot(ch), mf = light ? __ballot(chf) : m;
+        if (lane == 0) {
+            bits[i] = m;
+            if (light) bits[words + i] = mf;
+        }
+        pend |= mf != 0;
     }
-    if (found && lane == 0) flags[p & 63] = 1;
+    if (!light) {  // nothing is counted
+        if (pend && lane == 0) c->pend[p & 63] = 1;
+        return;
+    }
+    low = wave_sum32(low);
+    if (lane == 0) {
+        if (low) atomicAdd(&s_low, low);
+        if (pend) s_pend = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_low) atomicAdd(&c->low[p & 63], s_low);
+        if (s_pend) c->pend[p & 63] = 1;
+    }
 }
 
 template <class WT, class DT, int VEC>
@@ -3422,14 +3538,17 @@ __global__ __launch_bounds__(kActThreads) void k_el_active(const int32_t *__rest
                                                     const DT *__restrict__ w, int64_t E, DT *dist,
                                                     const unsigned long long *__restrict__ bits,
                                                     int32_t n_bits, int32_t mask,
-                                                    const int32_t *flags, int32_t p,
-                                                    int64_t per_block)
+                                                    ActCtl<DT> *c, int32_t p, int64_t per_block)
 {
     extern __shared__ uint32_t s_bits[];
-    if (flags[p & 63] == 0) return;
+    const int kind = act_kind(c, p);
+    if (kind == kPassIdle) return;
     const int tid = threadIdx.x;
+    if (blockIdx.x == 0 && tid == 0) c->kind[p & 63] = kind;
+    const DT thr = kind == kPassLight ? c->thr : (DT)~(DT)0;
     {
         const int words = (n_bits + 63) / 64;
+        if (kind == kPassFull && c->light) bits += words;
         uint64_t *s64 = reinterpret_cast<uint64_t *>(s_bits);
         for (int i = tid; i < words; i += kActThreads) s64[i] = bits[i];
     }
@@ -3471,11 +3590,21 @@ __global__ __launch_bounds__(kActThreads) void k_el_active(const int32_t *__rest
             v4i t[kActUnroll];
             v4w ww[kActUnroll];
             DT du[kActUnroll * 4];
+            if (kind == kPassLight) {
+                // weights first: most edges need no destination
+#pragma unroll
+                for (int u = 0; u < kActUnroll; u++)
+                    if (act >> (u * 4) & 15u)
+                        ww[u] = __builtin_nontemporal_load(&w4[g + u * kActThreads]);
+#pragma unroll
+                for (int e = 0; e < kActUnroll * 4; e++)
+                    if (act >> e & 1u && ww[e >> 2][e & 3] > thr) act &= ~(1u << e);
+            }
 #pragma unroll
             for (int u = 0; u < kActUnroll; u++) {
                 if (!(act >> (u * 4) & 15u)) continue;
                 t[u] = __builtin_nontemporal_load(&t4[g + u * kActThreads]);
-                ww[u] = __builtin_nontemporal_load(&w4[g + u * kActThreads]);
+                if (kind == kPassFull) ww[u] = __builtin_nontemporal_load(&w4[g + u * kActThreads]);
             }
 #pragma unroll
             for (int e = 0; e < kActUnroll * 4; e++)
@@ -3490,16 +3619,30 @@ __global__ __launch_bounds__(kActThreads) void k_el_active(const int32_t *__rest
         }
         if (b == 0 && tid < (E & 3)) {
             const int64_t e = ((E >> 2) << 2) + tid;
-            if (active(src[e])) relax(dist[src[e]], dist[dst[e]], dst[e], w[e]);
+            if (active(src[e]) && w[e] <= thr) relax(dist[src[e]], dist[dst[e]], dst[e], w[e]);
         }
     } else {
         const int64_t e0 = b * per_block, e1 = min(e0 + per_block, E);
         for (int64_t e = e0 + tid; e < e1; e += kActThreads) {
             const int32_t s = src[e];
-            if (active(s)) relax(dist[s], dist[dst[e]], dst[e], w[e]);
+            if (active(s) && w[e] <= thr) relax(dist[s], dist[dst[e]], dst[e], w[e]);
         }
     }
 }
+
+// Scratch of a call: state, two sets of bits, two copies of the distances.
+template <class DT>
+struct ActScratch {
+    size_t bits, last, full, bytes;
+    explicit ActScratch(int32_t V)
+    {
+        const size_t v = ((size_t)V * sizeof(DT) + 255) / 256 * 256;
+        bits = (sizeof(ActCtl<DT>) + 255) / 256 * 256;
+        last = bits + 2 * (kActBits / 8);
+        full = last + v;
+        bytes = full + v;
+    }
+};
 
 template <class WT, class DT>
 void ref_bf_active(const int32_t *src, const int32_t *dst, const DT *w, int32_t V, int64_t E, DT *d,
@@ -3510,40 +3653,48 @@ void ref_bf_active(const int32_t *src, const int32_t *dst, const DT *w, int32_t 
     SSSP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     const int32_t n_bits = std::min(V, kActBits), mask = V <= kActBits ? INT32_MAX : kActBits - 1;
     const size_t lds = ((size_t)n_bits + 63) / 64 * 8;
-    int32_t *flags = reinterpret_cast<int32_t *>(mem);
-    unsigned long long *bits = reinterpret_cast<unsigned long long *>(mem + kActFlagBytes);
-    DT *snap = reinterpret_cast<DT *>(mem + kActFlagBytes + kActBits / 8);
-    k_fill<int32_t><<<1, 64>>>(flags, 64, 0);
-    SSSP_LAUNCH_CHECK("clear change flags");
+    const ActScratch<DT> at(V);
+    ActCtl<DT> *const c = reinterpret_cast<ActCtl<DT> *>(mem);
+    unsigned long long *bits = reinterpret_cast<unsigned long long *>(mem + at.bits);
+    DT *last = reinterpret_cast<DT *>(mem + at.last), *full = reinterpret_cast<DT *>(mem + at.full);
+    k_act_begin<DT><<<1, kActSamples>>>(src, dst, w, V, E, WT::kWeighted ? 1 : 0,
+                                        (int32_t)(kLightStopFrac * V), c);
+    SSSP_LAUNCH_CHECK("k_act_begin");
     const bool vec = reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(dst) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(w) % 16 == 0;
     const int64_t units = vec ? E >> 2 : E;
-    const int64_t full = (int64_t)cus * (lds <= 80 * 1024 ? 2 : 1);
-    const int64_t nblocks = std::max<int64_t>(1, std::min(full, (units + kActThreads - 1) / kActThreads));
+    const int64_t grid = (int64_t)cus * (lds <= 80 * 1024 ? 2 : 1);
+    const int64_t nblocks = std::max<int64_t>(1, std::min(grid, (units + kActThreads - 1) / kActThreads));
     const int64_t per_block = (units + nblocks - 1) / nblocks;
-    const unsigned mgrid = grid_for(n_bits, 1024);
-    int32_t hc[64], pass = 0, done = -1;
-    while (done < 0) {
-        for (int i = 0; i < kActBatch; i++) {
-            k_mark_changed<DT><<<mgrid, kBlock>>>(d, snap, V, n_bits, bits, flags, pass + i,
-                                                  (DT)WT::INF);
+    const int64_t mgrid = std::min<int64_t>(cus, ((int64_t)n_bits + kActThreads - 1) / kActThreads);
+    ActCtl<DT> h;
+    int32_t pass = 0, fulls = 0;
+    bool done = false;
+    while (!done) {
+        const int batch = std::min(kActBatchMax, std::max(kActBatch, pass / 3));
+        for (int i = 0; i < batch; i++) {
+            k_mark_changed<DT><<<(unsigned)mgrid, kActThreads>>>(d, last, full, V, n_bits, bits, c,
+                                                                 pass + i, (DT)WT::INF);
             if (vec)
                 k_el_active<WT, DT, 4><<<(unsigned)nblocks, kActThreads, lds>>>(
-                    src, dst, w, E, d, bits, n_bits, mask, flags, pass + i, per_block);
+                    src, dst, w, E, d, bits, n_bits, mask, c, pass + i, per_block);
             else
                 k_el_active<WT, DT, 1><<<(unsigned)nblocks, kActThreads, lds>>>(
-                    src, dst, w, E, d, bits, n_bits, mask, flags, pass + i, per_block);
+                    src, dst, w, E, d, bits, n_bits, mask, c, pass + i, per_block);
             SSSP_LAUNCH_CHECK("bellman_ford pass");
         }
-        SSSP_HIP(hipMemcpy(hc, flags, sizeof(hc), hipMemcpyDeviceToHost));
-        for (int i = 0; i < kActBatch && done < 0; i++)
-            if (hc[(pass + i) & 63] == 0) done = pass + i;
-        pass += kActBatch;
-        if (done < 0 && pass >= V + 4)
+        SSSP_HIP(hipMemcpy(&h, c, sizeof(h), hipMemcpyDeviceToHost));
+        for (int i = 0; i < batch && !done; i++) {
+            done = h.pend[(pass + i) & 63] == 0;
+            if (!done && h.kind[(pass + i) & 63] == kPassFull) fulls++;
+        }
+        pass += batch;
+        // the reference loops at most V times (bellman_ford.cu:146)
+        if (!done && pass >= (int64_t)V + 4 + kLightMaxPasses)
             throw Error{SSSP_ERR_NOT_CONVERGED, "Bellman-Ford did not converge within V passes"};
     }
-    if (passes_out) *passes_out = std::max(done, 1);
+    if (passes_out) *passes_out = std::max(fulls, 1);
 }
 
 template <class WT, class DT>
@@ -3554,7 +3705,7 @@ void ref_bf(const int32_t *src, const int32_t *dst, const DT *w, int32_t V, int6
         // the passes that keep the distances of the pass before; when there
         // is no memory for those, the passes over every edge
         void *mem = nullptr;
-        if (hipMalloc(&mem, kActFlagBytes + kActBits / 8 + sizeof(DT) * (size_t)V) == hipSuccess) {
+        if (hipMalloc(&mem, ActScratch<DT>(V).bytes) == hipSuccess) {
             struct Free {
                 void *p;
                 ~Free() { dfree(p); }

@@ -131,6 +131,7 @@ struct WUnit {
 // 64-bit distances (f64 reference-shaped wrapper only).
 struct WF64 {
     static constexpr unsigned long long INF = 0x7FEFFFFFFFFFFFFFull;  // DBL_MAX
+    static constexpr bool kWeighted = true;
     __device__ __forceinline__ static unsigned long long add(unsigned long long d,
                                                              unsigned long long w)
     {

@@ -131,3 +131,25 @@ def test_wrapper_change_bits(gpu, lib, oracle, dtype, V, E, shift):
             assert getattr(lib, "sssp_bellman_ford_" + k)(*at, V, E, source, dist.ptr,
                                                            None) == S.OK, S.last_error()
             assert np.array_equal(_bits(dist.get()), _bits(ref))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("weights", ["random", "equal", "two", "mostly_zero"])
+@pytest.mark.parametrize("ends", ["hubs", "even", "sparse"])
+def test_wrapper_light_classes(gpu, lib, oracle, ends, weights):
+    """Wrapper passes with a light class of a graph with hubs, of one without,
+    and with none (few edges per vertex, equal weights, or too many of the
+    lightest): bit equality with the oracle."""
+    rng = np.random.default_rng(31)
+    E = (1 << 19) + 5
+    V = 200003 if ends == "sparse" else 40009
+    s, d = ((rng.random(E) ** (4 if ends == "hubs" else 1) * V).astype(np.int32)
+            for _ in range(2))
+    w = {"random": rng.random(E), "equal": np.full(E, 0.25), "two": rng.integers(1, 3, E) / 4,
+         "mostly_zero": np.where(rng.random(E) < 0.8, 0.0, rng.random(E))}[weights]
+    w = w.astype(np.float32)
+    source = int(s[0])
+    print(f"wrapper light class: {ends}, {weights}", flush=True)
+    _, got, passes = _run(lib, np.float32, s, d, w, V, source)
+    assert np.array_equal(_bits(got), _bits(oracle.bf(s, d, w, V, source)[0]))
+    assert 1 <= passes <= V
