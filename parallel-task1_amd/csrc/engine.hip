@@ -1490,13 +1490,7 @@ __device__ __forceinline__ int64_t blk_relax_tile(const BlkTile &t, const BlkLis
             const int32_t a1 = a0 + (int32_t)(pv.y >> kBlkBits);
             const int32_t a2 = a1 + (int32_t)(pv.z >> kBlkBits);
             const int32_t a3 = a2 + (int32_t)(pv.w >> kBlkBits);
-            int32_t incl = a3;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int32_t y = __shfl_up(incl, o);
-                if (lane >= o) incl += y;
-            }
-            const int32_t b0 = cb + (incl - a3);
+            const int32_t b0 = cb + (wave_scan32(a3) - a3);
             s0 = b0 + a0;
             s1 = b0 + a1;
             s2 = b0 + a2;
@@ -2000,13 +1994,7 @@ k_blk_local(const PassArgs a, const LocalArgs la, const BlkList L, uint32_t *dis
             a4[1] = a4[0] + (int32_t)(pv[h].y >> kBlkBits);
             a4[2] = a4[1] + (int32_t)(pv[h].z >> kBlkBits);
             a4[3] = a4[2] + (int32_t)(pv[h].w >> kBlkBits);
-            int32_t incl = a4[3];
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int32_t y = __shfl_up(incl, o);
-                if (lane >= o) incl += y;
-            }
-            const int32_t b0 = cb[h] + (incl - a4[3]);
+            const int32_t b0 = cb[h] + (wave_scan32(a4[3]) - a4[3]);
 #pragma unroll
             for (int j = 0; j < 4; j++) s[j] = b0 + a4[j];
         } else {

@@ -198,6 +198,20 @@ __device__ __forceinline__ long long wave_sum64(long long x)
     return x;
 }
 
+// Inclusive prefix sum over the wave in the vector unit (row shifts, then the
+// last lane of rows 0 and 2 to the row above, then lane 31 to the upper
+// half). Six shuffles go through the LDS unit, which the callers keep busy.
+__device__ __forceinline__ int wave_scan32(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return x;
+}
+
 __device__ __forceinline__ int wave_sum32(int x)
 {
 #pragma unroll
