@@ -250,8 +250,9 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * destination-blocked list: at most blk_tile_cap edge slots per tile (a
  * multiple of 256; default the smallest power of two from 2^13 that is at
  * least E / 512, up to 2^17, then doubled while more than 4096 tiles of it fit
- * in E) and the dispatch order 0 = smallest tiles first (default), 1 = by block,
- * 2 = largest first, 3 = by descending block. blk_range_bits > 0 (18-31)
+ * in E) and the dispatch order 0 = smallest tiles first, 1 = by block, 2 =
+ * largest first, 3 = by descending block (default: 2 for more than 512 tiles
+ * but in the plain schedule, else 0). blk_range_bits > 0 (18-31)
  * also cuts every block's tiles where their sources cross multiples of
  * 2^blk_range_bits and dispatches the tiles range by range, so that the
  * source gathers of the workgroups in flight stay in one range; the default

@@ -81,7 +81,7 @@ void graph_free(sssp_graph *g)
                     g->blk_a, g->blk_b, g->parent, g->ctrl, g->bdist, g->bscratch,
                     g->src_list, g->btasks, g->bcounter, g->bround, g->x_src, g->x_dst,
                     g->x_w, g->xgoff, g->pile[0], g->pile[1], g->farst, g->snap,
-                    g->b_pk, g->b_cbase, g->b_wide, g->b_w, g->b_tile, g->b_ltile, g->l_pk, g->l_cbase, g->l_wide, g->l_w, g->b_app, g->t_tile, g->t_state, g->t_seg, g->fbits, g->m_rec, g->m_tile, g->mdist,
+                    g->b_pk, g->b_cbase, g->b_wide, g->b_w, g->b_tile, g->b_ptile, g->b_ltile, g->l_pk, g->l_cbase, g->l_wide, g->l_w, g->b_app, g->t_tile, g->t_state, g->t_seg, g->fbits, g->m_rec, g->m_tile, g->mdist,
                     g->vperm, g->vinv, g->dout != g->dist ? g->dout : nullptr, g->msrc, g->mctl, g->mstamp, g->m_lrec, g->m_ltile, g->dvis, g->el_first};
     if (g->batch_exec) (void)hipGraphExecDestroy((hipGraphExec_t)g->batch_exec);
     for (auto &pair : g->mexec)
@@ -376,7 +376,8 @@ void graph_finish(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, con
     g->device_bytes = Ei * 12 + xe * 12 + (g->b_edges + g->l_edges) * 8 +
                       (g->b_edges + g->l_edges) / kBlkChunk * 4 +
                       (g->b_nwide + g->l_nwide) * kBlkChunk * 4 +
-                      (int64_t)(g->n_btile + g->n_ltile) * (int64_t)sizeof(BlkTile) +
+                      (int64_t)(g->n_btile * (g->b_ptile ? 2 : 1) + g->n_ltile) *
+                          (int64_t)sizeof(BlkTile) +
                       (int64_t)std::max(g->n_btile, g->n_ltile) * kBlkThreads * 2 +
                       (int64_t)g->n_ttile * (int64_t)(sizeof(BlkTile) + sizeof(TileState)) +
                       (int64_t)g->n_seg * 4 +
@@ -756,15 +757,17 @@ int sssp_set_param(sssp_graph *g, const char *name, double value)
             SSSP_REQUIRE(value >= (double)kBlkChunk && value <= 2147483648.0 &&
                              std::fmod(value, (double)kBlkChunk) == 0,
                          "blk_tile_cap must be a multiple of 256 in [256, 2^31]");
-            retile_blocked(g, (int64_t)value, g->blk_tile_order, g->blk_range_bits);
+            retile_blocked(g, (int64_t)value, g->blk_order_set ? g->blk_tile_order : -1,
+                           g->blk_range_bits);
         } else if (n == "blk_tile_order") {
             SSSP_REQUIRE(value == 0 || value == 1 || value == 2 || value == 3,
                          "blk_tile_order must be 0, 1, 2 or 3");
             retile_blocked(g, g->blk_tile_cap, (int)value, g->blk_range_bits);
+            g->blk_order_set = true;
         } else if (n == "blk_range_bits") {
             SSSP_REQUIRE(value == 0 || (value >= kBlkRangeFineBits && value <= 31),
                          "blk_range_bits must be 0 or in [18, 31]");
-            retile_blocked(g, g->blk_tile_cap, g->blk_tile_order, (int)value);
+            retile_blocked(g, g->blk_tile_cap, g->blk_order_set ? g->blk_tile_order : -1, (int)value);
         } else if (n == "decide_spin") {
             SSSP_REQUIRE(value == 0 || value == 1, "decide_spin must be 0 or 1");
             g->decide_spin = (int)value;

@@ -2293,7 +2293,7 @@ void frontier_to_queue(sssp_graph *g, int32_t r)
 constexpr int32_t kNotLocal = -1;
 template <class WT>
 void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st,
-                int32_t local = kNotLocal);
+                int32_t local = kNotLocal, const BlkTile *tiles = nullptr);
 
 template <class WT>
 bool run_round(sssp_graph *g, int mode, int kidx, int32_t r, int32_t tick0, const RoundSlot &cur,
@@ -2489,13 +2489,15 @@ constexpr int kPassAhead = 3;
 // With trace_events every pass is launched alone between events. Adds the
 // passes to the stats and the trace; full_limit: full passes at most (then
 // SSSP_ERR_NOT_CONVERGED). local: source of a run of local passes
-// (k_blk_local), or kNotLocal: k_blk_plain.
+// (k_blk_local), or kNotLocal: k_blk_plain. tiles: the full tiles in another
+// order.
 template <class WT>
-void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int32_t local)
+void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int32_t local,
+                const BlkTile *tiles)
 {
     hipStream_t s = g->stream;
     PassArgs a{};
-    a.full = g->b_tile;
+    a.full = tiles ? tiles : g->b_tile;
     a.light = g->b_ltile;
     a.n_full = g->n_btile;
     a.n_light = g->n_ltile;
@@ -2616,7 +2618,7 @@ void solve_plain(sssp_graph *g, bool mixed, int32_t source, sssp_stats *st)
     }
     if (plain_uses_blocked(g)) {
         run_passes<WT>(g, mixed && WT::kWeighted && g->n_ltile > 0 ? kRunMixed : kRunFull, limit,
-                       st);
+                       st, kNotLocal, mixed ? nullptr : g->b_ptile);
         return;
     }
     const int64_t ng = E >> 2;

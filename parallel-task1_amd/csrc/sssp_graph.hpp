@@ -239,6 +239,8 @@ struct sssp_graph {
     std::vector<int64_t> l_off_host;  // ... of the light list
     int64_t blk_tile_cap = 0;         // edges per tile at most
     int blk_tile_order = 0;           // dispatch order of the tiles (make_blk_tiles)
+    bool blk_order_set = false;       // by the caller, not by the tile count
+    sssp::BlkTile *b_ptile = nullptr; // smallest first for the plain schedule (null: b_tile)
     sssp::BlkRanges b_ranges;         // source-range cuts of the block runs (may be empty)
     int blk_range_bits = 0;           // tiles cut by source ranges of 2^bits vertices (0: no)
     int64_t b_edges = 0;  // edges in the blocked list, padding included

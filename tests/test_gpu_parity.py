@@ -683,6 +683,30 @@ def test_graphs_solved_whole_in_lds(gpu, oracle, V, E, kind):
 
 
 @pytest.mark.gpu
+def test_tile_order_by_count(gpu, oracle):
+    """More tiles than run at once are dispatched largest first (the plain
+    schedule's smallest first), fewer smallest first, unless the caller set an
+    order; all end on the oracle's fixpoint."""
+    src, dst, w = S.rmat(14, 16, seed=47, threads=16)
+    V = 1 << 14
+    ref = oracle.dijkstra(src, dst, w, V, 5)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        g.set_param("plain_kernel", 2)
+        for cap, order in ((1 << 17, 0), (256, 2), (512, 0), (256, 2)):
+            g.set_param("blk_tile_cap", cap)
+            print(f"tile order: cap {cap}, {g.get_param('blk_tiles')} tiles", flush=True)
+            assert (g.get_param("blk_tiles") > 512) == (order == 2)
+            assert g.get_param("blk_tile_order") == order
+            for below in (2.0 ** 26, 0.0):
+                g.set_param("plain_below_edges", below)
+                for sched in ("heuristic", "plain"):
+                    assert np.array_equal(bits(g.solve(5, sched)[0]), bits(ref)), (cap, sched)
+        g.set_param("blk_tile_order", 1)
+        g.set_param("blk_tile_cap", 1024)
+        assert g.get_param("blk_tile_order") == 1
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,cap", [(1, 1 << 13), (1 << 22, 1 << 13), ((1 << 22) + 1, 1 << 14),
                                    (1 << 23, 1 << 14), ((1 << 23) + 1, 1 << 15)])
 def test_default_tile_cap(gpu, oracle, E, cap):
