@@ -322,7 +322,7 @@ int sssp_init_distances_f64(double *d_dist, int32_t vertices, int32_t source);
 int sssp_init_distances_u32(uint32_t *d_dist, int32_t vertices, int32_t source);
 /* bellman_ford_wrapper<W> (bellman_ford.cu:103-144): all-edge passes over the
  * caller's edge list, in its order, until a pass changes nothing (at most
- * `vertices` passes). On lists of 2^19 edges or more a pass leaves out the edges
+ * `vertices` passes). On lists of 786432 edges or more a pass leaves out the edges
  * whose source did not change since it last relaxed them, told by two copies of
  * the distances allocated for the call (without memory for them every pass
  * relaxes every edge), and passes over the light edges alone run between them.

@@ -3369,8 +3369,9 @@ constexpr int kActUnroll = 2;
 constexpr int32_t kActBits = 1 << 20;
 constexpr int kActThreads = 1024;
 // Fewer edges run every edge in one launch a pass: R-MAT 14 x 16 0.287 ms against
-// 0.305, uniform 2000 x 4 0.26 against 0.30, power-law 100 K x 16 0.88 against 0.65.
-constexpr int64_t kActMinEdges = 1 << 19;
+// 0.305, uniform 90 K x 7 0.51 against 0.55, power-law 124 K x 8 (990 K edges)
+// 0.49 against 0.47, 100 K x 16 0.88 against 0.65.
+constexpr int64_t kActMinEdges = 3 << 18;
 // Passes queued per host check: a third of those that ran, between these (an
 // idle pass and mark take 4-8 us, a check 30).
 constexpr int kActBatch = 6, kActBatchMax = 32;

@@ -799,6 +799,38 @@ void radix_sort(const RsArrays<NA> &in, const RsArrays<NA> &fin, const RsArrays<
 
 inline uint32_t *u32p(const void *p) { return static_cast<uint32_t *>(const_cast<void *>(p)); }
 
+// Short-lived arrays of the build, cut from memory the sorts no longer need
+// (an allocation and its release cost 20 us and more, each); allocated where it
+// is used up. Used in stream order only.
+class Carve {
+  public:
+    Carve(void *base, size_t bytes) : p_(static_cast<char *>(base)), left_(bytes / 256 * 256) {}
+    Carve(const Carve &) = delete;
+    Carve &operator=(const Carve &) = delete;
+    ~Carve()
+    {
+        for (void *x : own_) dfree(x);
+    }
+    template <class T>
+    T *get(size_t n)
+    {
+        const size_t b = (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
+        if (b > left_) {
+            own_.push_back(dmalloc<char>(b));
+            return static_cast<T *>(own_.back());
+        }
+        T *at = reinterpret_cast<T *>(p_);
+        p_ += b;
+        left_ -= b;
+        return at;
+    }
+
+  private:
+    char *p_;
+    size_t left_;
+    std::vector<void *> own_;
+};
+
 void build_static_list(const int64_t *ptr, int32_t V, int64_t E, int64_t *tmp_flags,
                        int64_t *tmp_pos, int64_t *blk_a, int64_t *blk_b, int64_t n_blk,
                        hipStream_t s, int32_t **nz_v, int64_t **nz_scan, int32_t *n_nz,
@@ -1191,14 +1223,10 @@ static void build_local_tiles(sssp_graph *g)
 // With many equal weights the class can come out far from that share; below
 // half or above three times the target there are no classes (0xFFFFFFFF: every
 // edge is light and light passes do not run).
-static uint32_t light_threshold(sssp_graph *g)
+static uint32_t light_threshold(sssp_graph *g, Carve &tmp)
 {
     const int64_t n = std::min<int64_t>(g->E, kLightSample);
-    uint32_t *d = dmalloc<uint32_t>((size_t)n + 2);
-    struct F {
-        void *p;
-        ~F() { dfree(p); }
-    } f{d};
+    uint32_t *d = tmp.get<uint32_t>((size_t)n + 2);
     SSSP_HIP(hipMemsetAsync(d + n, 0, 8, g->stream));
     k_edge_sample<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, g->stream>>>(
         g->el_src, g->el_dst, g->el_w, g->E, (int32_t)n,
@@ -1235,20 +1263,11 @@ static uint32_t light_threshold(sssp_graph *g)
 }
 
 // Packs nch chunks of whole sources and destination offsets (k_blk_pack).
-static void pack_chunks(const int32_t *bs, const uint16_t *bd, int64_t nch, hipStream_t s,
+static void pack_chunks(const int32_t *bs, const uint16_t *bd, int64_t nch, hipStream_t s, Carve &tmp,
                         uint32_t **pk, int32_t **cbase, int32_t **wide, int64_t *nwide)
 {
-    uint8_t *wflag = dmalloc<uint8_t>((size_t)nch);
-    struct F {
-        void *p[2] = {};
-        ~F()
-        {
-            for (void *x : p) dfree(x);
-        }
-    } f;
-    f.p[0] = wflag;
-    int32_t *widx = dmalloc<int32_t>((size_t)nch);
-    f.p[1] = widx;
+    uint8_t *wflag = tmp.get<uint8_t>((size_t)nch);
+    int32_t *widx = tmp.get<int32_t>((size_t)nch);
     const unsigned chunk_grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
     k_blk_chunk_wide<<<chunk_grid, kBlock, 0, s>>>(bs, nch, wflag);
     SSSP_LAUNCH_CHECK("k_blk_chunk_wide");
@@ -1270,14 +1289,10 @@ static void pack_chunks(const int32_t *bs, const uint16_t *bd, int64_t nch, hipS
 
 // Source-range cuts of every block's run (k_blk_range_offsets), to the host.
 static void range_cuts(const int32_t *bs, const int64_t *boff, int32_t nblk, int32_t nfine,
-                       hipStream_t s, std::vector<int64_t> *out)
+                       hipStream_t s, Carve &tmp, std::vector<int64_t> *out)
 {
     const int64_t n_off = (int64_t)nblk * (nfine + 1);
-    int64_t *roff = dmalloc<int64_t>((size_t)n_off);
-    struct F {
-        void *p;
-        ~F() { dfree(p); }
-    } f{roff};
+    int64_t *roff = tmp.get<int64_t>((size_t)n_off);
     k_blk_range_offsets<<<grid_for(n_off), kBlock, 0, s>>>(bs, boff, nblk, kBlkRangeFineBits, nfine,
                                                           roff);
     SSSP_LAUNCH_CHECK("k_blk_range_offsets");
@@ -1292,22 +1307,14 @@ static void range_cuts(const int32_t *bs, const int64_t *boff, int32_t nblk, int
 // chunks as the blocked list's. (The padding of the blocked list may be light:
 // its copies of an edge are copied too.)
 static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *bd,
-                             const int64_t *boff, int32_t nblk, int64_t nch)
+                             const int64_t *boff, int32_t nblk, int64_t nch, Carve &tmp)
 {
     hipStream_t s = g->stream;
-    const uint32_t thr = light_threshold(g);
-    if (thr == 0xFFFFFFFFu) return;
-    struct F {
-        void *p[5] = {};
-        ~F()
-        {
-            for (void *x : p) dfree(x);
-        }
-    } f;
-    int64_t *pos = dmalloc<int64_t>((size_t)nch + 1);
-    f.p[0] = pos;
-    int64_t *lptr = dmalloc<int64_t>(2 * ((size_t)nblk + 1));
-    f.p[1] = lptr;
+    const uint32_t thr = light_threshold(g, tmp);
+    // none on graphs whose solves run in one workgroup (0.15 ms of the build)
+    if (thr == 0xFFFFFFFFu || (solo_fits(g) && g->E < kSoloEdges)) return;
+    int64_t *pos = tmp.get<int64_t>((size_t)nch + 1);
+    int64_t *lptr = tmp.get<int64_t>(2 * ((size_t)nblk + 1));
     int64_t *loff = lptr + nblk + 1;
     const unsigned chunk_grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
     k_light_count<<<chunk_grid, kBlock, 0, s>>>(g->b_w, nch * kBlkChunk, nch, thr, pos);
@@ -1324,10 +1331,8 @@ static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *b
     const int64_t Lp = lo[(size_t)nblk];
     if (Lp == 0) return;
     SSSP_HIP(hipMemcpyAsync(loff, lo.data(), 8 * lo.size(), hipMemcpyHostToDevice, s));
-    int32_t *ls = dmalloc<int32_t>((size_t)Lp);
-    f.p[2] = ls;
-    uint16_t *ld = dmalloc<uint16_t>((size_t)Lp);
-    f.p[3] = ld;
+    int32_t *ls = tmp.get<int32_t>((size_t)Lp);
+    uint16_t *ld = tmp.get<uint16_t>((size_t)Lp);
     g->l_w = dmalloc<uint32_t>((size_t)Lp);
     k_light_gather<<<chunk_grid, kBlock, 0, s>>>(bs, bd, g->b_w, nch, thr, pos, boff, nblk, lptr,
                                                  loff, ls, ld, g->l_w);
@@ -1335,9 +1340,9 @@ static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *b
     k_blk_pad<<<grid_for((int64_t)nblk * kBlkChunk), kBlock, 0, s>>>(lptr, loff, nblk, ls, ld,
                                                                      g->l_w);
     SSSP_LAUNCH_CHECK("k_blk_pad light");
-    pack_chunks(ls, ld, Lp / kBlkChunk, s, &g->l_pk, &g->l_cbase, &g->l_wide, &g->l_nwide);
+    pack_chunks(ls, ld, Lp / kBlkChunk, s, tmp, &g->l_pk, &g->l_cbase, &g->l_wide, &g->l_nwide);
     if (g->b_ranges.n_fine > 0)
-        range_cuts(ls, loff, nblk, g->b_ranges.n_fine, s, &g->b_ranges.loff);
+        range_cuts(ls, loff, nblk, g->b_ranges.n_fine, s, tmp, &g->b_ranges.loff);
     g->l_off_host = lo;
     g->l_edges = Lp;
     g->light_edges = lp[(size_t)nblk];
@@ -1573,16 +1578,17 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
         k_blk_pad<<<grid_for((int64_t)nblk * kBlkChunk), kBlock, 0, s>>>(bptr, boff, nblk, bs, bd,
                                                                          g->b_w);
         SSSP_LAUNCH_CHECK("k_blk_pad");
-        pack_chunks(bs, bd, nch, s, &g->b_pk, &g->b_cbase, &g->b_wide, &g->b_nwide);
+        Carve tmp(kA, 16 * (size_t)n_sort);  // the sorted arrays are placed
+        pack_chunks(bs, bd, nch, s, tmp, &g->b_pk, &g->b_cbase, &g->b_wide, &g->b_nwide);
         // source-range cuts of every block at 2^kBlkRangeFineBits granularity
         // (for tiles dispatched range by range), when the table is small
         const int64_t nfine = ((int64_t)V + (1 << kBlkRangeFineBits) - 1) >> kBlkRangeFineBits;
         if ((int64_t)nblk * (nfine + 1) <= kBlkRangeMaxEntries) {
-            range_cuts(bs, boff, nblk, (int32_t)nfine, s, &g->b_ranges.off);
+            range_cuts(bs, boff, nblk, (int32_t)nfine, s, tmp, &g->b_ranges.off);
             g->b_ranges.fine_bits = kBlkRangeFineBits;
             g->b_ranges.n_fine = (int32_t)nfine;
         }
-        build_light_list(g, bs, bd, boff, nblk, nch);
+        build_light_list(g, bs, bd, boff, nblk, nch, tmp);
         SSSP_HIP(hipStreamSynchronize(s));
         // Without hubs the d[src] gathers of a tile spread over the whole
         // distance array (degree order cannot gather them), so a graph whose

@@ -100,8 +100,8 @@ def test_wrappers_reject_bad_arrays(gpu, lib):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float64, np.uint32], ids=["f32", "f64", "u32"])
-@pytest.mark.parametrize("V,E,shift", [(1, 3, 0), (65, (1 << 19) - 1, 0),
-                                       (1, (1 << 19) + 3, 0), (65, 1 << 19, 1), (1 << 20, 3 << 20, 0), ((1 << 20) + 1, (3 << 20) + 2, 0),
+@pytest.mark.parametrize("V,E,shift", [(1, 3, 0), (65, (3 << 18) - 1, 0),
+                                       (1, (3 << 18) + 3, 0), (65, 3 << 18, 1), (1 << 20, 3 << 20, 0), ((1 << 20) + 1, (3 << 20) + 2, 0),
                                        (3000000, 4000003, 1)])
 def test_wrapper_change_bits(gpu, lib, oracle, dtype, V, E, shift):
     """The change bits of the wrappers' passes, on both sides of the edge count they
@@ -141,7 +141,7 @@ def test_wrapper_light_classes(gpu, lib, oracle, ends, weights):
     and with none (few edges per vertex, equal weights, or too many of the
     lightest): bit equality with the oracle."""
     rng = np.random.default_rng(31)
-    E = (1 << 19) + 5
+    E = (3 << 18) + 5
     V = 200003 if ends == "sparse" else 40009
     s, d = ((rng.random(E) ** (4 if ends == "hubs" else 1) * V).astype(np.int32)
             for _ in range(2))
