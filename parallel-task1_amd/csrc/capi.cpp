@@ -88,10 +88,8 @@ void graph_free(sssp_graph *g)
         for (void *e : pair)
             if (e) (void)hipGraphExecDestroy((hipGraphExec_t)e);
     for (void *p : ptrs) dfree(p);
-    for (int c = 0; c < kChunkCount; c++) {
-        dfree(g->nzo_tile[c]);
-        dfree(g->nzi_tile[c]);
-    }
+    dfree(g->nzo_tile[0]);  // the first table's allocation holds them all
+    dfree(g->nzi_tile[0]);
     if (g->ctrl_host) (void)hipHostFree(g->ctrl_host);
     for (hipEvent_t e : g->stage_ev)
         if (e) (void)hipEventDestroy(e);

@@ -851,11 +851,14 @@ void build_static_list(const int64_t *ptr, int32_t V, int64_t E, int64_t *tmp_fl
     *nz_scan = dmalloc<int64_t>((size_t)n + 1);
     k_nz_compact<<<grid_for(V), kBlock, 0, s>>>(ptr, V, tmp_pos, *nz_v, *nz_scan, n, E);
     SSSP_LAUNCH_CHECK("k_nz_compact");
+    // the tables in one allocation, tiles[0]'s
+    size_t at[kChunkCount + 1] = {};
+    auto count = [&](int c) { return (E + kBlock * kChunkK[c] - 1) / (kBlock * kChunkK[c]); };
+    for (int c = 0; c < kChunkCount; c++) at[c + 1] = at[c] + ((size_t)count(c) + 1 + 63) / 64 * 64;
+    tiles[0] = dmalloc<int32_t>(at[kChunkCount]);
     for (int c = 0; c < kChunkCount; c++) {
-        const int64_t TE = (int64_t)kBlock * kChunkK[c];
-        const int64_t ntiles = (E + TE - 1) / TE;
-        tiles[c] = dmalloc<int32_t>((size_t)ntiles + 1);
-        build_tile_table(*nz_scan, (int32_t)n, E, (int32_t)TE, tiles[c], s);
+        tiles[c] = tiles[0] + at[c];
+        build_tile_table(*nz_scan, (int32_t)n, E, kBlock * kChunkK[c], tiles[c], s);
     }
 }
 
