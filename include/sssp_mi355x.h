@@ -323,8 +323,8 @@ int sssp_init_distances_u32(uint32_t *d_dist, int32_t vertices, int32_t source);
 /* bellman_ford_wrapper<W> (bellman_ford.cu:103-144): all-edge passes over the
  * caller's edge list, in its order, until a pass changes nothing (at most
  * `vertices` passes). On lists of 786432 edges or more a pass leaves out the edges
- * whose source did not change since it last relaxed them, told by two copies of
- * the distances allocated for the call (without memory for them every pass
+ * whose source did not change since it last relaxed them, told by a copy of
+ * the distances allocated for the call (without memory for it every pass
  * relaxes every edge), and passes over the light edges alone run between them.
  * Convergence is tested on the device; *passes (may be NULL) receives the count
  * of passes over all weights. The edge arrays are checked on the device

@@ -3462,14 +3462,15 @@ __global__ __launch_bounds__(kActSamples) void k_act_begin(const int32_t *src, c
     }
 }
 
-// Before pass p: the vertices changed by the pass before (bits[0]) and since
-// the last full pass began (bits[1]), one bit each (bit v & mask; several
-// vertices share one where V exceeds the mask), against the copies last[] and
-// full[]. The first mark takes every vertex with a distance. A mark after one
-// that left nothing pending returns at once, and so does pass p.
+// Before pass p: the vertices changed by the pass before, against their copy
+// last[], one bit each (bit v & mask; several vertices share one where V
+// exceeds the mask), and, with a light class, those changed since the last full
+// pass began, the words after them: the union of the marks since. The first
+// mark takes every vertex with a distance. A mark after one that left nothing
+// pending returns at once, and so does pass p.
 template <class DT>
 __global__ __launch_bounds__(kActThreads) void k_mark_changed(const DT *__restrict__ dist, DT *last,
-                                                              DT *full, int32_t V, int32_t n_bits,
+                                                              int32_t V, int32_t n_bits,
                                                               unsigned long long *bits,
                                                               ActCtl<DT> *c, int32_t p, DT inf)
 {
@@ -3488,24 +3489,21 @@ __global__ __launch_bounds__(kActThreads) void k_mark_changed(const DT *__restri
     int low = 0;
     bool pend = false;
     for (int i = wave; i < words; i += (int)gridDim.x * (kActThreads / 64)) {
-        bool ch = false, chf = false;
+        bool ch = false;
+        unsigned long long since = light && p > 0 && !was_full ? bits[words + i] : 0;
         for (int64_t v = (int64_t)i * 64 + lane; v < V; v += n_bits) {
             const DT d = dist[v], l = p > 0 ? last[v] : inf;
             ch |= d != l;
             low += d != l ? 1 : 0;
             if (p == 0 || d != l) last[v] = d;
-            if (light) {
-                const DT f = p == 0 || was_full ? l : full[v];
-                if (p == 0 || was_full) full[v] = f;
-                chf |= d != f;
-            }
         }
-        const unsigned long long m = __ballot(ch), mf = light ? __ballot(chf) : m;
+        const unsigned long long m = __ballot(ch);
+        since |= m;
         if (lane == 0) {
             bits[i] = m;
-            if (light) bits[words + i] = mf;
+            if (light) bits[words + i] = since;
         }
-        pend |= mf != 0;
+        pend |= since != 0;
     }
     if (!light) {  // nothing is counted
         if (pend && lane == 0) c->pend[p & 63] = 1;
@@ -3621,17 +3619,15 @@ __global__ __launch_bounds__(kActThreads) void k_el_active(const int32_t *__rest
     }
 }
 
-// Scratch of a call: state, two sets of bits, two copies of the distances.
+// Scratch of a call: state, two sets of bits, a copy of the distances.
 template <class DT>
 struct ActScratch {
-    size_t bits, last, full, bytes;
+    size_t bits, last, bytes;
     explicit ActScratch(int32_t V)
     {
-        const size_t v = ((size_t)V * sizeof(DT) + 255) / 256 * 256;
         bits = (sizeof(ActCtl<DT>) + 255) / 256 * 256;
         last = bits + 2 * (kActBits / 8);
-        full = last + v;
-        bytes = full + v;
+        bytes = last + (size_t)V * sizeof(DT);
     }
 };
 
@@ -3647,7 +3643,7 @@ void ref_bf_active(const int32_t *src, const int32_t *dst, const DT *w, int32_t 
     const ActScratch<DT> at(V);
     ActCtl<DT> *const c = reinterpret_cast<ActCtl<DT> *>(mem);
     unsigned long long *bits = reinterpret_cast<unsigned long long *>(mem + at.bits);
-    DT *last = reinterpret_cast<DT *>(mem + at.last), *full = reinterpret_cast<DT *>(mem + at.full);
+    DT *last = reinterpret_cast<DT *>(mem + at.last);
     k_act_begin<DT><<<1, kActSamples>>>(src, dst, w, V, E, WT::kWeighted ? 1 : 0,
                                         (int32_t)(kLightStopFrac * V), c);
     SSSP_LAUNCH_CHECK("k_act_begin");
@@ -3665,8 +3661,8 @@ void ref_bf_active(const int32_t *src, const int32_t *dst, const DT *w, int32_t 
     while (!done) {
         const int batch = std::min(kActBatchMax, std::max(kActBatch, pass / 3));
         for (int i = 0; i < batch; i++) {
-            k_mark_changed<DT><<<(unsigned)mgrid, kActThreads>>>(d, last, full, V, n_bits, bits, c,
-                                                                 pass + i, (DT)WT::INF);
+            k_mark_changed<DT><<<(unsigned)mgrid, kActThreads>>>(d, last, V, n_bits, bits, c, pass + i,
+                                                                 (DT)WT::INF);
             if (vec)
                 k_el_active<WT, DT, 4><<<(unsigned)nblocks, kActThreads, lds>>>(
                     src, dst, w, E, d, bits, n_bits, mask, c, pass + i, per_block);
