@@ -3373,8 +3373,9 @@ constexpr int kActThreads = 1024;
 // 0.49 against 0.47, 100 K x 16 0.88 against 0.65.
 constexpr int64_t kActMinEdges = 3 << 18;
 // Passes queued per host check: a third of those that ran, between these (an
-// idle pass and mark take 4-8 us, a check 30).
-constexpr int kActBatch = 6, kActBatchMax = 32;
+// idle pass and mark take 4-8 us, a check 30). 6 / 12 / 16 at first, us a call: power-law
+// 1 M x 16 1780 / 1744 / 1770, f64 788 / 773 / 800, uniform 500 K x 16 1449 / 1389 / 1433.
+constexpr int kActBatch = 12, kActBatchMax = 32;
 
 // State of a run of passes on the device, rings of 64 by pass. Light edges
 // (weight pattern at most thr) are relaxed to near convergence between full
