@@ -3373,8 +3373,10 @@ constexpr int kActThreads = 1024;
 // 0.49 against 0.47, 100 K x 16 0.88 against 0.65.
 constexpr int64_t kActMinEdges = 3 << 18;
 // Passes queued per host check: a third of those that ran, between these (an
-// idle pass and mark take 4-8 us, a check 30). 6 / 12 / 16 at first, us a call: power-law
-// 1 M x 16 1780 / 1744 / 1770, f64 788 / 773 / 800, uniform 500 K x 16 1449 / 1389 / 1433.
+// idle pass and mark take 4-8 us, a check 30). 6 / 12 / 16 at first, us a call, means of two
+// runs: power-law 1 M x 16 1829 (1781, 1877) / 1744 / 1771, f64 300 K x 14 788 / 773 / 803,
+// uniform 500 K x 16 1449 / 1389 / 1433; 12 gives little or nothing on power-law 2 M x 5
+// (1721 / 1723 / 1673) and uniform 2 M x 16 (5339 / 5293 / 5269), where 16 is the better.
 constexpr int kActBatch = 12, kActBatchMax = 32;
 
 // State of a run of passes on the device, rings of 64 by pass. Light edges
