@@ -227,6 +227,14 @@ const char *sssp_last_error(void) { return g_last_error.c_str(); }
 
 int sssp_version(void) { return 10000; }
 
+int sssp_debug_wrapper_route(int32_t *changed_only)
+{
+    return guard([&] {
+        SSSP_REQUIRE(changed_only, "null output");
+        *changed_only = t_wrapper_active ? 1 : 0;
+    });
+}
+
 int sssp_debug_fail_next_alloc(void)
 {
     g_fail_next_alloc = 1;
@@ -664,8 +672,9 @@ int sssp_bfs_edges(const int32_t *d_src, const int32_t *d_dst, int32_t vertices,
         SSSP_REQUIRE(d_visited && vertices >= 1 && edges >= 0 && (edges == 0 || (d_src && d_dst)),
                      "bad arguments");
         SSSP_REQUIRE(source >= 0 && source < vertices, "source vertex out of range");
-        validate_edges(d_src, d_dst, nullptr, -1, edges, vertices, nullptr);
-        ref_bfs(d_src, d_dst, vertices, edges, d_visited, source, passes);
+        ListOrder order;
+        validate_edges(d_src, d_dst, nullptr, -1, edges, vertices, nullptr, nullptr, &order);
+        ref_bfs(d_src, d_dst, vertices, edges, d_visited, source, passes, order);
     });
 }
 
@@ -881,9 +890,10 @@ int sssp_bellman_ford_f32(const int32_t *d_src, const int32_t *d_dst, const floa
         SSSP_REQUIRE(d_dist && vertices >= 1 && edges >= 0 && (edges == 0 || (d_src && d_dst && d_w)),
                      "bad arguments");
         SSSP_REQUIRE(source >= 0 && source < vertices, "source vertex out of range");
-        validate_edges(d_src, d_dst, d_w, SSSP_W_F32, edges, vertices, nullptr);
+        ListOrder order;
+        validate_edges(d_src, d_dst, d_w, SSSP_W_F32, edges, vertices, nullptr, nullptr, &order);
         ref_bf<WF32, uint32_t>(d_src, d_dst, reinterpret_cast<const uint32_t *>(d_w), vertices, edges,
-                               reinterpret_cast<uint32_t *>(d_dist), passes);
+                               reinterpret_cast<uint32_t *>(d_dist), passes, order);
     });
 }
 
@@ -908,8 +918,9 @@ int sssp_bellman_ford_u32(const int32_t *d_src, const int32_t *d_dst, const uint
         SSSP_REQUIRE(d_dist && vertices >= 1 && edges >= 0 && (edges == 0 || (d_src && d_dst && d_w)),
                      "bad arguments");
         SSSP_REQUIRE(source >= 0 && source < vertices, "source vertex out of range");
-        validate_edges(d_src, d_dst, d_w, SSSP_W_U32, edges, vertices, nullptr);
-        ref_bf<WU32, uint32_t>(d_src, d_dst, d_w, vertices, edges, d_dist, passes);
+        ListOrder order;
+        validate_edges(d_src, d_dst, d_w, SSSP_W_U32, edges, vertices, nullptr, nullptr, &order);
+        ref_bf<WU32, uint32_t>(d_src, d_dst, d_w, vertices, edges, d_dist, passes, order);
     });
 }
 
@@ -921,11 +932,12 @@ int sssp_bellman_ford_f64(const int32_t *d_src, const int32_t *d_dst, const doub
         SSSP_REQUIRE(d_dist && vertices >= 1 && edges >= 0 && (edges == 0 || (d_src && d_dst && d_w)),
                      "bad arguments");
         SSSP_REQUIRE(source >= 0 && source < vertices, "source vertex out of range");
-        validate_edges(d_src, d_dst, d_w, SSSP_W_F64, edges, vertices, nullptr);
+        ListOrder order;
+        validate_edges(d_src, d_dst, d_w, SSSP_W_F64, edges, vertices, nullptr, nullptr, &order);
         ref_bf<WF64, unsigned long long>(d_src, d_dst,
                                          reinterpret_cast<const unsigned long long *>(d_w), vertices,
                                          edges, reinterpret_cast<unsigned long long *>(d_dist),
-                                         passes);
+                                         passes, order);
     });
 }
 

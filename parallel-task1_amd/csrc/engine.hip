@@ -3368,10 +3368,38 @@ void ref_init(DT *d, int32_t V, int32_t source)
 constexpr int kActUnroll = 2;
 constexpr int32_t kActBits = 1 << 20;
 constexpr int kActThreads = 1024;
-// Fewer edges run every edge in one launch a pass: R-MAT 14 x 16 0.287 ms against
-// 0.305, uniform 90 K x 7 0.51 against 0.55, power-law 124 K x 8 (990 K edges)
-// 0.49 against 0.47, 100 K x 16 0.88 against 0.65.
+// Which lists the passes over changed sources are for; the others run every edge
+// in one launch a pass (k_el_pass). They save the random reads of distances, and cost
+// a second launch a pass, the marks (0.1 ms a call at least) and what a pass over
+// every edge gains from its own changes. So the line follows what those
+// reads cost. Every edge / changed sources, ms a call:
+//  - a list in random order: 4-byte weights, 40 K vertices x 20 0.60 / 0.52, 200 K x 6
+//    0.76 / 0.65, 500 K x 2.4 0.64 / 0.78 and 1 M x 2 0.98 / 0.97 (none below 3 edges per
+//    vertex, then), from 2 M edges on 0.3-0.8 of the time; f64 200 K x 6 0.49 / 0.50, 1 K
+//    x 1200 0.29 / 0.38, from 2 M edges on 0.45-1.0;
+//  - in order of the sources or the destinations (one of the two reads stays in
+//    cache): 100 K x 12 0.45 / 0.69, 500 K x 2.4 0.47 / 0.75, 200 K x 10 0.64 / 0.65, 100 K
+//    x 20 0.60 / 0.51, from 4 M edges 0.5-1.06 of the time; f64 500 K x 8 0.99 / 1.20, from 8 M edges
+//    0.5-0.9 (once 1.11);
+//  - in order and between near ids (both stay in cache, and a pass carries a path
+//    over many edges): grid 8000 x 200 211 / 315, 5000 x 300 100 / 187, 700 x 700 16.8 / 20.7,
+//    band of 900 ids, 1 M x 12 and 1 % far edges 2.0 / 2.9; f64 650 x 650 11.1 / 19.0;
+//    with ids 1500 and more apart 1500 x 1500 103 / 84;
+//  - hops, whose few passes hardly repay the marks: 10 K x 120 0.16 / 0.28 and x 1600 0.39 / 0.54,
+//    500 K x 4 0.42 / 0.49, 500 K x 6 0.51 / 0.42, 1 M x 16 1.6 / 0.74; in order 100 K x 80
+//    0.36 / 0.42, 200 K x 20 0.38 / 0.35, 500 K x 16 0.54 / 0.50, 2 M x 4 1.4 / 0.84.
 constexpr int64_t kActMinEdges = 3 << 18;
+template <class WT, class DT>
+bool act_pays(int64_t V, int64_t E, const ListOrder &order)
+{
+    constexpr int64_t M = 15 << 16;  // 0.98 million
+    if (order.near || E < kActMinEdges) return false;
+    if (!WT::kWeighted)
+        return order.ordered ? E >= 8 * M && V >= 1 << 18 : E >= 3 * M && V >= 1 << 16;
+    if (sizeof(DT) == 8) return E >= (order.ordered ? 8 * M : 2 * M);
+    if (order.ordered) return E >= 4 * M || (E >= 2 * M && E >= 16 * V);
+    return E >= 2 * M || E >= 3 * V;
+}
 // Passes queued per host check: a third of those that ran, between these (an
 // idle pass and mark take 4-8 us, a check 30). 6 / 12 / 16 at first, us a call, means of two
 // runs: power-law 1 M x 16 1829 (1781, 1877) / 1744 / 1771, f64 300 K x 14 788 / 773 / 803,
@@ -3687,11 +3715,14 @@ void ref_bf_active(const int32_t *src, const int32_t *dst, const DT *w, int32_t 
     if (passes_out) *passes_out = std::max(fulls, 1);
 }
 
+thread_local bool t_wrapper_active = false;
+
 template <class WT, class DT>
 void ref_bf(const int32_t *src, const int32_t *dst, const DT *w, int32_t V, int64_t E, DT *d,
-            int32_t *passes_out, int32_t *changed_buf)
+            int32_t *passes_out, const ListOrder &order, int32_t *changed_buf)
 {
-    if (!changed_buf && E >= kActMinEdges) {
+    t_wrapper_active = false;
+    if (!changed_buf && act_pays<WT, DT>(V, E, order)) {
         // the passes that keep the distances of the pass before; when there
         // is no memory for those, the passes over every edge
         void *mem = nullptr;
@@ -3700,6 +3731,7 @@ void ref_bf(const int32_t *src, const int32_t *dst, const DT *w, int32_t V, int6
                 void *p;
                 ~Free() { dfree(p); }
             } fr{mem};
+            t_wrapper_active = true;
             ref_bf_active<WT, DT>(src, dst, w, V, E, d, passes_out,
                                   static_cast<unsigned char *>(mem));
             return;
@@ -3769,7 +3801,7 @@ void levels_to_visited(const uint32_t *lev, int32_t V, uint8_t *vis, hipStream_t
 // (unit-weight Bellman-Ford, the dst array stands in for the unused weights)
 // and end in the visited flags, 1 for every vertex reachable from source.
 void ref_bfs(const int32_t *src, const int32_t *dst, int32_t V, int64_t E, uint8_t *visited,
-             int32_t source, int32_t *passes_out)
+             int32_t source, int32_t *passes_out, const ListOrder &order)
 {
     uint32_t *lev = dmalloc<uint32_t>((size_t)V);
     struct Free {
@@ -3778,7 +3810,7 @@ void ref_bfs(const int32_t *src, const int32_t *dst, int32_t V, int64_t E, uint8
     } fr{lev};
     ref_init<WUnit, uint32_t>(lev, V, source);
     ref_bf<WUnit, uint32_t>(src, dst, reinterpret_cast<const uint32_t *>(dst), V, E, lev,
-                            passes_out);
+                            passes_out, order);
     levels_to_visited(lev, V, visited, nullptr);
     SSSP_HIP(hipDeviceSynchronize());
 }
@@ -3830,7 +3862,7 @@ void ref_bf_noalloc_f32(const int32_t *src, const int32_t *dst, const uint32_t *
     unsigned char *p = scratch_on_current_device();
     validate_edges(src, dst, w, SSSP_W_F32, E, V, nullptr,
                    reinterpret_cast<int64_t *>(p + kScratchBad));
-    ref_bf<WF32, uint32_t>(src, dst, w, V, E, d, passes_out,
+    ref_bf<WF32, uint32_t>(src, dst, w, V, E, d, passes_out, ListOrder{},
                            reinterpret_cast<int32_t *>(p + kScratchFlags));
 }
 
@@ -3838,11 +3870,12 @@ template void ref_init<WF32, uint32_t>(uint32_t *, int32_t, int32_t);
 template void ref_init<WU32, uint32_t>(uint32_t *, int32_t, int32_t);
 template void ref_init<WF64, unsigned long long>(unsigned long long *, int32_t, int32_t);
 template void ref_bf<WF32, uint32_t>(const int32_t *, const int32_t *, const uint32_t *, int32_t,
-                                     int64_t, uint32_t *, int32_t *, int32_t *);
+                                     int64_t, uint32_t *, int32_t *, const ListOrder &, int32_t *);
 template void ref_bf<WU32, uint32_t>(const int32_t *, const int32_t *, const uint32_t *, int32_t,
-                                     int64_t, uint32_t *, int32_t *, int32_t *);
+                                     int64_t, uint32_t *, int32_t *, const ListOrder &, int32_t *);
 template void ref_bf<WF64, unsigned long long>(const int32_t *, const int32_t *,
                                                const unsigned long long *, int32_t, int64_t,
-                                               unsigned long long *, int32_t *, int32_t *);
+                                               unsigned long long *, int32_t *, const ListOrder &,
+                                               int32_t *);
 
 }  // namespace sssp

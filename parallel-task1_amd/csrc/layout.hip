@@ -1032,17 +1032,39 @@ void build_multi_layout(sssp_graph *g)
 // which orders non-negative IEEE values only. The two counters live in
 // `bad_buf` when the caller brings one (device memory, 16 bytes), else in a
 // buffer allocated for the call; a kernel clears them either way.
+// out[0..3) += sampled edges whose source (destination) is near that of the
+// edge 256 further on, and edges between near ids. Ids may still be invalid.
+constexpr int kOrderSamples = 512;
+__global__ __launch_bounds__(kOrderSamples) void k_list_order(const int32_t *src, const int32_t *dst,
+                                                              int64_t E, int64_t V, int64_t *out)
+{
+    const int64_t e = threadIdx.x * E / kOrderSamples, f = min(e + 256, E - 1);
+    const int64_t s = src[e], t = dst[e], step = max((int64_t)1, V / 64);
+    const bool b[3] = {llabs(src[f] - s) <= step, llabs(dst[f] - t) <= step,
+                       llabs(t - s) <= min((int64_t)kListNear, V / 32)};
+    for (int i = 0; i < 3; i++) {
+        const unsigned long long m = __ballot(b[i]);
+        if (m != 0 && __lane_id() == 0)
+            atomicAdd((unsigned long long *)&out[i], (unsigned long long)__popcll(m));
+    }
+}
+
 void validate_edges(const int32_t *src, const int32_t *dst, const void *w, int wtype, int64_t E,
-                    int32_t V, hipStream_t s, int64_t *bad_buf)
+                    int32_t V, hipStream_t s, int64_t *bad_buf, ListOrder *order)
 {
     if (E <= 0) return;
-    int64_t *bad = bad_buf ? bad_buf : dmalloc<int64_t>(2);
+    const int n = order ? 5 : 2;
+    int64_t *bad = bad_buf ? bad_buf : dmalloc<int64_t>((size_t)n);
     struct Free {
         void *p;
         ~Free() { dfree(p); }
     } fr{bad_buf ? nullptr : bad};
-    k_zero_i64<<<1, 64, 0, s>>>(bad, 2);
+    k_zero_i64<<<1, 64, 0, s>>>(bad, n);
     SSSP_LAUNCH_CHECK("k_zero_i64");
+    if (order) {
+        k_list_order<<<1, kOrderSamples, 0, s>>>(src, dst, E, V, bad + 2);
+        SSSP_LAUNCH_CHECK("k_list_order");
+    }
     if (wtype == SSSP_W_F32)
         k_validate<float><<<grid_for(E), kBlock, 0, s>>>(src, dst, static_cast<const float *>(w), E,
                                                          V, bad);
@@ -1056,11 +1078,15 @@ void validate_edges(const int32_t *src, const int32_t *dst, const void *w, int w
     else
         k_validate<uint32_t><<<grid_for(E), kBlock, 0, s>>>(src, dst, nullptr, E, V, bad);
     SSSP_LAUNCH_CHECK("k_validate");
-    int64_t hb[2] = {0, 0};
-    SSSP_HIP(hipMemcpyAsync(hb, bad, 16, hipMemcpyDeviceToHost, s));
+    int64_t hb[5] = {0, 0, 0, 0, 0};
+    SSSP_HIP(hipMemcpyAsync(hb, bad, 8 * n, hipMemcpyDeviceToHost, s));
     SSSP_HIP(hipStreamSynchronize(s));
     if (hb[0]) throw Error{SSSP_ERR_ARG, std::to_string(hb[0]) + " edges have a vertex id outside [0, V)"};
     if (hb[1]) throw Error{SSSP_ERR_ARG, std::to_string(hb[1]) + " edges have a negative or NaN weight"};
+    if (order) {
+        order->ordered = std::max(hb[2], hb[3]) * 2 >= kOrderSamples;
+        order->near = order->ordered && hb[4] * 2 >= kOrderSamples;
+    }
 }
 
 // The tiles of the destination-blocked list: runs of at most `cap` edge slots

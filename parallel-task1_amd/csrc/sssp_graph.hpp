@@ -492,9 +492,17 @@ void rmat_device(int scale, int ef, int a, int b, int c, int d, uint32_t base_se
 // layout.hip
 // ids in [0, V), and for wtype SSSP_W_F32/F64/U32 weights >= 0 and not NaN
 // (any other wtype: ids only); throws SSSP_ERR_ARG. bad_buf: 2 device
-// counters to use, or null (allocated for the call)
+// counters to use, or null (allocated for the call). order (only without
+// bad_buf): what a sample of the list says about its order, read back with
+// the counters.
+struct ListOrder {
+    bool ordered = false;  // by source or by destination: edges that follow each other share lines
+    bool near = false;     // and most edges join ids closer than kListNear
+};
+constexpr int32_t kListNear = 1 << 10;
 void validate_edges(const int32_t *src, const int32_t *dst, const void *w, int wtype, int64_t E,
-                    int32_t V, hipStream_t s, int64_t *bad_buf = nullptr);
+                    int32_t V, hipStream_t s, int64_t *bad_buf = nullptr,
+                    ListOrder *order = nullptr);
 // in-place exclusive scan of two arrays of nb + 1 values (the last one
 // receives the total), one workgroup each, in one launch
 void scan_blocks_pair_inplace(int64_t *a, int64_t *b, int64_t nb, hipStream_t s);
@@ -530,7 +538,10 @@ void ref_init(DT *d, int32_t V, int32_t source);
 // changed_buf: the 64 change flags (device), or null (allocated for the call)
 template <class WT, class DT>
 void ref_bf(const int32_t *src, const int32_t *dst, const DT *w, int32_t V, int64_t E, DT *d,
-            int32_t *passes_out, int32_t *changed_buf = nullptr);
+            int32_t *passes_out, const ListOrder &order, int32_t *changed_buf = nullptr);
+// whether the last wrapper call of this thread ran the passes over changed
+// sources only (test hook)
+extern thread_local bool t_wrapper_active;
 // bellman_ford_wrapper<float> with its scratch in a file-scope device array:
 // no device allocation (sssp_bellman_ford_noalloc_f32)
 void ref_bf_noalloc_f32(const int32_t *src, const int32_t *dst, const uint32_t *w, int32_t V,
@@ -540,7 +551,7 @@ void bfs(sssp_graph *g, int32_t source, int sched, sssp_stats *st);
 void certify_levels(sssp_graph *g, int32_t source, int64_t *counts);
 void levels_to_visited(const uint32_t *lev, int32_t V, uint8_t *vis, hipStream_t s);
 void ref_bfs(const int32_t *src, const int32_t *dst, int32_t V, int64_t E, uint8_t *visited,
-             int32_t source, int32_t *passes_out);
+             int32_t source, int32_t *passes_out, const ListOrder &order);
 void reset_stamps(sssp_graph *g);  // stamps: 0 (out-edges) / kSinkStamp; pile states: 0
 void solve(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, sssp_stats *st);
 void certify(sssp_graph *g, const int32_t *sources, int32_t n_src, int64_t *counts);

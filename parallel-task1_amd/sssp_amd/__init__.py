@@ -114,6 +114,7 @@ _SIGS = {
     "sssp_collect_timings": (I32, [P, I32, I32, P, P, PI32]),
     "sssp_features": (I32, [F64, F64, F64, F64, F64, F64, F64, P]),
     "sssp_debug_fail_next_alloc": (I32, []),
+    "sssp_debug_wrapper_route": (I32, [C.POINTER(I32)]),
 }
 
 

@@ -153,3 +153,48 @@ def test_wrapper_light_classes(gpu, lib, oracle, ends, weights):
     _, got, passes = _run(lib, np.float32, s, d, w, V, source)
     assert np.array_equal(_bits(got), _bits(oracle.bf(s, d, w, V, source)[0]))
     assert 1 <= passes <= V
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,V,E,routes", [
+    ("random", 50000, (3 << 18) - 1, "0000"), ("random", 50000, 3 << 18, "1010"),
+    ("random", 300000, 800000, "0000"), ("random", 50000, 15 << 17, "1110"),
+    ("random", 70000, 45 << 16, "1111"), ("by_src", 50000, (15 << 17) - 1, "0000"),
+    ("by_src", 50000, 15 << 17, "1010"), ("by_dst", 50000, 15 << 17, "1010"),
+    ("by_src", 300000, (15 << 18) - 1, "0000"), ("by_dst", 300000, 15 << 18, "1010"),
+    ("by_src", 300000, 15 << 19, "1111"), ("near", 300000, 15 << 19, "0000"),
+    ("near_by_dst", 40000, 15 << 18, "0000"), ("near_shuffled", 70000, 15 << 18, "1111")])
+def test_wrapper_route_follows_the_list(gpu, lib, oracle, order, V, E, routes):
+    """Which passes a list gets (f32, f64, u32, hops; 1: over changed sources
+    only), on both sides of every line: lists in random order, by source, by
+    destination, and ordered ones between near ids, where the passes over every
+    edge are the faster. Bit equality with the oracle on both routes."""
+    rng = np.random.default_rng(E + V)
+    s = rng.integers(0, V, E).astype(np.int32)
+    if order.startswith("near"):
+        d = np.clip(s + rng.integers(-200, 201, E), 0, V - 1).astype(np.int32)
+        d[::100] = rng.integers(0, V, len(d[::100]))  # and a few far edges
+    else:
+        d = rng.integers(0, V, E).astype(np.int32)
+    if not order.endswith(("random", "shuffled")):
+        o = np.argsort(d if order.endswith("by_dst") else s, kind="stable")
+        s, d = s[o], d[o]
+    w = rng.integers(1, 256, E)
+    source, route = int(s[E // 3]), C.c_int32(-1)
+    ref = oracle.dijkstra(s, d, w.astype(np.uint32), V, source)
+    far = ref == S.U32_INF
+    with HipBuffer(s) as ds, HipBuffer(d) as dd:
+        for k, dtype in enumerate((np.float32, np.float64, np.uint32)):
+            print(f"wrapper route: {order} V {V} E {E} {SUFFIX[dtype]}", flush=True)
+            _, got, passes = _run(lib, dtype, s, d, w.astype(dtype), V, source)
+            assert lib.sssp_debug_wrapper_route(C.byref(route)) == S.OK
+            # whole weights: distances stay exact in every type
+            assert np.array_equal(got[~far], ref[~far].astype(dtype))
+            assert np.all(got[far] == INF[dtype]) and 1 <= passes <= V
+            assert route.value == int(routes[k]), SUFFIX[dtype]
+        with HipBuffer(np.zeros(V, np.uint8)) as vis:
+            print(f"wrapper route: {order} V {V} E {E} hops", flush=True)
+            assert lib.sssp_bfs_edges(ds.ptr, dd.ptr, V, E, vis.ptr, source, None) == S.OK
+            assert np.array_equal(vis.get(), (~far).astype(np.uint8))
+        assert lib.sssp_debug_wrapper_route(C.byref(route)) == S.OK
+        assert route.value == int(routes[3]), "hops"
