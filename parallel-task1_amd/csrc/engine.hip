@@ -1882,7 +1882,7 @@ __global__ __launch_bounds__(64) void k_tile_spans(const BlkTile *__restrict__ t
     state[blockIdx.x] = TileState{first >> kSegBits, last >> kSegBits, 1, 0};
 }
 
-// Before the first pass only the source's segment has changed.
+// Before the first pass only the sources' segments have changed.
 __global__ __launch_bounds__(kBlock) void k_local_reset(int32_t *seg, int32_t n_seg,
                                                         TileState *state, int32_t n_tiles,
                                                         int32_t source)
@@ -1893,6 +1893,13 @@ __global__ __launch_bounds__(kBlock) void k_local_reset(int32_t *seg, int32_t n_
         state[i].done = 1;
         state[i].work = 0;
     }
+}
+
+__global__ __launch_bounds__(kBlock) void k_local_sources(int32_t *seg, const int32_t *sources,
+                                                          int32_t n)
+{
+    const int32_t i = (int32_t)(blockIdx.x * kBlock + threadIdx.x);
+    if (i < n) seg[sources[i] >> kSegBits] = 1;
 }
 
 // A pass of graphs whose edges join near ids and whose paths are long (grids,
@@ -2293,7 +2300,7 @@ void frontier_to_queue(sssp_graph *g, int32_t r)
 constexpr int32_t kNotLocal = -1;
 template <class WT>
 void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st,
-                int32_t local = kNotLocal, const BlkTile *tiles = nullptr);
+                int32_t local = kNotLocal, int32_t n_src = 1, const BlkTile *tiles = nullptr);
 
 template <class WT>
 bool run_round(sssp_graph *g, int mode, int kidx, int32_t r, int32_t tick0, const RoundSlot &cur,
@@ -2489,11 +2496,11 @@ constexpr int kPassAhead = 3;
 // With trace_events every pass is launched alone between events. Adds the
 // passes to the stats and the trace; full_limit: full passes at most (then
 // SSSP_ERR_NOT_CONVERGED). local: source of a run of local passes
-// (k_blk_local), or kNotLocal: k_blk_plain. tiles: the full tiles in another
-// order.
+// (k_blk_local; the first of n_src in src_list), or kNotLocal: k_blk_plain.
+// tiles: the full tiles in another order.
 template <class WT>
 void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int32_t local,
-                const BlkTile *tiles)
+                int32_t n_src, const BlkTile *tiles)
 {
     hipStream_t s = g->stream;
     PassArgs a{};
@@ -2530,6 +2537,10 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int3
         k_local_reset<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(
             la.seg, g->n_seg, la.state, g->n_ttile, local);
         SSSP_LAUNCH_CHECK("k_local_reset");
+        if (n_src > 1) {
+            k_local_sources<<<grid_for(n_src, 1 << 20), kBlock, 0, s>>>(la.seg, g->src_list, n_src);
+            SSSP_LAUNCH_CHECK("k_local_sources");
+        }
     }
     // the mirror still holds the last run's word (another tag) or none
     volatile unsigned long long *pos = &g->ctrl_host->ph_pos;
@@ -2604,21 +2615,21 @@ int64_t plain_limit(const sssp_graph *g)
 
 // The plain pass loop: full passes until one changes nothing (mixed: with
 // light passes between them, see k_blk_plain, or local passes where the graph
-// has their tiles: one source then).
+// has their tiles).
 template <class WT>
-void solve_plain(sssp_graph *g, bool mixed, int32_t source, sssp_stats *st)
+void solve_plain(sssp_graph *g, bool mixed, int32_t source, int32_t n_src, sssp_stats *st)
 {
     hipStream_t s = g->stream;
     const int64_t E = g->E;
     const int64_t limit = plain_limit(g);
     st->verify_passes = 1;  // the last pass changed nothing: the fixpoint check
     if (mixed && g->n_ttile > 0 && g->plain_kernel != 1) {
-        run_passes<WT>(g, kRunFull, limit, st, source);
+        run_passes<WT>(g, kRunFull, limit, st, source, n_src);
         return;
     }
     if (plain_uses_blocked(g)) {
         run_passes<WT>(g, mixed && WT::kWeighted && g->n_ltile > 0 ? kRunMixed : kRunFull, limit,
-                       st, kNotLocal, mixed ? nullptr : g->b_ptile);
+                       st, kNotLocal, 1, mixed ? nullptr : g->b_ptile);
         return;
     }
     const int64_t ng = E >> 2;
@@ -2952,13 +2963,18 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
     // Measured (learned, ms): R-MAT 21 x 16 (2^25 edges) 2.98 plain against
     // 3.66 in rounds, BFS 0.79 against 0.95; at 2^26 edges about even (R-MAT
     // 22 x 16 5.12 / 5.00, R-MAT 21 x 32 4.46 / 4.71); R-MAT 22 x 32 (2^27)
-    // 7.1 against 5.6 in rounds.
+    // 7.1 against 5.6 in rounds. Several sources (the larger graphs of a pack
+    // solved together) fill the rounds better: from half as many edges on.
+    // Rounds / passes, ms: 5 R-MAT 19 x 8 (21 M edges) 1.71 / 1.60, 100 R-MAT 16 x 8 (52 M)
+    // 1.63 / 2.34, 2 of them 1.0 / 0.43, 100 uniform 40 K x 5 2.49 / 1.37; 20 grids
+    // 200 x 200 24 / 7.6 with scattered ids, 23 / 0.98 in local passes with near
+    // ones (a round costs 25 us however few vertices it holds).
     const bool small = (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) &&
-                       n_src == 1 && g->E < g->plain_below_edges;
+                       g->E < g->plain_below_edges / (n_src > 1 && g->n_ttile == 0 ? 2 : 1);
     if (n_src > 1) upload_sources(g, sources, n_src);
     g->trace.clear();
     g->snap_round = -1;
-    if (small && solo_fits(g) && g->plain_kernel == 0 && !g->trace_events) {
+    if (small && n_src == 1 && solo_fits(g) && g->plain_kernel == 0 && !g->trace_events) {
         solve_solo<WT>(g, source, st);
         return;
     }
@@ -2974,7 +2990,7 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
         SSSP_LAUNCH_CHECK("k_init_sources");
     }
     if (sched == SSSP_SCHED_PLAIN || small) {
-        solve_plain<WT>(g, small, source, st);
+        solve_plain<WT>(g, small, source, n_src, st);
         g->tick = tick0 + 1;
     } else {
         if (g->pile_dirty) {

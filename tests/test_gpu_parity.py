@@ -1261,3 +1261,68 @@ def test_batch_policy_1_in_lds_u32(gpu, oracle, V):
         D, _ = g.solve_batch(sources, policy=1)
         for i, s in enumerate(sources):
             assert np.array_equal(D[i], oracle.dijkstra(src, dst, w, V, int(s))), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("near", [True, False], ids=["near", "scattered"])
+def test_pack_of_large_grids_runs_passes(gpu, oracle, near):
+    """The graphs of a pack that are too large for LDS are solved together in
+    passes, as one of them alone would be (local passes where ids are near), not
+    in rounds that cost a host check per hop: four grids and a small graph
+    between them take a few times one grid's time (rounds took 5 and 30 times).
+    Bit equality with the oracle."""
+    rng = np.random.default_rng(53)
+    r, c = 200, 200
+    v = np.arange(r * c, dtype=np.int32).reshape(r, c)
+    a = np.concatenate([v[:, :-1].ravel(), v[:-1].ravel()])
+    b = np.concatenate([v[:, 1:].ravel(), v[1:].ravel()])
+    gs = []
+    for k in range(4):
+        q = v.ravel() if near else rng.permutation(r * c).astype(np.int32)
+        s, d = q[np.concatenate([a, b])], q[np.concatenate([b, a])]
+        gs.append((s, d, rng.random(len(s), dtype=np.float32), r * c, int(q[k])))
+    s, d = (rng.integers(0, 900, 5000).astype(np.int32) for _ in range(2))
+    gs.insert(2, (s, d, rng.random(5000, dtype=np.float32), 900, int(s[0])))
+    refs = [oracle.dijkstra(s, d, w, n, x) for s, d, w, n, x in gs]
+    with S.DeviceGraph(*gs[0][:4]) as g:
+        one = min(g.solve(gs[0][4], "heuristic")[1]["t_solve_ms"] for _ in range(4))
+    offs = np.concatenate([[0], np.cumsum([len(x[0]) for x in gs])]).astype(np.int64)
+    vc = np.array([x[3] for x in gs], np.int32)
+    srcs = np.array([x[4] for x in gs], np.int32)
+    voff = np.concatenate([[0], np.cumsum(vc)])
+    p = S.GraphPack(*(np.concatenate([x[i] for x in gs]) for i in range(3)), offs, vc)
+    try:
+        for policy in (1, 2):
+            times = []
+            for rep in range(4):
+                print(f"pack of grids: near {near} policy {policy} {rep}", flush=True)
+                D, st = p.solve(srcs, policy=policy)
+                times.append(st["t_solve_ms"])
+                for k, ref in enumerate(refs):
+                    assert np.array_equal(bits(D[voff[k]:voff[k + 1]]), bits(ref)), (policy, k)
+            assert min(times) < 3 * one, (policy, times, one)
+    finally:
+        p.close()
+
+
+@pytest.mark.gpu
+def test_pack_merged_in_rounds(gpu, oracle):
+    """From 2^25 edges on the graphs of a pack that are too large for LDS share
+    the rounds of the engine: bit equality with the oracle."""
+    scales = np.full(65, 16, np.int32)
+    s, d, w, offs = S.rmat_many(scales, 8, seed0=3)
+    assert len(s) > 1 << 25
+    vc = (1 << scales).astype(np.int32)
+    srcs = np.minimum.reduceat(s, offs[:-1]).astype(np.int32)
+    voff = np.concatenate([[0], np.cumsum(vc)])
+    p = S.GraphPack(s, d, w, offs, vc)
+    try:
+        for policy in (1, 2):
+            print(f"merged pack in rounds: policy {policy}", flush=True)
+            D, _ = p.solve(srcs, policy=policy)
+            for k in range(0, 65, 4):
+                e0, e1 = offs[k], offs[k + 1]
+                ref = oracle.dijkstra(s[e0:e1], d[e0:e1], w[e0:e1], int(vc[k]), int(srcs[k]))
+                assert np.array_equal(bits(D[voff[k]:voff[k + 1]]), bits(ref)), (policy, k)
+    finally:
+        p.close()
