@@ -846,6 +846,7 @@ int sssp_get_param(const sssp_graph *g, const char *name, double *value)
         else if (n == "tail_blocks") *value = g->tail_blocks;
         else if (n == "push_bits_edges") *value = (double)g->push_bits_edges;
         else if (n == "multi_passes") *value = g->multi_passes;
+        else if (n == "multi_tiles") *value = g->n_mtile;
         else if (n == "rollout_policy") *value = g->rollout_policy;
         else if (n == "collect_kind") *value = g->collect_kind;
         else if (n == "collect_budget") *value = (double)g->collect_budget;

@@ -948,13 +948,17 @@ static void build_records(sssp_graph *g, const int32_t *src, const int32_t *dst,
     std::vector<int64_t> bp((size_t)nblk + 1);
     SSSP_HIP(hipMemcpyAsync(bp.data(), bptr, 8 * bp.size(), hipMemcpyDeviceToHost, s));
     SSSP_HIP(hipStreamSynchronize(s));
+    int64_t most = 0;
+    for (int32_t b = 0; b < nblk; b++) most = std::max(most, bp[(size_t)b + 1] - bp[(size_t)b]);
+    const int64_t cap =
+        nblk >= kMEvenBlocks && most * nblk <= 4 * n ? kMTileEven : kMTileEdges;
     std::vector<BlkTile> tiles;
     for (int32_t b = 0; b < nblk; b++) {
         const int64_t c = bp[(size_t)b + 1] - bp[(size_t)b];
-        const int64_t nt = (c + kMTileEdges - 1) / kMTileEdges;
+        const int64_t nt = (c + cap - 1) / cap;
         for (int64_t k = 0; k < nt; k++) {
-            const int64_t e0 = bp[(size_t)b] + k * kMTileEdges;
-            tiles.push_back(BlkTile{b, nt > 1 ? 1 : 0, e0, std::min(e0 + kMTileEdges, bp[(size_t)b + 1])});
+            const int64_t e0 = bp[(size_t)b] + k * cap;
+            tiles.push_back(BlkTile{b, nt > 1 ? 1 : 0, e0, std::min(e0 + cap, bp[(size_t)b + 1])});
         }
     }
     BlkTile *td = dmalloc<BlkTile>(std::max<size_t>(tiles.size(), 1));

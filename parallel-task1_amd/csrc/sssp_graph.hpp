@@ -154,11 +154,15 @@ struct BlkRanges {
 // relaxes a record in about 0.25 us; ms at 4096 / 1024 / 512 / 256 / 128 / 64 edges:
 // R-MAT 20 x 16 with 256 sources 59 / 54.9 / 17.9 / 16.7 / 17.3 / 20.7 -- the last four
 // without the pass counter's contention --, R-MAT 16 x 12 with 33 6.2 / 3.3 / 2.0 /
-// 1.4 / 1.2 / 0.94).
+// 1.4 / 1.2 / 0.94). Where no block is much larger than the mean a tile may hold
+// the whole block (kMTileEven): cut in two it is written back twice, with atomics (uniform,
+// 256 sources, 128 / 512 edges: 20 K x 10 2.24 / 1.71 ms, 100 K x 9 4.7 / 3.6, 400 K x 10 11.7 /
+// 10.3), unless the blocks alone do not fill the chip (4 K x 12 0.66 / 0.73).
 constexpr int kMBits = 4;
 constexpr int kMultiSlots = 4;  // captured chunk launches kept per graph
 constexpr int kMultiKey = 10;
-constexpr int64_t kMTileEdges = 128;
+constexpr int64_t kMTileEdges = 128, kMTileEven = 512;
+constexpr int32_t kMEvenBlocks = 1024;
 struct MRec {
     int32_t src;
     uint32_t w;

@@ -1326,3 +1326,34 @@ def test_pack_merged_in_rounds(gpu, oracle):
                 assert np.array_equal(bits(D[voff[k]:voff[k + 1]]), bits(ref)), (policy, k)
     finally:
         p.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,E,n,kind", [(16384, 400003, 257, "even"), (16368, 150001, 40, "below_u32"),
+                                        (16385, 600007, 65, "one_block"), (20000, 20000, 33, "even")])
+def test_batch_tiles_of_even_blocks(gpu, oracle, V, E, n, kind):
+    """Policy 3 on graphs without hubs, whose tiles hold whole destination blocks
+    from 1024 blocks on, and with one large block, whose tiles stay short: below, at
+    and past the line, part of a wave, a chunk and a part, u32, groups of records
+    that are and are not whole eights. Captured and queued; bit equality."""
+    rng = np.random.default_rng(E + n)
+    src, dst = (rng.integers(0, V, E).astype(np.int32) for _ in range(2))
+    if kind == "one_block":
+        dst[::3] = rng.integers(48, 64, len(dst[::3]))
+    w = rng.random(E, dtype=np.float32)
+    if kind.endswith("u32"):
+        w = rng.integers(1, 256, E).astype(np.uint32)
+    sources = src[rng.integers(0, E, n)].astype(np.int32)
+    refs = {i: oracle.dijkstra(src, dst, w, V, int(sources[i])) for i in (0, n // 2, n - 1)}
+    nblk = (V + 15) // 16
+    per = np.bincount(dst // 16, minlength=nblk)
+    cap = 512 if nblk >= 1024 and per.max() * nblk <= 4 * E else 128
+    assert (cap == 512) == (kind == "even")
+    with S.DeviceGraph(src, dst, w, V) as g:
+        for capture in (1, 0):
+            g.set_param("batch_capture", capture)
+            print(f"batch tiles: {kind} V {V} E {E} n {n} capture {capture}", flush=True)
+            D, _ = g.solve_batch(sources, policy=3)
+            assert g.get_param("multi_tiles") == ((per + cap - 1) // cap).sum()
+            for i, ref in refs.items():
+                assert np.array_equal(bits(D[i]), bits(ref)), (capture, i)
