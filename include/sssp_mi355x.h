@@ -188,8 +188,11 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * "batch_capture", "decide_spin", "blk_tile_cap", "blk_tile_order",
  * "blk_range_bits", "plain_kernel", "tail_edges", "tail_group", "tail_blocks",
  * "push_bits_edges", "trace_events"; "cu_count",
- * "collect_rounds", "multi_passes", "multi_tiles", "blk_tiles", "blk_wide_chunks"
- * and "plain_blocked" read-only).
+ * "collect_rounds", "multi_passes", "multi_tiles", "multi_light_tiles",
+ * "light_edges", "blk_tiles", "blk_wide_chunks" and "plain_blocked" read-only).
+ * "light_edges" = edges in the list of the light passes (0: the graph has none, or
+ * its solves run in one workgroup and none needed it yet), "multi_light_tiles" =
+ * tiles over the light records of policy-3 batches (0 before the first).
  * dense_all_frac (default 0.15, or 0.4 for a graph without hubs: no block of
  * 2^14 destinations with twice the mean in-edges) and dense_unreached
  * (default 0.5): an all-edge round whose frontier has at least

@@ -182,6 +182,7 @@ __global__ __launch_bounds__(BS) void k_wg_solve(const BatchTask *__restrict__ t
 // bitmaps), largest class first; class 0 is solved in global memory.
 constexpr int kLdsClasses = 4;
 constexpr int32_t kLdsVerts[kLdsClasses] = {0, 1 << 15, 1 << 14, 1 << 11};
+static_assert(kLdsVerts[1] == kSoloVerts, "one task may be a whole graph");
 
 inline int lds_class(int64_t nv)
 {
@@ -503,6 +504,7 @@ void launch_solo_t(sssp_graph *g, int32_t source, int32_t limit)
     auto reg = [&](auto kernel) {
         kernel<<<1, kSoloThreads, 0, g->stream>>>(a, g->el_src, g->el_dst, g->el_w, E, g->dist);
     };
+    static_assert(kRegEdges == 32 * kSoloThreads, "more edges need el_first");
     if (E <= 8 * kSoloThreads) reg(k_reg_solve<WT, 8>);
     else if (E <= 16 * kSoloThreads) reg(k_reg_solve<WT, 16>);
     else if (E <= 32 * kSoloThreads) reg(k_reg_solve<WT, 32>);
@@ -1351,7 +1353,7 @@ void check_pack_sources(const sssp_pack *p, const int32_t *sources)
 
 bool solo_fits(const sssp_graph *g)
 {
-    return g->V <= kLdsVerts[1] && g->E <= (g->n_ttile > 0 ? kSoloLocalEdges : kSoloEdges);
+    return g->V <= kSoloVerts && g->E <= (g->n_ttile > 0 ? kSoloLocalEdges : kSoloEdges);
 }
 
 void ensure_chunk_sources(sssp_graph *g)

@@ -324,6 +324,25 @@ sssp_graph *graph_begin(int32_t weight_type, int32_t vertices, int64_t edges, in
 
 // Builds the layouts from edge arrays already in device memory and allocates
 // the solve state.
+int64_t resident_bytes(const sssp_graph *g)
+{
+    // resident arrays: the three edge orders and the CSC, row offsets, the
+    // per-vertex arrays (dist, stamp, piles, pile state, snapshot, parent,
+    // queues, load-balancing entries, static entry lists)
+    const int64_t Ei = g->E, Vi = g->V;
+    const int64_t xe = g->xgoff_host.empty() ? 0 : g->xgoff_host.back();
+    return Ei * 12 + xe * 12 + (g->b_edges + g->l_edges) * 8 +
+           (g->b_edges + g->l_edges) / kBlkChunk * 4 +
+           (g->b_nwide + g->l_nwide) * kBlkChunk * 4 +
+           (int64_t)(g->n_btile * (g->b_ptile ? 2 : 1) + g->n_ltile) *
+               (int64_t)sizeof(BlkTile) +
+           (int64_t)g->n_btile * kBlkThreads * 2 +
+           (int64_t)g->n_ttile * (int64_t)(sizeof(BlkTile) + sizeof(TileState)) +
+           (int64_t)g->n_seg * 4 +
+           (Vi + 1) * 8 + (g->has_csc ? Ei * 8 + (Vi + 1) * 8 : 0) + Vi * 4 * 7 +
+           (Vi + 1) * 4 * 3 + (Vi + 1) * 8 * 2 + Vi * 24 + (g->relabel ? Vi * 12 : 0);
+}
+
 void graph_finish(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, const uint32_t *d_w,
                   uint32_t flags)
 {
@@ -374,21 +393,6 @@ void graph_finish(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, con
     SSSP_HIP(hipEventCreate(&g->ev_r0));
     SSSP_HIP(hipEventCreate(&g->ev_r1));
     SSSP_HIP(hipStreamSynchronize(s));
-    // resident arrays: the three edge orders and the CSC, row offsets, the
-    // per-vertex arrays (dist, stamp, piles, pile state, snapshot, parent,
-    // queues, load-balancing entries, static entry lists)
-    const int64_t Ei = g->E, Vi = g->V;
-    const int64_t xe = g->xgoff_host.empty() ? 0 : g->xgoff_host.back();
-    g->device_bytes = Ei * 12 + xe * 12 + (g->b_edges + g->l_edges) * 8 +
-                      (g->b_edges + g->l_edges) / kBlkChunk * 4 +
-                      (g->b_nwide + g->l_nwide) * kBlkChunk * 4 +
-                      (int64_t)(g->n_btile * (g->b_ptile ? 2 : 1) + g->n_ltile) *
-                          (int64_t)sizeof(BlkTile) +
-                      (int64_t)std::max(g->n_btile, g->n_ltile) * kBlkThreads * 2 +
-                      (int64_t)g->n_ttile * (int64_t)(sizeof(BlkTile) + sizeof(TileState)) +
-                      (int64_t)g->n_seg * 4 +
-                      (Vi + 1) * 8 + (g->has_csc ? Ei * 8 + (Vi + 1) * 8 : 0) + Vi * 4 * 7 +
-                      (Vi + 1) * 4 * 3 + (Vi + 1) * 8 * 2 + Vi * 24 + (g->relabel ? Vi * 12 : 0);
 }
 
 struct DevBuf {
@@ -575,7 +579,7 @@ int sssp_graph_info(const sssp_graph *g, int32_t *vertices, int64_t *edges, int3
         if (vertices) *vertices = g->V;
         if (edges) *edges = g->E;
         if (weight_type) *weight_type = g->wtype;
-        if (device_bytes) *device_bytes = g->device_bytes;
+        if (device_bytes) *device_bytes = resident_bytes(g);
     });
 }
 
@@ -847,6 +851,8 @@ int sssp_get_param(const sssp_graph *g, const char *name, double *value)
         else if (n == "push_bits_edges") *value = (double)g->push_bits_edges;
         else if (n == "multi_passes") *value = g->multi_passes;
         else if (n == "multi_tiles") *value = g->n_mtile;
+        else if (n == "multi_light_tiles") *value = g->n_mltile;
+        else if (n == "light_edges") *value = (double)g->light_edges;
         else if (n == "rollout_policy") *value = g->rollout_policy;
         else if (n == "collect_kind") *value = g->collect_kind;
         else if (n == "collect_budget") *value = (double)g->collect_budget;

@@ -2978,6 +2978,7 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
         solve_solo<WT>(g, source, st);
         return;
     }
+    if (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) ensure_pass_lists(g);
     SSSP_HIP(hipEventRecord(g->ev_a, s));
     k_fill<uint32_t><<<grid_for(g->V), kBlock, 0, s>>>(g->dist, g->V, WT::INF);
     SSSP_LAUNCH_CHECK("k_fill dist");
@@ -3099,6 +3100,7 @@ void collect_t(sssp_graph *g, int32_t source, int32_t cap, float *feats, float *
         k_fill<int32_t><<<grid_for(g->V), kBlock, 0, s>>>(g->farst, g->V, 0);
         SSSP_LAUNCH_CHECK("pile state reset");
     }
+    ensure_pass_lists(g);
     const int32_t tick0 = g->tick;
     const size_t V = (size_t)g->V;
     struct Saved {

@@ -968,68 +968,6 @@ static void build_records(sssp_graph *g, const int32_t *src, const int32_t *dst,
     *n_tile = (int32_t)tiles.size();
 }
 
-void build_multi_layout(sssp_graph *g)
-{
-    if (g->m_rec || g->E == 0) return;
-    hipStream_t s = g->stream;
-    struct Made {
-        void *p[4] = {};
-        ~Made()
-        {
-            for (void *x : p) dfree(x);
-        }
-    } made;
-    MRec *rec = nullptr, *lrec = nullptr;
-    BlkTile *tile = nullptr, *ltile = nullptr;
-    int32_t nt = 0, nlt = 0;
-    auto hold = [&] { made.p[0] = rec, made.p[1] = lrec, made.p[2] = tile, made.p[3] = ltile; };
-    try {
-        build_records(g, g->el_src, g->el_dst, g->el_w, g->E, &rec, &tile, &nt);
-        if (g->light_thr != 0xFFFFFFFFu) {
-            // the light edges of the src-sorted list, in order
-            const int64_t E = g->E, nch = (E + kBlkChunk - 1) / kBlkChunk;
-            int64_t *pos = dmalloc<int64_t>((size_t)nch + 1);
-            struct F {
-                void *p[4] = {};
-                ~F()
-                {
-                    for (void *x : p) dfree(x);
-                }
-            } f;
-            f.p[0] = pos;
-            const unsigned grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
-            k_light_count<<<grid, kBlock, 0, s>>>(g->el_w, E, nch, g->light_thr, pos);
-            SSSP_LAUNCH_CHECK("k_light_count");
-            k_fill_i64<<<1, 64, 0, s>>>(pos + nch, 1, 0);
-            device_exclusive_scan_i64(pos, pos, nch + 1, g->blk_a, g->blk_b, g->n_blk, s);
-            int64_t nl = 0;
-            SSSP_HIP(hipMemcpyAsync(&nl, pos + nch, 8, hipMemcpyDeviceToHost, s));
-            SSSP_HIP(hipStreamSynchronize(s));
-            if (nl > 0) {
-                int32_t *ls = dmalloc<int32_t>((size_t)nl);
-                f.p[1] = ls;
-                int32_t *ld = dmalloc<int32_t>((size_t)nl);
-                f.p[2] = ld;
-                uint32_t *lw = dmalloc<uint32_t>((size_t)nl);
-                f.p[3] = lw;
-                k_light_select<<<grid, kBlock, 0, s>>>(g->el_src, g->el_dst, g->el_w, E, nch,
-                                                       g->light_thr, pos, ls, ld, lw);
-                SSSP_LAUNCH_CHECK("k_light_select");
-                build_records(g, ls, ld, lw, nl, &lrec, &ltile, &nlt);
-            }
-        }
-    } catch (...) {
-        hold();
-        throw;
-    }
-    g->m_rec = rec;
-    g->m_tile = tile;
-    g->n_mtile = nt;
-    g->m_lrec = lrec;
-    g->m_ltile = ltile;
-    g->n_mltile = nlt;
-}
-
 // Edge-list check on the device: every id in [0, V) and (wtype >= 0) every
 // weight >= 0 and not NaN (unsigned weights always are); throws SSSP_ERR_ARG.
 // The relaxations rely on it: distances are compared as unsigned bit patterns,
@@ -1201,10 +1139,9 @@ void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits)
     } own;
     BlkTile *td = upload(tiles);
     own.p[0] = td;
-    BlkTile *ltd = upload(ltiles);
+    BlkTile *ltd = ltiles.empty() ? nullptr : upload(ltiles);
     own.p[1] = ltd;
-    const size_t n_mask = std::max<size_t>(std::max(tiles.size(), ltiles.size()), 1);
-    uint16_t *ad = dmalloc<uint16_t>(n_mask * kBlkThreads);
+    uint16_t *ad = dmalloc<uint16_t>(std::max<size_t>(tiles.size(), 1) * kBlkThreads);
     own.p[2] = ad;
     BlkTile *ptd = ptiles.empty() ? nullptr : upload(ptiles);
     own.p[3] = ptd;
@@ -1228,13 +1165,13 @@ void retile_blocked(sssp_graph *g, int64_t cap, int order, int range_bits)
 // The tiles of the local passes (k_blk_local), on graphs they are for.
 static void build_local_tiles(sssp_graph *g)
 {
-    if (!g->local_graph) return;
+    if (!g->local_graph || g->n_ttile > 0) return;
     const std::vector<BlkTile> tiles =
         make_blk_tiles(g->b_off_host, kLocalTileMax, 0, BlkRanges{}, {});
     const size_t n_seg = (g->b_off_host.size() - 1) << (kBlkBits - kSegBits);
-    g->t_tile = dmalloc<BlkTile>(tiles.size());
-    g->t_state = dmalloc<TileState>(tiles.size());
-    g->t_seg = dmalloc<int32_t>(n_seg);
+    if (!g->t_tile) g->t_tile = dmalloc<BlkTile>(tiles.size());
+    if (!g->t_state) g->t_state = dmalloc<TileState>(tiles.size());
+    if (!g->t_seg) g->t_seg = dmalloc<int32_t>(n_seg);
     SSSP_HIP(hipMemcpyAsync(g->t_tile, tiles.data(), sizeof(BlkTile) * tiles.size(),
                             hipMemcpyHostToDevice, g->stream));
     tile_spans(g, g->t_tile, (int32_t)tiles.size(), g->t_state);
@@ -1258,6 +1195,7 @@ static void build_local_tiles(sssp_graph *g)
 // edge is light and light passes do not run).
 static uint32_t light_threshold(sssp_graph *g, Carve &tmp)
 {
+    if (g->E == 0) return 0xFFFFFFFFu;
     const int64_t n = std::min<int64_t>(g->E, kLightSample);
     uint32_t *d = tmp.get<uint32_t>((size_t)n + 2);
     SSSP_HIP(hipMemsetAsync(d + n, 0, 8, g->stream));
@@ -1272,6 +1210,7 @@ static uint32_t light_threshold(sssp_graph *g, Carve &tmp)
     SSSP_HIP(hipStreamSynchronize(g->stream));
     const double mean = (double)g->E / std::max(g->n_nzo, 1);
     const bool hubs = (double)s[(size_t)n] >= 16.0 * mean;
+    g->out_hubs = hubs;
     if (!hubs && mean < kLightMinDegree) {
         // local passes: half the sampled edges join near ids (on random graphs
         // of 2000-7000 vertices, whose edges all lie in one block, they took
@@ -1293,6 +1232,13 @@ static uint32_t light_threshold(sssp_graph *g, Carve &tmp)
     const double got = use_lo ? (double)lo : (double)up;
     if (got < 0.5 * target || got > 3.0 * target || got > 0.75 * (double)n) return 0xFFFFFFFFu;
     return use_lo ? at - 1 : at;
+}
+
+static void sample_weights(sssp_graph *g, Carve &tmp)
+{
+    if (g->weights_known) return;
+    g->light_thr = light_threshold(g, tmp);
+    g->weights_known = true;
 }
 
 // Packs nch chunks of whole sources and destination offsets (k_blk_pack).
@@ -1343,9 +1289,8 @@ static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *b
                              const int64_t *boff, int32_t nblk, int64_t nch, Carve &tmp)
 {
     hipStream_t s = g->stream;
-    const uint32_t thr = light_threshold(g, tmp);
-    // none on graphs whose solves run in one workgroup (0.15 ms of the build)
-    if (thr == 0xFFFFFFFFu || (solo_fits(g) && g->E < kSoloEdges)) return;
+    const uint32_t thr = g->light_thr;
+    if (thr == 0xFFFFFFFFu) return;
     int64_t *pos = tmp.get<int64_t>((size_t)nch + 1);
     int64_t *lptr = tmp.get<int64_t>(2 * ((size_t)nblk + 1));
     int64_t *loff = lptr + nblk + 1;
@@ -1379,7 +1324,150 @@ static void build_light_list(sssp_graph *g, const int32_t *bs, const uint16_t *b
     g->l_off_host = lo;
     g->l_edges = Lp;
     g->light_edges = lp[(size_t)nblk];
-    g->light_thr = thr;
+}
+
+// f(), which builds what solves can do without: false, with nothing of it
+// kept, when there is no memory for it.
+template <class F, class Undo>
+static bool without_memory_skip(F &&f, Undo &&undo)
+{
+    try {
+        f();
+        return true;
+    } catch (const Error &e) {
+        undo();
+        if (e.code != SSSP_ERR_OOM) throw;
+        (void)hipGetLastError();
+        return false;
+    }
+}
+
+static bool light_list_if_room(sssp_graph *g, const int32_t *bs, const uint16_t *bd,
+                               const int64_t *boff, int32_t nblk, int64_t nch, Carve &tmp)
+{
+    return without_memory_skip([&] { build_light_list(g, bs, bd, boff, nblk, nch, tmp); },
+                               [&] {
+                                   (void)hipStreamSynchronize(g->stream);
+                                   for (void *p : {(void *)g->l_w, (void *)g->l_pk,
+                                                   (void *)g->l_cbase, (void *)g->l_wide})
+                                       dfree(p);
+                                   g->l_w = g->l_pk = nullptr;
+                                   g->l_cbase = g->l_wide = nullptr;
+                                   g->l_edges = g->l_nwide = g->light_edges = 0;
+                                   g->b_ranges.loff.clear();
+                               });
+}
+
+// The blocked list's edges again as whole sources and destination offsets
+// (one wave per chunk).
+__global__ __launch_bounds__(kBlock) void k_blk_unpack(const uint32_t *pk, const int32_t *cbase,
+                                                       const int32_t *wide, int64_t nch,
+                                                       int32_t *bs, uint16_t *bd)
+{
+    const int64_t c = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+    if (c >= nch) return;  // wave-uniform
+    const int64_t e = c * kBlkChunk + 4 * __lane_id();
+    const int32_t cb = cbase[c];
+    uint32_t p[4];
+    int32_t sum = 0;
+    for (int k = 0; k < 4; k++) {
+        p[k] = pk[e + k];
+        sum += (int32_t)(p[k] >> kBlkBits);
+    }
+    int32_t at = cb + wave_scan32(sum) - sum;
+    for (int k = 0; k < 4; k++) {
+        at += (int32_t)(p[k] >> kBlkBits);
+        bs[e + k] = cb >= 0 ? at : wide[(int64_t)(-1 - cb) * kBlkChunk + 4 * __lane_id() + k];
+        bd[e + k] = (uint16_t)(p[k] & ((1u << kBlkBits) - 1));
+    }
+}
+
+void ensure_pass_lists(sssp_graph *g)
+{
+    if (g->pass_lists || g->E == 0) return;
+    hipStream_t s = g->stream;
+    const size_t Ep = (size_t)g->b_edges, nblk = g->b_off_host.size() - 1;
+    const bool built = without_memory_skip(
+        [&] {
+            Carve tmp(nullptr, 0);
+            sample_weights(g, tmp);
+            build_local_tiles(g);
+            if (g->light_thr == 0xFFFFFFFFu) return;
+            int32_t *bs = tmp.get<int32_t>(Ep);
+            uint16_t *bd = tmp.get<uint16_t>(Ep);
+            int64_t *boff = tmp.get<int64_t>(nblk + 1);
+            SSSP_HIP(hipMemcpyAsync(boff, g->b_off_host.data(), 8 * (nblk + 1),
+                                    hipMemcpyHostToDevice, s));
+            const int64_t nch = (int64_t)Ep / kBlkChunk;
+            k_blk_unpack<<<(unsigned)((nch * 64 + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+                g->b_pk, g->b_cbase, g->b_wide, nch, bs, bd);
+            SSSP_LAUNCH_CHECK("k_blk_unpack");
+            if (light_list_if_room(g, bs, bd, boff, (int32_t)nblk, nch, tmp) && g->light_edges > 0)
+                retile_blocked(g, g->blk_tile_cap, g->blk_order_set ? g->blk_tile_order : -1,
+                               g->blk_range_bits);
+            SSSP_HIP(hipStreamSynchronize(s));
+        },
+        [&] { (void)hipStreamSynchronize(s); });
+    g->pass_lists = built;
+}
+
+// The light edges of the src-sorted list as records of their own, where they
+// pay (kMLightEdges).
+static void build_light_records(sssp_graph *g, MRec **rec, BlkTile **tile, int32_t *n_tile)
+{
+    hipStream_t s = g->stream;
+    Carve tmp(nullptr, 0);
+    sample_weights(g, tmp);
+    if (g->light_thr == 0xFFFFFFFFu ||
+        g->E < (g->out_hubs ? kMLightEdges : kMLightEvenEdges) || g->E < kMLightMean * g->n_nzo)
+        return;
+    const int64_t E = g->E, nch = (E + kBlkChunk - 1) / kBlkChunk;
+    int64_t *pos = tmp.get<int64_t>((size_t)nch + 1);
+    const unsigned grid = (unsigned)((nch * 64 + kBlock - 1) / kBlock);
+    k_light_count<<<grid, kBlock, 0, s>>>(g->el_w, E, nch, g->light_thr, pos);
+    SSSP_LAUNCH_CHECK("k_light_count");
+    k_fill_i64<<<1, 64, 0, s>>>(pos + nch, 1, 0);
+    device_exclusive_scan_i64(pos, pos, nch + 1, g->blk_a, g->blk_b, g->n_blk, s);
+    int64_t nl = 0;
+    SSSP_HIP(hipMemcpyAsync(&nl, pos + nch, 8, hipMemcpyDeviceToHost, s));
+    SSSP_HIP(hipStreamSynchronize(s));
+    if (nl == 0) return;
+    int32_t *ls = tmp.get<int32_t>((size_t)nl), *ld = tmp.get<int32_t>((size_t)nl);
+    uint32_t *lw = tmp.get<uint32_t>((size_t)nl);
+    k_light_select<<<grid, kBlock, 0, s>>>(g->el_src, g->el_dst, g->el_w, E, nch, g->light_thr, pos,
+                                           ls, ld, lw);
+    SSSP_LAUNCH_CHECK("k_light_select");
+    build_records(g, ls, ld, lw, nl, rec, tile, n_tile);
+}
+
+void build_multi_layout(sssp_graph *g)
+{
+    if (g->m_rec || g->E == 0) return;
+    MRec *rec[2] = {};
+    BlkTile *tile[2] = {};
+    int32_t n[2] = {};
+    auto drop = [&](int i) {
+        (void)hipStreamSynchronize(g->stream);
+        dfree(rec[i]);
+        dfree(tile[i]);
+        rec[i] = nullptr;
+        tile[i] = nullptr;
+        n[i] = 0;
+    };
+    try {
+        build_records(g, g->el_src, g->el_dst, g->el_w, g->E, &rec[0], &tile[0], &n[0]);
+        (void)without_memory_skip([&] { build_light_records(g, &rec[1], &tile[1], &n[1]); },
+                                  [&] { drop(1); });
+    } catch (...) {
+        drop(0);
+        throw;
+    }
+    g->m_rec = rec[0];
+    g->m_tile = tile[0];
+    g->n_mtile = n[0];
+    g->m_lrec = rec[1];
+    g->m_ltile = tile[1];
+    g->n_mltile = n[1];
 }
 
 void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, const uint32_t *d_w,
@@ -1621,7 +1709,15 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
             g->b_ranges.fine_bits = kBlkRangeFineBits;
             g->b_ranges.n_fine = (int32_t)nfine;
         }
-        build_light_list(g, bs, bd, boff, nblk, nch, tmp);
+        // The light list, unless solves of the graph run in one workgroup
+        // (ensure_pass_lists builds it for those that do not; the sample of the
+        // weights and the list are 0.1 and 0.15 ms of a build of 0.7 ms).
+        if (V > kSoloVerts || E > std::min(kSoloLocalEdges, kRegEdges)) sample_weights(g, tmp);
+        const bool solo = V <= kSoloVerts && E <= (g->local_graph ? kSoloLocalEdges : kSoloEdges);
+        if (!solo) {
+            (void)light_list_if_room(g, bs, bd, boff, nblk, nch, tmp);
+            g->pass_lists = true;
+        }
         SSSP_HIP(hipStreamSynchronize(s));
         // Without hubs the d[src] gathers of a tile spread over the whole
         // distance array (degree order cannot gather them), so a graph whose
@@ -1639,9 +1735,10 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
             range_bits = std::max(kBlkRangeFineBits, lg - 3);
         }
         retile_blocked(g, tcap, -1, range_bits);
-        build_local_tiles(g);
+        if (g->pass_lists)
+            (void)without_memory_skip([&] { build_local_tiles(g); }, [] {});
     }
-    if (solo_fits(g)) ensure_chunk_sources(g);
+    if (solo_fits(g) && E > kRegEdges) ensure_chunk_sources(g);
 
     // ---- CSC ----
     if (build_csc) {

@@ -163,6 +163,16 @@ constexpr int kMultiSlots = 4;  // captured chunk launches kept per graph
 constexpr int kMultiKey = 10;
 constexpr int64_t kMTileEdges = 128, kMTileEven = 512;
 constexpr int32_t kMEvenBlocks = 1024;
+// Light records pay from these counts and means of edges per vertex with
+// out-edges on: below, a pass takes its launch and one tile's chain whatever
+// it reads, and light passes are more of them. With / without, ms, 33 and 256
+// sources: with hubs R-MAT 12 x 16 0.49 / 0.37 and 0.78 / 0.57, 14 x 16 0.74 / 0.73 and 1.76 /
+// 1.74, 16 x 12 1.30 / 1.35 and 2.54 / 2.72, 17 x 16 1.62 / 2.52 and 3.50 / 4.06, 18 x 16 2.8 / 5.0 and
+// 6.4 / 7.5, power-law 60 K x 8 2.9 / 1.3 and 8.5 / 3.5, 200 K x 6 3.0 / 2.0 and 7.4 / 3.4; without
+// hubs (tiles of kMTileEven) uniform 50 K x 16 1.71 / 1.75 and 4.9 / 3.9, 400 K x 10 6.2 / 5.5
+// and 12.3 / 10.3, 200 K x 16 3.8 / 4.4 and 7.0 / 7.6.
+constexpr int64_t kMLightEdges = (int64_t)1 << 19, kMLightEvenEdges = (int64_t)1 << 21;
+constexpr int64_t kMLightMean = 12;
 struct MRec {
     int32_t src;
     uint32_t w;
@@ -238,7 +248,12 @@ struct sssp_graph {
     int32_t n_ttile = 0, n_seg = 0;
     bool local_graph = false;  // sparse, no hubs, most edges between near ids
     int64_t light_edges = 0;      // edges in the light list
-    uint32_t light_thr = 0xFFFFFFFFu;  // its largest weight pattern (0xFFFFFFFF: no light list)
+    // largest weight pattern of the light class (0xFFFFFFFF: none), once the
+    // edges were sampled (weights_known); pass_lists: the light list or the
+    // local tiles, where the graph has them, are built
+    uint32_t light_thr = 0xFFFFFFFFu;
+    bool weights_known = false, pass_lists = false;
+    bool out_hubs = false;  // a vertex with 16 times the mean of the out-edges (sampled too)
     std::vector<int64_t> b_off_host;  // padded block offsets (tiles are rebuilt from them)
     std::vector<int64_t> l_off_host;  // ... of the light list
     int64_t blk_tile_cap = 0;         // edges per tile at most
@@ -384,8 +399,6 @@ struct sssp_graph {
     hipEvent_t stage_ev[sssp::kStageBufs] = {};
     uint8_t *dvis = nullptr;  // visited flags of a BFS (on demand)
 
-    int64_t device_bytes = 0;
-
     // multi-source solves: device copy of the source list
     int32_t *src_list = nullptr;
     int32_t src_cap = 0;
@@ -485,6 +498,8 @@ class Prefault {
 // (39600 edges) 331 / 527.
 constexpr int64_t kSoloEdges = (int64_t)1 << 17;
 constexpr int64_t kSoloLocalEdges = (int64_t)1 << 15;
+constexpr int32_t kSoloVerts = 1 << 15;
+constexpr int64_t kRegEdges = (int64_t)1 << 15;  // edges a workgroup holds in registers
 bool solo_fits(const sssp_graph *g);
 void ensure_chunk_sources(sssp_graph *g);
 void launch_solo(sssp_graph *g, int32_t source, bool hops, int32_t limit);
@@ -515,6 +530,11 @@ void split_records(const uint32_t *rec, int64_t n, int32_t *src, int32_t *dst, u
                    hipStream_t s);
 void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, const uint32_t *d_w,
                    bool build_csc);
+// The light list and the tiles of the local passes, where the graph has them.
+// Built with the graph, or, on graphs whose solves run in one workgroup, by
+// the first solve that does not (traced, another plain kernel, in rounds,
+// many sources at once). Without memory for the light list there is none.
+void ensure_pass_lists(sssp_graph *g);
 // the multi-source records and tiles (m_rec, m_tile), built once per graph
 void build_multi_layout(sssp_graph *g);
 // rebuilds the destination-blocked list's tile table (cap: edge slots per

@@ -5,6 +5,8 @@ is unique for w >= 0, so every schedule must land on the same bits as the
 oracle's restatement of cpu_bellman_ford, sssp.hpp:3-71), plus the
 shortest-path certificate (all edges satisfied, tight parent tree).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -1355,5 +1357,115 @@ def test_batch_tiles_of_even_blocks(gpu, oracle, V, E, n, kind):
             print(f"batch tiles: {kind} V {V} E {E} n {n} capture {capture}", flush=True)
             D, _ = g.solve_batch(sources, policy=3)
             assert g.get_param("multi_tiles") == ((per + cap - 1) // cap).sum()
+            for i, ref in refs.items():
+                assert np.array_equal(bits(D[i]), bits(ref)), (capture, i)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,E,kind", [(4099, 45089, "f32"), (4099, 45089, "u32"),
+                                      (1 << 14, 1 << 17, "f32"), (900, 30000, "f32"),
+                                      (20011, 220121, "f32"), (4099, 45089, "equal")])
+def test_light_list_of_graphs_solved_in_one_workgroup(gpu, oracle, V, E, kind):
+    """Graphs whose single solves run in one workgroup are built without the
+    light list; a solve that does run passes (traced, in rounds) builds it then,
+    and the light passes are in its trace. Without memory for it the solve runs
+    without. A larger graph has it from the start. Bit equality with the oracle."""
+    rng = np.random.default_rng(E)
+    src = (rng.random(E) ** 2 * V).astype(np.int32)
+    dst = rng.integers(0, V, E).astype(np.int32)
+    w = rng.random(E, dtype=np.float32)
+    if kind == "u32":
+        w = rng.integers(1, 256, E).astype(np.uint32)
+    elif kind == "equal":
+        w[:] = 0.5
+    solo = V <= 1 << 15 and E <= 1 << 17
+    source = int(src[0])
+
+    def resident(graph):
+        b = C.c_int64(0)
+        assert S.lib().sssp_graph_info(graph.handle, None, None, None, C.byref(b)) == S.OK
+        return b.value
+
+    ref = oracle.dijkstra(src, dst, w, V, source)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        light = g.get_param("light_edges")
+        assert (light > 0) == (not solo)
+        d, _ = g.solve(source, "heuristic")
+        assert np.array_equal(bits(d), bits(ref)) and g.get_param("light_edges") == light
+        g.set_param("trace_events", 1)
+        g.set_param("plain_kernel", 2)
+        if solo and kind != "equal":
+            print(f"light list on demand: {kind} V {V} E {E}, no memory", flush=True)
+            S.lib().sssp_debug_fail_next_alloc()  # of the light list's build
+            d, _ = g.solve(source, "heuristic")
+            assert np.array_equal(bits(d), bits(ref))
+            assert not (g.trace()["mode"] == S.MODE_LIGHT).any()
+        size = resident(g)
+        for below in (2 ** 26, 0):  # pass loop, rounds
+            print(f"light list on demand: {kind} V {V} E {E}, below {below}", flush=True)
+            g.set_param("plain_below_edges", below)
+            g.set_param("dense_unreached", 0.0)
+            d, _ = g.solve(source, "heuristic")
+            assert np.array_equal(bits(d), bits(ref)), below
+            assert (g.trace()["mode"] == S.MODE_LIGHT).any() == (kind != "equal"), below
+        assert (g.get_param("light_edges") > 0) == (kind != "equal")
+        assert (resident(g) > size) == (solo and kind != "equal")
+
+
+@pytest.mark.gpu
+def test_local_tiles_of_graphs_solved_in_one_workgroup(gpu, oracle):
+    """The same for the tiles of the local passes: built by the first solve of
+    a small grid that runs passes, which are then the local ones."""
+    rng = np.random.default_rng(59)
+    v = np.arange(3000, dtype=np.int32).reshape(60, 50)
+    a = np.concatenate([v[:, :-1].ravel(), v[:-1].ravel()])
+    b = np.concatenate([v[:, 1:].ravel(), v[1:].ravel()])
+    src, dst = np.concatenate([a, b]), np.concatenate([b, a])
+    w = rng.random(len(src), dtype=np.float32)
+    ref = oracle.dijkstra(src, dst, w, 3000, 0)
+    with S.DeviceGraph(src, dst, w, 3000) as g:
+        for rep in range(2):  # in one workgroup, before and after
+            d, st = g.solve(0, "heuristic")
+            assert np.array_equal(bits(d), bits(ref))
+            g.set_param("trace_events", 1)
+            for fail in (1, 0) if rep == 0 else (0,):
+                print(f"local tiles on demand: {rep} no memory {fail}", flush=True)
+                if fail:
+                    S.lib().sssp_debug_fail_next_alloc()
+                d, st = g.solve(0, "heuristic")
+                assert np.array_equal(bits(d), bits(ref))
+                plain = g.solve(0, "plain")[1]
+                assert (st["iterations"] * 2 < plain["iterations"]) == (fail == 0)
+            g.set_param("trace_events", 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,E,n,kind,light", [
+    (4099, 60000, 65, "hubs", False), (30011, (1 << 19) - 1, 33, "hubs", False),
+    (30011, 1 << 19, 65, "hubs", True), (30011, 1 << 19, 300, "hubs_u32", True),
+    (30011, 1 << 19, 64, "equal", False), (60000, 1 << 19, 33, "hubs", False),
+    (100003, (1 << 21) - 1, 33, "even", False), (100003, 1 << 21, 40, "even_u32", True),
+    (190000, 1 << 21, 33, "even", False), (16384, 400003, 257, "even", False)])
+def test_batch_light_records_where_they_pay(gpu, oracle, V, E, n, kind, light):
+    """Policy 3 has light records from the edge counts and mean degrees on where
+    they pay, on graphs with hubs and without, and none with equal weights: part of a
+    wave, a chunk and a part, u32, tiles that hold whole blocks, captured and
+    queued. Bit equality with the oracle."""
+    rng = np.random.default_rng(E + n)
+    src = (rng.random(E) ** (1 if kind.startswith("even") else 2) * V).astype(np.int32)
+    dst = rng.integers(0, V, E).astype(np.int32)
+    w = rng.random(E, dtype=np.float32)
+    if kind.endswith("u32"):
+        w = rng.integers(1, 256, E).astype(np.uint32)
+    elif kind == "equal":
+        w[:] = 0.5
+    sources = rng.integers(0, V, n).astype(np.int32)
+    refs = {i: oracle.dijkstra(src, dst, w, V, int(sources[i])) for i in (0, n // 2, n - 1)}
+    with S.DeviceGraph(src, dst, w, V) as g:
+        for capture in (1, 0):
+            g.set_param("batch_capture", capture)
+            print(f"light records: {kind} V {V} E {E} n {n} capture {capture}", flush=True)
+            D, _ = g.solve_batch(sources, policy=3)
+            assert (g.get_param("multi_light_tiles") > 0) == light
             for i, ref in refs.items():
                 assert np.array_equal(bits(D[i]), bits(ref)), (capture, i)
