@@ -33,7 +33,9 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <numeric>
+#include <optional>
 #include <string>
 
 #include "sssp_graph.hpp"
@@ -660,14 +662,20 @@ TaskCounts upload_tasks(sssp_graph *g, const std::vector<BatchTask> &tasks,
     return tc;
 }
 
+void prepare_multi(sssp_graph *g, int32_t n);
 double run_multi(sssp_graph *g, const int32_t *sources, int32_t n);
 
 // ---- many sources on one graph ----------------------------------------------
-double batch_sources(sssp_graph *g, const int32_t *sources, int32_t n, const Config &c)
+// ready: called when every allocation is made, before the solves.
+using Ready = std::function<void()>;
+double batch_sources(sssp_graph *g, const int32_t *sources, int32_t n, const Config &c,
+                     const Ready &ready = {})
 {
     const int64_t V = g->V;
     if (c.policy == 3) {
         ensure_batch_buffers(g, (int64_t)n * V, 0, 0, 0);
+        prepare_multi(g, n);
+        if (ready) ready();
         return run_multi(g, sources, n);
     }
     if (c.policy == 1) {
@@ -675,6 +683,8 @@ double batch_sources(sssp_graph *g, const int32_t *sources, int32_t n, const Con
         const int32_t nwg =
             lds_class(V) == 0 ? std::min<int32_t>(n, g->cu_count * c.wgpcu) : 0;
         ensure_batch_buffers(g, (int64_t)n * V, n, nwg, V);
+        ensure_chunk_sources(g);
+        if (ready) ready();
         std::vector<BatchTask> tasks((size_t)n);
         std::vector<int64_t> work((size_t)n, 1);
         for (int32_t i = 0; i < n; i++) tasks[(size_t)i] = BatchTask{0, (int64_t)i * V, (int32_t)V, sources[i]};
@@ -699,6 +709,7 @@ double batch_sources(sssp_graph *g, const int32_t *sources, int32_t n, const Con
         return ms;
     }
     ensure_batch_buffers(g, (int64_t)n * V, 0, 0, 0);
+    if (ready) ready();
     const double saved = g->push_edge_frac;
     const int saved_chunk = g->push_chunk;
     g->push_edge_frac = c.frac;
@@ -1037,14 +1048,43 @@ void launch_multi_init(sssp_graph *g, const MultiArgs &a, const int32_t *sources
 
 // The captured launches of one chunk of at most 256 sources, keyed on chunk
 // shape and buffers: `first` initialises the vertex-major distances, the stamps
-// and the pass state, runs kMultiRun passes and transposes the result into the per-source output; `more` advances the pass
+// and the pass state, runs kMultiRun passes and transposes the result into the per-source output; `more` (captured when a
+// chunk first needs it) advances the pass
 // base by kMultiRun and runs the next kMultiRun passes and the transpose.
 // Passes after the fixpoint return at once.
-struct MultiGraphs {
-    hipGraphExec_t first, more;
-};
+hipGraphExec_t capture_multi(sssp_graph *g, int32_t c0, int32_t m, bool first)
+{
+    hipStream_t s = g->stream;
+    const int64_t V = g->V;
+    SSSP_HIP(hipStreamSynchronize(s));
+    const MultiArgs a = multi_args(g, m);
+    hipGraph_t graph;
+    SSSP_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+    if (first) {
+        launch_multi_init(g, a, g->msrc + c0, s);
+    } else {
+        k_advance_base<<<1, 64, 0, s>>>(&a.ctl->base, kMultiRun);
+    }
+    if (g->n_mtile > 0)
+        for (int32_t k = 0; k < kMultiRun; k++) launch_multi_pass(g, a, k, s);
+    k_multi_out<<<dim3((unsigned)((V + 63) / 64), (unsigned)((m + 63) / 64)), kBlock, 0, s>>>(
+        g->mdist, m, V, g->vperm, g->bdist + (int64_t)c0 * V);
+    const hipError_t le = hipGetLastError();
+    const hipError_t ce = hipStreamEndCapture(s, &graph);
+    if (le != hipSuccess || ce != hipSuccess) {
+        if (ce == hipSuccess) (void)hipGraphDestroy(graph);
+        throw Error{SSSP_ERR_HIP, std::string("capturing the batch launch failed: ") +
+                                      hipGetErrorString(le != hipSuccess ? le : ce)};
+    }
+    hipGraphExec_t exec;
+    const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    SSSP_HIP(ie);
+    return exec;
+}
 
-MultiGraphs multi_graphs(sssp_graph *g, int32_t c0, int32_t m)
+// The slot of a chunk's captured launches, `first` captured.
+int multi_graphs(sssp_graph *g, int32_t c0, int32_t m)
 {
     const int64_t V = g->V;
     const int64_t key[kMultiKey] = {m,
@@ -1058,8 +1098,7 @@ MultiGraphs multi_graphs(sssp_graph *g, int32_t c0, int32_t m)
                                     g->wtype,
                                     (int64_t)(uintptr_t)g->m_tile};
     for (int i = 0; i < kMultiSlots; i++)
-        if (g->mexec[i][0] && std::memcmp(key, g->mkey[i], sizeof(key)) == 0)
-            return MultiGraphs{(hipGraphExec_t)g->mexec[i][0], (hipGraphExec_t)g->mexec[i][1]};
+        if (g->mexec[i][0] && std::memcmp(key, g->mkey[i], sizeof(key)) == 0) return i;
     const int slot = g->mnext;
     g->mnext = (g->mnext + 1) % kMultiSlots;
     for (int j = 0; j < 2; j++)
@@ -1067,36 +1106,9 @@ MultiGraphs multi_graphs(sssp_graph *g, int32_t c0, int32_t m)
             (void)hipGraphExecDestroy((hipGraphExec_t)g->mexec[slot][j]);
             g->mexec[slot][j] = nullptr;
         }
-    hipStream_t s = g->stream;
-    SSSP_HIP(hipStreamSynchronize(s));
-    const MultiArgs a = multi_args(g, m);
-    for (int j = 0; j < 2; j++) {
-        hipGraph_t graph;
-        SSSP_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        if (j == 0) {
-            launch_multi_init(g, a, g->msrc + c0, s);
-        } else {
-            k_advance_base<<<1, 64, 0, s>>>(&a.ctl->base, kMultiRun);
-        }
-        if (g->n_mtile > 0)
-            for (int32_t k = 0; k < kMultiRun; k++) launch_multi_pass(g, a, k, s);
-        k_multi_out<<<dim3((unsigned)((V + 63) / 64), (unsigned)((m + 63) / 64)), kBlock, 0, s>>>(
-            g->mdist, m, V, g->vperm, g->bdist + (int64_t)c0 * V);
-        const hipError_t le = hipGetLastError();
-        const hipError_t ce = hipStreamEndCapture(s, &graph);
-        if (le != hipSuccess || ce != hipSuccess) {
-            if (ce == hipSuccess) (void)hipGraphDestroy(graph);
-            throw Error{SSSP_ERR_HIP, std::string("capturing the batch launch failed: ") +
-                                          hipGetErrorString(le != hipSuccess ? le : ce)};
-        }
-        hipGraphExec_t exec;
-        const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        SSSP_HIP(ie);
-        g->mexec[slot][j] = exec;
-    }
+    g->mexec[slot][0] = capture_multi(g, c0, m, true);
     std::memcpy(g->mkey[slot], key, sizeof(key));
-    return MultiGraphs{(hipGraphExec_t)g->mexec[slot][0], (hipGraphExec_t)g->mexec[slot][1]};
+    return slot;
 }
 
 // Passes among [first, first + count) that did work, from the host's copy of
@@ -1133,9 +1145,9 @@ int32_t multi_passes_launched(sssp_graph *g, const MultiArgs &a)
     return ran;
 }
 
-double run_multi(sssp_graph *g, const int32_t *sources, int32_t n)
+// Layout, buffers and the first chunk's captured launches of a policy-3 batch.
+void prepare_multi(sssp_graph *g, int32_t n)
 {
-    hipStream_t s = g->stream;
     build_multi_layout(g);
     const int64_t V = g->V;
     const int32_t chunk = std::min<int32_t>(n, kMThreads);
@@ -1153,22 +1165,30 @@ double run_multi(sssp_graph *g, const int32_t *sources, int32_t n)
     }
     if (!g->mctl) g->mctl = dmalloc<MultiCtl>(1);
     if (!g->mstamp) g->mstamp = dmalloc<int32_t>((size_t)V);
+    if (g->batch_capture) (void)multi_graphs(g, 0, chunk);
+}
+
+double run_multi(sssp_graph *g, const int32_t *sources, int32_t n)
+{
+    hipStream_t s = g->stream;
+    const int64_t V = g->V;
     SSSP_HIP(hipMemcpyAsync(g->msrc, sources, 4 * (size_t)n, hipMemcpyHostToDevice, s));
     float total = 0.f;
     g->multi_passes = 0;
     for (int32_t c0 = 0; c0 < n; c0 += kMThreads) {
         const int32_t m = std::min<int32_t>(kMThreads, n - c0);
         if (g->batch_capture) {
-            const MultiGraphs mg = multi_graphs(g, c0, m);
+            void **const mg = g->mexec[multi_graphs(g, c0, m)];
             SSSP_HIP(hipEventRecord(g->ev_a, s));
             bool done = g->n_mtile == 0;
-            if (done) SSSP_HIP(hipGraphLaunch(mg.first, s));
+            if (done) SSSP_HIP(hipGraphLaunch((hipGraphExec_t)mg[0], s));
             // replay until a run holds an idle pass (at most V + 1 passes and the
             // light ones, as the pass loop)
             for (int32_t run = 0; !done; run++) {
                 if ((int64_t)run * kMultiRun > V + 1 + kLightMaxPasses)
                     throw Error{SSSP_ERR_NOT_CONVERGED, "multi-source passes exceeded V passes"};
-                SSSP_HIP(hipGraphLaunch(run == 0 ? mg.first : mg.more, s));
+                if (run == 1 && !mg[1]) mg[1] = capture_multi(g, c0, m, false);
+                SSSP_HIP(hipGraphLaunch((hipGraphExec_t)mg[run > 0], s));
                 SSSP_HIP(hipMemcpyAsync(g->ctrl_host->changed,
                                         static_cast<MultiCtl *>(g->mctl)->kind, 4 * 64,
                                         hipMemcpyDeviceToHost, s));
@@ -1396,10 +1416,14 @@ int sssp_solve_batch(sssp_graph *g, const int32_t *sources, int32_t n, int32_t p
                                 : Config{2, 256, 2, g->push_edge_frac, g->push_chunk};
         const std::vector<int32_t> slots = source_slots(g, sources, n);
         const size_t bytes = 4 * (size_t)n * (size_t)g->V;
-        Prefault pages(dist_out, bytes);
-        const double ms = batch_sources(g, slots.data(), n, c);
+        // the pages are faulted in under the solves alone: an allocation beside
+        // it waits for the address space's lock (the first batch of R-MAT 20 x 16
+        // with 256 sources, which makes some twenty, 84 ms against 42)
+        std::optional<Prefault> pages;
+        const double ms = batch_sources(g, slots.data(), n, c,
+                                        [&] { pages.emplace(dist_out, bytes); });
         if (dist_out) {
-            pages.join();
+            pages->join();
             download(g, dist_out, g->bdist, bytes);
         }
         fill_stats(stats, ms, (double)g->E * n);
@@ -1496,6 +1520,7 @@ int sssp_pack_solve(sssp_pack *p, const int32_t *sources, int32_t policy, float 
         Config c{p->policy ? p->policy : 1, p->bs, p->wgpcu, p->frac, p->push_chunk};
         if (policy == 1) c = Config{1, p->policy == 1 ? p->bs : 1024, p->policy == 1 ? p->wgpcu : 1, 0.05, 1};
         if (policy == 2) c = Config{2, 256, 2, p->policy == 2 ? p->frac : 0.05, p->policy == 2 ? p->push_chunk : 1};
+        ensure_batch_buffers(p->g, p->g->V, 0, 0, 0);
         Prefault pages(dist_out, 4 * (size_t)p->g->V);
         const double ms = pack_run(p, sources, c);
         if (dist_out) {

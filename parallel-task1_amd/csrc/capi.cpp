@@ -649,15 +649,13 @@ int sssp_bfs(sssp_graph *g, int32_t source, int32_t schedule, uint8_t *visited_o
         std::memset(&st, 0, sizeof(st));
         g->have_result = false;
         g->bfs_result = false;
+        if (visited_out && !g->dvis) g->dvis = dmalloc<uint8_t>((size_t)g->V);
         Prefault lev_pages(levels_out, 4 * (size_t)g->V), vis_pages(visited_out, (size_t)g->V);
         bfs(g, slot_of(g, source), schedule, &st);
         g->last_source = source;
         g->last_sched = schedule;
         g->bfs_result = true;
-        if (visited_out) {
-            if (!g->dvis) g->dvis = dmalloc<uint8_t>((size_t)g->V);
-            levels_to_visited(g->dout, g->V, g->dvis, g->stream);
-        }
+        if (visited_out) levels_to_visited(g->dout, g->V, g->dvis, g->stream);
         lev_pages.join();
         vis_pages.join();
         if (levels_out) download(g, levels_out, g->dout, 4 * (size_t)g->V);

@@ -6,6 +6,7 @@ oracle's restatement of cpu_bellman_ford, sssp.hpp:3-71), plus the
 shortest-path certificate (all edges satisfied, tight parent tree).
 """
 import ctypes as C
+import mmap
 
 import numpy as np
 import pytest
@@ -1469,3 +1470,71 @@ def test_batch_light_records_where_they_pay(gpu, oracle, V, E, n, kind, light):
             assert (g.get_param("multi_light_tiles") > 0) == light
             for i, ref in refs.items():
                 assert np.array_equal(bits(D[i]), bits(ref)), (capture, i)
+
+
+def _fresh(n, dtype):
+    """An array in memory just mapped, none of it touched."""
+    return np.frombuffer(mmap.mmap(-1, n * np.dtype(dtype).itemsize,
+                                   flags=mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS), dtype)
+
+
+def _resident(a):
+    """Pages of an array that are in memory, by mincore(2)."""
+    libc = C.CDLL(None, use_errno=True)
+    page = 4096
+    lo = (a.ctypes.data + page - 1) // page * page
+    n = (a.ctypes.data + a.nbytes - lo) // page
+    vec = (C.c_ubyte * n)()
+    assert libc.mincore(C.c_void_p(lo), C.c_size_t(n * page), vec) == 0
+    return sum(v & 1 for v in vec), n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["batch1", "batch2", "batch3", "bfs", "pack"])
+def test_result_pages_wait_for_the_allocations(gpu, oracle, call):
+    """The pages of a large result are faulted in only once the call's device
+    buffers are there (each allocation would wait for the page faults): when
+    the first one fails, the call returns SSSP_ERR_OOM with the result's pages untouched. The
+    next call succeeds, with every word written."""
+    src, dst, w = S.rmat(17, 4, seed=5, threads=8)
+    V, n = 1 << 17, 40
+    L, sources = S.lib(), S.pick_sources(src, 1 << 17, 2, 40)
+    if call == "pack":
+        k = 40
+        offs = np.arange(k + 1, dtype=np.int64) * len(src)
+        many = [np.tile(x, k) for x in (src, dst, w)]
+        p = S.GraphPack(*many, offs, np.full(k, V, np.int32))
+        same = np.full(k, int(sources[0]), np.int32)
+        out, rows, want = _fresh(k * V, np.float32), k, [int(sources[0])] * k
+        run = lambda: L.sssp_pack_solve(p._h, S._ptr(same), 0, S._ptr(out), None)  # noqa: E731
+        close = p.close
+    else:
+        if call == "bfs":
+            V = 1 << 21
+        g = S.DeviceGraph(src, dst, w, V)
+        close = g.close
+        if call == "bfs":
+            out, vis = _fresh(V, np.uint32), np.empty(V, np.uint8)
+            run = lambda: L.sssp_bfs(g.handle, int(sources[0]), S.SCHED_HEURISTIC,  # noqa: E731
+                                     S._ptr(vis), S._ptr(out), None)
+        else:
+            out, rows, want = _fresh(n * V, np.float32), n, [int(x) for x in sources]
+            run = lambda: L.sssp_solve_batch(g.handle, S._ptr(sources), n, int(call[5:]),  # noqa: E731
+                                             S._ptr(out), None)
+    try:
+        print(f"result pages: {call}", flush=True)
+        before, pages = _resident(out)
+        assert pages > 1024 and before * 20 < pages
+        L.sssp_debug_fail_next_alloc()
+        assert run() == S.ERR_OOM
+        assert _resident(out)[0] * 20 < pages
+        assert run() == S.OK, S.last_error()
+        if call == "bfs":
+            ref = oracle.bfs(src, dst, V, int(sources[0]))
+            assert np.array_equal(out, ref[1]) and np.array_equal(vis, ref[0])
+        else:
+            for i in range(0, rows, 13):
+                ref = oracle.dijkstra(src, dst, w, V, want[i])
+                assert np.array_equal(bits(out.reshape(rows, V)[i]), bits(ref)), i
+    finally:
+        close()
