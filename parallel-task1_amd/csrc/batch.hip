@@ -591,9 +591,8 @@ double run_wg(sssp_graph *g, const TaskCounts &tc, int64_t maxv, int bs, int wgp
     if (ntasks > 0 && maxv > g->bscratch_stride)
         throw Error{SSSP_ERR_INTERNAL, "batch scratch too small"};
     maxv = g->bscratch_stride;
-    int32_t nwg = g->cu_count * wgpcu;
-    if (nwg > ntasks) nwg = ntasks;
-    if (nwg < 1) nwg = 1;
+    const int32_t nwg = std::min(g->cu_count * wgpcu, ntasks);
+    if (ntasks == 0) bs = 0;  // no launch reads it: one capture serves every setting
     ensure_chunk_sources(g);
     const int64_t key[10] = {ntasks, maxv, bs, nwg, (int64_t)(uintptr_t)g->bdist,
                              (int64_t)(uintptr_t)g->bscratch, (int64_t)(uintptr_t)g->btasks,
@@ -1217,22 +1216,40 @@ double run_multi(sssp_graph *g, const int32_t *sources, int32_t n)
     return total;
 }
 
-// one_graph: many sources on one graph (policy 3 applies); else a pack
-std::vector<Config> candidates(bool one_graph)
+// What a tuning call may choose from. one_graph: many sources on one graph
+// (policy 3 applies); else a pack. workgroups: policy 1 has tasks for the
+// persistent kernel, whose block size and workgroups per CU matter; rounds1,
+// rounds2: policy 1 / 2 solves in rounds, whose threshold and chunk matter.
+// What nothing reads has one candidate.
+struct Choices {
+    bool one_graph, workgroups, rounds1, rounds2;
+};
+
+std::vector<Config> candidates(const Choices &k)
 {
     std::vector<Config> c;
-    if (one_graph) c.push_back(Config{3, kMThreads, 1, 0.0, 0});
+    if (k.one_graph) c.push_back(Config{3, kMThreads, 1, 0.0, 0});
+    auto thresholds = [&](int policy, int bs, int w, bool rounds) {
+        if (!rounds) c.push_back(Config{policy, bs, w, 0.05, 1});
+        for (double f : {0.02, 0.05, 0.15})
+            for (int pc : {1, 2})
+                if (rounds) c.push_back(Config{policy, bs, w, f, pc});
+    };
+    if (!k.workgroups) thresholds(1, 1024, 1, k.rounds1);
     for (int bs : {256, 512, 1024})
-        for (int w : {1, 2, 4}) c.push_back(Config{1, bs, w, 0.05, 1});
-    for (double f : {0.02, 0.05, 0.15})
-        for (int pc : {1, 2}) c.push_back(Config{2, 256, 2, f, pc});
+        for (int w : {1, 2, 4})
+            if (k.workgroups) c.push_back(Config{1, bs, w, 0.05, 1});
+    thresholds(2, 256, 2, k.rounds2);
     return c;
 }
 
-std::string describe(const Config &c)
+std::string describe(const Config &c, const Choices &k)
 {
     char buf[160];
-    if (c.policy == 1)
+    if (c.policy == 1 && !k.workgroups)
+        std::snprintf(buf, sizeof(buf), k.rounds1 ? "policy=workgroup_per_task push_edge_frac=%.3f push_chunk=%d"
+                                                  : "policy=workgroup_per_task", c.frac, c.push_chunk);
+    else if (c.policy == 1)
         std::snprintf(buf, sizeof(buf), "policy=workgroup_per_task block=%d wg_per_cu=%d", c.bs, c.wgpcu);
     else if (c.policy == 3)
         std::snprintf(buf, sizeof(buf), "policy=vertex_major_all_edge sources_per_chunk=%d", c.bs);
@@ -1243,9 +1260,9 @@ std::string describe(const Config &c)
 }
 
 template <class Run>
-Config autotune(Run &&run, const char *file, double *best_ms, const char *what, bool one_graph)
+Config autotune(Run &&run, const char *file, double *best_ms, const char *what, const Choices &k)
 {
-    std::vector<Config> cs = candidates(one_graph);
+    std::vector<Config> cs = candidates(k);
     std::vector<double> t(cs.size(), 1e300);
     for (size_t i = 0; i < cs.size(); i++) {
         (void)run(cs[i]);  // warm-up (and graph capture)
@@ -1257,7 +1274,7 @@ Config autotune(Run &&run, const char *file, double *best_ms, const char *what, 
         if (!f) throw Error{SSSP_ERR_IO, std::string("cannot open tuning file ") + file};
         std::fprintf(f, "# autotune %s: min of 2 timed runs after 1 warm-up, device ms\n", what);
         for (size_t i = 0; i < cs.size(); i++)
-            std::fprintf(f, "%s ms=%.4f%s\n", describe(cs[i]).c_str(), t[i], i == b ? " best" : "");
+            std::fprintf(f, "%s ms=%.4f%s\n", describe(cs[i], k).c_str(), t[i], i == b ? " best" : "");
         std::fclose(f);
     }
     if (best_ms) *best_ms = t[b];
@@ -1441,7 +1458,8 @@ int sssp_autotune_batch(sssp_graph *g, const int32_t *sources, int32_t n, const 
         SSSP_HIP(hipSetDevice(g->device));
         const std::vector<int32_t> slots = source_slots(g, sources, n);
         const Config b = autotune([&](const Config &c) { return batch_sources(g, slots.data(), n, c); },
-                                  tuning_file, best_ms, "batch of sources", true);
+                                  tuning_file, best_ms, "batch of sources",
+                                  Choices{true, lds_class(g->V) == 0, false, !runs_passes(g, 1)});
         g->batch_policy = b.policy;
         g->batch_bs = b.bs;
         g->batch_wgpcu = b.wgpcu;
@@ -1517,9 +1535,9 @@ int sssp_pack_solve(sssp_pack *p, const int32_t *sources, int32_t policy, float 
         SSSP_REQUIRE(policy >= 0 && policy <= 2, "policy must be 0, 1 or 2");
         check_pack_sources(p, sources);
         SSSP_HIP(hipSetDevice(p->g->device));
-        Config c{p->policy ? p->policy : 1, p->bs, p->wgpcu, p->frac, p->push_chunk};
-        if (policy == 1) c = Config{1, p->policy == 1 ? p->bs : 1024, p->policy == 1 ? p->wgpcu : 1, 0.05, 1};
-        if (policy == 2) c = Config{2, 256, 2, p->policy == 2 ? p->frac : 0.05, p->policy == 2 ? p->push_chunk : 1};
+        Config c{p->policy ? p->policy : 1, p->bs, p->wgpcu, p->frac, p->push_chunk};  // as tuned
+        if (policy != 0 && policy != p->policy)
+            c = policy == 1 ? Config{1, 1024, 1, 0.05, 1} : Config{2, 256, 2, 0.05, 1};
         ensure_batch_buffers(p->g, p->g->V, 0, 0, 0);
         Prefault pages(dist_out, 4 * (size_t)p->g->V);
         const double ms = pack_run(p, sources, c);
@@ -1539,8 +1557,12 @@ int sssp_autotune_pack(sssp_pack *p, const int32_t *sources, const char *tuning_
         SSSP_REQUIRE(p && p->g, "null pack");
         check_pack_sources(p, sources);
         SSSP_HIP(hipSetDevice(p->g->device));
+        int32_t large = 0;  // graphs that policy 1 solves together
+        for (int32_t k = 0; k < p->n; k++) large += lds_class(p->voff[k + 1] - p->voff[k]) == 0;
+        const bool together = !runs_passes(p->g, p->n);
         const Config b = autotune([&](const Config &c) { return pack_run(p, sources, c); },
-                                  tuning_file, best_ms, "pack of graphs", false);
+                                  tuning_file, best_ms, "pack of graphs",
+                                  Choices{false, false, large > 0 && !runs_passes(p->g, large), together});
         p->policy = b.policy;
         p->bs = b.bs;
         p->wgpcu = b.wgpcu;

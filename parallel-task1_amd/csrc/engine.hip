@@ -2970,7 +2970,7 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
     // 200 x 200 24 / 7.6 with scattered ids, 23 / 0.98 in local passes with near
     // ones (a round costs 25 us however few vertices it holds).
     const bool small = (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) &&
-                       g->E < g->plain_below_edges / (n_src > 1 && g->n_ttile == 0 ? 2 : 1);
+                       runs_passes(g, n_src);
     if (n_src > 1) upload_sources(g, sources, n_src);
     g->trace.clear();
     g->snap_round = -1;

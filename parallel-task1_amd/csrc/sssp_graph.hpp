@@ -485,6 +485,13 @@ class Prefault {
     std::vector<std::thread> threads_;
 };
 
+// Whether a heuristic or learned solve from n_src sources runs the plain pass
+// loop, not the rounds (see solve_t; a bound, not what may be forced).
+inline bool runs_passes(const sssp_graph *g, int32_t n_src)
+{
+    return g->E < g->plain_below_edges / (n_src > 1 && g->n_ttile == 0 ? 2 : 1);
+}
+
 // batch.hip
 // Graphs solved whole in one workgroup's LDS (launch_solo): one launch and one
 // wait, where the pass loop has a launch per pass and a wait per four. One

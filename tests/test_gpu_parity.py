@@ -1538,3 +1538,40 @@ def test_result_pages_wait_for_the_allocations(gpu, oracle, call):
                 assert np.array_equal(bits(out.reshape(rows, V)[i]), bits(ref)), i
     finally:
         close()
+
+
+@pytest.mark.gpu
+def test_autotuners_try_each_setting_once(gpu, tmp_path):
+    """The tuning files list no two candidates that run the same launches: block size
+    and workgroups per CU only where a task is too large for LDS, thresholds of the rounds
+    only where a solve runs in rounds; the tuned setting solves as the others."""
+    def lines(path):
+        text = [x for x in path.read_text().splitlines() if not x.startswith("#")]
+        assert len({x.split(" ms=")[0] for x in text}) == len(text)
+        return [sum(x.startswith("policy=" + k) for x in text)
+                for k in ("workgroup_per_task", "merged_frontier", "vertex_major_all_edge")]
+
+    for scale, below, want in ((12, 2 ** 26, [1, 1, 1]), (12, 0, [1, 6, 1]), (16, 2 ** 26, [9, 1, 1])):
+        src, dst, w = S.rmat(scale, 8, seed=2, threads=8)
+        sources = S.pick_sources(src, 1 << scale, 2, 6)
+        print(f"autotune batch: scale {scale} below {below}", flush=True)
+        with S.DeviceGraph(src, dst, w, 1 << scale) as g:
+            g.set_param("plain_below_edges", below)
+            g.autotune_batch(sources, tmp_path / "b.txt")
+            assert lines(tmp_path / "b.txt") == want
+            a, b = (g.solve_batch(sources, policy=p)[0] for p in (0, 2))
+            assert np.array_equal(bits(a), bits(b))
+    for scales, want in ((np.full(9, 9), [1, 1, 0]), (np.array([9, 16, 17]), [1, 1, 0]),
+                         (np.append(np.full(65, 16), 10), [6, 6, 0])):
+        scales = scales.astype(np.int32)
+        s, d, w, offs = S.rmat_many(scales, 8, seed0=3)
+        srcs = np.minimum.reduceat(s, offs[:-1]).astype(np.int32)
+        print(f"autotune pack: {len(scales)} graphs, {len(s)} edges", flush=True)
+        p = S.GraphPack(s, d, w, offs, (1 << scales).astype(np.int32))
+        try:
+            p.autotune(srcs, tmp_path / "p.txt")
+            assert lines(tmp_path / "p.txt") == want
+            a, b = (p.solve(srcs, policy=q)[0] for q in (0, 2))
+            assert np.array_equal(bits(a), bits(b))
+        finally:
+            p.close()
