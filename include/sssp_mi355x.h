@@ -189,7 +189,8 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * "blk_range_bits", "plain_kernel", "tail_edges", "tail_group", "tail_blocks",
  * "push_bits_edges", "trace_events"; "cu_count",
  * "collect_rounds", "multi_passes", "multi_tiles", "multi_light_tiles",
- * "light_edges", "blk_tiles", "blk_wide_chunks" and "plain_blocked" read-only).
+ * "light_edges", "blk_tiles", "blk_wide_chunks", "host_polls" and "plain_blocked"
+ * read-only).
  * "light_edges" = edges in the list of the light passes (0: the graph has none, or
  * its solves run in one workgroup and none needed it yet), "multi_light_tiles" =
  * tiles over the light records of policy-3 batches (0 before the first).
@@ -240,9 +241,11 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * hub_degree waits in the pile instead of being relaxed; 0 (default) = off.
  * max_rounds (default 100000) is bounded to [1, 2^28]; a solve that needs more
  * rounds returns SSSP_ERR_NOT_CONVERGED.
- * The plain schedule queues its passes four at a time (the change flags are
- * kept and tested on the device; the host reads them after each four); with
- * trace_events = 1 each pass is launched alone between HIP events.
+ * The plain schedule's passes find out on the device whether the one before
+ * changed anything. Edge-list passes are queued four at a time (the host reads
+ * the change flags after each four), passes over blocked tiles ahead of the
+ * one the host has seen begin; with trace_events = 1 each pass is launched alone
+ * between HIP events.
  * batch_capture (default 1): a batch of policy 3 runs each chunk of up to 256
  * sources as captured hipGraph launches -- init and a run of 32 passes (one
  * launch each, the pass number read from device memory, passes after the
@@ -261,9 +264,11 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * source gathers of the workgroups in flight stay in one range; the default
  * is 0, or, for a graph of 2^22 vertices or more without hub blocks, the size
  * that makes 8 ranges. "blk_wide_chunks" (read-only) = chunks of 256 edges
- * whose sources are stored whole (a gap of 2^18 or more between two of them). decide_spin (default 1): the host polls the
- * mapped control block for each round's decision instead of synchronizing
- * the stream.
+ * whose sources are stored whole (a gap of 2^18 or more between two of them).
+ * decide_spin (default 1): the host polls the mapped control block for each
+ * round's decision and for the progress of passes over blocked tiles; 0: it
+ * synchronizes the stream instead, per round or per four passes. "host_polls" (read-only) =
+ * polls of the last solve.
  * Distances do not depend on any knob. */
 int sssp_set_param(sssp_graph *g, const char *name, double value);
 int sssp_get_param(const sssp_graph *g, const char *name, double *value);

@@ -856,6 +856,7 @@ int sssp_get_param(const sssp_graph *g, const char *name, double *value)
         else if (n == "collect_budget") *value = (double)g->collect_budget;
         else if (n == "collect_rounds") *value = (double)g->collect_rounds;
         else if (n == "trace_events") *value = g->trace_events;
+        else if (n == "host_polls") *value = (double)g->host_polls;
         else if (n == "cu_count") *value = g->cu_count;
         else throw Error{SSSP_ERR_ARG, "unknown parameter '" + n + "'"};
     });

@@ -2477,6 +2477,7 @@ void wait_decision(sssp_graph *g, int32_t seq)
 {
     volatile int32_t *p = &g->ctrl_host->dec_seq;
     for (int64_t i = 0; g->decide_spin && i < kSpinPolls; i++) {
+        g->host_polls++;
         if (*p == seq) {
             std::atomic_thread_fence(std::memory_order_acquire);
             return;
@@ -2490,9 +2491,11 @@ void wait_decision(sssp_graph *g, int32_t seq)
 // host's poll and launch, few enough that the idle ones left in the queue
 // when a run ends (3-6 us each) cost little.
 constexpr int kPassAhead = 3;
+constexpr int kPassGroup = 4;  // passes queued per stream synchronize without polls
 
 // Runs a run of blocked passes (k_blk_plain) to its end on the device, the
-// host queueing passes as it sees them begin in the mirror's progress word.
+// host queueing passes as it sees them begin in the mirror's progress word, or,
+// without decide_spin, a group per stream synchronize.
 // With trace_events every pass is launched alone between events. Adds the
 // passes to the stats and the trace; full_limit: full passes at most (then
 // SSSP_ERR_NOT_CONVERGED). local: source of a run of local passes
@@ -2545,7 +2548,7 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int3
     // the mirror still holds the last run's word (another tag) or none
     volatile unsigned long long *pos = &g->ctrl_host->ph_pos;
     const unsigned long long mine = pass_word(a.tag, 0, 0, 0) >> 58;
-    const int ahead = g->trace_events ? 1 : kPassAhead;
+    const int ahead = g->trace_events ? 1 : g->decide_spin ? kPassAhead : kPassGroup;
     int32_t queued = 0, begun = 0, full = 0;
     int kind = 0;
     while (kind != kPassIdle) {
@@ -2562,15 +2565,17 @@ void run_passes(sssp_graph *g, int run, int64_t full_limit, sssp_stats *st, int3
         unsigned long long w = 0;
         bool drained = false;
         for (int64_t i = 0;; i++) {
+            if (!drained && (!g->decide_spin || i >= kSpinPolls ||
+                             ((i & 1023) == 1023 && hipStreamQuery(s) != hipErrorNotReady))) {
+                SSSP_HIP(hipStreamSynchronize(s));  // reports a failed kernel
+                drained = true;                      // the word is final
+            }
+            if (!drained) g->host_polls++;
             w = *pos;
             if (w >> 58 == mine && ((int32_t)(w >> 30 & 0xFFFFFFF) > begun ||
                                     (int)(w & 3) == kPassIdle))
                 break;
             if (drained) throw Error{SSSP_ERR_INTERNAL, "blocked passes made no progress"};
-            if ((i & 1023) == 1023 && hipStreamQuery(s) != hipErrorNotReady) {
-                SSSP_HIP(hipStreamSynchronize(s));  // reports a failed kernel
-                drained = true;                      // the word is final: read it once more
-            }
         }
         const int32_t was = begun;
         begun = (int32_t)(w >> 30 & 0xFFFFFFF);
@@ -2974,6 +2979,7 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
     if (n_src > 1) upload_sources(g, sources, n_src);
     g->trace.clear();
     g->snap_round = -1;
+    g->host_polls = 0;
     if (small && n_src == 1 && solo_fits(g) && g->plain_kernel == 0 && !g->trace_events) {
         solve_solo<WT>(g, source, st);
         return;

@@ -343,7 +343,8 @@ struct sssp_graph {
     int32_t tick = 1;
     int32_t dec_seq = 0;  // sequence number of the last decision enqueued
     int32_t ph_tag = 0;   // tag of the last run of blocked passes
-    int decide_spin = 1;  // 1: poll the mirror for the decision; 0: stream synchronize
+    int decide_spin = 1;  // 1: poll the mirror for decisions and passes; 0: stream synchronize
+    int64_t host_polls = 0;  // polls of the mirror in the last solve
     hipEvent_t ev_a = nullptr, ev_b = nullptr, ev_r0 = nullptr, ev_r1 = nullptr;
 
     // knobs

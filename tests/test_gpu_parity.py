@@ -1575,3 +1575,40 @@ def test_autotuners_try_each_setting_once(gpu, tmp_path):
             assert np.array_equal(bits(a), bits(b))
         finally:
             p.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["plain", "light", "local", "rounds"])
+def test_decide_spin_off_never_polls(gpu, oracle, kind):
+    """decide_spin 0: the host synchronizes the stream, in passes over blocked tiles
+    (plain schedule, light and local passes) as in rounds, and polls nothing; 1:
+    it polls. Distances are the same, traced or not, and a limit below the solve's
+    passes still gives up and leaves the graph usable."""
+    if kind == "local":
+        V, src, dst = _local_graph("grid", np.random.default_rng(1))
+        src, dst = src.astype(np.int32), dst.astype(np.int32)
+        w = np.random.default_rng(2).random(len(src), dtype=np.float32)
+    else:
+        src, dst, w = S.rmat(16, 16, seed=5, threads=8)
+        V = 1 << 16
+    source, sched = int(src[0]), "plain" if kind == "plain" else "heuristic"
+    ref = oracle.dijkstra(src, dst, w, V, source)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        g.set_param("plain_kernel", 2 if kind == "plain" else 0)
+        if kind == "rounds":
+            g.set_param("plain_below_edges", 0)
+        for spin in (0, 1, 0):
+            g.set_param("decide_spin", spin)
+            for traced in (0, 1):
+                g.set_param("trace_events", traced)
+                print(f"decide_spin {spin}: {kind} traced {traced}", flush=True)
+                d, st = g.solve(source, sched)
+                assert np.array_equal(bits(d), bits(ref)), (spin, traced)
+                assert (g.get_param("host_polls") > 0) == (spin == 1), (spin, traced)
+            g.set_param("trace_events", 0)
+            if kind == "plain":
+                g.set_param("max_rounds", 1)
+                with pytest.raises(S.SSSPError) as e:
+                    g.solve(source, sched)
+                assert e.value.code == S.ERR_NOT_CONVERGED
+                g.set_param("max_rounds", 100000)
