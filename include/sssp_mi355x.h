@@ -221,8 +221,9 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * plain_kernel picks the plain pass: 0 (default) the destination-blocked pass
  * (block minima in LDS, as the dense rounds) once the blocked list has 64
  * tiles or more, else the XCD-partitioned edge-list pass; 1 always the
- * edge-list pass (also for those graphs), 2 always the blocked pass. "plain_blocked" (read-only) = 1
- * when plain solves use the blocked pass.
+ * edge-list pass (also for those graphs), 2 always the blocked pass (light ones
+ * among them, local ones never). "plain_blocked" (read-only) = 1 when plain solves
+ * use the blocked pass.
  * tail_edges (default 2^23): once a heuristic or learned solve's frontier has
  * had more than tail_edges out-edges, a round decided as a push round over a
  * frontier with at most that many (far pile off) starts the tail rounds: push

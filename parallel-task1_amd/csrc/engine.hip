@@ -2628,7 +2628,7 @@ void solve_plain(sssp_graph *g, bool mixed, int32_t source, int32_t n_src, sssp_
     const int64_t E = g->E;
     const int64_t limit = plain_limit(g);
     st->verify_passes = 1;  // the last pass changed nothing: the fixpoint check
-    if (mixed && g->n_ttile > 0 && g->plain_kernel != 1) {
+    if (mixed && g->n_ttile > 0 && g->plain_kernel == 0) {
         run_passes<WT>(g, kRunFull, limit, st, source, n_src);
         return;
     }

@@ -1612,3 +1612,22 @@ def test_decide_spin_off_never_polls(gpu, oracle, kind):
                     g.solve(source, sched)
                 assert e.value.code == S.ERR_NOT_CONVERGED
                 g.set_param("max_rounds", 100000)
+
+
+@pytest.mark.gpu
+def test_plain_kernel_forces_every_kind_of_graph(gpu, oracle):
+    """plain_kernel 2 runs the blocked pass and 1 the edge-list pass also on
+    graphs that have local passes: each of their passes relaxes every edge, local ones
+    leave tiles out."""
+    V, src, dst = _local_graph("grid", np.random.default_rng(1))
+    src, dst = src.astype(np.int32), dst.astype(np.int32)
+    w = np.random.default_rng(2).random(len(src), dtype=np.float32)
+    ref = oracle.dijkstra(src, dst, w, V, 7)
+    with S.DeviceGraph(src, dst, w, V) as g:
+        for kernel in (0, 1, 2):
+            g.set_param("plain_kernel", kernel)
+            print(f"plain kernel {kernel} on a grid", flush=True)
+            d, st = g.solve(7, "heuristic")
+            assert np.array_equal(bits(d), bits(ref)), kernel
+            every = st["edges_relaxed"] == st["iterations"] * len(src)
+            assert every == (kernel != 0), kernel
