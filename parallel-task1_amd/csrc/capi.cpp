@@ -4,11 +4,13 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
+#include <thread>
 
 #include "mlp_dev.hpp"
 #include "sssp_graph.hpp"
@@ -31,19 +33,156 @@ int fail(int code, const std::string &msg)
 
 namespace {
 
-// The pinned buffers that large results are staged through: one set for the
-// process (16 MB), allocated at the first such result and freed with the last
-// graph. A download that finds another thread using them copies directly.
+// Threads that empty the staging buffers, beside the caller: as many as could be
+// made (none is needed). A chunk is cut into one part per thread and the
+// caller; each copies its own (the caller's memory stays in that CPU's cache
+// from call to call), and the caller those that nobody has begun.
+class Crew {
+  public:
+    void start()
+    {
+        try {
+            while (n_ < kThreads) {
+                const int id = n_ + 1;  // 0: the caller
+                threads_[n_] = std::thread([this, id] { serve(id); });
+                n_++;
+            }
+        } catch (...) {  // no thread to be had: fewer do
+        }
+    }
+    void stop()
+    {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            quit_ = true;
+        }
+        cv_.notify_all();
+        while (n_ > 0) threads_[--n_].join();
+        quit_ = false;
+        run_ = 0;
+    }
+    // One download of `bytes` through the ring at `ring`; closed (and left by
+    // every thread) when the Run ends.
+    class Run {
+      public:
+        Run(Crew &c, char *dst, const char *ring, size_t bytes) : c_(c)
+        {
+            c.dst_ = dst;
+            c.ring_ = ring;
+            c.bytes_ = bytes;
+            c.chunks_ = (bytes + kStageBytes - 1) / kStageBytes;
+            c.filled_ = 0;
+            c.ended_ = false;
+            {
+                std::lock_guard<std::mutex> lock(c.mu_);
+                c.run_++;
+                c.open_ = true;
+            }
+            c.cv_.notify_all();
+        }
+        ~Run()
+        {
+            c_.ended_ = true;
+            std::unique_lock<std::mutex> lock(c_.mu_);
+            c_.open_ = false;
+            c_.gone_.wait(lock, [&] { return c_.in_ == 0; });
+        }
+        // Chunk k is in its buffer: returns once it is copied out.
+        void chunk(size_t k)
+        {
+            c_.done_.store(0, std::memory_order_relaxed);
+            c_.claims_.store((uint64_t)k << kParts, std::memory_order_relaxed);
+            c_.filled_.store(k + 1, std::memory_order_release);
+            for (int id = 0; id < kParts; id++)
+                if (c_.claim(k, id)) c_.copy(k, id);
+            while (c_.done_.load(std::memory_order_acquire) < kParts) __builtin_ia32_pause();
+        }
+
+      private:
+        Crew &c_;
+    };
+
+  private:
+    static constexpr int kThreads = 7, kParts = kThreads + 1;
+    static constexpr size_t kPart = kStageBytes / kParts;
+    static constexpr int kSpins = 1 << 12;  // before a thread gives its CPU away: 100 us, a chunk's copy
+
+    // Part id of chunk k, unless it is taken, or the chunk is over.
+    bool claim(size_t k, int id)
+    {
+        uint64_t w = claims_.load(std::memory_order_relaxed);
+        while (w >> kParts == k && !(w >> id & 1))
+            if (claims_.compare_exchange_weak(w, w | (uint64_t)1 << id)) return true;
+        return false;
+    }
+    void copy(size_t k, int id)
+    {
+        const size_t o = k * kStageBytes + id * kPart;
+        if (o < bytes_)
+            std::memcpy(dst_ + o, ring_ + k % kStageBufs * kStageBytes + id * kPart,
+                        std::min(kPart, bytes_ - o));
+        done_.fetch_add(1, std::memory_order_release);
+    }
+    void serve(int id)
+    {
+        uint64_t seen = 0;
+        std::unique_lock<std::mutex> lock(mu_);
+        for (;;) {
+            cv_.wait(lock, [&] { return quit_ || (open_ && run_ != seen); });
+            if (quit_) return;
+            seen = run_;
+            in_++;
+            lock.unlock();
+            int spins = 0;
+            for (size_t k = 0; k < chunks_ && !ended_;) {
+                const size_t filled = filled_.load(std::memory_order_acquire);
+                if (filled > k) {
+                    k = filled - 1;  // earlier ones are over
+                    if (claim(k, id)) copy(k, id);
+                    k++;
+                    spins = 0;
+                } else if (++spins < kSpins) {
+                    __builtin_ia32_pause();
+                } else {
+                    std::this_thread::yield();
+                }
+            }
+            lock.lock();
+            if (--in_ == 0) gone_.notify_all();
+        }
+    }
+
+    std::thread threads_[kThreads];
+    int n_ = 0;
+    std::mutex mu_;
+    std::condition_variable cv_, gone_;
+    bool quit_ = false, open_ = false;
+    uint64_t run_ = 0;
+    int in_ = 0;  // threads in the open run
+    char *dst_ = nullptr;
+    const char *ring_ = nullptr;
+    size_t bytes_ = 0, chunks_ = 0;
+    std::atomic<bool> ended_{false};
+    alignas(64) std::atomic<size_t> filled_{0};
+    alignas(64) std::atomic<uint64_t> claims_{0};  // chunk, and a bit per part
+    alignas(64) std::atomic<int> done_{0};
+};
+
+// The pinned buffers that large results are staged through, and the threads
+// that empty them: one set for the process (16 MB), made at the first such
+// result and given back with the last graph. A download that finds another thread
+// using them copies directly.
 struct Stage {
     std::mutex mu;
     char *mem = nullptr;
     int graphs = 0;
+    Crew crew;
 };
 
 Stage &stage()
 {
-    static Stage s;
-    return s;
+    static Stage *s = new Stage;  // a program that exits with graphs left leaves its threads
+    return *s;
 }
 
 void stage_retain()
@@ -56,6 +195,7 @@ void stage_release()
 {
     std::lock_guard<std::mutex> lock(stage().mu);
     if (--stage().graphs == 0 && stage().mem) {
+        stage().crew.stop();
         (void)hipHostFree(stage().mem);
         stage().mem = nullptr;
     }
@@ -120,7 +260,6 @@ bool pageable(const void *p)
 // allocate once per graph.
 constexpr size_t kStagedMin = kStageBytes + 1;
 constexpr size_t kPrefaultPerThread = (size_t)16 << 20;
-constexpr int kPrefaultThreads = 8;
 constexpr uintptr_t kPrefaultStep = (uintptr_t)4 << 20;
 
 }  // namespace
@@ -135,15 +274,15 @@ Prefault::Prefault(void *dst, size_t bytes)
     const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE), huge = (uintptr_t)2 << 20;
     const uintptr_t lo = ((uintptr_t)dst + page - 1) / page * page;
     const uintptr_t hi = ((uintptr_t)dst + bytes) / page * page;
-    const int n = (int)std::min<size_t>(kPrefaultThreads, bytes / kPrefaultPerThread + 1);
+    const int n = (int)std::min<size_t>(kThreads, bytes / kPrefaultPerThread + 1);
     try {
         for (int i = 0; i < n; i++) {
             const uintptr_t span = hi - lo;
             uintptr_t a = lo + span / n * i, b = i == n - 1 ? hi : lo + span / n * (i + 1);
             if (i > 0) a = std::min((a + huge - 1) / huge * huge, hi);
             if (i < n - 1) b = std::min((b + huge - 1) / huge * huge, hi);
-            if (a < b)
-                threads_.emplace_back([this, a, b] {
+            if (a < b) {
+                threads_[n_] = std::thread([this, a, b] {
                     while (!go_.load(std::memory_order_acquire)) std::this_thread::yield();
                     // an older kernel refuses this advice: the copy faults the
                     // pages in then
@@ -152,8 +291,10 @@ Prefault::Prefault(void *dst, size_t bytes)
                                     MADV_POPULATE_WRITE) != 0)
                             break;
                 });
+                n_++;
+            }
         }
-    } catch (const std::system_error &) {  // no thread to be had: not needed
+    } catch (...) {  // no thread, or no memory for one: not needed
     }
     // all threads exist before the first page is touched: making one maps its
     // stack, which waits for the address space's lock behind a population (3 ms
@@ -163,8 +304,7 @@ Prefault::Prefault(void *dst, size_t bytes)
 
 void Prefault::join()
 {
-    for (std::thread &t : threads_) t.join();
-    threads_.clear();
+    while (n_ > 0) threads_[--n_].join();
 }
 
 Prefault::~Prefault() { join(); }
@@ -177,11 +317,14 @@ void download(sssp_graph *g, void *dst, const void *src, size_t bytes)
 {
     std::unique_lock<std::mutex> lock(stage().mu, std::defer_lock);
     const bool staged = bytes >= kStagedMin && pageable(dst) && lock.try_lock();
-    if (staged && !stage().mem &&
-        hipHostMalloc((void **)&stage().mem, kStageBufs * kStageBytes, hipHostMallocPortable) !=
-            hipSuccess) {
-        (void)hipGetLastError();
-        stage().mem = nullptr;
+    if (staged && !stage().mem) {
+        if (hipHostMalloc((void **)&stage().mem, kStageBufs * kStageBytes,
+                          hipHostMallocPortable) == hipSuccess) {
+            stage().crew.start();
+        } else {
+            (void)hipGetLastError();
+            stage().mem = nullptr;
+        }
     }
     if (!staged || !stage().mem) {
         SSSP_HIP(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
@@ -205,14 +348,11 @@ void download(sssp_graph *g, void *dst, const void *src, size_t bytes)
         SSSP_HIP(hipEventRecord(g->stage_ev[k % kStageBufs], s));
     };
     for (size_t k = 0; k < n && k < (size_t)kStageBufs; k++) fetch(k);
+    // (waking the threads takes as long as the first chunk's way here)
+    Crew::Run run(stage().crew, static_cast<char *>(dst), ring, bytes);
     for (size_t k = 0; k < n; k++) {
         SSSP_HIP(hipEventSynchronize(g->stage_ev[k % kStageBufs]));
-        const char *from = ring + k % kStageBufs * kStageBytes;
-        char *to = static_cast<char *>(dst) + k * kStageBytes;
-        const int64_t len = (int64_t)size(k), part = (int64_t)512 << 10;
-#pragma omp parallel for schedule(static) num_threads(8)
-        for (int64_t o = 0; o < len; o += part)
-            std::memcpy(to + o, from + o, (size_t)std::min(part, len - o));
+        run.chunk(k);
         if (k + kStageBufs < n) fetch(k + kStageBufs);
     }
 }

@@ -472,9 +472,11 @@ __device__ inline int64_t block_excl_scan_i64(int64_t x, int64_t *total, int64_t
 void download(sssp_graph *g, void *dst, const void *src, size_t bytes);
 // Faults in a large host buffer's pages on helper threads while the GPU
 // solves (the first touch of fresh memory costs more than the copy into it);
-// its contents stay as they are. Joined by the destructor.
+// its contents stay as they are. Joined by the destructor. Never throws: without
+// threads, or memory for them, the copy faults the pages in.
 class Prefault {
   public:
+    static constexpr int kThreads = 8;
     Prefault(void *dst, size_t bytes);
     ~Prefault();
     Prefault(const Prefault &) = delete;
@@ -483,7 +485,8 @@ class Prefault {
 
   private:
     std::atomic<bool> go_{false};
-    std::vector<std::thread> threads_;
+    std::thread threads_[kThreads];
+    int n_ = 0;
 };
 
 // Whether a heuristic or learned solve from n_src sources runs the plain pass
