@@ -2633,8 +2633,9 @@ void solve_plain(sssp_graph *g, bool mixed, int32_t source, int32_t n_src, sssp_
         return;
     }
     if (plain_uses_blocked(g)) {
-        run_passes<WT>(g, mixed && WT::kWeighted && g->n_ltile > 0 ? kRunMixed : kRunFull, limit,
-                       st, kNotLocal, 1, mixed ? nullptr : g->b_ptile);
+        const bool light = mixed && WT::kWeighted && g->n_ltile > 0 &&
+                           (g->plain_kernel == 2 || light_pays(g));
+        run_passes<WT>(g, light ? kRunMixed : kRunFull, limit, st, kNotLocal, 1, mixed ? nullptr : g->b_ptile);
         return;
     }
     const int64_t ng = E >> 2;
@@ -2984,7 +2985,10 @@ void solve_t(sssp_graph *g, const int32_t *sources, int32_t n_src, int sched, ss
         solve_solo<WT>(g, source, st);
         return;
     }
-    if (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) ensure_pass_lists(g);
+    if (small) ensure_local_tiles(g);
+    if (WT::kWeighted && (sched == SSSP_SCHED_HEURISTIC || sched == SSSP_SCHED_LEARNED) &&
+        (!small || g->plain_kernel == 2 || light_pays(g)))
+        ensure_light_list(g);
     SSSP_HIP(hipEventRecord(g->ev_a, s));
     k_fill<uint32_t><<<grid_for(g->V), kBlock, 0, s>>>(g->dist, g->V, WT::INF);
     SSSP_LAUNCH_CHECK("k_fill dist");
@@ -3106,7 +3110,7 @@ void collect_t(sssp_graph *g, int32_t source, int32_t cap, float *feats, float *
         k_fill<int32_t><<<grid_for(g->V), kBlock, 0, s>>>(g->farst, g->V, 0);
         SSSP_LAUNCH_CHECK("pile state reset");
     }
-    ensure_pass_lists(g);
+    ensure_light_list(g);
     const int32_t tick0 = g->tick;
     const size_t V = (size_t)g->V;
     struct Saved {

@@ -1342,20 +1342,15 @@ static bool without_memory_skip(F &&f, Undo &&undo)
     }
 }
 
-static bool light_list_if_room(sssp_graph *g, const int32_t *bs, const uint16_t *bd,
-                               const int64_t *boff, int32_t nblk, int64_t nch, Carve &tmp)
+static void drop_light_list(sssp_graph *g)
 {
-    return without_memory_skip([&] { build_light_list(g, bs, bd, boff, nblk, nch, tmp); },
-                               [&] {
-                                   (void)hipStreamSynchronize(g->stream);
-                                   for (void *p : {(void *)g->l_w, (void *)g->l_pk,
-                                                   (void *)g->l_cbase, (void *)g->l_wide})
-                                       dfree(p);
-                                   g->l_w = g->l_pk = nullptr;
-                                   g->l_cbase = g->l_wide = nullptr;
-                                   g->l_edges = g->l_nwide = g->light_edges = 0;
-                                   g->b_ranges.loff.clear();
-                               });
+    (void)hipStreamSynchronize(g->stream);
+    for (void *p : {(void *)g->l_w, (void *)g->l_pk, (void *)g->l_cbase, (void *)g->l_wide}) dfree(p);
+    g->l_w = g->l_pk = nullptr;
+    g->l_cbase = g->l_wide = nullptr;
+    g->l_edges = g->l_nwide = g->light_edges = 0;
+    g->l_off_host.clear();
+    g->b_ranges.loff.clear();
 }
 
 // The blocked list's edges again as whole sources and destination offsets
@@ -1382,16 +1377,15 @@ __global__ __launch_bounds__(kBlock) void k_blk_unpack(const uint32_t *pk, const
     }
 }
 
-void ensure_pass_lists(sssp_graph *g)
+void ensure_light_list(sssp_graph *g)
 {
-    if (g->pass_lists || g->E == 0) return;
+    if (g->light_built || g->E == 0) return;
     hipStream_t s = g->stream;
     const size_t Ep = (size_t)g->b_edges, nblk = g->b_off_host.size() - 1;
-    const bool built = without_memory_skip(
+    g->light_built = without_memory_skip(
         [&] {
             Carve tmp(nullptr, 0);
             sample_weights(g, tmp);
-            build_local_tiles(g);
             if (g->light_thr == 0xFFFFFFFFu) return;
             int32_t *bs = tmp.get<int32_t>(Ep);
             uint16_t *bd = tmp.get<uint16_t>(Ep);
@@ -1402,13 +1396,25 @@ void ensure_pass_lists(sssp_graph *g)
             k_blk_unpack<<<(unsigned)((nch * 64 + kBlock - 1) / kBlock), kBlock, 0, s>>>(
                 g->b_pk, g->b_cbase, g->b_wide, nch, bs, bd);
             SSSP_LAUNCH_CHECK("k_blk_unpack");
-            if (light_list_if_room(g, bs, bd, boff, (int32_t)nblk, nch, tmp) && g->light_edges > 0)
+            build_light_list(g, bs, bd, boff, (int32_t)nblk, nch, tmp);
+            if (g->light_edges > 0)
                 retile_blocked(g, g->blk_tile_cap, g->blk_order_set ? g->blk_tile_order : -1,
                                g->blk_range_bits);
             SSSP_HIP(hipStreamSynchronize(s));
         },
-        [&] { (void)hipStreamSynchronize(s); });
-    g->pass_lists = built;
+        [&] { drop_light_list(g); });
+}
+
+void ensure_local_tiles(sssp_graph *g)
+{
+    if (g->local_built || g->E == 0) return;
+    g->local_built = without_memory_skip(
+        [&] {
+            Carve tmp(nullptr, 0);
+            sample_weights(g, tmp);
+            build_local_tiles(g);
+        },
+        [] {});
 }
 
 // The light edges of the src-sorted list as records of their own, where they
@@ -1709,15 +1715,15 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
             g->b_ranges.fine_bits = kBlkRangeFineBits;
             g->b_ranges.n_fine = (int32_t)nfine;
         }
-        // The light list, unless solves of the graph run in one workgroup
-        // (ensure_pass_lists builds it for those that do not; the sample of the
-        // weights and the list are 0.1 and 0.15 ms of a build of 0.7 ms).
+        // What the graph's solves run passes over, unless they run in one
+        // workgroup: the light list where light passes pay (the sample of the
+        // weights and the list are 0.1 and 0.15 ms of a small build of 0.7 ms)
         if (V > kSoloVerts || E > std::min(kSoloLocalEdges, kRegEdges)) sample_weights(g, tmp);
         const bool solo = V <= kSoloVerts && E <= (g->local_graph ? kSoloLocalEdges : kSoloEdges);
-        if (!solo) {
-            (void)light_list_if_room(g, bs, bd, boff, nblk, nch, tmp);
-            g->pass_lists = true;
-        }
+        if (!solo && (light_pays(g) || E >= g->plain_below_edges))
+            g->light_built =
+                without_memory_skip([&] { build_light_list(g, bs, bd, boff, nblk, nch, tmp); },
+                                    [&] { drop_light_list(g); });
         SSSP_HIP(hipStreamSynchronize(s));
         // Without hubs the d[src] gathers of a tile spread over the whole
         // distance array (degree order cannot gather them), so a graph whose
@@ -1735,8 +1741,8 @@ void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, co
             range_bits = std::max(kBlkRangeFineBits, lg - 3);
         }
         retile_blocked(g, tcap, -1, range_bits);
-        if (g->pass_lists)
-            (void)without_memory_skip([&] { build_local_tiles(g); }, [] {});
+        if (!solo)
+            g->local_built = without_memory_skip([&] { build_local_tiles(g); }, [] {});
     }
     if (solo_fits(g) && E > kRegEdges) ensure_chunk_sources(g);
 

@@ -125,6 +125,18 @@ struct TileState {
 // lines: uniform 1 M x 16 2.26 -> 2.77 ms of plain passes.)
 constexpr int kLightSample = 1 << 12;        // weights sampled for the threshold
 constexpr double kLightMinDegree = 8;        // no light class on sparser graphs without hubs
+// The pass loop runs light passes from these edge counts, and without hubs
+// this mean of edges per vertex with out-edges, on: below, a pass costs its launch
+// and one tile's chain, and light passes are a third more passes. Time with
+// light passes over time without, heuristic solves: hubs, power-law 100 K x 8-16 1.09-1.21,
+// 200 K x 10 (2.0 M) 1.06, 200 K x 12 0.95, 400 K x 8 0.92, 1 M x 8 0.77, 4 M x 16 0.50,
+// R-MAT 16 x 8 1.05, 16 x 16 1.00, 17 x 8 0.99, 17 x 16 (2^21) 0.90, 19 x 16 0.63; none,
+// uniform 400 K x 8 / 10 / 12 / 16 1.15-1.30 / 1.21-1.26 / 1.04-1.09 / 1.02-1.09, 1 M 1.20-1.27 / 1.05-1.10 /
+// 0.97-1.01 / 0.94, 2 M 1.00-1.17 / 1.04-1.14 / 0.81-0.85 / 0.86-0.90, 4 M 0.92 / 0.94-1.00 /
+// 0.91-0.97 / 0.68-0.74, 7.9 M x 8 1.00-1.18. (Rounds gain from kLightMinDegree on:
+// uniform 16 M x 8 0.77.)
+constexpr int64_t kLightLoopEdges = (int64_t)1 << 21, kLightLoopEvenEdges = (int64_t)3 << 22;
+constexpr int64_t kLightLoopMean = 11;
 constexpr int64_t kLightTileMin = 1 << 12;   // edge slots of a light tile at least
 constexpr int64_t kLightTiles = 1024;        // ... and the tile count its cap aims at
 constexpr int kLightMaxPasses = 64;          // light passes stop after this many passes of a run
@@ -249,10 +261,10 @@ struct sssp_graph {
     bool local_graph = false;  // sparse, no hubs, most edges between near ids
     int64_t light_edges = 0;      // edges in the light list
     // largest weight pattern of the light class (0xFFFFFFFF: none), once the
-    // edges were sampled (weights_known); pass_lists: the light list or the
-    // local tiles, where the graph has them, are built
+    // edges were sampled (weights_known); the light list and the local tiles, where
+    // the graph has them, are built
     uint32_t light_thr = 0xFFFFFFFFu;
-    bool weights_known = false, pass_lists = false;
+    bool weights_known = false, light_built = false, local_built = false;
     bool out_hubs = false;  // a vertex with 16 times the mean of the out-edges (sampled too)
     std::vector<int64_t> b_off_host;  // padded block offsets (tiles are rebuilt from them)
     std::vector<int64_t> l_off_host;  // ... of the light list
@@ -489,6 +501,13 @@ class Prefault {
     int n_ = 0;
 };
 
+inline bool light_pays(const sssp_graph *g)
+{
+    return g->light_thr != 0xFFFFFFFFu &&
+           (g->out_hubs ? g->E >= kLightLoopEdges
+                        : g->E >= kLightLoopEvenEdges && g->E >= kLightLoopMean * g->n_nzo);
+}
+
 // Whether a heuristic or learned solve from n_src sources runs the plain pass
 // loop, not the rounds (see solve_t; a bound, not what may be forced).
 inline bool runs_passes(const sssp_graph *g, int32_t n_src)
@@ -542,10 +561,11 @@ void split_records(const uint32_t *rec, int64_t n, int32_t *src, int32_t *dst, u
 void build_layouts(sssp_graph *g, const int32_t *d_src, const int32_t *d_dst, const uint32_t *d_w,
                    bool build_csc);
 // The light list and the tiles of the local passes, where the graph has them.
-// Built with the graph, or, on graphs whose solves run in one workgroup, by
-// the first solve that does not (traced, another plain kernel, in rounds,
-// many sources at once). Without memory for the light list there is none.
-void ensure_pass_lists(sssp_graph *g);
+// Built with the graph where its solves use them, else by the first solve
+// that does (traced, another plain kernel, in rounds, many sources at once).
+// Without memory for them there are none.
+void ensure_light_list(sssp_graph *g);
+void ensure_local_tiles(sssp_graph *g);
 // the multi-source records and tiles (m_rec, m_tile), built once per graph
 void build_multi_layout(sssp_graph *g);
 // rebuilds the destination-blocked list's tile table (cap: edge slots per

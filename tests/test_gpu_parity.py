@@ -1367,10 +1367,10 @@ def test_batch_tiles_of_even_blocks(gpu, oracle, V, E, n, kind):
                                       (1 << 14, 1 << 17, "f32"), (900, 30000, "f32"),
                                       (20011, 220121, "f32"), (4099, 45089, "equal")])
 def test_light_list_of_graphs_solved_in_one_workgroup(gpu, oracle, V, E, kind):
-    """Graphs whose single solves run in one workgroup are built without the
-    light list; a solve that does run passes (traced, in rounds) builds it then,
-    and the light passes are in its trace. Without memory for it the solve runs
-    without. A larger graph has it from the start. Bit equality with the oracle."""
+    """Graphs whose solves run in one workgroup, or whose passes are too short for
+    light ones, are built without the light list; a solve that uses it (plain_kernel
+    2, rounds) builds it then, and the light passes are in its trace. Without
+    memory for it the solve runs without. Bit equality with the oracle."""
     rng = np.random.default_rng(E)
     src = (rng.random(E) ** 2 * V).astype(np.int32)
     dst = rng.integers(0, V, E).astype(np.int32)
@@ -1379,7 +1379,6 @@ def test_light_list_of_graphs_solved_in_one_workgroup(gpu, oracle, V, E, kind):
         w = rng.integers(1, 256, E).astype(np.uint32)
     elif kind == "equal":
         w[:] = 0.5
-    solo = V <= 1 << 15 and E <= 1 << 17
     source = int(src[0])
 
     def resident(graph):
@@ -1389,13 +1388,13 @@ def test_light_list_of_graphs_solved_in_one_workgroup(gpu, oracle, V, E, kind):
 
     ref = oracle.dijkstra(src, dst, w, V, source)
     with S.DeviceGraph(src, dst, w, V) as g:
-        light = g.get_param("light_edges")
-        assert (light > 0) == (not solo)
-        d, _ = g.solve(source, "heuristic")
-        assert np.array_equal(bits(d), bits(ref)) and g.get_param("light_edges") == light
+        for traced in (0, 1):
+            g.set_param("trace_events", traced)
+            d, _ = g.solve(source, "heuristic")
+            assert np.array_equal(bits(d), bits(ref)) and g.get_param("light_edges") == 0
         g.set_param("trace_events", 1)
         g.set_param("plain_kernel", 2)
-        if solo and kind != "equal":
+        if E > 1 << 15 and kind != "equal":
             print(f"light list on demand: {kind} V {V} E {E}, no memory", flush=True)
             S.lib().sssp_debug_fail_next_alloc()  # of the light list's build
             d, _ = g.solve(source, "heuristic")
@@ -1410,7 +1409,7 @@ def test_light_list_of_graphs_solved_in_one_workgroup(gpu, oracle, V, E, kind):
             assert np.array_equal(bits(d), bits(ref)), below
             assert (g.trace()["mode"] == S.MODE_LIGHT).any() == (kind != "equal"), below
         assert (g.get_param("light_edges") > 0) == (kind != "equal")
-        assert (resident(g) > size) == (solo and kind != "equal")
+        assert (resident(g) > size) == (kind != "equal")
 
 
 @pytest.mark.gpu
@@ -1631,3 +1630,33 @@ def test_plain_kernel_forces_every_kind_of_graph(gpu, oracle):
             assert np.array_equal(bits(d), bits(ref)), kernel
             every = st["edges_relaxed"] == st["iterations"] * len(src)
             assert every == (kernel != 0), kernel
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,E,ends,light", [
+    (100003, (1 << 21) - 1, "hubs", False), (100003, 1 << 21, "hubs", True),
+    (900001, (3 << 22) - 1, "even", False), (900001, 3 << 22, "even", True),
+    (1400003, 3 << 22, "even", False)])
+def test_light_passes_where_they_pay(gpu, oracle, V, E, ends, light):
+    """The pass loop runs light passes from 2^21 edges on, without hubs from 3 * 2^22
+    and a mean of 11 edges; plain_kernel 2 runs them below too. f32, u32 and hops;
+    bit equality with the oracle."""
+    rng = np.random.default_rng(E)
+    src, dst = ((rng.random(E) ** (2 if ends == "hubs" else 1) * V).astype(np.int32)
+                for _ in range(2))
+    w = rng.random(E, dtype=np.float32) if V % 2 else rng.integers(1, 256, E).astype(np.uint32)
+    source = int(src[0])
+    ref = oracle.dijkstra(src, dst, w, V, source)
+    with S.DeviceGraph(src, dst, w, V, csc=False) as g:
+        assert (g.get_param("light_edges") > 0) == light
+        for traced in (0, 1):
+            g.set_param("trace_events", traced)
+            print(f"light line: {ends} V {V} E {E} traced {traced}", flush=True)
+            d, st = g.solve(source, "heuristic")
+            assert np.array_equal(bits(d), bits(ref)), traced
+        assert (g.trace()["mode"] == S.MODE_LIGHT).any() == light
+        assert (g.get_param("light_edges") > 0) == light
+        g.set_param("plain_kernel", 2)
+        d, st = g.solve(source, "heuristic")
+        assert np.array_equal(bits(d), bits(ref))
+        assert (g.trace()["mode"] == S.MODE_LIGHT).any() and st["n_all"] == st["iterations"]
