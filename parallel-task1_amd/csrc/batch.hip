@@ -881,7 +881,6 @@ struct MultiArgs {
     int32_t n_tile, n_ltile;  // n_ltile 0: full passes only
     uint32_t *D;
     int32_t n;
-    int64_t V;
     int32_t *stamp;
     MultiCtl *ctl;
     int32_t every;       // a power of two: blocks whose hash is 0 modulo it count their rows
@@ -1017,7 +1016,6 @@ MultiArgs multi_args(sssp_graph *g, int32_t m)
     a.n_ltile = g->n_mltile;
     a.D = g->mdist;
     a.n = m;
-    a.V = g->V;
     a.stamp = g->mstamp;
     a.ctl = static_cast<MultiCtl *>(g->mctl);
     a.every = 1;

@@ -1578,8 +1578,8 @@ __device__ __forceinline__ void flush_acc_lds(const RoundAcc &acc, RoundSlot *s,
 // round's counters.
 template <class WT>
 __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blk_pass(
-    const BlkTile *__restrict__ tiles, const BlkList L, uint32_t *dist, int64_t V,
-    int32_t *stamp, int32_t tick_cur, const int64_t *row_ptr, uint16_t *app_bits, RoundSlot *slot)
+    const BlkTile *__restrict__ tiles, const BlkList L, uint32_t *dist, int32_t *stamp,
+    int32_t tick_cur, const int64_t *row_ptr, uint16_t *app_bits, RoundSlot *slot)
 {
     __shared__ uint32_t s_d[1 << kBlkBits];
     static_assert((1 << kBlkBits) >= 5 * kBlkThreads, "the counters' LDS fits the block's");
@@ -2345,8 +2345,8 @@ bool run_round(sssp_graph *g, int mode, int kidx, int32_t r, int32_t tick0, cons
                     run_passes<WT>(g, kRunLight, INT64_MAX, st);
                 if (g->trace_events) SSSP_HIP(hipEventRecord(g->ev_r0, s));
                 k_blk_pass<WT><<<(unsigned)g->n_btile, kBlkThreads, 0, s>>>(
-                    g->b_tile, blk_list(g), g->dist, g->V, g->stamp, a.tick_cur,
-                    g->row_ptr, g->b_app, a.slot);
+                    g->b_tile, blk_list(g), g->dist, g->stamp, a.tick_cur, g->row_ptr, g->b_app,
+                    a.slot);
                 SSSP_LAUNCH_CHECK("k_blk_pass");
                 g->frontier_bits = true;
                 return false;
@@ -3581,7 +3581,7 @@ __global__ __launch_bounds__(kActThreads) void k_mark_changed(const DT *__restri
 }
 
 template <class WT, class DT, int VEC>
-__global__ __launch_bounds__(kActThreads) void k_el_active(const int32_t *__restrict__ src,
+__global__ __launch_bounds__(kActThreads) void k_el_changed(const int32_t *__restrict__ src,
                                                     const int32_t *__restrict__ dst,
                                                     const DT *__restrict__ w, int64_t E, DT *dist,
                                                     const unsigned long long *__restrict__ bits,
@@ -3723,10 +3723,10 @@ void ref_bf_active(const int32_t *src, const int32_t *dst, const DT *w, int32_t 
             k_mark_changed<DT><<<(unsigned)mgrid, kActThreads>>>(d, last, V, n_bits, bits, c, pass + i,
                                                                  (DT)WT::INF);
             if (vec)
-                k_el_active<WT, DT, 4><<<(unsigned)nblocks, kActThreads, lds>>>(
+                k_el_changed<WT, DT, 4><<<(unsigned)nblocks, kActThreads, lds>>>(
                     src, dst, w, E, d, bits, n_bits, mask, c, pass + i, per_block);
             else
-                k_el_active<WT, DT, 1><<<(unsigned)nblocks, kActThreads, lds>>>(
+                k_el_changed<WT, DT, 1><<<(unsigned)nblocks, kActThreads, lds>>>(
                     src, dst, w, E, d, bits, n_bits, mask, c, pass + i, per_block);
             SSSP_LAUNCH_CHECK("bellman_ford pass");
         }

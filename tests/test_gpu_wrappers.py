@@ -198,3 +198,36 @@ def test_wrapper_route_follows_the_list(gpu, lib, oracle, order, V, E, routes):
             assert np.array_equal(vis.get(), (~far).astype(np.uint8))
         assert lib.sssp_debug_wrapper_route(C.byref(route)) == S.OK
         assert route.value == int(routes[3]), "hops"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("weights", ["random", "light_path", "heavy_path"])
+def test_wrapper_passes_beyond_the_rings(gpu, lib, oracle, weights):
+    """Passes over changed sources past number 64, where the light ones end and
+    the rings of pass states wrap, several times over: a path of 300 hops, whose
+    edges are light, heavy or mixed, in front of a random graph, listed in random
+    order; f32, f64, u32 and hops. Bit equality with the oracle."""
+    V, E, hops = 70000, 3000001, 300
+    rng = np.random.default_rng(61)
+    s, d = (rng.integers(hops, V, E).astype(np.int32) for _ in range(2))
+    w = rng.integers(1, 256, E)
+    at = rng.permutation(E)[:hops]
+    s[at], d[at] = np.arange(hops), np.arange(1, hops + 1)
+    if weights != "random":
+        w[at] = 1 if weights == "light_path" else 255
+    ref = oracle.dijkstra(s, d, w.astype(np.uint32), V, 0)
+    far, route = ref == S.U32_INF, C.c_int32(0)
+    for dtype in (np.float32, np.float64, np.uint32):
+        print(f"wrapper past the rings: {weights} {SUFFIX[dtype]}", flush=True)
+        _, got, passes = _run(lib, dtype, s, d, w.astype(dtype), V, 0)
+        assert lib.sssp_debug_wrapper_route(C.byref(route)) == S.OK and route.value == 1
+        assert np.array_equal(got[~far], ref[~far].astype(dtype))  # whole weights: exact
+        assert np.all(got[far] == INF[dtype])
+        # light passes follow a path of light edges for the first 64 passes at most
+        assert hops - 64 <= passes <= V
+    print(f"wrapper past the rings: {weights} hops", flush=True)
+    with HipBuffer(s) as ds, HipBuffer(d) as dd, HipBuffer(np.zeros(V, np.uint8)) as vis:
+        passes = C.c_int32(0)
+        assert lib.sssp_bfs_edges(ds.ptr, dd.ptr, V, E, vis.ptr, 0, C.byref(passes)) == S.OK
+        assert lib.sssp_debug_wrapper_route(C.byref(route)) == S.OK and route.value == 1
+        assert np.array_equal(vis.get(), (~far).astype(np.uint8)) and passes.value >= hops
