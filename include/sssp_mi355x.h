@@ -214,8 +214,8 @@ int sssp_certify(sssp_graph *g, int32_t source, int32_t *parent_out, int64_t *co
  * plain_below_edges (default 2^26): a single-source heuristic or learned
  * solve (or BFS) of a graph with fewer edges runs the plain pass loop, whose
  * passes then cost less than the rounds with their fixed per-round cost: light
- * passes (the lightest edges alone) before and between the passes over all
- * edges, or, on sparse graphs without hubs whose edges mostly join near ids
+ * passes (the lightest edges alone; on graphs large enough to gain from them) before
+ * and between the passes over all edges, or, on sparse graphs without hubs whose edges mostly join near ids
  * (grids, road networks), passes that relax each tile of edges several times
  * and leave out the tiles no source of which changed.
  * plain_kernel picks the plain pass: 0 (default) the destination-blocked pass
@@ -295,13 +295,13 @@ int sssp_bfs(sssp_graph *g, int32_t source, int32_t schedule, uint8_t *visited_o
 int sssp_bfs_edges(const int32_t *d_src, const int32_t *d_dst, int32_t vertices, int64_t edges,
                    uint8_t *d_visited, int32_t source, int32_t *passes);
 
-/* ---- batched solves (one persistent launch, replayed through a hipGraph) -- */
+/* ---- batched solves ------------------------------------------------------- */
 /* Many sources on one graph. dist_out: n*V elements (host) or NULL.
  * policy 0 = autotuned (untuned: 3 for n >= 32, else 2), 1 = one workgroup
  * per source, 2 = the sources solved one after another on the full chip,
  * 3 = vertex-major all-edge passes: the distances of up to 256 sources are
- * held per vertex as one row, each pass reads every edge once for all of
- * them; the layout it needs (16 bytes per edge) is built on its first use,
+ * held per vertex as one row, a pass relaxes each edge once for all of
+ * them, unless no source lowered its source vertex since; the layout it needs (16 bytes per edge) is built on its first use,
  * and 256 * V distances are kept on the device. stats->iterations = the
  * policy run. */
 int sssp_solve_batch(sssp_graph *g, const int32_t *sources, int32_t n, int32_t policy,
@@ -313,7 +313,10 @@ int sssp_pack_create(const int32_t *src, const int32_t *dst, const float *weight
                      const int64_t *edge_offsets, const int32_t *vertex_counts,
                      int32_t n_graphs, int32_t device, sssp_pack **out);
 int sssp_pack_destroy(sssp_pack *p);
-/* sources[k] is local to graph k. dist_out: sum(vertex_counts) floats or NULL. */
+/* sources[k] is local to graph k. dist_out: sum(vertex_counts) floats or NULL.
+ * policy 0 = autotuned (untuned: graphs of up to 2^15 vertices as 1, the
+ * larger ones together as 2), 1 = one workgroup per graph, 2 = all graphs as
+ * one union graph on the full chip. */
 int sssp_pack_solve(sssp_pack *p, const int32_t *sources, int32_t policy, float *dist_out,
                     sssp_stats *stats);
 /* Autotuner: times candidate (policy, block size, chunk width, frontier

@@ -11,25 +11,28 @@
 //   appends to the next frontier through an LDS counter, deduplicated by a
 //   per-workgroup stamp array. The launches are captured once in a hipGraph
 //   and replayed.
-// Policy 2 (merged frontier): many disjoint graphs are one union graph, so all
-//   their sources share one full-chip frontier solve; many sources on one
-//   graph are solved one after another on the full chip.
+// Policy 2 (full chip): many disjoint graphs are one union graph, whose solve
+//   starts from all their sources: in passes over its blocked list (the pass
+//   loop) below 2^25 edges, in frontier rounds from there on. Many sources on one
+//   graph are solved one after another, each as sssp_solve does it.
 // Policy 3 (many sources on one graph, vertex-major): the distances of up to
 //   256 sources are one array D[v * n + s], so a vertex's distances are one
 //   contiguous row. All-edge passes over the edges sorted by 16-vertex
 //   destination block: a 256-thread workgroup (thread s = source s) holds its
-//   block's 16 x 256 minima in LDS, reads each edge record once for all its
-//   sources (a wave-uniform load), gathers the source vertex's row (coalesced,
-//   eight rows in flight) unless no source lowered it since the record was
-//   last relaxed,
-//   and lowers its own LDS column -- no atomics inside a block; the block is
-//   written back at the end (atomicMin for blocks split over several tiles).
-//   Passes over the light edges alone alternate with full ones until a full
-//   pass changes nothing, the Bellman-Ford fixpoint of every source; the rows
-//   are then transposed into the per-source output.
+//   block's 16 x 256 minima in LDS (they start unreached, not at the distances).
+//   Each of its waves reads the records 64 at a time, one per lane, and takes
+//   them in turn (readlane): gather the source vertex's row (coalesced, eight
+//   rows in flight) unless no source lowered it since the record was last
+//   relaxed, and lower the own LDS column -- no atomics inside a block. The
+//   minima below the block's distances are written at the end (atomicMin for
+//   blocks split over several tiles).
+//   Where light records pay (kMLightEdges), passes over the light edges alone
+//   alternate with full ones; they end with a full pass that changes nothing,
+//   the Bellman-Ford fixpoint of every source, and the rows are then transposed
+//   into the per-source output.
 // The autotuner times block size x workgroups per CU for policy 1, frontier
 // threshold x push chunk width for policy 2, and policy 3, and keeps the
-// fastest.
+// fastest; a setting that none of a solve's kernels reads is timed once.
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -1284,7 +1287,7 @@ Config default_config(sssp_graph *g, int32_t n)
     if (g->batch_policy)
         return Config{g->batch_policy, g->batch_bs, g->batch_wgpcu, g->push_edge_frac, g->push_chunk};
     // untuned: policy 3 for 32 or more sources on one graph (R-MAT scale 20
-    // x 256 sources: 54.7 GTEPS against 10.5 for policy 1), policy 2 below
+    // x 256 sources: 171-180 GTEPS against 11-12 for policy 1, 22-24 for policy 2), policy 2 below
     if (n >= 32) return Config{3, kMThreads, 1, 0.0, 0};
     return Config{2, 256, 2, g->push_edge_frac, g->push_chunk};
 }

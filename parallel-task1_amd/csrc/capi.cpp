@@ -257,7 +257,7 @@ bool pageable(const void *p)
 
 // Results below this go through hipMemcpy, and their pages are not faulted in
 // ahead: 4 MB take 0.3-0.5 ms that way, about what the staging buffers cost to
-// allocate once per graph.
+// allocate once per process.
 constexpr size_t kStagedMin = kStageBytes + 1;
 constexpr size_t kPrefaultPerThread = (size_t)16 << 20;
 constexpr uintptr_t kPrefaultStep = (uintptr_t)4 << 20;

@@ -1739,8 +1739,8 @@ __global__ __launch_bounds__(kBlock) void k_frontier_from_bits(const BlkTile *__
 // Why light passes: a shortest path takes mostly light edges, so relaxing the
 // lightest sixteenth of the edges to near convergence costs a fraction of the
 // full passes it replaces, and the full passes after it find the distances
-// nearly final. R-MAT 25 x 16: 13 light passes of 0.15 ms and one dense round
-// instead of 9 dense rounds of 1.1 ms (a learned solve 13.4 -> 5.6 ms); R-MAT
+// nearly final. R-MAT 25 x 16: 14 light passes of 0.09-0.13 ms and two dense rounds
+// instead of 9 of 1.05 ms (a learned solve 13.4 -> 5.7 ms); R-MAT
 // 22 x 32 4.75 -> 2.1; uniform 6 M x 16, u32 6.85 -> 4.8; power-law 1.2 M x 9 in the
 // pass loop 2.33 -> 1.2.
 // A tile counts a vertex as lowered only when its minimum is below the
@@ -3388,7 +3388,8 @@ void ref_init(DT *d, int32_t V, int32_t source)
 // distance reads per edge (a distance array as large as an XCD's L2), 16 passes,
 // 4.8 ms a call. With the bits 22 passes, since a pass no longer sees the changes
 // of its own, six of them 0.14-0.41 ms and the others 0.02-0.09: 2.7 ms. With
-// light passes between them 1.9. Uniform 500 K x 16, u32 2.9 / 1.6 / 1.4 ms,
+// light passes between them 1.9-2.3: 24 passes, the longest two 0.33 and 0.14 ms,
+// 1.6 ms of kernels. Uniform 500 K x 16, u32 2.9 / 1.6 / 1.4 ms,
 // power-law 300 K x 14 f64 1.15 / 0.86 / 0.79. kActBits bits fill most of a CU's
 // LDS; half of them with two workgroups per CU 3.0 ms without light passes, a
 // quarter 3.2. kActUnroll 1 / 2 / 4 groups of four edges in flight per lane:

@@ -968,12 +968,6 @@ static void build_records(sssp_graph *g, const int32_t *src, const int32_t *dst,
     *n_tile = (int32_t)tiles.size();
 }
 
-// Edge-list check on the device: every id in [0, V) and (wtype >= 0) every
-// weight >= 0 and not NaN (unsigned weights always are); throws SSSP_ERR_ARG.
-// The relaxations rely on it: distances are compared as unsigned bit patterns,
-// which orders non-negative IEEE values only. The two counters live in
-// `bad_buf` when the caller brings one (device memory, 16 bytes), else in a
-// buffer allocated for the call; a kernel clears them either way.
 // out[0..3) += sampled edges whose source (destination) is near that of the
 // edge 256 further on, and edges between near ids. Ids may still be invalid.
 constexpr int kOrderSamples = 512;
@@ -991,6 +985,13 @@ __global__ __launch_bounds__(kOrderSamples) void k_list_order(const int32_t *src
     }
 }
 
+// Edge-list check on the device: every id in [0, V) and (wtype >= 0) every
+// weight >= 0 and not NaN (unsigned weights always are); throws SSSP_ERR_ARG.
+// The relaxations rely on it: distances are compared as unsigned bit patterns,
+// which orders non-negative IEEE values only. The two counters live in
+// `bad_buf` when the caller brings one (device memory, 16 bytes), else in a
+// buffer allocated for the call; a kernel clears them either way.
+// With `order` (and no bad_buf), the order of the list is sampled on the way.
 void validate_edges(const int32_t *src, const int32_t *dst, const void *w, int wtype, int64_t E,
                     int32_t V, hipStream_t s, int64_t *bad_buf, ListOrder *order)
 {
