@@ -3388,7 +3388,7 @@ void ref_init(DT *d, int32_t V, int32_t source)
 // distance reads per edge (a distance array as large as an XCD's L2), 16 passes,
 // 4.8 ms a call. With the bits 22 passes, since a pass no longer sees the changes
 // of its own, six of them 0.14-0.41 ms and the others 0.02-0.09: 2.7 ms. With
-// light passes between them 1.9-2.3: 24 passes, the longest two 0.33 and 0.14 ms,
+// light passes between them 1.8-2.3: 24 passes, the longest two 0.33 and 0.14 ms,
 // 1.6 ms of kernels. Uniform 500 K x 16, u32 2.9 / 1.6 / 1.4 ms,
 // power-law 300 K x 14 f64 1.15 / 0.86 / 0.79. kActBits bits fill most of a CU's
 // LDS; half of them with two workgroups per CU 3.0 ms without light passes, a
